@@ -1477,6 +1477,297 @@ __global__ __launch_bounds__(kVecBlock) void k_accum_cols(
 }
 
 // ============================================================================
+// Many small operators on a few vectors, and inner products of many columns
+// ============================================================================
+
+// Y[:, l * n_vec + v] = O_l psi_v for the operators l of this workgroup's
+// chunk (blockIdx.y).  One lane per row: the row's state is read once for all
+// operators, and a term's rank is looked up once for all vectors (kEachVecs of
+// them per round).  Per output the sum runs in term order, then the diagonal,
+// as in the apply kernels, so the columns have the same bits.
+constexpr int kEachVecs = 4;
+constexpr int kEachOps = 8;  // operators of one workgroup
+
+template <int NW>
+__global__ __launch_bounds__(kApplyBlock) void k_apply_each(
+    BasisView b, const EachOp* __restrict__ ops, int n_ops, const double* __restrict__ psi,
+    int64_t ld, int n_vec, double* __restrict__ Y, int64_t ldy) {
+  const int64_t i = static_cast<int64_t>(xcd_remap(blockIdx.x, gridDim.x)) * kApplyBlock +
+                    threadIdx.x;
+  if (i >= b.dim) return;
+  const State<NW> s = load_state_cached<NW>(b.states, i);
+  const int l1 = min(n_ops, static_cast<int>(blockIdx.y + 1) * kEachOps);
+  for (int l = blockIdx.y * kEachOps; l < l1; ++l) {
+    const EachOp O = ops[l];
+    for (int v0 = 0; v0 < n_vec; v0 += kEachVecs) {
+      const double* x = psi + v0 * ld;
+      double acc[kEachVecs] = {};
+      for (int t = 0; t < O.n_off; ++t) {
+        const OffTerm& T = O.off[t];
+        if (!term_ok<NW>(T, s)) continue;
+        const int64_t J = basis_lookup<NW>(b, xor_state<NW>(s, T.X));
+        if (J < 0) continue;
+        double c = T.c * T.sgn;
+        if (parity_notz<NW>(s, T.Z)) c = -c;
+#pragma unroll
+        for (int v = 0; v < kEachVecs; ++v) {
+          if (v0 + v < n_vec) {
+            const double xj = x[v * ld + J];
+            if (fabs(xj) > kApplyTol) acc[v] += c * xj;
+          }
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < kEachVecs; ++v) {
+        if (v0 + v < n_vec) {
+          if (O.n_diag > 0)
+            acc[v] = diag_accumulate<NW>(acc[v], x[v * ld + i], s, O.dg, O.n_diag);
+          Y[static_cast<int64_t>(l * n_vec + v0 + v) * ldy + i] = acc[v];
+        }
+      }
+    }
+  }
+}
+
+// Inner products of the columns of A (pa) and B (pb) over n rows, on the FP64
+// matrix cores.  blockIdx.y is a pair of 64-column blocks (of the upper triangle
+// when A and B are the same matrix), blockIdx.x a slab of rows.  A wavefront
+// takes 16 rows at a time: lane l reads four consecutive rows 4 (l / 16) of
+// column l % 16 (a whole 128-byte line per column), and the four rows feed four
+// 16x16x4 products per pair of 16-column blocks; which rows share a product does
+// not matter to the sum.  The four wavefronts' 64 x 64 sums meet in LDS in a fixed
+// order, and part[(slab, pair)] holds the slab's result.  Reading the columns
+// once per pair of blocks instead of once per 16 columns and output column is
+// what it is for.
+constexpr int kGramCols = 64;
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
+// The column blocks (ba, bb) of a pair: row by row of the upper triangle (same)
+// or of all nbb columns of blocks.
+__device__ __forceinline__ void gram_pair(int64_t pair, int nbb, int same, int* ba, int* bb) {
+  if (same) {
+    int a = 0;
+    while (pair >= nbb - a) pair -= nbb - a++;
+    *ba = a;
+    *bb = a + static_cast<int>(pair);
+  } else {
+    *ba = static_cast<int>(pair / nbb);
+    *bb = static_cast<int>(pair % nbb);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_gram(const double* __restrict__ A, int64_t lda, int pa,
+                                              const double* __restrict__ B, int64_t ldb, int pb,
+                                              int64_t n, int64_t slab, int same, int64_t pairs,
+                                              double* __restrict__ part) {
+  __shared__ double sum[kGramCols * kGramCols];
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int64_t pair = static_cast<int64_t>(blockIdx.z) * gridDim.y + blockIdx.y;
+  if (pair >= pairs) return;
+  int ba, bb;
+  gram_pair(pair, (pb + kGramCols - 1) / kGramCols, same, &ba, &bb);
+  const int a0 = ba * kGramCols, b0 = bb * kGramCols;
+  const int ta = min(4, (pa - a0 + 15) / 16), tb = min(4, (pb - b0 + 15) / 16);
+  const int c = lane & 15, k = lane >> 4;
+  f64x4 acc[4][4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+#pragma unroll
+    for (int v = 0; v < 4; ++v) acc[u][v] = f64x4{0.0, 0.0, 0.0, 0.0};
+  const int64_t r_end = min<int64_t>(n, (blockIdx.x + 1) * slab);
+  for (int64_t r = blockIdx.x * slab + wid * 16; r < r_end; r += 64) {
+    double fa[4][4], fb[4][4];
+    // columns past the last repeat it (their sums are not stored); rows past
+    // the end count as zero
+    auto load = [&](const double* M, int64_t ld, int col, double (&f)[4]) {
+      const double* p = M + static_cast<int64_t>(col) * ld + r + 4 * k;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f[j] = r + 4 * k + j < r_end ? p[j] : 0.0;
+    };
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      if (u < ta) load(A, lda, min(a0 + 16 * u + c, pa - 1), fa[u]);
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (v < tb) load(B, ldb, min(b0 + 16 * v + c, pb - 1), fb[v]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int v = 0; v < 4; ++v)
+        if (u < ta && v < tb) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            acc[u][v] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[u][j], fb[v][j], acc[u][v], 0, 0, 0);
+        }
+  }
+  // lane l holds rows l / 16 + 4 q and column l % 16 of each 16 x 16 product
+  for (int w = 0; w < 4; ++w) {
+    if (wid == w) {
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            double& o = sum[(16 * u + k + 4 * q) * kGramCols + 16 * v + c];
+            o = w == 0 ? acc[u][v][q] : o + acc[u][v][q];
+          }
+    }
+    __syncthreads();
+  }
+  double* out = part + (blockIdx.x * pairs + pair) * (kGramCols * kGramCols);
+  for (int t = threadIdx.x; t < kGramCols * kGramCols; t += 256) out[t] = sum[t];
+}
+
+// out[b * pa + a] = the slabs' sums of (a, b) (and its mirror image when the two
+// matrices are the same) for T-column blocks: a workgroup sums 32 neighbouring
+// entries, eight groups of slabs side by side (every eighth slab each), which
+// are added in a fixed order.
+template <int T>
+__global__ __launch_bounds__(256) void k_gram_sum(const double* __restrict__ part, int n_slab,
+                                                  int pa, int pb, int same, int64_t pairs,
+                                                  double* __restrict__ out) {
+  __shared__ double red[8][32];
+  const int64_t e = static_cast<int64_t>(blockIdx.x) * 32 + (threadIdx.x & 31);
+  const int g = threadIdx.x >> 5;
+  double v = 0.0;
+  for (int s = g; s < n_slab; s += 8) v += part[s * pairs * (T * T) + e];
+  red[g][threadIdx.x & 31] = v;
+  __syncthreads();
+  if (g != 0) return;
+#pragma unroll
+  for (int k = 1; k < 8; ++k) v += red[k][threadIdx.x];
+  int ba, bb;
+  gram_pair(e / (T * T), (pb + T - 1) / T, same, &ba, &bb);
+  const int k = static_cast<int>(e % (T * T));
+  const int a = ba * T + k / T, b = bb * T + k % T;
+  if (a >= pa || b >= pb) return;
+  out[static_cast<int64_t>(b) * pa + a] = v;
+  if (same && ba != bb) out[static_cast<int64_t>(a) * pa + b] = v;
+}
+
+// The same inner products for operators of a few terms each, without the
+// columns O_l psi_v ever going to memory: a workgroup takes 64 rows at a time,
+// forms those rows of every column in LDS (lane = row, wavefront w the
+// operators of list w; four lookups in flight per lane; sums in term order,
+// then the diagonal), and multiplies them on the matrix cores, each wavefront
+// with the 16 x 16 products w, w + 4, ... of its own.  part[(workgroup, product)]
+// holds the workgroup's sums.  With stored columns the products read every
+// column once per output column and 64-column block: 48 operators on two 48-spin
+// vectors took 6.9 ms for expectations and correlations, 96 launches of 4 us and
+// 98 of 28 us each; this way 0.38 ms, 2 x 80 us of it on the device, bound by the
+// latency of the lookups.  Columns [0, P) are the operators', and for
+// expectations (same = 0) n_vec columns of psi follow at the next multiple of 16.
+constexpr int kObsCols = 128;  // most columns of the operators
+constexpr int kObsVecs = 16;   // most columns of psi for expectations
+constexpr int kObsTiles = kObsCols / 16 * (kObsCols / 16 + 1) / 2;
+constexpr int kObsLd = 66;     // LDS rows of a column: 64 and two that spread the banks
+
+template <int NW>
+__global__ __launch_bounds__(256) void k_observe(BasisView b, ObserveArgs q,
+                                                 const double* __restrict__ psi, int64_t ld,
+                                                 double* __restrict__ part) {
+  extern __shared__ double col[];  // [column][kObsLd]
+  constexpr int G = 4;
+  const int lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int nb = (q.P + 15) / 16;
+  const int n_cols = 16 * nb + (q.same ? 0 : 16);
+  const int c = lane & 15, k = lane >> 4;
+  // this wavefront's products
+  constexpr int kMine = kObsTiles / 4;
+  int tu[kMine], tv[kMine], mine = 0;
+  for (int t = wid; t < q.tiles; t += 4) {
+    int u = t, v = nb;  // expectations: block u against psi's
+    if (q.same) gram_pair(t, nb, 1, &u, &v);
+#pragma unroll
+    for (int m = 0; m < kMine; ++m)
+      if (m == mine) {
+        tu[m] = u;
+        tv[m] = v;
+      }
+    ++mine;
+  }
+  f64x4 acc[kMine];
+#pragma unroll
+  for (int m = 0; m < kMine; ++m) acc[m] = f64x4{0.0, 0.0, 0.0, 0.0};
+  // columns that no operator writes stay zero
+  for (int e = threadIdx.x; e < n_cols * kObsLd; e += 256) col[e] = 0.0;
+  __syncthreads();
+  const int64_t chunks = (b.dim + 63) / 64;
+  for (int64_t ch = blockIdx.x; ch < chunks; ch += gridDim.x) {
+    const int64_t i = ch * 64 + lane;
+    const bool row_ok = i < b.dim;
+    const State<NW> s = load_state_cached<NW>(b.states, row_ok ? i : ch * 64);
+    for (int e = q.col_begin[wid]; e < q.col_begin[wid + 1]; ++e) col[q.cols[e] * kObsLd + lane] = 0.0;
+    if (!q.same && wid == 0)
+      for (int v = 0; v < q.n_vec; ++v)
+        col[(16 * nb + v) * kObsLd + lane] = row_ok ? psi[v * ld + i] : 0.0;
+    const int t1 = q.off_begin[wid + 1];
+    for (int t0 = q.off_begin[wid]; t0 < t1; t0 += 64) {
+      uint64_t mask = connect_mask<NW>(q.off + t0, min(64, t1 - t0), s);
+      if (!row_ok) mask = 0;
+      while (mask) {
+        int tt[G];
+        bool act[G];
+        State<NW> key[G];
+        uint32_t rk[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          act[g] = mask != 0;
+          const int z = act[g] ? __builtin_clzll(mask) : 0;
+          tt[g] = t0 + z;
+          mask &= ~(uint64_t{1} << 63 >> z);
+          key[g] = xor_state<NW>(s, q.off[tt[g]].X);
+        }
+        lookup_batch<NW, G>(b, key, act, rk);
+        for (int v = 0; v < q.n_vec; ++v) {
+          double xj[G];
+#pragma unroll
+          for (int g = 0; g < G; ++g) xj[g] = rk[g] != kNoRank ? psi[v * ld + rk[g]] : 0.0;
+#pragma unroll
+          for (int g = 0; g < G; ++g) {
+            if (rk[g] != kNoRank && fabs(xj[g]) > kApplyTol) {
+              const OffTerm& T = q.off[tt[g]];
+              double cg = T.c * T.sgn;
+              if (parity_notz<NW>(s, T.Z)) cg = -cg;
+              col[(T.slot + v) * kObsLd + lane] += cg * xj[g];
+            }
+          }
+        }
+      }
+    }
+    for (int d = q.diag_begin[wid]; d < q.diag_begin[wid + 1]; ++d) {
+      const EachOp& O = q.diag[d];
+      if (row_ok)
+        for (int v = 0; v < q.n_vec; ++v) {
+          double& y = col[(O.col + v) * kObsLd + lane];
+          y = diag_accumulate<NW>(y, psi[v * ld + i], s, O.dg, O.n_diag);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < kMine; ++m) {
+      if (m < mine) {
+        const double* A = col + (16 * tu[m] + c) * kObsLd + k;
+        const double* B = col + (16 * tv[m] + c) * kObsLd + k;
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+          acc[m] = __builtin_amdgcn_mfma_f64_16x16x4f64(A[4 * j], B[4 * j], acc[m], 0, 0, 0);
+      }
+    }
+    __syncthreads();
+  }
+  double* out = part + static_cast<int64_t>(blockIdx.x) * q.tiles * 256;
+#pragma unroll
+  for (int m = 0; m < kMine; ++m)
+    if (m < mine)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) out[(wid + 4 * m) * 256 + (k + 4 * e) * 16 + c] = acc[m][e];
+}
+
+// ============================================================================
 // Host helpers
 // ============================================================================
 
@@ -1872,6 +2163,87 @@ int launch_accum_cols(const double* v, double* Psi, int64_t ld, int nb, const do
                       int64_t n, hipStream_t s, const double* vs_dev) {
   hipLaunchKernelGGL(k_accum_cols, dim3(vec_blocks(n)), dim3(kVecBlock), 0, s, v, Psi, ld, nb,
                      c, n, vs_dev);
+  QSI_CHECK_LAUNCH();
+  return QSI_OK;
+}
+
+int launch_apply_each(const qsi_basis_s* basis, const EachOp* ops, int n_ops, const double* psi,
+                      int64_t ld, int n_vec, double* Y, int64_t ldy, hipStream_t s) {
+  const dim3 grid(static_cast<uint32_t>((basis->dim + kApplyBlock - 1) / kApplyBlock),
+                  static_cast<uint32_t>((n_ops + kEachOps - 1) / kEachOps));
+  if (basis->nw == 1)
+    hipLaunchKernelGGL(k_apply_each<1>, grid, dim3(kApplyBlock), 0, s, basis->view(), ops, n_ops,
+                       psi, ld, n_vec, Y, ldy);
+  else
+    hipLaunchKernelGGL(k_apply_each<2>, grid, dim3(kApplyBlock), 0, s, basis->view(), ops, n_ops,
+                       psi, ld, n_vec, Y, ldy);
+  QSI_CHECK_LAUNCH();
+  return QSI_OK;
+}
+
+namespace {
+int64_t gram_pairs(int pa, int pb, bool same) {
+  const int64_t na = (pa + kGramCols - 1) / kGramCols, nb = (pb + kGramCols - 1) / kGramCols;
+  return same ? na * (na + 1) / 2 : na * nb;
+}
+// Rows of a slab: 1024 workgroups over all pairs, at least 256 rows each.
+int64_t gram_slab(int pa, int pb, bool same, int64_t n) {
+  const int64_t want = std::max<int64_t>(1, 1024 / gram_pairs(pa, pb, same));
+  return std::max<int64_t>(256, ((n + want - 1) / want + 63) / 64 * 64);
+}
+}  // namespace
+
+size_t gram_partials(int pa, int pb, bool same, int64_t n) {
+  const int64_t slab = gram_slab(pa, pb, same, n);
+  return static_cast<size_t>((n + slab - 1) / slab * gram_pairs(pa, pb, same)) * kGramCols *
+         kGramCols;
+}
+
+int launch_gram(const double* A, int64_t lda, int pa, const double* B, int64_t ldb, int pb,
+                int64_t n, double* partials, double* out, hipStream_t s) {
+  const bool same = A == B && pa == pb && lda == ldb;
+  const int64_t pairs = gram_pairs(pa, pb, same), slab = gram_slab(pa, pb, same, n);
+  const int64_t n_slab = (n + slab - 1) / slab;
+  const uint32_t py = static_cast<uint32_t>(std::min<int64_t>(pairs, 65535));
+  const uint32_t pz = static_cast<uint32_t>((pairs + py - 1) / py);
+  hipLaunchKernelGGL(k_gram, dim3(static_cast<uint32_t>(n_slab), py, pz), dim3(256), 0, s, A, lda,
+                     pa, B, ldb, pb, n, slab, same ? 1 : 0, pairs, partials);
+  QSI_CHECK_LAUNCH();
+  hipLaunchKernelGGL(k_gram_sum<kGramCols>,
+                     dim3(static_cast<uint32_t>(pairs * (kGramCols * kGramCols / 32))), dim3(256),
+                     0, s, partials, static_cast<int>(n_slab), pa, pb, same ? 1 : 0, pairs, out);
+  QSI_CHECK_LAUNCH();
+  return QSI_OK;
+}
+
+bool observe_fits(int P, int n_vec, bool gram) {
+  return P <= kObsCols && (gram || n_vec <= kObsVecs);
+}
+
+int observe_blocks(int64_t n) {
+  // one workgroup per CU while the partial sums they leave would be most of the
+  // traffic (and while their buffer, 11 MB for 96 columns, stays cheap to
+  // allocate: a 22 MB one costs 0.3 ms a call), three on large bases
+  return static_cast<int>(std::min<int64_t>((n + 63) / 64, n > (1 << 20) ? 768 : 256));
+}
+
+int observe_tiles(int P, bool gram) {
+  const int nb = (P + 15) / 16;
+  return gram ? nb * (nb + 1) / 2 : nb;
+}
+
+int launch_observe(const qsi_basis_s* basis, const ObserveArgs& q, const double* psi, int64_t ld,
+                   double* partials, double* out, hipStream_t s) {
+  const int nb = (q.P + 15) / 16, blocks = observe_blocks(basis->dim);
+  const size_t lds = static_cast<size_t>(16 * nb + (q.same ? 0 : 16)) * kObsLd * sizeof(double);
+  auto kern = basis->nw == 1 ? k_observe<1> : k_observe<2>;
+  QSI_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    static_cast<int>(lds)));
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), lds, s, basis->view(), q, psi, ld, partials);
+  QSI_CHECK_LAUNCH();
+  hipLaunchKernelGGL(k_gram_sum<16>, dim3(q.tiles * 8), dim3(256), 0, s, partials, blocks, q.P,
+                     q.same ? q.P : q.n_vec, q.same, static_cast<int64_t>(q.tiles), out);
   QSI_CHECK_LAUNCH();
   return QSI_OK;
 }

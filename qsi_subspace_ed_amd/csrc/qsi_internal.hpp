@@ -217,6 +217,41 @@ int launch_axpy_dev(const double* s_dev, double c, const double* x, double* y,
 int launch_accum_cols(const double* v, double* Psi, int64_t ld, int nb, const double* c,
                       int64_t n, hipStream_t s, const double* vs_dev = nullptr);
 
+// One of several operators applied together (device pointers of a qsi_op_s).
+struct EachOp {
+  const OffTerm* off;
+  const DiagTerm* dg;
+  int n_off;
+  int n_diag;
+  int col;  // first output column (k_observe)
+};
+// Y[:, l * n_vec + v] = O_l psi[:, v] (ops: n_ops records on the device; psi and
+// Y column-major): one launch for many operators of a few terms each.
+int launch_apply_each(const qsi_basis_s* basis, const EachOp* ops, int n_ops, const double* psi,
+                      int64_t ld, int n_vec, double* Y, int64_t ldy, hipStream_t s);
+// out[b * pa + a] = A[:, a] . B[:, b] over n rows (column-major); partials holds
+// gram_partials() doubles, with same = (A is B).
+size_t gram_partials(int pa, int pb, bool same, int64_t n);
+int launch_gram(const double* A, int64_t lda, int pa, const double* B, int64_t ldb, int pb,
+                int64_t n, double* partials, double* out, hipStream_t s);
+
+// Expectations (same = 0: columns O_l psi_v against psi) or correlations (same
+// = 1: against each other) of operators of a few terms without storing the
+// columns: wavefront w of a workgroup forms the columns of list w.
+struct ObserveArgs {
+  const OffTerm* off;  // list by list, slot = the operator's first column
+  const EachOp* diag;  // operators with diagonal terms, list by list
+  const int* cols;     // columns, list by list
+  int off_begin[5], diag_begin[5], col_begin[5];
+  int P, n_vec, same, tiles;
+};
+bool observe_fits(int P, int n_vec, bool gram);
+int observe_blocks(int64_t n);
+int observe_tiles(int P, bool gram);
+// out[b * P + a] as launch_gram; partials: observe_blocks() * observe_tiles() * 256
+int launch_observe(const qsi_basis_s* basis, const ObserveArgs& q, const double* psi, int64_t ld,
+                   double* partials, double* out, hipStream_t s);
+
 // The 3-term Lanczos coefficient run behind qsi_lanczos_coeffs on
 // caller-provided device buffers: v (D, the start vector, normalised here;
 // clobbered), u (D), partials (lanczos_coeffs_partials(op) doubles), ab

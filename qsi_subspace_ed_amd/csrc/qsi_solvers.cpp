@@ -639,10 +639,16 @@ int qsi_eigsh(qsi_op_t op, int nev, int ncv, double tol, int max_restarts,
 
 namespace {
 
+// Operators of up to this many off-diagonal terms go through one launch for all
+// (ring operators have one term, partial volumes six): at 48 spins an apply of
+// its own costs 4 us and a launch each.  Longer ones keep the apply kernels,
+// which have several lookups in flight per row.
+constexpr int kEachTerms = 16;
+
 // Y[:, l*n_vec + i] = O_l psi_i for every operator and vector (Y column-major
 // with leading dimension ldy), then out[b*P + a] = Y[:, a] . W[:, b] for the
-// P = n_ops*n_vec columns a and the n_w columns b of W (ldw), by multi-dots
-// of up to 64 columns.  Synchronises.
+// P = n_ops*n_vec columns a and the n_w columns b of W (Y itself or psi).
+// Synchronises.
 int observe(const qsi_op_t* ops, int n_ops, const double* d_psi, int64_t ld, int n_vec,
             bool gram, std::vector<double>& out, int* P_out) {
   QSI_REQUIRE(ops && d_psi && n_ops >= 1 && n_vec >= 1, "observables: bad arguments");
@@ -655,23 +661,82 @@ int observe(const qsi_op_t* ops, int n_ops, const double* d_psi, int64_t ld, int
   const int P = n_ops * n_vec;
   const int64_t ldy = (D + 63) / 64 * 64;
   hipStream_t s = nullptr;
-  DevBuf bY, bpart, bout;
-  QSI_CHECK_HIP(bY.alloc(static_cast<size_t>(ldy) * P * sizeof(double)));
-  QSI_CHECK_HIP(bpart.alloc(static_cast<size_t>(multidot_partials()) * sizeof(double)));
+  DevBuf bY, bpart, bout, bops;
   const int n_w = gram ? P : n_vec;
   QSI_CHECK_HIP(bout.alloc(static_cast<size_t>(P) * n_w * sizeof(double)));
-  double* Y = bY.d();
-  for (int l = 0; l < n_ops; ++l)
-    for (int i = 0; i < n_vec; ++i)
-      QSI_TRY(launch_apply(ops[l], d_psi + static_cast<int64_t>(i) * ld,
-                           Y + static_cast<int64_t>(l * n_vec + i) * ldy, nullptr, 0.0, nullptr,
-                           nullptr, s));
-  for (int b = 0; b < n_w; ++b) {
-    const double* w = gram ? Y + static_cast<int64_t>(b) * ldy : d_psi + static_cast<int64_t>(b) * ld;
-    for (int a0 = 0; a0 < P; a0 += 64)
-      QSI_TRY(launch_multidot(Y + static_cast<int64_t>(a0) * ldy, ldy, std::min(64, P - a0), w, D,
-                              bpart.d(), bout.d() + static_cast<int64_t>(b) * P + a0, nullptr, s));
+  bool small = true;
+  for (int l = 0; l < n_ops; ++l) small = small && ops[l]->n_off <= kEachTerms;
+  if (small && observe_fits(P, n_vec, gram)) {
+    // four lists of operators, dealt round robin, in one upload
+    std::vector<OffTerm> off;
+    std::vector<EachOp> diag;
+    std::vector<int> cols;
+    ObserveArgs q{};
+    q.P = P;
+    q.n_vec = n_vec;
+    q.same = gram ? 1 : 0;
+    q.tiles = observe_tiles(P, gram);
+    for (int w = 0; w < 4; ++w) {
+      q.off_begin[w] = static_cast<int>(off.size());
+      q.diag_begin[w] = static_cast<int>(diag.size());
+      q.col_begin[w] = static_cast<int>(cols.size());
+      for (int l = w; l < n_ops; l += 4) {
+        for (OffTerm t : ops[l]->h_off) {
+          t.slot = l * n_vec;
+          off.push_back(t);
+        }
+        if (ops[l]->n_diag > 0)
+          diag.push_back({nullptr, ops[l]->d_diag, 0, ops[l]->n_diag, l * n_vec});
+        for (int v = 0; v < n_vec; ++v) cols.push_back(l * n_vec + v);
+      }
+    }
+    q.off_begin[4] = static_cast<int>(off.size());
+    q.diag_begin[4] = static_cast<int>(diag.size());
+    q.col_begin[4] = static_cast<int>(cols.size());
+    const size_t n_off = off.size() * sizeof(OffTerm), n_diag = diag.size() * sizeof(EachOp);
+    std::vector<char> up(n_off + n_diag + cols.size() * sizeof(int));
+    if (n_off) std::memcpy(up.data(), off.data(), n_off);
+    if (n_diag) std::memcpy(up.data() + n_off, diag.data(), n_diag);
+    std::memcpy(up.data() + n_off + n_diag, cols.data(), cols.size() * sizeof(int));
+    QSI_CHECK_HIP(bops.alloc(up.size()));
+    QSI_CHECK_HIP(hipMemcpy(bops.p, up.data(), up.size(), hipMemcpyHostToDevice));
+    const char* base = static_cast<const char*>(bops.p);
+    q.off = reinterpret_cast<const OffTerm*>(base);
+    q.diag = reinterpret_cast<const EachOp*>(base + n_off);
+    q.cols = reinterpret_cast<const int*>(base + n_off + n_diag);
+    QSI_CHECK_HIP(bpart.alloc(static_cast<size_t>(observe_blocks(D)) * q.tiles * 256 *
+                              sizeof(double)));
+    QSI_TRY(launch_observe(basis, q, d_psi, ld, bpart.d(), bout.d(), s));
+    out.resize(static_cast<size_t>(P) * n_w);
+    QSI_CHECK_HIP(
+        hipMemcpy(out.data(), bout.d(), out.size() * sizeof(double), hipMemcpyDeviceToHost));
+    *P_out = P;
+    return QSI_OK;
   }
+  QSI_CHECK_HIP(bY.alloc(static_cast<size_t>(ldy) * P * sizeof(double)));
+  QSI_CHECK_HIP(bpart.alloc(gram_partials(P, n_w, gram, D) * sizeof(double)));
+  double* Y = bY.d();
+  if (small) {
+    std::vector<EachOp> each(n_ops);
+    for (int l = 0; l < n_ops; ++l)
+      each[l] = {ops[l]->d_off, ops[l]->d_diag, ops[l]->n_off, ops[l]->n_diag, 0};
+    QSI_CHECK_HIP(bops.alloc(each.size() * sizeof(EachOp)));
+    QSI_CHECK_HIP(hipMemcpy(bops.p, each.data(), each.size() * sizeof(EachOp),
+                            hipMemcpyHostToDevice));
+    for (int l0 = 0; l0 < n_ops; l0 += 1 << 18) {  // at most 2^15 workgroups of operators
+      const int nl = std::min(n_ops - l0, 1 << 18);
+      QSI_TRY(launch_apply_each(basis, static_cast<const EachOp*>(bops.p) + l0, nl, d_psi, ld,
+                                n_vec, Y + static_cast<int64_t>(l0) * n_vec * ldy, ldy, s));
+    }
+  } else {
+    for (int l = 0; l < n_ops; ++l)
+      for (int i = 0; i < n_vec; ++i)
+        QSI_TRY(launch_apply(ops[l], d_psi + static_cast<int64_t>(i) * ld,
+                             Y + static_cast<int64_t>(l * n_vec + i) * ldy, nullptr, 0.0, nullptr,
+                             nullptr, s));
+  }
+  QSI_TRY(launch_gram(Y, ldy, P, gram ? Y : d_psi, gram ? ldy : ld, n_w, D, bpart.d(), bout.d(),
+                      s));
   out.resize(static_cast<size_t>(P) * n_w);
   QSI_CHECK_HIP(hipMemcpy(out.data(), bout.d(), out.size() * sizeof(double), hipMemcpyDeviceToHost));
   *P_out = P;
