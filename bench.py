@@ -39,7 +39,7 @@ PMC_SUMMARY_96 = os.path.join(ROOT, "profiles", "apply_96spin_pmc.json")
 _VARIANT_KERNEL = {"lane": ("lane", 1), "lane2": ("lane", 2), "lane4": ("lane", 4),
                    "lane8": ("lane", 8), "low2": ("low", 2), "low4": ("low", 4),
                    "low8": ("low", 8), "slot2": ("slot", 2), "slot3": ("slot", 3),
-                   "slot4": ("slot", 4), "window": ("win", 4), "hash": ("hash", 1),
+                   "slot4": ("slot", 4), "window": ("win", 0), "hash": ("hash", 1),
                    "hash4": ("hash", 4)}
 
 
@@ -49,6 +49,8 @@ def variant_kernel(variant, nw, cached_pipe=None, low_mode=0):
     if variant == "cached":
         return f"k_apply_cached<{nw}, false, {cached_pipe},"
     kind, g = _VARIANT_KERNEL[variant]
+    if kind == "win":  # without the compare after a mode-2 check
+        return f"k_apply_win<{nw}, false, false, {'false' if low_mode == 2 else 'true'}>"
     if kind == "low":
         return f"k_apply_low<{nw}, false, false, {g}, {int(low_mode or 0)}>"
     return f"k_apply_{kind}<{nw}, false, false, {g}>"

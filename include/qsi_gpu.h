@@ -152,8 +152,10 @@ int qsi_op_n_diag(qsi_op_t op);
  * QSI_APPLY_HASH{,4}: each lane owns a row and finds its connected states in
  * the hash index, 1/4 lookups in flight per lane.  QSI_APPLY_LANE{,2,4,8}: the
  * same through the bucket table and a bisection of the bucket.
- * QSI_APPLY_WINDOW: per wavefront, one bucket lookup per term, then the
- * connected rows search a 64-state window staged in LDS.  QSI_APPLY_CACHED:
+ * QSI_APPLY_WINDOW: per wavefront of 128 rows, two bucket lookups per term (its
+ * first and last connected state), then the rows are matched in order with the
+ * basis states between them that the reversed flip connects (bases below 128
+ * states: as LANE4).  QSI_APPLY_CACHED:
  * gathers through the cached connectivity (qsi_op_cache_connectivity; setting
  * it requires the cache, dropping the cache resets it to AUTO).
  * QSI_APPLY_SLOT{2,3,4}: as LANE*, through the slot index under each bucket
@@ -162,9 +164,12 @@ int qsi_op_n_diag(qsi_op_t op);
  * LANE4 (SLOT4) or LANE2.  QSI_APPLY_LOW{2,4,8}: as LANE*, bisecting each
  * bucket on the basis's low keys (qsi_basis_build_lowkeys); setting one
  * requires them, and without them later the apply falls back to LANE* of the
- * same depth.  AUTO = CACHED when the connectivity is cached, else, when the
- * basis has low keys, LOW8 after qsi_op_verify_lowkeys found mode 2 and LOW4
- * otherwise, else LANE4.
+ * same depth.  AUTO = CACHED when the connectivity is cached; else WINDOW on
+ * bases of at least 2^21 states whose connected states are mostly in the basis
+ * and whose terms flip no spin outside their projectors (after
+ * qsi_op_verify_lowkeys found mode 2: one-word states, or at least 2^28
+ * of two words, and a term list that holds every flip's reverse); else, when the
+ * basis has low keys, LOW8 after mode 2 and LOW4 otherwise, else LANE4.
  * All give bit-identical y. */
 enum {
   QSI_APPLY_AUTO = 0,

@@ -165,17 +165,6 @@ __host__ __device__ __forceinline__ uint32_t low_key(const BasisView& b, const S
   return static_cast<uint32_t>(k);
 }
 
-// true if the state has a bit at or above n_spins (it is then larger than
-// every basis state)
-template <int NW>
-__device__ __forceinline__ bool above_range(const State<NW>& s, int n_spins) {
-  if constexpr (NW == 1) {
-    return n_spins < 64 && (s.w[0] >> n_spins) != 0;
-  } else {
-    return n_spins < 128 && (s.w[1] >> (n_spins - 64)) != 0;
-  }
-}
-
 template <int NW>
 __device__ __forceinline__ bool st_lt(const State<NW>& a, const State<NW>& b) {
   if constexpr (NW == 1) {
@@ -312,37 +301,6 @@ __device__ __forceinline__ int64_t hash_lookup(const HashView& h,
     }
     p = (p + 1) & h.mask;
   }
-}
-
-// First rank whose state is >= key (dim if none): bucket from the table,
-// then a lower-bound bisection inside it.  A state outside the basis may
-// differ from the basis at a position the key leaves out, so its bucket need
-// not bound its place: the result is checked against its neighbours and, if
-// it is off, the bisection is redone over the whole basis.
-template <int NW>
-__device__ __forceinline__ int64_t basis_lower_bound(const BasisView& b,
-                                                     const State<NW>& key) {
-  if (above_range<NW>(key, b.n_spins)) return b.dim;
-  auto bisect = [&](int64_t lo, int64_t n) {
-    while (n > 0) {
-      const int64_t half = n >> 1;
-      const State<NW> m = load_state_cached<NW>(b.states, lo + half);
-      if (st_lt<NW>(m, key)) {
-        lo += half + 1;
-        n -= half + 1;
-      } else {
-        n = half;
-      }
-    }
-    return lo;
-  };
-  const uint32_t k = bucket_key<NW>(b, key);
-  const int64_t lo0 = b.table[k];
-  const int64_t lo = bisect(lo0, static_cast<int64_t>(b.table[static_cast<uint64_t>(k) + 1]) - lo0);
-  const bool below_ok = lo == 0 || st_lt<NW>(load_state_cached<NW>(b.states, lo - 1), key);
-  const bool above_ok = lo == b.dim || !st_lt<NW>(load_state_cached<NW>(b.states, lo), key);
-  if (below_ok && above_ok) return lo;
-  return bisect(0, b.dim);
 }
 
 }  // namespace qsi

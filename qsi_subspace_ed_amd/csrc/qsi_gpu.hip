@@ -20,10 +20,12 @@
 #include <hipcub/hipcub.hpp>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <mutex>
 #include <new>
+#include <set>
 #include <vector>
 
 #include "qsi_blockk.hpp"
@@ -165,6 +167,24 @@ __global__ void k_verify_lowkeys(BasisView b, const OffTerm* __restrict__ off, i
     else if (!st_eq<NW>(load_state_cached<NW>(b.states, lo), key)) clash = true;
   }
   if (clash || absent) atomicOr(bad, (clash ? 1u : 0u) | (absent ? 2u : 0u));
+}
+
+// cnt[0] += connecting (row, term) pairs of gridDim.x * blockDim.x rows spread
+// evenly over the basis, cnt[1] += those whose target is in the basis.
+template <int NW>
+__global__ void k_sample_closed(BasisView b, const OffTerm* __restrict__ off, int n_off,
+                                unsigned int* __restrict__ cnt) {
+  const int64_t n = static_cast<int64_t>(gridDim.x) * blockDim.x;
+  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+  const State<NW> s = load_state_cached<NW>(b.states, b.dim / n * k);
+  unsigned int conn = 0, found = 0;
+  for (int t = 0; t < n_off; ++t) {
+    if (!term_ok<NW>(off[t], s)) continue;
+    ++conn;
+    found += basis_lookup<NW>(b, xor_state<NW>(s, off[t].X)) >= 0 ? 1u : 0u;
+  }
+  atomicAdd(cnt, conn);
+  atomicAdd(cnt + 1, found);
 }
 
 // lowkeys[i] = low key of state i (qsi_basis_build_lowkeys)
@@ -917,48 +937,269 @@ __global__ __launch_bounds__(kApplyBlock) void k_apply_hash(
 }
 
 // ----------------------------------------------------------------------------
-// Window variant (default).  A wavefront owns 64 consecutive rows.  For one
-// term, the rows it connects share the term's precondition bits, so their
-// targets s ^ X are increasing in lane order and fall in a short run of the
-// sorted basis (median ~40 ranks on the 64-spin ice basis).  Per chunk of 64
-// terms the wavefront
-//   1. tests every term on every row; a ballot gives each term's lane mask,
-//   2. finds each term's anchor rank (lower bound of its first target) with
-//      the 64 lookups spread over the 64 lanes,
-//   3. per term, stages basis[r .. r+63] and x[r .. r+63] in LDS with one
-//      coalesced load each, and every connected lane bisects the staged window
-//      (targets past the window fall back to a full lookup).
-// Contributions are added in term order, then the diagonal, exactly as in the
-// lane variant, so both variants give bit-identical y.
+// Window variant.  A wavefront owns 128 consecutive rows, two per lane (lane l
+// holds rows l and 64 + l).  For one term, the rows it connects share the
+// term's projector bits, so their targets s ^ X increase with the row, and
+// every basis state between the first and the last target that the reversed
+// flip connects (its projector bits are v ^ X) is the target of one of those
+// rows: the p-th connected row's target is the p-th such state.  So a
+// wavefront looks up two ranks per term (first and last target) instead of one
+// per row and term, reads the basis states and x between them with coalesced
+// loads (a window: 128 ranks, two per lane), and matches rows to states by
+// counting bits of lane masks, with no search and no key compare.  On the
+// 64-spin ice basis 128 rows connect through 39 of the 128 terms, 36 rows each,
+// and a term's targets span 80 ranks at the median (a quarter span more than
+// one window).  Per batch of up to 64 terms that the bits shared by all 128
+// rows do not rule out:
+//   1. one compare per term and 64 rows gives the row masks, kept in lane q
+//      for the q-th term;
+//   2. lane q looks up the ranks of its first and last target (both
+//      bisections in flight together) and lists its windows in LDS;
+//   3. the windows are taken in order with P of them in flight; a window's
+//      matching lanes write x to LDS compacted, the term's rows read it back
+//      by their own index, and add it in term order.
+// A target may be missing from the basis, or a state in the range may have no
+// partner row (a sector the terms do not close).  CHECK also passes the
+// matched states through LDS and compares them with the rows' targets; a term
+// with a mismatch (also one that flips a spin its projector leaves open, whose
+// targets do not keep the rows' order), an end that is not found or a range
+// beyond kWinMax windows is done by per-row lookups.  Without CHECK (every
+// connected state is in the basis, every flip's reverse is a term too, every
+// flipped spin under the projector) only the last can be.
+// What bounds it is the L2's misses: states and x of a window are 16 or 24 bytes
+// a rank, a third of them matched, and the rows in flight on an XCD reach more
+// ranks than its L2 holds (72 spins: 8.4 GB per apply at 7 TB/s).  Wider tiles,
+// fewer or more windows in flight and fewer wavefronts measured no better.
+// Against four lookups in flight per row (LANE4, no low keys): 64 spins 266 ->
+// 200 us, 72 spins 2.09 -> 1.47 ms, 80 spins 17.6 -> 10.1 ms, 96 spins 543 -> 301 ms.
+// Contributions are added in term order, then the diagonal, and the dot
+// product's partials are those of 256 rows, exactly as in the lane variant, so
+// y and the partials are bit-identical.
 // ----------------------------------------------------------------------------
 
 constexpr int kWavesPerBlock = kApplyBlock / 64;
-
-
+// windows in flight per wavefront, and wavefronts per SIMD
+// (7 wavefronts of 4 windows measured best at 64 spins: 8 x 2 188, 6 x 4 200, 4 x 8
+// 220 us)
+template <int NW, bool CHECK>
+constexpr int kWinItems = NW == 1 ? 4 : 2;
+template <int NW, bool CHECK>
+constexpr int kWinWaves = NW == 1 ? 7 : 5;
+// AUTO takes the window kernel from this many states on; against LOW8 on two-word
+// states only from the second
+constexpr int64_t kWinMinDim = int64_t{1} << 21;
+constexpr int64_t kWinMinDimLow2 = int64_t{1} << 28;
+constexpr int kWinRows = 128;  // rows of a wavefront, and ranks of a window
+constexpr int kWinMax = 8;     // windows of one term (a wider range: per-row lookups)
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-__device__ __forceinline__ uint64_t readlane64(uint64_t v, int lane) {
-  const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(v), lane);
-  const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(v >> 32), lane);
+__device__ __forceinline__ uint32_t readlane32(uint32_t v, int lane) {
+  return __builtin_amdgcn_readlane(v, lane);
+}
+
+// v with lane `lane`'s value replaced by val (val and lane wave-uniform); the
+// compiler intrinsic, which has no builtin of its own.
+extern "C" __device__ int qsi_amdgcn_writelane(int val, int lane, int v) __asm(
+    "llvm.amdgcn.writelane.i32");
+
+__device__ __forceinline__ uint32_t writelane32(uint32_t val, int lane, uint32_t v) {
+  return static_cast<uint32_t>(
+      qsi_amdgcn_writelane(static_cast<int>(val), lane, static_cast<int>(v)));
+}
+
+__device__ __forceinline__ uint64_t first_lane64(uint64_t v) {
+  const uint32_t lo = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v));
+  const uint32_t hi = __builtin_amdgcn_readfirstlane(static_cast<uint32_t>(v >> 32));
   return (static_cast<uint64_t>(hi) << 32) | lo;
 }
 
-template <int NW, bool HAS_Z, bool DOT, int P>
-__global__ __launch_bounds__(kApplyBlock) void k_apply_win(
-    BasisView b, const OffTerm* __restrict__ off, int n_off,
-    const DiagTerm* __restrict__ dg, int n_diag, const double* __restrict__ x,
+// OR of v over the wavefront (row shifts and row broadcasts, result uniform).
+__device__ __forceinline__ uint32_t wave_or32(uint32_t v) {
+  v |= __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v |= __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v |= __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v |= __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v |= __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v |= __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return readlane32(v, 63);
+}
+
+__device__ __forceinline__ uint64_t wave_or64(uint64_t v) {
+  const uint32_t lo = wave_or32(static_cast<uint32_t>(v));
+  const uint32_t hi = wave_or32(static_cast<uint32_t>(v >> 32));
+  return (static_cast<uint64_t>(hi) << 32) | lo;
+}
+
+// Set bits of m below this lane, plus base.
+__device__ __forceinline__ uint32_t lanes_below(uint64_t m, uint32_t base) {
+  return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
+                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), base));
+}
+
+// Inclusive sum of v over the wavefront's lanes.
+__device__ __forceinline__ uint32_t wave_scan_add(uint32_t v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);  // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);  // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);  // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
+  return v;
+}
+
+// Elements 2 lane and 2 lane + 1 from a wave-uniform address, read in 16-byte
+// pieces (8-byte aligned).  The empty asm keeps the address in scalar registers
+// (the load adds the lane's offset); otherwise the compiler adds in the vector
+// unit.
+template <typename T>
+__device__ __forceinline__ void load_window(const void* p, int lane, T (&v)[2]) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(8)));
+  typedef const __attribute__((address_space(1))) char* gptr;
+  gptr g = (gptr)p;
+  asm("" : "+s"(g));
+  constexpr uint32_t kBytes = 2 * sizeof(T);
+  u32x4 piece[kBytes / 16];
+#pragma unroll
+  for (uint32_t k = 0; k < kBytes / 16; ++k)
+    piece[k] = *(const __attribute__((address_space(1))) u32x4*)(
+        g + static_cast<uint32_t>(lane) * kBytes + 16 * k);
+  __builtin_memcpy(&v[0], &piece[0], kBytes);
+}
+
+// Lanes whose state the term connects, and whose state its reverse connects.
+template <int NW>
+__device__ __forceinline__ uint64_t rec_lanes(const State<NW>& s, const TermRec<NW>& A) {
+  uint64_t b = ~uint64_t{0};
+#pragma unroll
+  for (int w = 0; w < NW; ++w) b &= __builtin_amdgcn_ballot_w64((s.w[w] & A.m[w]) == A.v[w]);
+  return b;
+}
+template <int NW>
+__device__ __forceinline__ uint64_t rec_hits(const State<NW>& s, const TermRec<NW>& A) {
+  uint64_t b = ~uint64_t{0};
+#pragma unroll
+  for (int w = 0; w < NW; ++w) b &= __builtin_amdgcn_ballot_w64((s.w[w] & A.m[w]) == A.u[w]);
+  return b;
+}
+
+// The listed terms (term t_k in lane k, nq of them; also in LDS at list[k].x, as
+// a lane may not read a register of one that has finished) by per-row lookups, G in
+// flight per lane, as the lane variant's rounds: acc gains this lane's row's
+// contributions.  What a batch takes when most of its terms lead out of the
+// basis.
+template <int NW, bool HAS_Z>
+__device__ __forceinline__ void win_batch_by_rows(
+    const BasisView& b, const OffTerm* __restrict__ off, const TermPlanes& tp,
+    const TermRec<NW>* __restrict__ tr, int t, const uint2* list, int nq,
+    const double* __restrict__ x, double xs, const State<NW>& s, uint32_t ks, bool row_ok, double& acc) {
+  constexpr int G = NW == 1 ? 4 : 2;
+  uint32_t word[2] = {0, 0};
+  for (int k = 0; k < 64; ++k) {
+    uint64_t m = 0;
+    if (k < nq) m = rec_lanes<NW>(s, tr[readlane32(t, k)]);
+    word[k >> 5] = shift_in_lane(word[k >> 5], m);
+  }
+  uint64_t mask = row_ok ? static_cast<uint64_t>(word[0]) << 32 | word[1] : 0;
+  while (mask) {
+    int tt[G];
+    uint32_t lo[G], n[G];
+    State<NW> key[G];
+    uint2 p[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      const bool act = mask != 0;
+      const int z = act ? __builtin_clzll(mask) : 0;
+      mask &= ~(uint64_t{1} << 63 >> z);
+      tt[g] = static_cast<int>(list[z].x);
+      p[g] = make_uint2(0u, 0u);
+#pragma unroll
+      for (int w = 0; w < NW; ++w) key[g].w[w] = s.w[w] ^ tp.X(w)[tt[g]];
+      if (act)
+        __builtin_memcpy(&p[g], b.table + (ks ^ static_cast<uint32_t>(tp.key()[tt[g]])),
+                         sizeof(uint2));
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) asm volatile("" : "+v"(p[g].x), "+v"(p[g].y));
+    bool more = false;
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      lo[g] = p[g].x;
+      n[g] = p[g].y - p[g].x;
+      more |= n[g] > 1;
+    }
+    while (more) {
+      State<NW> m[G];
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        m[g] = State<NW>{};
+        if (n[g] > 1) m[g] = load_state_cached<NW>(b.states, lo[g] + (n[g] >> 1));
+      }
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+#pragma unroll
+        for (int w = 0; w < NW; ++w) asm volatile("" : "+v"(m[g].w[w]));
+      more = false;
+#pragma unroll
+      for (int g = 0; g < G; ++g) {
+        const uint32_t half = n[g] >> 1;
+        lo[g] = st_le<NW>(m[g], key[g]) ? lo[g] + half : lo[g];
+        n[g] -= half;
+        more |= n[g] > 1;
+      }
+    }
+    double xj[G];
+    State<NW> f[G];
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      xj[g] = 0.0;
+      if (n[g] == 1) {
+        f[g] = load_state_cached<NW>(b.states, lo[g]);
+        xj[g] = x[lo[g]];
+      }
+    }
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+      xj[g] *= xs;
+      if (n[g] == 1 && st_eq<NW>(f[g], key[g]) && fabs(xj[g]) > kApplyTol) {
+        double cg = tr[tt[g]].c;
+        if constexpr (HAS_Z) {
+          if (parity_notz<NW>(s, off[tt[g]].Z)) cg = -cg;
+        }
+        acc += cg * xj[g];
+      }
+    }
+  }
+}
+
+template <int NW, bool HAS_Z, bool DOT, bool CHECK>
+__global__ __launch_bounds__(kApplyBlock)
+__attribute__((amdgpu_waves_per_eu(kWinWaves<NW, CHECK>))) void k_apply_win(
+    BasisView b, const OffTerm* __restrict__ off, int n_off, TermPlanes tp,
+    const TermRec<NW>* __restrict__ tr, const DiagTerm* __restrict__ dg, int n_diag, const double* __restrict__ x,
     double* y, const double* y_in, double yscale,
     const double* __restrict__ yscale_dev, double* __restrict__ partials,
     const double* __restrict__ xs_dev, const double* __restrict__ ys_dev) {
-  __shared__ uint64_t rows_lds[kWavesPerBlock][64 * NW];
-  __shared__ uint64_t win_lds[kWavesPerBlock][P][64 * NW];
-  __shared__ double xwin_lds[kWavesPerBlock][P][64];
+  constexpr int P = kWinItems<NW, CHECK>;
+  constexpr int R = 2;  // rows of a lane, and ranks of a lane's window share
+  // the 64 listed windows are whole groups of P: a group past lane 63 would wrap
+  static_assert(64 % P == 0, "P divides the windows listed at a time");
+  // a term's matched x (and states), compacted: fewer than 128 before its last
+  // window, and at most 128 more from that one
+  constexpr int kEx = 2 * kWinRows;
+  __shared__ double ex[kWavesPerBlock][kEx];
+  __shared__ State<NW> exs[CHECK ? kWavesPerBlock : 1][CHECK ? kEx : 1];
+  __shared__ int list[kWavesPerBlock][128];    // terms not ruled out
+  __shared__ uint2 item[kWavesPerBlock][64];   // windows: first rank, flags
+  // flags of a window: first / last window of its term, term for per-row
+  // lookups; the last lane to read in bits 3-8; the term from bit 9 on
+  constexpr uint32_t kFirst = 1u, kLast = 2u, kSlow = 4u;
+  constexpr int kLane = 3, kTerm = 9;
   const int lane = threadIdx.x & 63;
-  const int wid = threadIdx.x >> 6;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const uint32_t blk = xcd_remap(blockIdx.x, gridDim.x);
   if (yscale_dev) yscale *= yscale_dev[0];
   // x and y_in are read as xs * x and ys * y_in.  Only the dot-product
@@ -966,141 +1207,292 @@ __global__ __launch_bounds__(kApplyBlock) void k_apply_win(
   // constant 1 and the multiplies fold away.
   const double xs = (DOT && xs_dev) ? xs_dev[0] : 1.0;
   const double ys = (DOT && ys_dev) ? ys_dev[0] : 1.0;
-  const int64_t i = static_cast<int64_t>(blk) * kApplyBlock + threadIdx.x;
-  const bool row_ok = i < b.dim;
-  const State<NW> s = load_state_cached<NW>(b.states, row_ok ? i : 0);
+  const int64_t r0 = (static_cast<int64_t>(blk) * kWavesPerBlock + wid) * kWinRows;
+  double prod[R] = {0.0, 0.0};
+  if (r0 < b.dim) {  // wave-uniform
+    State<NW> s[R];
+    double acc[R];
+    uint32_t ks[R];
+    uint64_t rows[R];  // lanes with a row
+    uint64_t same[NW], s0[NW];  // the bits all rows share; the first row
 #pragma unroll
-  for (int w = 0; w < NW; ++w) rows_lds[wid][lane * NW + w] = s.w[w];
-  double acc = 0.0;
-  double xi = 0.0;
-  if (row_ok) {
-    xi = x[i] * xs;
-    acc = y_in ? yscale * (y_in[i] * ys) : 0.0;
-  }
-  wave_sync();
-  for (int t0 = 0; t0 < n_off; t0 += 64) {
-    const int tn = min(64, n_off - t0);
-    // 1. lane masks: lane k keeps the mask of term t0 + k
-    uint64_t my_mask = 0;
-    for (int k = 0; k < tn; ++k) {
-      const uint64_t m = __ballot(row_ok && term_ok<NW>(off[t0 + k], s));
-      my_mask = (lane == k) ? m : my_mask;
+    for (int q = 0; q < R; ++q) {
+      // lanes past the end hold the first row's state and connect to nothing
+      const int64_t i = r0 + 64 * q + lane;
+      const int64_t left = b.dim - (r0 + 64 * q);
+      rows[q] = left >= 64 ? ~uint64_t{0} : left > 0 ? ~uint64_t{0} >> (64 - left) : 0;
+      s[q] = load_state_cached<NW>(b.states, i < b.dim ? i : r0);
+      acc[q] = 0.0;
+      if (y_in && i < b.dim) acc[q] = yscale * (y_in[i] * ys);
+      ks[q] = bucket_key<NW>(b, s[q]);
     }
-    // 2. anchors: lower bound of the first connected row's target, one
-    //    lookup per lane, all in flight together
-    uint32_t anchor = 0;
-    if (lane < tn && my_mask != 0) {
-      const int a = __builtin_ctzll(my_mask);
-      State<NW> key;
 #pragma unroll
-      for (int w = 0; w < NW; ++w) key.w[w] = rows_lds[wid][a * NW + w] ^ off[t0 + lane].X[w];
-      anchor = static_cast<uint32_t>(basis_lower_bound<NW>(b, key));
+    for (int w = 0; w < NW; ++w) {
+      s0[w] = first_lane64(s[0].w[w]);
+      same[w] = ~wave_or64((s[0].w[w] ^ s0[w]) | (s[1].w[w] ^ s0[w]));
     }
-    // 3. groups of P terms: stage P windows with back-to-back loads, then run
-    //    the P bisections interleaved
-    for (int kb = 0; kb < tn; kb += P) {
-      uint64_t gm[P];
-      int64_t gr[P];
-      uint64_t any = 0;
+    const uint32_t dim32 = static_cast<uint32_t>(b.dim);
+    const uint32_t top = dim32 - kWinRows;  // the basis has at least kWinRows states
+    int n_list = 0;
+    for (int t0 = 0; t0 < n_off || n_list > 0; t0 += 64) {
+      if (t0 < n_off) {
+        // terms that the shared bits do not rule out (the planes are padded
+        // to whole chunks)
+        const int t = t0 + lane;
+        bool alive = t < n_off;
 #pragma unroll
-      for (int j = 0; j < P; ++j) {
-        const int k = kb + j;
-        gm[j] = (k < tn) ? readlane64(my_mask, k) : 0;
-        gr[j] = gm[j] ? static_cast<int64_t>(__builtin_amdgcn_readlane(anchor, k)) : 0;
-        any |= gm[j];
+        for (int w = 0; w < NW; ++w)
+          alive = alive && ((s0[w] ^ tp.v(w)[t]) & tp.m(w)[t] & same[w]) == 0;
+        const uint64_t live = __builtin_amdgcn_ballot_w64(alive);
+        const uint32_t at = lanes_below(live, n_list);
+        if (alive) list[wid][at] = t;
+        n_list += __popcll(live);
+        if (n_list < 64 && t0 + 64 < n_off) continue;
+        wave_sync();
       }
-      if (any == 0) continue;
-      State<NW> wv[P];
-      double xv[P];
-#pragma unroll
-      for (int j = 0; j < P; ++j) {
-        const int64_t idx = gr[j] + lane;
-        if (gm[j] != 0 && idx < b.dim) {
-          wv[j] = load_state_cached<NW>(b.states, idx);
-          xv[j] = x[idx] * xs;
-        }
-      }
-#pragma unroll
-      for (int j = 0; j < P; ++j) {
-        const int64_t idx = gr[j] + lane;
-        if (gm[j] != 0 && idx < b.dim) {
-#pragma unroll
-          for (int w = 0; w < NW; ++w) win_lds[wid][j][lane * NW + w] = wv[j].w[w];
-          xwin_lds[wid][j][lane] = xv[j];
-        }
+      if (n_list == 0) break;
+      const int nq = min(n_list, 64);
+      // lanes past the list hold the record that connects nothing
+      const int t = lane < nq ? list[wid][lane] : n_off;
+      n_list -= nq;
+      if (n_list > 0) {  // the rest moves to the front
+        const int t2 = list[wid][64 + lane];
+        wave_sync();
+        list[wid][lane] = t2;
       }
       wave_sync();
-      int lo[P], n[P], nv[P];
+      // 1. row masks of the q-th term in lane q
+      uint32_t mlo[R] = {0, 0}, mhi[R] = {0, 0};
+      for (int k0 = 0; k0 < nq; k0 += 4) {
+        TermRec<NW> A[4];
 #pragma unroll
-      for (int j = 0; j < P; ++j) {
-        nv[j] = gm[j] ? static_cast<int>(min<int64_t>(64, b.dim - gr[j])) : 0;
-        lo[j] = 0;
-        n[j] = ((gm[j] >> lane) & 1) ? nv[j] : 0;
+        for (int u = 0; u < 4; ++u) A[u] = tr[readlane32(t, k0 + u)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+#pragma unroll
+          for (int q = 0; q < R; ++q) {
+            const uint64_t mk = rec_lanes<NW>(s[q], A[u]) & rows[q];
+            mlo[q] = writelane32(static_cast<uint32_t>(mk), k0 + u, mlo[q]);
+            mhi[q] = writelane32(static_cast<uint32_t>(mk >> 32), k0 + u, mhi[q]);
+          }
+        }
       }
-      // lower-bound bisection of each key in its window (<= 7 rounds)
+      // 2. ranks of the first and the last connected row's targets
+      const bool a_hi = (mlo[0] | mhi[0]) == 0, z_hi = (mlo[1] | mhi[1]) != 0;
+      const uint64_t ma = a_hi ? static_cast<uint64_t>(mhi[1]) << 32 | mlo[1]
+                               : static_cast<uint64_t>(mhi[0]) << 32 | mlo[0];
+      const uint64_t mz = z_hi ? static_cast<uint64_t>(mhi[1]) << 32 | mlo[1]
+                               : static_cast<uint64_t>(mhi[0]) << 32 | mlo[0];
+      const bool has = ma != 0;
+      const int ra = has ? __builtin_ctzll(ma) : 0, rz = has ? 63 - __builtin_clzll(mz) : 0;
+      State<NW> ka, kz;
 #pragma unroll
-      for (int step = 0; step < 7; ++step) {
+      for (int w = 0; w < NW; ++w) {
+        const uint64_t X = tp.X(w)[t];
+        const uint64_t a0 = __shfl(s[0].w[w], ra, 64), a1 = __shfl(s[1].w[w], ra, 64);
+        const uint64_t z0 = __shfl(s[0].w[w], rz, 64), z1 = __shfl(s[1].w[w], rz, 64);
+        ka.w[w] = (a_hi ? a1 : a0) ^ X;
+        kz.w[w] = (z_hi ? z1 : z0) ^ X;
+      }
+      const uint32_t kx = static_cast<uint32_t>(tp.key()[t]);
+      const uint32_t ba0 = __shfl(ks[0], ra, 64), ba1 = __shfl(ks[1], ra, 64);
+      const uint32_t bz0 = __shfl(ks[0], rz, 64), bz1 = __shfl(ks[1], rz, 64);
+      uint2 pa = make_uint2(0u, 0u), pz = make_uint2(0u, 0u);
+      if (has) {
+        __builtin_memcpy(&pa, b.table + ((a_hi ? ba1 : ba0) ^ kx), sizeof(uint2));
+        __builtin_memcpy(&pz, b.table + ((z_hi ? bz1 : bz0) ^ kx), sizeof(uint2));
+      }
+      asm volatile("" : "+v"(pa.x), "+v"(pa.y), "+v"(pz.x), "+v"(pz.y));
+      uint32_t la = pa.x, na = pa.y - pa.x, lz = pz.x, nz = pz.y - pz.x;
+      while (na > 1 || nz > 1) {
+        State<NW> fa{}, fz{};
+        if (na > 1) fa = load_state_cached<NW>(b.states, la + (na >> 1));
+        if (nz > 1) fz = load_state_cached<NW>(b.states, lz + (nz >> 1));
 #pragma unroll
-        for (int j = 0; j < P; ++j) {
-          if (n[j] > 0) {
-            const State<NW> key = xor_state<NW>(s, off[t0 + kb + j].X);
-            const int half = n[j] >> 1;
-            State<NW> m;
+        for (int w = 0; w < NW; ++w) asm volatile("" : "+v"(fa.w[w]), "+v"(fz.w[w]));
+        const uint32_t ha = na >> 1, hz = nz >> 1;
+        la = st_le<NW>(fa, ka) ? la + ha : la;
+        lz = st_le<NW>(fz, kz) ? lz + hz : lz;
+        na -= ha;
+        nz -= hz;
+      }
+      bool good = has;
+      if constexpr (CHECK) {
+        good = na == 1 && nz == 1;
+        if (good) {
+          const State<NW> fa = load_state_cached<NW>(b.states, la);
+          const State<NW> fz = load_state_cached<NW>(b.states, lz);
+          good = st_eq<NW>(fa, ka) && st_eq<NW>(fz, kz);
+        }
+      }
+      // every window of the term lies inside the arrays
+      uint32_t n_win = (lz - la) / kWinRows + 1;
+      good = good && n_win <= kWinMax && la + n_win * kWinRows <= dim32;
+      if constexpr (CHECK) {
+        const int bad = __popcll(__builtin_amdgcn_ballot_w64(has && !good));
+        if (2 * bad > __popcll(__builtin_amdgcn_ballot_w64(has))) {
+          item[wid][lane] = make_uint2(static_cast<uint32_t>(t), 0u);
+          wave_sync();
 #pragma unroll
-            for (int w = 0; w < NW; ++w) m.w[w] = win_lds[wid][j][(lo[j] + half) * NW + w];
-            if (st_lt<NW>(m, key)) {
-              lo[j] += half + 1;
-              n[j] -= half + 1;
+          for (int q = 0; q < R; ++q)
+            win_batch_by_rows<NW, HAS_Z>(b, off, tp, tr, t, item[wid], nq, x, xs, s[q], ks[q],
+                                         __builtin_amdgcn_inverse_ballot_w64(rows[q]), acc[q]);
+          wave_sync();
+          continue;
+        }
+      }
+      n_win = good ? n_win : has ? 1u : 0u;
+      const uint32_t end = wave_scan_add(n_win);
+      const int n_items = static_cast<int>(readlane32(end, 63));
+      // contribution of term tt to this lane's row q
+      auto add = [&](int q, uint32_t tt, double c, double xj) {
+        if constexpr (HAS_Z) {
+          if (parity_notz<NW>(s[q], off[tt].Z)) c = -c;
+          if (fabs(xj) > kApplyTol) acc[q] += c * xj;
+        } else {
+          // under a branch: as a select it costs two more vector instructions
+          if (fabs(xj) > kApplyTol)
+            asm volatile("v_fma_f64 %0, %1, %2, %0" : "+v"(acc[q]) : "v"(xj), "s"(c));
+        }
+      };
+      // 3. the windows, 64 listed at a time (all of this loop's control is
+      //    wave-uniform)
+      uint32_t base = 0;  // matches in the current term's windows so far
+      for (int i0 = 0; i0 < n_items; i0 += 64) {
+        for (uint32_t w = 0; w < n_win; ++w) {
+          const uint32_t id = end - n_win + w - i0;
+          if (id < 64) {
+            item[wid][id] = make_uint2(
+                min(la + w * kWinRows, top),  // below top unless the term is slow
+                static_cast<uint32_t>(t) << kTerm | (w == 0 ? kFirst : 0u) |
+                    (w + 1 == n_win ? kLast : 0u) | (good ? 0u : kSlow) |
+                    (min(lz - la - w * kWinRows, kWinRows - 1u) >> 1) << kLane);
+          }
+        }
+        wave_sync();
+        const int n = min(n_items - i0, 64);
+        // entries past the end hold the term that matches nothing
+        const uint2 it = lane < n ? item[wid][lane]
+                                  : make_uint2(0u, static_cast<uint32_t>(n_off) << kTerm);
+        wave_sync();
+        State<NW> ws[P][R];
+        double wx[P][R];
+        auto issue = [&](int p, int id) {
+          // no load is under a condition: it could not be counted, only waited
+          // for with all others.  Lanes past the last target read its line again
+          // and match after every row's state.
+          const uint32_t from = readlane32(it.x, id & 63);
+          const int wl = min(lane, static_cast<int>(readlane32(it.y, id & 63) >> kLane & 63));
+          load_window<State<NW>>(b.states + static_cast<int64_t>(from) * NW, wl, ws[p]);
+          load_window<double>(x + from, wl, wx[p]);
+          // the order of the windows' loads is what their waits count
+          __builtin_amdgcn_sched_barrier(0);
+        };
+        // a term by per-row lookups
+        auto by_rows = [&](int tt, const TermRec<NW>& A) {
+#pragma unroll 1
+          for (int q = 0; q < R; ++q) {
+            const State<NW> sq = q == 0 ? s[0] : s[1];
+            if (__builtin_amdgcn_inverse_ballot_w64(rec_lanes<NW>(sq, A) & (q == 0 ? rows[0] : rows[1]))) {
+              const State<NW> want = xor_state<NW>(sq, off[tt].X);
+              const int64_t r = basis_lookup<NW>(b, want);
+              const double xj = r >= 0 ? x[r] * xs : 0.0;
+              if (r >= 0 && q == 0) add(0, tt, A.c, xj);
+              if (r >= 0 && q == 1) add(1, tt, A.c, xj);
+            }
+          }
+        };
+#pragma unroll
+        for (int p = 0; p < P; ++p) issue(p, p);
+        for (int id0 = 0; id0 < n; id0 += P) {
+#pragma unroll
+          for (int p = 0; p < P; ++p) {
+            const uint32_t f = readlane32(it.y, id0 + p);
+            const int tt = static_cast<int>(f >> kTerm);
+            const TermRec<NW> A = tr[tt];
+            if (f & kSlow) {
+              by_rows(tt, A);
             } else {
-              n[j] = half;
+              if (f & kFirst) base = 0;
+              uint64_t hit[R];
+#pragma unroll
+              for (int q = 0; q < R; ++q) hit[q] = rec_hits<NW>(ws[p][q], A);  // ranks 2 l + q
+              uint32_t at = lanes_below(hit[1], lanes_below(hit[0], base));
+              if (__builtin_amdgcn_inverse_ballot_w64(hit[0])) {
+                ex[wid][at] = wx[p][0];
+                if constexpr (CHECK) exs[wid][at] = ws[p][0];
+                ++at;
+              }
+              if (__builtin_amdgcn_inverse_ballot_w64(hit[1])) {
+                ex[wid][at] = wx[p][1];
+                if constexpr (CHECK) exs[wid][at] = ws[p][1];
+              }
+              if (!(f & kLast)) {
+                base += static_cast<uint32_t>(__popcll(hit[0]) + __popcll(hit[1]));
+                if constexpr (CHECK) {
+                  // no row reads past entry 127: more matches than that
+                  // (without a partner row each) only need to stay inside
+                  base = base < kWinRows ? base : kWinRows;
+                }
+              } else {
+                wave_sync();
+                uint64_t msk[R];
+                double xj[R];
+                uint64_t bad = 0;
+#pragma unroll
+                for (int q = 0; q < R; ++q) {
+                  msk[q] = rec_lanes<NW>(s[q], A) & rows[q];
+                  const uint32_t from = lanes_below(msk[q], q == 0 ? 0u : __popcll(msk[0]));
+                  xj[q] = ex[wid][from];
+                  if constexpr (CHECK) {
+                    const State<NW> fs = exs[wid][from];
+                    const State<NW> want = xor_state<NW>(s[q], off[tt].X);
+                    bad |= msk[q] & ~__builtin_amdgcn_ballot_w64(st_eq<NW>(fs, want));
+                  }
+                }
+                if (CHECK && bad != 0) {
+                  by_rows(tt, A);
+                } else {
+#pragma unroll
+                  for (int q = 0; q < R; ++q)
+                    if (__builtin_amdgcn_inverse_ballot_w64(msk[q])) add(q, tt, A.c, xj[q] * xs);
+                }
+                wave_sync();
+              }
             }
+            issue(p, id0 + p + P);
           }
         }
       }
-      // contributions in term order
-#pragma unroll
-      for (int j = 0; j < P; ++j) {
-        if ((gm[j] >> lane) & 1) {
-          const OffTerm& T = off[t0 + kb + j];
-          const State<NW> key = xor_state<NW>(s, T.X);
-          bool found = false;
-          double xj = 0.0;
-          if (lo[j] < nv[j]) {
-            State<NW> m;
-#pragma unroll
-            for (int w = 0; w < NW; ++w) m.w[w] = win_lds[wid][j][lo[j] * NW + w];
-            if (st_eq<NW>(m, key)) {
-              found = true;
-              xj = xwin_lds[wid][j][lo[j]];
-            }
-          } else {
-            const int64_t J = basis_lookup<NW>(b, key);
-            if (J >= 0) {
-              found = true;
-              xj = x[J] * xs;
-            }
-          }
-          if (found && fabs(xj) > kApplyTol) {
-            double c = T.c * T.sgn;
-            if constexpr (HAS_Z) {
-              if (parity_notz<NW>(s, T.Z)) c = -c;
-            }
-            acc += c * xj;
-          }
-        }
-      }
-      wave_sync();
     }
-  }
-  double prod = 0.0;
-  if (row_ok) {
-    acc = diag_accumulate<NW>(acc, xi, s, dg, n_diag);
-    y[i] = acc;
-    if constexpr (DOT) prod = xi * acc;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int64_t i = r0 + 64 * q + lane;
+      if (i < b.dim) {
+        const double xi = x[i] * xs;
+        acc[q] = diag_accumulate<NW>(acc[q], xi, s[q], dg, n_diag);
+        y[i] = acc[q];
+        if constexpr (DOT) prod[q] = xi * acc[q];
+      }
+    }
   }
   if constexpr (DOT) {
-    const double bs = block_sum<kApplyBlock>(prod);
-    if (threadIdx.x == 0) partials[blk] = bs;
+    // one partial per 256 rows, summed as block_sum does
+    __shared__ double red[kWavesPerBlock * R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const double v = wave_sum(prod[q]);
+      if (lane == 0) red[wid * R + q] = v;
+    }
+    __syncthreads();
+    constexpr int kPer = kApplyBlock / 64;  // 64-row sums of one partial
+    const int64_t pb = static_cast<int64_t>(blk) * R + threadIdx.x;
+    if (threadIdx.x < R && pb * kApplyBlock < b.dim) {
+      double v = 0.0;
+#pragma unroll
+      for (int w = 0; w < kPer; ++w) v += red[threadIdx.x * kPer + w];
+      partials[pb] = v;
+    }
   }
 }
 
@@ -1814,19 +2206,33 @@ static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
                            const double* xs_dev, const double* ys_dev, hipStream_t s) {
   const int64_t nb = apply_num_blocks(op);
   const dim3 grid(static_cast<uint32_t>(nb)), block(kApplyBlock);
+  // the window kernel's workgroups take two blocks of rows
+  const dim3 wgrid(static_cast<uint32_t>((nb + 1) / 2));
   const auto v = op->basis->view();
   int variant = op->variant;
-  // AUTO: the cached gathers when the connectivity is cached, else LANE4 (the
-  // fastest search kernel measured on the 64- and 96-spin bases, with or
-  // without the slot index and low keys; the autotuner times them all)
-  // AUTO: the cached connectivity when it exists, else the low-key kernel
-  // (eight lookups per lane once the candidates need no compare, four
-  // otherwise), else the lane kernel
-  if (variant == QSI_APPLY_AUTO)
-    variant = op->conn_nnz >= 0         ? QSI_APPLY_CACHED
-              : !op->basis->d_lowkeys   ? QSI_APPLY_LANE4
-              : op->lowkeys_check == kLowTrusted ? QSI_APPLY_LOW8
-                                                 : QSI_APPLY_LOW4;
+  // AUTO: the cached connectivity when it exists.  Else, without low keys whose
+  // candidates need no compare, the window kernel on bases large enough to fill
+  // the chip with its 128-row wavefronts (WINDOW / LANE4 / LOW4 in us: 32 spins
+  // 35 / 12 / 13, 293394 states 33 / 25 / 25, 1062882 states 55 / 52 / 53, 64 spins 200 /
+  // 266 / 273, 72 spins 1467 / 2089 / 1831; 80 spins 10.1 / 17.6 / 14.3 and 96 spins
+  // 301 / 543 ms), if the sampled rows' targets are mostly in the basis (64 spins
+  // with single flips, which all leave it, 678 / 456).  With them LOW8, except where WINDOW
+  // without its compare is the faster: one-word states on large bases (WINDOW /
+  // LOW8: 293394 states 33 / 21, 64 spins 181 / 190, 60 spins 166 / 191 us) and bases so
+  // large that the 31-bit bucket key leaves long bisections (72 spins 1.21 / 1.18,
+  // 80 spins 9.47 / 9.38, 96 spins 278 / 292 ms).
+  if (variant == QSI_APPLY_AUTO) {
+    const int64_t dim = op->basis->dim;
+    const bool trusted = op->basis->d_lowkeys && op->lowkeys_check == kLowTrusted;
+    const bool window = 
+        dim >= kWinMinDim && op->ordered &&
+        (trusted ? op->paired && (NW == 1 || dim >= kWinMinDimLow2) : op->mostly_closed);
+    variant = op->conn_nnz >= 0        ? QSI_APPLY_CACHED
+              : window                 ? QSI_APPLY_WINDOW
+              : trusted                ? QSI_APPLY_LOW8
+              : op->basis->d_lowkeys   ? QSI_APPLY_LOW4
+                                       : QSI_APPLY_LANE4;
+  }
   // a slot or low-key variant chosen while the basis had that index, which
   // has been dropped since, falls back to the lane kernel (LANE4 for SLOT4,
   // LANE2 for SLOT2 and SLOT3; the same depth for LOW*)
@@ -1856,9 +2262,23 @@ static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
                          y_in, yscale, yscale_dev, partials, xs_dev, ys_dev);
       break;
     case QSI_APPLY_WINDOW:
-      hipLaunchKernelGGL((k_apply_win<NW, HAS_Z, DOT, 4>), grid, block, 0, s, v,
-                         op->d_off, op->n_off, op->d_diag, op->n_diag, x, y,
-                         y_in, yscale, yscale_dev, partials, xs_dev, ys_dev);
+      // a window holds kWinRows states.  No compare of matched states when
+      // every connected state is in the basis, every flip's reverse is a term
+      // of the operator too, and targets keep the rows' order
+      if (op->basis->dim < kWinRows)
+        hipLaunchKernelGGL((k_apply_lane<NW, HAS_Z, DOT, 4>), grid, block, 0, s, v,
+                           op->d_off, op->n_off, op->d_diag, op->n_diag, x, y,
+                           y_in, yscale, yscale_dev, partials, xs_dev, ys_dev);
+      else if (op->lowkeys_check == kLowTrusted && op->paired && op->ordered)
+        hipLaunchKernelGGL((k_apply_win<NW, HAS_Z, DOT, false>), wgrid, block, 0, s, v,
+                           op->d_off, op->n_off, op->planes(),
+                           reinterpret_cast<const TermRec<NW>*>(op->planes().rec()), op->d_diag, op->n_diag, x, y,
+                           y_in, yscale, yscale_dev, partials, xs_dev, ys_dev);
+      else
+        hipLaunchKernelGGL((k_apply_win<NW, HAS_Z, DOT, true>), wgrid, block, 0, s, v,
+                           op->d_off, op->n_off, op->planes(),
+                           reinterpret_cast<const TermRec<NW>*>(op->planes().rec()), op->d_diag, op->n_diag, x, y,
+                           y_in, yscale, yscale_dev, partials, xs_dev, ys_dev);
       break;
     case QSI_APPLY_LANE8:
       hipLaunchKernelGGL((k_apply_lane<NW, HAS_Z, DOT, 8>), grid, block, 0, s, v,
@@ -2826,7 +3246,68 @@ int qsi_op_create(qsi_basis_t b, const qsi_term_t* terms, int n_terms,
   op->n_off = static_cast<int>(op->h_off.size());
   op->n_diag = static_cast<int>(op->h_diag.size());
   op->n_slots = n_slots;
-  hipError_t e = hipMalloc(&op->d_off, std::max<size_t>(1, op->h_off.size()) * sizeof(OffTerm));
+  // every flipped spin is under the term's projector, so targets keep the
+  // rows' order; and every term's reverse (the same flip from the flipped
+  // projector values) is a term too
+  op->ordered = op->paired = true;
+  {
+    for (auto& o : op->h_off)
+      op->ordered = op->ordered && ((o.X[0] & ~o.m[0]) | (o.X[1] & ~o.m[1])) == 0;
+    auto key = [](const OffTerm& o, bool rev) {
+      std::array<uint64_t, 6> k{};
+      for (int w = 0; w < 2; ++w) {
+        k[w] = o.X[w];
+        k[2 + w] = o.m[w];
+        k[4 + w] = rev ? o.v[w] ^ (o.X[w] & o.m[w]) : o.v[w];
+      }
+      return k;
+    };
+    std::set<std::array<uint64_t, 6>> have;
+    for (auto& o : op->h_off) have.insert(key(o, false));
+    for (auto& o : op->h_off) op->paired = op->paired && have.count(key(o, true)) != 0;
+  }
+  // the terms field by field and as TermRec records, behind the full records
+  // and padded to whole chunks of 64
+  op->n_plane = op->n_off / 64 * 64 + 64;
+  const size_t off_bytes = (std::max<size_t>(1, op->h_off.size()) * sizeof(OffTerm) + 63) / 64 * 64;
+  std::vector<uint64_t> planes(static_cast<size_t>(op->n_plane) *
+                                   (TermPlanes::kCount + sizeof(TermRec<2>) / sizeof(uint64_t)),
+                               0);
+  for (int t = 0; t < op->n_off; ++t) {
+    const OffTerm& o = op->h_off[t];
+    const double cs = o.c * o.sgn;
+    uint64_t cw;
+    std::memcpy(&cw, &cs, sizeof(cw));
+    const uint64_t bk = nw == 1 ? bucket_key<1>(b->view(), State<1>{{o.X[0]}})
+                                : bucket_key<2>(b->view(), State<2>{{o.X[0], o.X[1]}});
+    const uint64_t field[TermPlanes::kCount] = {o.m[0], o.v[0], o.X[0], o.m[1],
+                                                o.v[1], o.X[1], bk};
+    for (int q = 0; q < TermPlanes::kCount; ++q)
+      planes[static_cast<size_t>(q) * op->n_plane + t] = field[q];
+    uint64_t* rec = planes.data() + static_cast<size_t>(TermPlanes::kCount) * op->n_plane +
+                    static_cast<size_t>(t) * (nw == 1 ? sizeof(TermRec<1>) : sizeof(TermRec<2>)) /
+                        sizeof(uint64_t);
+    for (int w = 0; w < nw; ++w) {
+      rec[w] = o.m[w];
+      rec[nw + w] = o.v[w];
+      rec[2 * nw + w] = o.v[w] ^ (o.X[w] & o.m[w]);
+    }
+    rec[3 * nw] = cw;
+  }
+  // record n_off connects nothing and has no match
+  {
+    uint64_t* rec = planes.data() + static_cast<size_t>(TermPlanes::kCount) * op->n_plane +
+                    static_cast<size_t>(op->n_off) * (nw == 1 ? sizeof(TermRec<1>) : sizeof(TermRec<2>)) /
+                        sizeof(uint64_t);
+    rec[nw] = rec[2 * nw] = 1;
+  }
+  hipError_t e = hipMalloc(&op->d_off, off_bytes + planes.size() * sizeof(uint64_t));
+  if (e == hipSuccess) {
+    op->d_planes = reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(op->d_off) + off_bytes);
+  }
+  if (e == hipSuccess && !planes.empty())
+    e = hipMemcpy(op->d_planes, planes.data(), planes.size() * sizeof(uint64_t),
+                  hipMemcpyHostToDevice);
   if (e == hipSuccess)
     e = hipMalloc(&op->d_diag, std::max<size_t>(1, op->h_diag.size()) * sizeof(DiagTerm));
   if (e == hipSuccess && op->n_off)
@@ -2847,6 +3328,34 @@ int qsi_op_create(qsi_basis_t b, const qsi_term_t* terms, int n_terms,
     delete op;
     set_error(std::string("qsi_op_create: ") + hipGetErrorString(e));
     return e == hipErrorOutOfMemory ? QSI_E_NOMEM : QSI_E_HIP;
+  }
+  if (b->dim >= kWinMinDim && op->n_off > 0) {
+    // whether the terms mostly stay in the basis, by 4096 rows: AUTO's choice
+    // between kernels of equal results
+    unsigned int* cnt = nullptr;
+    unsigned int h[2] = {0, 0};
+    e = hipMalloc(&cnt, sizeof(h));
+    if (e == hipSuccess) e = hipMemset(cnt, 0, sizeof(h));
+    if (e == hipSuccess) {
+      if (nw == 1)
+        hipLaunchKernelGGL(k_sample_closed<1>, dim3(64), dim3(64), 0, 0, b->view(), op->d_off,
+                           op->n_off, cnt);
+      else
+        hipLaunchKernelGGL(k_sample_closed<2>, dim3(64), dim3(64), 0, 0, b->view(), op->d_off,
+                           op->n_off, cnt);
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipMemcpy(h, cnt, sizeof(h), hipMemcpyDeviceToHost);
+    if (cnt) (void)hipFree(cnt);
+    if (e != hipSuccess) {
+      (void)hipFree(op->d_off);
+      (void)hipFree(op->d_diag);
+      (void)hipFree(op->d_cls);
+      delete op;
+      set_error(std::string("qsi_op_create: ") + hipGetErrorString(e));
+      return QSI_E_HIP;
+    }
+    op->mostly_closed = h[1] >= h[0] - h[0] / 8;
   }
   basis_retain(b);
   op->basis = b;

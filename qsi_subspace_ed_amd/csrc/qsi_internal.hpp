@@ -54,6 +54,32 @@ struct DiagTerm {
   int32_t slot;
 };
 
+// What a wavefront needs of an off-diagonal term as one scalar load: projector
+// mask and value, the reversed flip's value v ^ (X & m), c * sgn.
+template <int NW>
+struct alignas(32 * NW) TermRec {
+  uint64_t m[NW];
+  uint64_t v[NW];
+  uint64_t u[NW];
+  double c;
+};
+static_assert(sizeof(TermRec<1>) == 32 && sizeof(TermRec<2>) == 64, "4 or 8 words");
+
+// The off-diagonal terms field by field, n entries each (a multiple of 64, the
+// tail zero), so a wavefront's lanes read one field of 64 terms with one
+// coalesced load (projector mask, value and flip mask per word, and the flip
+// mask's bucket key), and then as TermRec records.
+struct TermPlanes {
+  static constexpr int kCount = 7;
+  const uint64_t* p;
+  int n;
+  __host__ __device__ const uint64_t* m(int w) const { return p + (3 * w) * n; }
+  __host__ __device__ const uint64_t* v(int w) const { return p + (3 * w + 1) * n; }
+  __host__ __device__ const uint64_t* X(int w) const { return p + (3 * w + 2) * n; }
+  __host__ __device__ const uint64_t* key() const { return p + 6 * n; }
+  __host__ __device__ const uint64_t* rec() const { return p + kCount * n; }
+};
+
 }  // namespace qsi
 
 struct qsi_basis_s {
@@ -117,6 +143,11 @@ struct qsi_op_s {
   int variant = 0;     // apply kernel: one of the QSI_APPLY_* values
   qsi::OffTerm* d_off = nullptr;
   qsi::DiagTerm* d_diag = nullptr;
+  uint64_t* d_planes = nullptr;  // TermPlanes data (in the allocation of d_off)
+  int n_plane = 0;
+  bool ordered = false;          // every off-diagonal term's X lies under its m
+  bool paired = false;           // every off-diagonal term's reverse is a term too
+  bool mostly_closed = false;    // sampled: most connected states are in the basis
   std::vector<qsi::OffTerm> h_off;
   std::vector<qsi::DiagTerm> h_diag;
   int n_cls = 0;  // coefficient classes (0: more than kMaxCoefClasses)
@@ -139,6 +170,8 @@ struct qsi_op_s {
   // compare (every connected state is in the basis).  A property of the terms
   // and the basis, both fixed, so it holds for any build of the keys.
   int lowkeys_check = 0;
+
+  qsi::TermPlanes planes() const { return {d_planes, n_plane}; }
 };
 
 namespace qsi {

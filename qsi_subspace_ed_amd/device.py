@@ -210,12 +210,12 @@ class GpuOp:
 
     def set_variant(self, variant):
         """Choose the apply kernel: 'auto' ('cached' when the connectivity is
-        cached, else with low keys 'low8' after verify_lowkeys() gave 2 and
-        'low4' otherwise, else 'lane4'),
+        cached, else 'window' on large bases, else with low keys 'low8' after
+        verify_lowkeys() gave 2 and 'low4' otherwise, else 'lane4'),
         'cached', 'hash', 'hash4' (hash-index lookups; the basis needs
         hash_index=True), 'lane', 'lane2', 'lane4',
         'lane8' (bucket-table lookups, 1-8 in flight per lane), 'window'
-        (LDS-staged bucket windows per wavefront), 'slot2/3/4' (slot index)
+        (states between a term's first and last target matched in order), 'slot2/3/4' (slot index)
         or 'low2/4/8' (low keys)."""
         v = _lib.VARIANTS[variant]
         check(_lib.load().qsi_op_set_variant(self._h, v), "qsi_op_set_variant")

@@ -88,8 +88,7 @@ def diagonalise_real(op: GpuOp, opts: Options = Options()):
     the basis size.  The matrix-free solve (mfsparse) builds the basis's low
     keys if it has none (4 bytes per state, kept on the basis) and checks them
     against the operator once (about one apply), so its applies run on the
-    low-key kernel; a basis whose low keys cannot be built keeps the lane
-    kernel.  Every kernel gives the same bits, so the same eigenpairs."""
+    kernels that need no compare.  Every kernel gives the same bits, so the same eigenpairs."""
     import torch
     D = op.rows()
     algo = opts.algorithm or choose_algorithm(D)
@@ -119,9 +118,10 @@ def diagonalise_real(op: GpuOp, opts: Options = Options()):
         op.cache_connectivity(True)
         op.set_variant("cached")
     elif saved in (_lib.QSI_APPLY_AUTO, _lib.QSI_APPLY_CACHED):
-        # matrix-free even when the operator holds a connectivity cache: the
-        # low-key kernel, eight lookups per lane when candidates need no
-        # compare (check mode 2), else four; the lane kernel without low keys
+        # the automatic choice, with the basis's low keys built and checked if
+        # they can be; matrix-free even when the operator holds a connectivity
+        # cache: then the low-key kernel, eight lookups per lane when candidates
+        # need no compare (check mode 2), else four, or the lane kernel
         variant = "lane4"
         try:
             if not op.basis.has_lowkeys():
@@ -129,7 +129,7 @@ def diagonalise_real(op: GpuOp, opts: Options = Options()):
             variant = "low8" if op.verify_lowkeys() == 2 else "low4"
         except _lib.QsiError:
             pass
-        op.set_variant(variant)
+        op.set_variant("auto" if op.connectivity_padding() < 0 else variant)
     try:
         evals, vecs, nconv, _ = op.eigsh(nev=n_eigvals, ncv=ncv, tol=10.0 ** opts.atol,
                                          max_restarts=opts.max_iters, seed=opts.rng_seed,
