@@ -47,10 +47,9 @@ __device__ __forceinline__ double sum_over_groups(double v, int G) {
   return v;
 }
 
-constexpr int kBlkCap = 512;         // LDS flip entries per wavefront and round
+constexpr int kBlkCap = 1024;        // LDS flip entries per wavefront and round
 constexpr int kBlkSuper = 256;       // off-diagonal terms per round (4 masks)
 constexpr int kBlkBatch = 4;         // lookups in flight per lane (phase A)
-constexpr int kBlkPipe = 4;          // X loads in flight per lane (phase B)
 
 __device__ __forceinline__ void blk_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -58,83 +57,143 @@ __device__ __forceinline__ void blk_wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Factor of a diagonal term on state s, without its coefficient.
+template <int NW>
+__device__ __forceinline__ double diag_factor(const DiagTerm& d, const State<NW>& s) {
+  if (d.kind == 0) return diag_ok<NW>(d, s) ? d.sgn * (1 - 2 * parity_notz<NW>(s, d.Z)) : 0.0;
+  int nz = __popcll(d.Z[0]);
+  if constexpr (NW == 2) nz += __popcll(d.Z[1]);
+  return d.sgn * static_cast<double>(2 * popc_and<NW>(s, d.Z) - nz);
+}
+
+// CPL neighbouring columns of one row of X or of the coefficient table (8-byte
+// aligned; two columns are one 16-byte load).
+template <int CPL>
+struct ColVec {
+  double v[CPL];
+};
+template <int CPL>
+__device__ __forceinline__ ColVec<CPL> load_cols(const double* p) {
+  ColVec<CPL> r;
+  __builtin_memcpy(&r, p, sizeof(r));
+  return r;
+}
+
 // Y[:, c] = H_c X[:, c] (or Y += H_c X) for R columns of row-major blocks,
 // and (partials != null) per-wave, per-sector partials of <X[:, c], Y[:, c]>.
 //
 // Each wavefront takes a 64-row tile in two phases per round:
 //   A  one lane per row finds the row's connected terms, looks up the
-//      pre-image ranks BATCH at a time and writes (rank, term, sign)
-//      entries to LDS in term order;
-//   B  G lanes per row (one per column) walk the row's entries and read
-//      X[J, 0:R] as one coalesced segment per connected state.
+//      pre-image ranks BATCH at a time and writes (rank, term or class, sign)
+//      entries to LDS in term order; the lookup keys are the row's bucket key
+//      and state XOR the flip's, staged in LDS;
+//   B  G lanes per row, CPL columns each, walk the row's entries and read X's
+//      row as one coalesced segment per connected state, kPipe entries in
+//      flight.
 // A round covers up to kBlkSuper terms and as many rows as fit kBlkCap LDS
-// entries; partial sums of rows cut by a round boundary go through Y.
+// entries (a whole tile on the lattices up to 72 spins: half as many entries
+// cut most tiles in two, and a round's phase A runs half empty); partial sums
+// of rows cut by a round boundary go through Y.  The classes' column
+// coefficients are read from LDS, one copy per workgroup: the tiles of a
+// workgroup's wavefronts are neighbours, and sectors start at multiples of
+// kBlkWaves tiles, so all its wavefronts are in one sector at a time.  With
+// two columns per lane an odd last column is computed by a lane that repeats
+// the column before it (R >= 2), so every load stays inside its row.
 // Contributions are added in term order, then the diagonal terms in order, so
 // column c's result depends only on X[:, c] and its coefficients.
-template <int NW, int BATCH>
-__global__ __launch_bounds__(kBlkThreads) void k_blk_apply(
+//
+// Bound: phase A is the lookups of a single-vector apply (one column: 366 us
+// at 64 spins, 2.76 M rows, where that apply takes 266), phase B the gather of
+// X's rows through the L2 misses.  64 spins, 1 / 7 / 16 / 64 columns, one
+// (g, B) each: 0.37 / 0.64 / 0.98 / 3.1 ms; 2.00 ms for seven columns when the
+// flip tests' term loads were vector loads (they alone took 300 us), a round
+// held 512 entries, a lane had one column and chose its coefficient in
+// registers.  Four wavefronts per SIMD: with five, the LDS of one workgroup
+// more does not fit and a persistent grid leaves a second wave of workgroups;
+// six at 768 entries a round takes 0.75 ms for seven columns.
+template <int NW, int BATCH, int CPL>
+__global__ __launch_bounds__(kBlkThreads) __attribute__((amdgpu_waves_per_eu(4)))
+void k_blk_apply(
     BlkArgs a, const double* __restrict__ X, double* __restrict__ Y,
     double* __restrict__ partials) {
-  // entry: rank (bits 0-31, kNoRank if absent), term - round base (32-39),
-  // coefficient class (40-47), total sign negative (bit 48)
-  __shared__ uint64_t lds_ent[kBlkWaves][kBlkCap];
+  constexpr int kPipe = 6;
+  // entry: rank (kNoRank if absent); class, or term - round base without
+  // classes (bits 0-7), total sign negative (bit 8)
+  __shared__ uint32_t lds_rank[kBlkWaves][kBlkCap];
+  __shared__ uint16_t lds_meta[kBlkWaves][kBlkCap];
+  __shared__ double coef[kMaxCoefClasses][64];
+  // flip masks, and bucket keys with class and sign, of the sector's first
+  // kBlkSuper terms (later ones are read from the planes)
+  __shared__ uint64_t flip[NW][kBlkSuper];
+  __shared__ uint64_t tkey[kBlkSuper];
   const int lane = threadIdx.x & 63;
   // wave-uniform values kept in scalar registers
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  uint64_t* ent = lds_ent[wv];
+  uint32_t* ent = lds_rank[wv];
+  uint16_t* met = lds_meta[wv];
   const int G = a.G, R = a.R;
   const int lg = __builtin_ctz(G);
-  const int grp = lane >> lg, col = lane & (G - 1);
-  const bool col_ok = col < R;
+  const int grp = lane >> lg;
+  const int c_out = CPL * (lane & (G - 1));           // first column it writes
+  const bool col_ok = c_out < R;
+  const int col = CPL == 1 ? (col_ok ? c_out : 0) : max(0, min(c_out, R - CPL));  // first it reads
+  const int skip = CPL == 1 ? 0 : (col_ok ? c_out - col : 0);  // repeated columns
   const int64_t wave = static_cast<int64_t>(blockIdx.x) * kBlkWaves + wv;
   const int64_t n_waves = static_cast<int64_t>(gridDim.x) * kBlkWaves;
   const int rpp = 64 >> lg;  // rows per phase-B pass
   // tiles are visited in increasing order, so sectors come in order: one
   // running dot product, flushed when the sector changes
-  double dot = 0.0;
+  ColVec<CPL> dot{};
   int flushed = 0;  // sectors [0, flushed) have their partial written
   auto flush_to = [&](int upto, int cur) {
     for (; flushed < upto; ++flushed) {
-      const double v = sum_over_groups(flushed == cur ? dot : 0.0, G);
-      if (partials && grp == 0 && col_ok) partials[(flushed * n_waves + wave) * R + col] = v;
+#pragma unroll
+      for (int u = 0; u < CPL; ++u) {
+        const double v = sum_over_groups(flushed == cur ? dot.v[u] : 0.0, G);
+        if (partials && grp == 0 && col_ok && u >= skip)
+          partials[(flushed * n_waves + wave) * R + col + u] = v;
+      }
     }
   };
   int cur = -1;
-  double cc[kMaxCoefClasses];
-  for (int64_t t = wave; t < a.n_tiles; t += n_waves) {
-    const int s = __builtin_amdgcn_readfirstlane(find_sector(a, t));
+  for (int64_t tb0 = wave - wv; tb0 < a.n_tiles; tb0 += n_waves) {
+    const int s = __builtin_amdgcn_readfirstlane(find_sector(a, tb0));  // the workgroup's
     const BlkSector& S = a.sec[s];
     if (s != cur) {
       flush_to(s, cur);
       cur = s;
-      dot = 0.0;
-      // this lane's column coefficient of every class
-#pragma unroll
-      for (int k = 0; k < kMaxCoefClasses; ++k) {
-        cc[k] = 0.0;
-        if (k < S.n_cls && col_ok) {
-          const CoefClass& K = S.cls[k];
-          cc[k] = (S.coeffs && K.slot >= 0) ? S.coeffs[K.slot * R + col] : K.c;
-        }
+      dot = ColVec<CPL>{};
+      __syncthreads();  // no wavefront still reads the last sector's
+      for (int e = threadIdx.x; e < S.n_cls * R; e += kBlkThreads) {
+        const CoefClass& K = S.cls[e / R];
+        coef[e / R][e % R] = (S.coeffs && K.slot >= 0) ? S.coeffs[K.slot * R + e % R] : K.c;
       }
+      for (int e = threadIdx.x; e < min(S.n_off, kBlkSuper); e += kBlkThreads) {
+#pragma unroll
+        for (int w = 0; w < NW; ++w) flip[w][e] = S.tp.X(w)[e];
+        tkey[e] = S.tp.key()[e];
+      }
+      __syncthreads();
     }
+    const int64_t t = tb0 + wv;
     const int64_t r_begin = (t - S.tile_begin) * kTileRows;
     const int n_rows = static_cast<int>(min<int64_t>(kTileRows, S.b.dim - r_begin));
+    if (t >= a.n_tiles || n_rows <= 0) continue;  // padding tiles
     const bool row_ok = lane < n_rows;
     const State<NW> st = load_state_cached<NW>(S.b.states, r_begin + (row_ok ? lane : 0));
+    const uint32_t ks = bucket_key<NW>(S.b, st);
     const int n_sc = max(1, (S.n_off + kBlkSuper - 1) / kBlkSuper);
     for (int sc = 0; sc < n_sc; ++sc) {
       const int tb = sc * kBlkSuper;
       const int tn = min(kBlkSuper, S.n_off - tb);
-      // connected terms of this lane's row
+      // connected terms of this lane's row: term tb + 64 q + u at bit 63 - u
       uint64_t conn[4];
       int cnt = 0;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        conn[q] = 0;
-        const int qn = row_ok ? min(64, tn - q * 64) : 0;
-        for (int u = 0; u < qn; ++u)
-          conn[q] |= static_cast<uint64_t>(term_ok<NW>(S.off[tb + q * 64 + u], st)) << u;
+        const int qn = min(64, tn - q * 64);
+        conn[q] = qn > 0 ? connect_mask<NW>(S.off + tb + q * 64, qn, st) : 0;
+        if (!row_ok) conn[q] = 0;
         cnt += __popcll(conn[q]);
       }
       int incl = cnt;
@@ -150,30 +209,39 @@ __global__ __launch_bounds__(kBlkThreads) void k_blk_apply(
         // phase A: this lane's connected terms, in term order
         if (lane >= ra && lane < rb && cnt > 0) {
           int pos = excl - base;
+#pragma unroll
           for (int q = 0; q < 4; ++q) {
             uint64_t m = conn[q];
             while (m) {
               State<NW> key[BATCH];
+              uint32_t bk[BATCH], cs[BATCH];
               bool act[BATCH];
               int tl[BATCH];
               uint32_t rk[BATCH];
 #pragma unroll
               for (int g = 0; g < BATCH; ++g) {
                 act[g] = m != 0;
-                tl[g] = q * 64 + (act[g] ? __builtin_ctzll(m) : 0);
-                m &= m - 1;
-                key[g] = xor_state<NW>(st, S.off[tb + tl[g]].X);
+                const int z = act[g] ? __builtin_clzll(m) : 0;
+                tl[g] = q * 64 + z;
+                m &= ~(uint64_t{1} << 63 >> z);
+#pragma unroll
+                for (int w = 0; w < NW; ++w)
+                  key[g].w[w] = st.w[w] ^ (sc == 0 ? flip[w][tl[g]] : S.tp.X(w)[tb + tl[g]]);
+                const uint64_t k = sc == 0 ? tkey[tl[g]] : S.tp.key()[tb + tl[g]];
+                bk[g] = ks ^ static_cast<uint32_t>(k);
+                cs[g] = static_cast<uint32_t>(k >> 32);
               }
-              lookup_batch<NW, BATCH>(S.b, key, act, rk);
+              lookup_batch_at<NW, BATCH>(S.b, key, bk, act, rk);
 #pragma unroll
               for (int g = 0; g < BATCH; ++g) {
                 if (act[g]) {
-                  const OffTerm& T = S.off[tb + tl[g]];
-                  const bool ng = (T.sgn < 0.0) != static_cast<bool>(parity_notz<NW>(st, T.Z));
-                  ent[pos++] = static_cast<uint64_t>(rk[g]) |
-                               (static_cast<uint64_t>(tl[g]) << 32) |
-                               (static_cast<uint64_t>(T.cls & 0xFF) << 40) |
-                               (static_cast<uint64_t>(ng) << 48);
+                  bool ng = cs[g] & TermPlanes::kNegative;
+                  if (cs[g] & TermPlanes::kHasZ)
+                    ng ^= parity_notz<NW>(st, S.off[tb + tl[g]].Z) != 0;
+                  ent[pos] = rk[g];
+                  met[pos] = static_cast<uint16_t>((S.n_cls > 0 ? cs[g] & 255 : tl[g]) |
+                                                   (ng ? 256 : 0));
+                  ++pos;
                 }
               }
             }
@@ -189,62 +257,64 @@ __global__ __launch_bounds__(kBlkThreads) void k_blk_apply(
           const int e1 = __shfl(incl, rs, 64) - base;
           if (r < rb && r < n_rows && col_ok) {
             const int64_t row = S.row_off + r_begin + r;
-            const int64_t gi = a.y_colmajor ? col * a.ldy + row : row * a.ldy + col;
-            double acc = (sc > 0 || a.accumulate) ? Y[gi] : 0.0;
-            // kBlkPipe entries at a time: their X and coefficient loads are
-            // issued together, the sum is taken in entry order
-            for (int e = e0; e < e1; e += kBlkPipe) {
-              uint64_t en[kBlkPipe];
-              bool ok[kBlkPipe];
-              double xj[kBlkPipe], c[kBlkPipe];
+            double* yp[CPL];
+            ColVec<CPL> acc;
 #pragma unroll
-              for (int u = 0; u < kBlkPipe; ++u) {
-                en[u] = e + u < e1 ? ent[e + u] : static_cast<uint64_t>(kNoRank);
-                ok[u] = static_cast<uint32_t>(en[u]) != kNoRank;
+            for (int u = 0; u < CPL; ++u) {
+              yp[u] = Y + (a.y_colmajor ? (col + u) * a.ldy + row : row * a.ldy + col + u);
+              acc.v[u] = (sc > 0 || a.accumulate) && u >= skip ? *yp[u] : 0.0;
+            }
+            for (int e = e0; e < e1; e += kPipe) {
+              uint32_t J[kPipe];
+              uint32_t mt[kPipe];
+              ColVec<CPL> xj[kPipe];
+#pragma unroll
+              for (int u = 0; u < kPipe; ++u) {
+                J[u] = e + u < e1 ? ent[e + u] : kNoRank;
+                mt[u] = e + u < e1 ? met[e + u] : 0u;
               }
 #pragma unroll
-              for (int u = 0; u < kBlkPipe; ++u) {
-                const int64_t J = ok[u] ? static_cast<int64_t>(static_cast<uint32_t>(en[u])) : 0;
-                xj[u] = ok[u] ? X[(S.row_off + J) * a.ldx + col] : 0.0;
+              for (int u = 0; u < kPipe; ++u)
+                xj[u] = J[u] != kNoRank
+                            ? load_cols<CPL>(X + (S.row_off + static_cast<int64_t>(J[u])) * a.ldx + col)
+                            : ColVec<CPL>{};
+#pragma unroll
+              for (int u = 0; u < kPipe; ++u) {
+                if (J[u] == kNoRank) continue;
+                ColVec<CPL> c;
                 if (S.n_cls > 0) {
-                  const int k = static_cast<int>((en[u] >> 40) & 0xFF);
-                  double ck = cc[0];
-#pragma unroll
-                  for (int q = 1; q < kMaxCoefClasses; ++q)
-                    if (k == q) ck = cc[q];
-                  c[u] = ck;
+                  c = load_cols<CPL>(&coef[mt[u] & 255][col]);
                 } else {
-                  const OffTerm& T = S.off[tb + static_cast<int>((en[u] >> 32) & 0xFF)];
-                  c[u] = (S.coeffs && T.slot >= 0) ? S.coeffs[T.slot * R + col] : T.c;
-                }
-              }
+                  const OffTerm& T = S.off[tb + static_cast<int>(mt[u] & 255)];
 #pragma unroll
-              for (int u = 0; u < kBlkPipe; ++u) {
-                if (ok[u] && fabs(xj[u]) > kApplyTol) {
-                  const double cu = ((en[u] >> 48) & 1) ? -c[u] : c[u];
-                  acc += cu * xj[u];
+                  for (int v = 0; v < CPL; ++v)
+                    c.v[v] = (S.coeffs && T.slot >= 0) ? S.coeffs[T.slot * R + col + v] : T.c;
                 }
+#pragma unroll
+                for (int v = 0; v < CPL; ++v)
+                  if (fabs(xj[u].v[v]) > kApplyTol)
+                    acc.v[v] += (mt[u] & 256 ? -c.v[v] : c.v[v]) * xj[u].v[v];
               }
             }
             if (sc == n_sc - 1) {
               const State<NW> sr = load_state_cached<NW>(S.b.states, r_begin + r);
-              const double xi = X[row * a.ldx + col];
+              const ColVec<CPL> xi = load_cols<CPL>(X + row * a.ldx + col);
               for (int k = 0; k < S.n_diag; ++k) {
-                const DiagTerm& d = S.dg[k];
-                double f;
-                if (d.kind == 0) {
-                  f = diag_ok<NW>(d, sr) ? d.sgn * (1 - 2 * parity_notz<NW>(sr, d.Z)) : 0.0;
-                } else {
-                  int nz = __popcll(d.Z[0]);
-                  if constexpr (NW == 2) nz += __popcll(d.Z[1]);
-                  f = d.sgn * static_cast<double>(2 * popc_and<NW>(sr, d.Z) - nz);
+                const DiagTerm d = const_load(S.dg + k);
+                const double f = diag_factor<NW>(d, sr);
+#pragma unroll
+                for (int v = 0; v < CPL; ++v) {
+                  const double c =
+                      (S.coeffs && d.slot >= 0) ? S.coeffs[d.slot * R + col + v] : d.c;
+                  acc.v[v] += c * xi.v[v] * f;
                 }
-                const double c = (S.coeffs && d.slot >= 0) ? S.coeffs[d.slot * R + col] : d.c;
-                acc += c * xi * f;
               }
-              dot += xi * acc;
+#pragma unroll
+              for (int v = 0; v < CPL; ++v) dot.v[v] += xi.v[v] * acc.v[v];
             }
-            Y[gi] = acc;
+#pragma unroll
+            for (int v = 0; v < CPL; ++v)
+              if (v >= skip) *yp[v] = acc.v[v];
           }
         }
         blk_wave_sync();
@@ -428,15 +498,8 @@ __global__ __launch_bounds__(kBlkThreads) void k_blk_capply(
       const State<NW> sr = load_state_cached<NW>(S.b.states, i);
       const double xi = X[row * a.ldx + col];
       for (int k = 0; k < S.n_diag; ++k) {
-        const DiagTerm& d = S.dg[k];
-        double f;
-        if (d.kind == 0) {
-          f = diag_ok<NW>(d, sr) ? d.sgn * (1 - 2 * parity_notz<NW>(sr, d.Z)) : 0.0;
-        } else {
-          int nz = __popcll(d.Z[0]);
-          if constexpr (NW == 2) nz += __popcll(d.Z[1]);
-          f = d.sgn * static_cast<double>(2 * popc_and<NW>(sr, d.Z) - nz);
-        }
+        const DiagTerm d = const_load(S.dg + k);
+        const double f = diag_factor<NW>(d, sr);
         const double c = (S.coeffs && d.slot >= 0) ? S.coeffs[d.slot * R + col] : d.c;
         acc += c * xi * f;
       }
@@ -546,15 +609,8 @@ __global__ __launch_bounds__(kBlkThreads) void k_blk_capply2(
       const State<NW> sr = load_state_cached<NW>(S.b.states, i);
       const double2 xi = *reinterpret_cast<const double2*>(X + row * a.ldx + c0);
       for (int k = 0; k < S.n_diag; ++k) {
-        const DiagTerm& d = S.dg[k];
-        double f;
-        if (d.kind == 0) {
-          f = diag_ok<NW>(d, sr) ? d.sgn * (1 - 2 * parity_notz<NW>(sr, d.Z)) : 0.0;
-        } else {
-          int nz = __popcll(d.Z[0]);
-          if constexpr (NW == 2) nz += __popcll(d.Z[1]);
-          f = d.sgn * static_cast<double>(2 * popc_and<NW>(sr, d.Z) - nz);
-        }
+        const DiagTerm d = const_load(S.dg + k);
+        const double f = diag_factor<NW>(d, sr);
         const bool slot = S.coeffs && d.slot >= 0;
         const double ca = slot ? S.coeffs[d.slot * R + c0] : d.c;
         const double cb = ok1 ? (slot ? S.coeffs[d.slot * R + c0 + 1] : d.c) : 0.0;
@@ -742,8 +798,12 @@ BlkKernel blk_kernel(int nw, bool cached, int cfg, bool pairs) {
     if (nw == 1) return k == 0 ? k_blk_capply<1, 4> : (k == 2 ? k_blk_capply<1, 16> : k_blk_capply<1, 8>);
     return k == 0 ? k_blk_capply<2, 4> : (k == 2 ? k_blk_capply<2, 16> : k_blk_capply<2, 8>);
   }
-  if (nw == 1) return k == 2 ? k_blk_apply<1, 2> : k_blk_apply<1, 4>;
-  return k == 2 ? k_blk_apply<2, 2> : k_blk_apply<2, 4>;
+  if (pairs) {
+    if (nw == 1) return k == 2 ? k_blk_apply<1, 2, 2> : k_blk_apply<1, 6, 2>;
+    return k == 2 ? k_blk_apply<2, 2, 2> : k_blk_apply<2, 4, 2>;
+  }
+  if (nw == 1) return k == 2 ? k_blk_apply<1, 2, 1> : k_blk_apply<1, 6, 1>;
+  return k == 2 ? k_blk_apply<2, 2, 1> : k_blk_apply<2, 4, 1>;
 }
 
 }  // namespace
@@ -767,7 +827,7 @@ int blk_apply_blocks(int nw, int64_t n_tiles, bool cached, int cfg) {
       cu = 256;
     return cu;
   }();
-  const bool pairs = cached && blk_cfg_pairs(cfg);
+  const bool pairs = !cached || blk_cfg_pairs(cfg);
   std::atomic<int>& occ = per_cu[cached ? 1 : 0][nw - 1][blk_cfg_kernel(cfg)][pairs ? 1 : 0];
   int o_cu = occ.load(std::memory_order_relaxed);
   if (o_cu == 0) {
@@ -785,6 +845,16 @@ int blk_apply_blocks(int nw, int64_t n_tiles, bool cached, int cfg) {
 
 int launch_blk_apply(const BlkArgs& a, int nw, int n_blocks, const double* X, double* Y,
                      double* partials, hipStream_t s) {
+  if (!blk_cached(a) && a.R >= 2) {
+    // two columns per lane, a power of two of lanes per row
+    BlkArgs b = a;
+    b.G = 1;
+    while (2 * b.G < a.R) b.G <<= 1;
+    hipLaunchKernelGGL(blk_kernel(nw, false, a.cfg, true), dim3(n_blocks), dim3(kBlkThreads), 0,
+                       s, b, X, Y, partials);
+    QSI_CHECK_LAUNCH();
+    return QSI_OK;
+  }
   if (blk_pairs(a, X)) {
     // ceil(R / 2) lanes per row; a power of two when the partials cross
     // row groups by butterfly
@@ -924,6 +994,7 @@ BlkArgs sector_args(const qsi_op_t* ops, int n_sectors, int R, const double* con
     BlkSector& S = args.sec[s];
     S.b = op->basis->view();
     S.off = op->d_off;
+    S.tp = op->planes();
     S.dg = op->d_diag;
     S.cls = op->d_cls;
     S.n_cls = op->n_cls;
@@ -935,7 +1006,8 @@ BlkArgs sector_args(const qsi_op_t* ops, int n_sectors, int R, const double* con
     S.coeffs = d_coeffs ? d_coeffs[s] : nullptr;
     S.tile_begin = tiles;
     S.row_off = rows;
-    tiles += (op->basis->dim + kTileRows - 1) / kTileRows;
+    // whole workgroups of tiles (the last ones may be empty)
+    tiles += (op->basis->dim + kTileRows * kBlkWaves - 1) / (kTileRows * kBlkWaves) * kBlkWaves;
     rows += op->basis->dim;
   }
   args.n_tiles = tiles;

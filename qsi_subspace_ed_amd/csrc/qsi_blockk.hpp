@@ -20,13 +20,14 @@ constexpr int kMaxSectors = 8;
 struct BlkSector {
   BasisView b;
   const OffTerm* off;
+  TermPlanes tp;
   const DiagTerm* dg;
   const double* coeffs;  // n_slots x R, or null
   const CoefClass* cls;  // coefficient classes of the off-diagonal terms
   int n_cls;             // 0: per-term coefficients
   int n_off;
   int n_diag;
-  int64_t tile_begin;  // first global tile of this sector
+  int64_t tile_begin;  // first global tile of this sector, a multiple of kBlkWaves
   int64_t row_off;     // first row of this sector in the concatenated blocks
   // cached connectivity of the operator, or null (see qsi_op_s)
   const uint64_t* rowptr;

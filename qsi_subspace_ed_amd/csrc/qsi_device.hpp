@@ -38,9 +38,25 @@ struct TermMV {
 };
 static_assert(offsetof(OffTerm, m) == 0 && offsetof(OffTerm, v) == sizeof(TermMV::m),
               "OffTerm must start with its m and v words");
+// *p from memory that no kernel writes while it runs (term tables), read as
+// constant memory: at a wave-uniform address that is a scalar load even where
+// the pointer comes out of a kernel argument structure, about which the compiler
+// cannot know that the kernel's stores leave it alone (it would load every term
+// into vector registers, 256 vector loads per 64-row tile of a 64-spin basis).
+template <typename T>
+__device__ __forceinline__ T const_load(const T* p) {
+  static_assert(sizeof(T) % 8 == 0 && alignof(T) >= 8);
+  const auto* w = (const __attribute__((address_space(4))) uint64_t*)p;
+  uint64_t word[sizeof(T) / 8];
+#pragma unroll
+  for (unsigned i = 0; i < sizeof(T) / 8; ++i) word[i] = w[i];
+  T out;
+  __builtin_memcpy(&out, word, sizeof(T));
+  return out;
+}
 template <int NW>
 __device__ __forceinline__ TermMV load_mv(const OffTerm* __restrict__ t) {
-  return *reinterpret_cast<const TermMV*>(t);
+  return const_load(reinterpret_cast<const TermMV*>(t));
 }
 
 // Lanes of the wavefront whose s & m (u) equals v.
@@ -153,15 +169,17 @@ constexpr uint32_t kNoRank = 0xFFFFFFFFu;
 // that reads each loaded value after the last load keeps the compiler from
 // moving a use next to its load (which would make each load wait for the
 // one before).
+// bk: the keys' bucket keys.
 template <int NW, int B>
-__device__ __forceinline__ void lookup_batch(const BasisView& b, const State<NW>* key,
-                                             const bool* act, uint32_t* rank) {
+__device__ __forceinline__ void lookup_batch_at(const BasisView& b, const State<NW>* key,
+                                                const uint32_t* bk, const bool* act,
+                                                uint32_t* rank) {
   uint32_t lo[B], n[B];
   uint2 p[B];
 #pragma unroll
   for (int g = 0; g < B; ++g) {
     p[g] = make_uint2(0u, 0u);
-    if (act[g]) __builtin_memcpy(&p[g], b.table + bucket_key<NW>(b, key[g]), sizeof(uint2));
+    if (act[g]) __builtin_memcpy(&p[g], b.table + bk[g], sizeof(uint2));
   }
 #pragma unroll
   for (int g = 0; g < B; ++g) asm volatile("" : "+v"(p[g].x), "+v"(p[g].y));
@@ -204,6 +222,15 @@ __device__ __forceinline__ void lookup_batch(const BasisView& b, const State<NW>
     for (int w = 0; w < NW; ++w) asm volatile("" : "+v"(f[g].w[w]));
 #pragma unroll
   for (int g = 0; g < B; ++g) rank[g] = n[g] == 1 && st_eq<NW>(f[g], key[g]) ? lo[g] : kNoRank;
+}
+
+template <int NW, int B>
+__device__ __forceinline__ void lookup_batch(const BasisView& b, const State<NW>* key,
+                                             const bool* act, uint32_t* rank) {
+  uint32_t bk[B];
+#pragma unroll
+  for (int g = 0; g < B; ++g) bk[g] = bucket_key<NW>(b, key[g]);
+  lookup_batch_at<NW, B>(b, key, bk, act, rank);
 }
 
 }  // namespace qsi

@@ -3278,8 +3278,12 @@ int qsi_op_create(qsi_basis_t b, const qsi_term_t* terms, int n_terms,
     const double cs = o.c * o.sgn;
     uint64_t cw;
     std::memcpy(&cw, &cs, sizeof(cw));
-    const uint64_t bk = nw == 1 ? bucket_key<1>(b->view(), State<1>{{o.X[0]}})
-                                : bucket_key<2>(b->view(), State<2>{{o.X[0], o.X[1]}});
+    const uint32_t info = (o.cls >= 0 ? static_cast<uint32_t>(o.cls) : 0u) |
+                          (o.sgn < 0.0 ? TermPlanes::kNegative : 0u) |
+                          ((o.Z[0] | o.Z[1]) ? TermPlanes::kHasZ : 0u);
+    const uint64_t bk = static_cast<uint64_t>(info) << 32 |
+                        (nw == 1 ? bucket_key<1>(b->view(), State<1>{{o.X[0]}})
+                                 : bucket_key<2>(b->view(), State<2>{{o.X[0], o.X[1]}}));
     const uint64_t field[TermPlanes::kCount] = {o.m[0], o.v[0], o.X[0], o.m[1],
                                                 o.v[1], o.X[1], bk};
     for (int q = 0; q < TermPlanes::kCount; ++q)
@@ -3512,6 +3516,7 @@ int qsi_op_apply_block(qsi_op_t op, const double* d_X, int64_t ldx, double* d_Y,
   a.y_colmajor = 0;
   a.sec[0].b = op->basis->view();
   a.sec[0].off = op->d_off;
+  a.sec[0].tp = op->planes();
   a.sec[0].dg = op->d_diag;
   a.sec[0].cls = op->d_cls;
   a.sec[0].n_cls = op->n_cls;

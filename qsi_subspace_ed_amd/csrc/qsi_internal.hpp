@@ -67,10 +67,12 @@ static_assert(sizeof(TermRec<1>) == 32 && sizeof(TermRec<2>) == 64, "4 or 8 word
 
 // The off-diagonal terms field by field, n entries each (a multiple of 64, the
 // tail zero), so a wavefront's lanes read one field of 64 terms with one
-// coalesced load (projector mask, value and flip mask per word, and the flip
-// mask's bucket key), and then as TermRec records.
+// coalesced load (projector mask, value and flip mask per word; the flip mask's
+// bucket key with the term's class, sign and whether it has a Z string in the
+// upper half), and then as TermRec records.
 struct TermPlanes {
   static constexpr int kCount = 7;
+  static constexpr uint32_t kNegative = 256, kHasZ = 512;  // class in bits 0-7
   const uint64_t* p;
   int n;
   __host__ __device__ const uint64_t* m(int w) const { return p + (3 * w) * n; }

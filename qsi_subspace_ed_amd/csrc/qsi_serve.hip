@@ -704,6 +704,7 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
   a.y_colmajor = 1;
   a.sec[0].b = op->basis->view();
   a.sec[0].off = op->d_off;
+  a.sec[0].tp = op->planes();
   a.sec[0].dg = op->d_diag;
   a.sec[0].cls = op->d_cls;
   a.sec[0].n_cls = op->n_cls;
