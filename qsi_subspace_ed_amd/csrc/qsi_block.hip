@@ -5,18 +5,19 @@
 // recurrence (components/linalg_routines/src/lanczos.cpp:111-146, without the
 // convergence checks) side by side, M steps, no reorthogonalisation, which is
 // what FTLM needs: the (alpha, beta) coefficients of every sample.  Sectors of
-// different basis size share each launch: their rows are cut into tiles of 64
+// different basis size share each launch: their rows are cut into tiles
 // and one persistent grid of wavefronts walks the concatenated tile list, so
 // each basis state's flip tests and rank lookups serve all R columns.
 //
 // Per step (three rotating D x R blocks holding v_{j-1}, v_j unnormalised,
 // A = w_{j-1}, B = w_j with v = scale * column, and C):
-//   k_blk_apply      C = H B, per-wave partials of <B_c, C_c>
+//   k_blk_apply      C = H B, per-workgroup partials of <B_c, C_c>
 //   k_blk_finalize   alpha[s][c] = scale_B^2 <B_c, C_c>
-//   k_blk_update     C = scale_B (C - alpha B) - beta scale_A A, partials of |C_c|^2
-//   k_blk_finalize   beta[s][c] = |C_c|, scale_C = 1/beta (0 when beta underflows)
-//   k_blk_step       history index += 1;  then (A, B, C) <- (B, C, A)
-// No pass rewrites a block to normalise it.  The five launches of a step are
+//   k_blk_update     C = scale_B (C - alpha B) - beta scale_A A, partials of |C_c|^2,
+//                    history index += 1
+//   k_blk_finalize   beta[s][c] = |C_c|, scale_C = 1/beta (0 when beta underflows);
+//                    then (A, B, C) <- (B, C, A)
+// No pass rewrites a block to normalise it.  The four launches of a step are
 // captured once per rotation phase as a HIP graph and replayed.
 #include <hip/hip_runtime.h>
 
@@ -47,6 +48,18 @@ __device__ __forceinline__ double sum_over_groups(double v, int G) {
   return v;
 }
 
+constexpr int kBlkVecBlocks = 2048;  // workgroups of a vector pass
+// A tile is one wavefront's work.  With 64 rows each, a 48-spin sector (87 546
+// rows) is 1368 wavefronts on 1024 SIMDs, each waiting for one gather after the
+// other, so smaller bases are cut finer: down to the rows of one pass and no
+// further than kTileRowsMin, until there are kBlkFill* tiles.  48 spins, cached:
+// 16 columns 47 -> 24 us, 64 columns 169 -> 76 us; at 2.76 M rows the tiles stay
+// whole.  The searching kernel finds the entries with one lane per row, so short
+// tiles leave its lanes idle: 64 columns 195 us whole, 138 us cut for 4096 tiles,
+// and a two-sector recurrence of 16 columns (131 us a step) takes 187 us when
+// cut for 16384.
+constexpr int kTileRowsMin = 8;
+constexpr int64_t kBlkFillSearch = 4096, kBlkFillCached = 32768;
 constexpr int kBlkCap = 1024;        // LDS flip entries per wavefront and round
 constexpr int kBlkSuper = 256;       // off-diagonal terms per round (4 masks)
 constexpr int kBlkBatch = 4;         // lookups in flight per lane (phase A)
@@ -79,10 +92,63 @@ __device__ __forceinline__ ColVec<CPL> load_cols(const double* p) {
   return r;
 }
 
+// A wavefront's place in a row-major block: G lanes per row, CPL neighbouring
+// columns each.  An odd last column is computed by a lane that also reads the
+// column before it and leaves that one alone (R >= 2), so every load stays
+// inside its row.
+template <int CPL>
+struct ColLane {
+  int grp;    // row within the pass
+  int col;    // first column it reads
+  int skip;   // leading columns that another lane writes
+  int rpp;    // rows per pass
+  bool ok;    // it has a column and a row
+  __device__ __forceinline__ ColLane(int lane, int G, int R) {
+    grp = lane / G;
+    rpp = 64 / G;
+    const int c = CPL * (lane % G);
+    ok = c < R && grp < rpp;
+    col = CPL == 1 ? (ok ? c : 0) : max(0, min(c, R - CPL));
+    skip = CPL == 1 ? 0 : (ok ? c - col : 0);
+  }
+};
+
+// out[c] = the workgroup's sum of column c's v: over the row groups by
+// butterfly (G a power of two), over the wavefronts in order through LDS.
+// Every thread of the workgroup calls it.
+template <int CPL>
+__device__ __forceinline__ void store_partials(double (&red)[kBlkWaves][64], const ColLane<CPL>& q,
+                                               int G, int R, const ColVec<CPL>& v,
+                                               double* __restrict__ out) {
+#pragma unroll
+  for (int u = 0; u < CPL; ++u) {
+    const double t = sum_over_groups(v.v[u], G);
+    if (q.grp == 0 && q.ok && u >= q.skip) red[threadIdx.x >> 6][q.col + u] = t;
+  }
+  __syncthreads();
+  if (static_cast<int>(threadIdx.x) < R) {
+    double t = red[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < kBlkWaves; ++w) t += red[w][threadIdx.x];
+    out[threadIdx.x] = t;
+  }
+  __syncthreads();
+}
+
+// coef[k][c] = column c's coefficient of class k, by the whole workgroup.
+__device__ __forceinline__ void load_coefs(double (&coef)[kMaxCoefClasses][64], const BlkSector& S,
+                                           int R) {
+  for (int e = threadIdx.x; e < S.n_cls * R; e += kBlkThreads) {
+    const CoefClass& K = S.cls[e / R];
+    coef[e / R][e % R] = (S.coeffs && K.slot >= 0) ? S.coeffs[K.slot * R + e % R] : K.c;
+  }
+}
+
 // Y[:, c] = H_c X[:, c] (or Y += H_c X) for R columns of row-major blocks,
-// and (partials != null) per-wave, per-sector partials of <X[:, c], Y[:, c]>.
+// and (partials != null) per-workgroup, per-sector partials of
+// <X[:, c], Y[:, c]>.
 //
-// Each wavefront takes a 64-row tile in two phases per round:
+// Each wavefront takes a tile of up to 64 rows in two phases per round:
 //   A  one lane per row finds the row's connected terms, looks up the
 //      pre-image ranks BATCH at a time and writes (rank, term or class, sign)
 //      entries to LDS in term order; the lookup keys are the row's bucket key
@@ -96,9 +162,7 @@ __device__ __forceinline__ ColVec<CPL> load_cols(const double* p) {
 // of rows cut by a round boundary go through Y.  The classes' column
 // coefficients are read from LDS, one copy per workgroup: the tiles of a
 // workgroup's wavefronts are neighbours, and sectors start at multiples of
-// kBlkWaves tiles, so all its wavefronts are in one sector at a time.  With
-// two columns per lane an odd last column is computed by a lane that repeats
-// the column before it (R >= 2), so every load stays inside its row.
+// kBlkWaves tiles, so all its wavefronts are in one sector at a time.
 // Contributions are added in term order, then the diagonal terms in order, so
 // column c's result depends only on X[:, c] and its coefficients.
 //
@@ -131,32 +195,24 @@ void k_blk_apply(
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   uint32_t* ent = lds_rank[wv];
   uint16_t* met = lds_meta[wv];
+  __shared__ double red[kBlkWaves][64];
   const int G = a.G, R = a.R;
-  const int lg = __builtin_ctz(G);
-  const int grp = lane >> lg;
-  const int c_out = CPL * (lane & (G - 1));           // first column it writes
-  const bool col_ok = c_out < R;
-  const int col = CPL == 1 ? (col_ok ? c_out : 0) : max(0, min(c_out, R - CPL));  // first it reads
-  const int skip = CPL == 1 ? 0 : (col_ok ? c_out - col : 0);  // repeated columns
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * kBlkWaves + wv;
+  const ColLane<CPL> q(lane, G, R);
+  const int grp = q.grp, col = q.col, skip = q.skip, rpp = q.rpp;
+  const bool col_ok = q.ok;
   const int64_t n_waves = static_cast<int64_t>(gridDim.x) * kBlkWaves;
-  const int rpp = 64 >> lg;  // rows per phase-B pass
   // tiles are visited in increasing order, so sectors come in order: one
-  // running dot product, flushed when the sector changes
+  // running dot product, flushed when the workgroup's sector changes
   ColVec<CPL> dot{};
   int flushed = 0;  // sectors [0, flushed) have their partial written
   auto flush_to = [&](int upto, int cur) {
-    for (; flushed < upto; ++flushed) {
-#pragma unroll
-      for (int u = 0; u < CPL; ++u) {
-        const double v = sum_over_groups(flushed == cur ? dot.v[u] : 0.0, G);
-        if (partials && grp == 0 && col_ok && u >= skip)
-          partials[(flushed * n_waves + wave) * R + col + u] = v;
-      }
-    }
+    for (; partials && flushed < upto; ++flushed)
+      store_partials(red, q, G, R, flushed == cur ? dot : ColVec<CPL>{},
+                     partials + (static_cast<int64_t>(flushed) * gridDim.x + blockIdx.x) * R);
   };
   int cur = -1;
-  for (int64_t tb0 = wave - wv; tb0 < a.n_tiles; tb0 += n_waves) {
+  for (int64_t tb0 = static_cast<int64_t>(blockIdx.x) * kBlkWaves; tb0 < a.n_tiles;
+       tb0 += n_waves) {
     const int s = __builtin_amdgcn_readfirstlane(find_sector(a, tb0));  // the workgroup's
     const BlkSector& S = a.sec[s];
     if (s != cur) {
@@ -164,10 +220,7 @@ void k_blk_apply(
       cur = s;
       dot = ColVec<CPL>{};
       __syncthreads();  // no wavefront still reads the last sector's
-      for (int e = threadIdx.x; e < S.n_cls * R; e += kBlkThreads) {
-        const CoefClass& K = S.cls[e / R];
-        coef[e / R][e % R] = (S.coeffs && K.slot >= 0) ? S.coeffs[K.slot * R + e % R] : K.c;
-      }
+      load_coefs(coef, S, R);
       for (int e = threadIdx.x; e < min(S.n_off, kBlkSuper); e += kBlkThreads) {
 #pragma unroll
         for (int w = 0; w < NW; ++w) flip[w][e] = S.tp.X(w)[e];
@@ -176,8 +229,8 @@ void k_blk_apply(
       __syncthreads();
     }
     const int64_t t = tb0 + wv;
-    const int64_t r_begin = (t - S.tile_begin) * kTileRows;
-    const int n_rows = static_cast<int>(min<int64_t>(kTileRows, S.b.dim - r_begin));
+    const int64_t r_begin = (t - S.tile_begin) * a.tile_rows;
+    const int n_rows = static_cast<int>(min<int64_t>(a.tile_rows, S.b.dim - r_begin));
     if (t >= a.n_tiles || n_rows <= 0) continue;  // padding tiles
     const bool row_ok = lane < n_rows;
     const State<NW> st = load_state_cached<NW>(S.b.states, r_begin + (row_ok ? lane : 0));
@@ -420,207 +473,97 @@ __device__ __forceinline__ void load_entries(const BlkSector& S, uint64_t e, uin
 }
 
 // The block apply over cached connectivity: same arithmetic, order and
-// results as k_blk_apply.  G lanes per row (one per column), PIPE entries'
+// results as k_blk_apply.  G lanes per row, CPL columns each, PIPE entries'
 // gathers in flight.  G may be any width up to 64 when no partials are asked
 // for (a wavefront then serves floor(64 / G) rows per pass); with partials it
 // must be a power of two (the per-column sums cross row groups by butterfly).
-template <int NW, int PIPE>
+// The class's coefficients come from LDS: one read of CPL columns instead of a
+// choice among eight registers per column and entry (2.76 M rows of 64 spins, 16
+// columns in pairs 0.87 -> 0.68 ms, 64 columns 3.4 -> 2.7 ms; then bound by the
+// gathers' L2 misses, 15.5 GB of X's rows at 5.7 TB/s).
+template <int NW, int PIPE, int CPL>
 __global__ __launch_bounds__(kBlkThreads) void k_blk_capply(
     BlkArgs a, const double* __restrict__ X, double* __restrict__ Y,
     double* __restrict__ partials) {
+  __shared__ double coef[kMaxCoefClasses][64];
+  __shared__ double red[kBlkWaves][64];
   const int lane = threadIdx.x & 63;
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int G = a.G, R = a.R;
-  const int grp = lane / G, col = lane % G;
-  const int rpp = 64 / G;
-  const bool col_ok = col < R && grp < rpp;
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * kBlkWaves + wv;
+  const ColLane<CPL> q(lane, G, R);
+  const int col = q.col;
   const int64_t n_waves = static_cast<int64_t>(gridDim.x) * kBlkWaves;
-  double dot = 0.0;
+  ColVec<CPL> dot{};
   int flushed = 0;
   auto flush_to = [&](int upto, int cur) {
-    for (; flushed < upto; ++flushed) {
-      if (!partials) continue;
-      const double v = sum_over_groups(flushed == cur ? dot : 0.0, G);
-      if (grp == 0 && col_ok) partials[(flushed * n_waves + wave) * R + col] = v;
-    }
+    for (; partials && flushed < upto; ++flushed)
+      store_partials(red, q, G, R, flushed == cur ? dot : ColVec<CPL>{},
+                     partials + (static_cast<int64_t>(flushed) * gridDim.x + blockIdx.x) * R);
   };
   int cur = -1;
-  double cc[kMaxCoefClasses];
-  for (int64_t t = wave; t < a.n_tiles; t += n_waves) {
-    const int s = __builtin_amdgcn_readfirstlane(find_sector(a, t));
+  for (int64_t tb0 = static_cast<int64_t>(blockIdx.x) * kBlkWaves; tb0 < a.n_tiles;
+       tb0 += n_waves) {
+    const int s = __builtin_amdgcn_readfirstlane(find_sector(a, tb0));  // the workgroup's
     const BlkSector& S = a.sec[s];
     if (s != cur) {
       flush_to(s, cur);
       cur = s;
-      dot = 0.0;
-#pragma unroll
-      for (int k = 0; k < kMaxCoefClasses; ++k) {
-        cc[k] = 0.0;
-        if (k < S.n_cls && col_ok) {
-          const CoefClass& K = S.cls[k];
-          cc[k] = (S.coeffs && K.slot >= 0) ? S.coeffs[K.slot * R + col] : K.c;
-        }
-      }
+      dot = ColVec<CPL>{};
+      __syncthreads();  // no wavefront still reads the last sector's
+      load_coefs(coef, S, R);
+      __syncthreads();
     }
-    const int64_t r_begin = (t - S.tile_begin) * kTileRows;
-    const int n_rows = static_cast<int>(min<int64_t>(kTileRows, S.b.dim - r_begin));
-    const int n_pass = (n_rows + rpp - 1) / rpp;
-    for (int p = 0; p < n_pass; ++p) {
-      const int r = p * rpp + grp;
-      if (r >= n_rows || !col_ok) continue;
+    const int64_t t = tb0 + wv;
+    const int64_t r_begin = (t - S.tile_begin) * a.tile_rows;
+    const int n_rows = static_cast<int>(min<int64_t>(a.tile_rows, S.b.dim - r_begin));
+    if (t >= a.n_tiles || n_rows <= 0 || !q.ok) continue;  // padding tiles
+    for (int r = q.grp; r < n_rows; r += q.rpp) {
       const int64_t i = r_begin + r;
       const int64_t row = S.row_off + i;
-      const int64_t gi = a.y_colmajor ? col * a.ldy + row : row * a.ldy + col;
-      double acc = a.accumulate ? Y[gi] : 0.0;
+      double* yp[CPL];
+      ColVec<CPL> acc;
+#pragma unroll
+      for (int u = 0; u < CPL; ++u) {
+        yp[u] = Y + (a.y_colmajor ? (col + u) * a.ldy + row : row * a.ldy + col + u);
+        acc.v[u] = a.accumulate && u >= q.skip ? *yp[u] : 0.0;
+      }
       const uint64_t e0 = S.rowptr[i], e1 = S.rowptr[i + 1];
       for (uint64_t e = e0 & ~uint64_t{3}; e < e1; e += PIPE) {
         uint32_t J[PIPE];
         uint8_t mt[PIPE];
-        double xj[PIPE];
-        load_entries<PIPE>(S, e, e0, e1, J, mt);
-#pragma unroll
-        for (int u = 0; u < PIPE; ++u)
-          xj[u] = J[u] != kNoRank ? X[(S.row_off + static_cast<int64_t>(J[u])) * a.ldx + col] : 0.0;
-#pragma unroll
-        for (int u = 0; u < PIPE; ++u) {
-          if (J[u] != kNoRank && fabs(xj[u]) > kApplyTol) {
-            const int k = mt[u] & 0x7F;
-            double c = cc[0];
-#pragma unroll
-            for (int q = 1; q < kMaxCoefClasses; ++q)
-              if (k == q) c = cc[q];
-            if (mt[u] & 0x80) c = -c;
-            acc += c * xj[u];
-          }
-        }
-      }
-      const State<NW> sr = load_state_cached<NW>(S.b.states, i);
-      const double xi = X[row * a.ldx + col];
-      for (int k = 0; k < S.n_diag; ++k) {
-        const DiagTerm d = const_load(S.dg + k);
-        const double f = diag_factor<NW>(d, sr);
-        const double c = (S.coeffs && d.slot >= 0) ? S.coeffs[d.slot * R + col] : d.c;
-        acc += c * xi * f;
-      }
-      dot += xi * acc;
-      Y[gi] = acc;
-    }
-  }
-  flush_to(a.n_sec, cur);
-}
-
-// Column pairs: each lane of a row group serves columns c0 = 2q and c0 + 1
-// with one 16-byte gather per entry, so a wavefront covers twice the rows per
-// pass of k_blk_capply for the same number of memory instructions (G here is
-// the number of lanes per row, ceil(R / 2), a power of two when partials are
-// asked for).  Needs 16-byte aligned rows of X that hold both columns of
-// every lane: even ldx >= R rounded up to even.  Per column the arithmetic
-// and its order are those of k_blk_capply, so Y is identical; partials sum
-// the row groups in another order.
-template <int NW, int PIPE>
-__global__ __launch_bounds__(kBlkThreads) void k_blk_capply2(
-    BlkArgs a, const double* __restrict__ X, double* __restrict__ Y,
-    double* __restrict__ partials) {
-  const int lane = threadIdx.x & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int G = a.G, R = a.R;
-  const int grp = lane / G, c0 = 2 * (lane % G);
-  const int rpp = 64 / G;
-  const bool ok0 = c0 < R && grp < rpp;
-  const bool ok1 = ok0 && c0 + 1 < R;
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * kBlkWaves + wv;
-  const int64_t n_waves = static_cast<int64_t>(gridDim.x) * kBlkWaves;
-  double dot0 = 0.0, dot1 = 0.0;
-  int flushed = 0;
-  auto flush_to = [&](int upto, int cur) {
-    for (; flushed < upto; ++flushed) {
-      if (!partials) continue;
-      const double v0 = sum_over_groups(flushed == cur ? dot0 : 0.0, G);
-      const double v1 = sum_over_groups(flushed == cur ? dot1 : 0.0, G);
-      if (grp == 0 && ok0) partials[(flushed * n_waves + wave) * R + c0] = v0;
-      if (grp == 0 && ok1) partials[(flushed * n_waves + wave) * R + c0 + 1] = v1;
-    }
-  };
-  int cur = -1;
-  double cc0[kMaxCoefClasses], cc1[kMaxCoefClasses];
-  for (int64_t t = wave; t < a.n_tiles; t += n_waves) {
-    const int s = __builtin_amdgcn_readfirstlane(find_sector(a, t));
-    const BlkSector& S = a.sec[s];
-    if (s != cur) {
-      flush_to(s, cur);
-      cur = s;
-      dot0 = dot1 = 0.0;
-#pragma unroll
-      for (int k = 0; k < kMaxCoefClasses; ++k) {
-        cc0[k] = cc1[k] = 0.0;
-        if (k < S.n_cls) {
-          const CoefClass& K = S.cls[k];
-          const bool slot = S.coeffs && K.slot >= 0;
-          if (ok0) cc0[k] = slot ? S.coeffs[K.slot * R + c0] : K.c;
-          if (ok1) cc1[k] = slot ? S.coeffs[K.slot * R + c0 + 1] : K.c;
-        }
-      }
-    }
-    const int64_t r_begin = (t - S.tile_begin) * kTileRows;
-    const int n_rows = static_cast<int>(min<int64_t>(kTileRows, S.b.dim - r_begin));
-    const int n_pass = (n_rows + rpp - 1) / rpp;
-    for (int p = 0; p < n_pass; ++p) {
-      const int r = p * rpp + grp;
-      if (r >= n_rows || !ok0) continue;
-      const int64_t i = r_begin + r;
-      const int64_t row = S.row_off + i;
-      const int64_t g0 = a.y_colmajor ? c0 * a.ldy + row : row * a.ldy + c0;
-      const int64_t g1 = a.y_colmajor ? g0 + a.ldy : g0 + 1;
-      double acc0 = a.accumulate ? Y[g0] : 0.0;
-      double acc1 = a.accumulate && ok1 ? Y[g1] : 0.0;
-      const uint64_t e0 = S.rowptr[i], e1 = S.rowptr[i + 1];
-      for (uint64_t e = e0 & ~uint64_t{3}; e < e1; e += PIPE) {
-        uint32_t J[PIPE];
-        uint8_t mt[PIPE];
-        double2 xj[PIPE];
+        ColVec<CPL> xj[PIPE];
         load_entries<PIPE>(S, e, e0, e1, J, mt);
 #pragma unroll
         for (int u = 0; u < PIPE; ++u)
           xj[u] = J[u] != kNoRank
-                      ? *reinterpret_cast<const double2*>(
-                            X + (S.row_off + static_cast<int64_t>(J[u])) * a.ldx + c0)
-                      : make_double2(0.0, 0.0);
+                      ? load_cols<CPL>(X + (S.row_off + static_cast<int64_t>(J[u])) * a.ldx + col)
+                      : ColVec<CPL>{};
 #pragma unroll
         for (int u = 0; u < PIPE; ++u) {
-          if (J[u] != kNoRank) {
-            const int k = mt[u] & 0x7F;
-            double ca = cc0[0], cb = cc1[0];
+          if (J[u] == kNoRank) continue;
+          const ColVec<CPL> c = load_cols<CPL>(&coef[mt[u] & 0x7F][col]);
 #pragma unroll
-            for (int q = 1; q < kMaxCoefClasses; ++q)
-              if (k == q) {
-                ca = cc0[q];
-                cb = cc1[q];
-              }
-            if (mt[u] & 0x80) {
-              ca = -ca;
-              cb = -cb;
-            }
-            if (fabs(xj[u].x) > kApplyTol) acc0 += ca * xj[u].x;
-            if (fabs(xj[u].y) > kApplyTol) acc1 += cb * xj[u].y;
-          }
+          for (int v = 0; v < CPL; ++v)
+            if (fabs(xj[u].v[v]) > kApplyTol)
+              acc.v[v] += (mt[u] & 0x80 ? -c.v[v] : c.v[v]) * xj[u].v[v];
         }
       }
       const State<NW> sr = load_state_cached<NW>(S.b.states, i);
-      const double2 xi = *reinterpret_cast<const double2*>(X + row * a.ldx + c0);
+      const ColVec<CPL> xi = load_cols<CPL>(X + row * a.ldx + col);
       for (int k = 0; k < S.n_diag; ++k) {
         const DiagTerm d = const_load(S.dg + k);
         const double f = diag_factor<NW>(d, sr);
-        const bool slot = S.coeffs && d.slot >= 0;
-        const double ca = slot ? S.coeffs[d.slot * R + c0] : d.c;
-        const double cb = ok1 ? (slot ? S.coeffs[d.slot * R + c0 + 1] : d.c) : 0.0;
-        acc0 += ca * xi.x * f;
-        acc1 += cb * xi.y * f;
+#pragma unroll
+        for (int v = 0; v < CPL; ++v) {
+          const double c = (S.coeffs && d.slot >= 0) ? S.coeffs[d.slot * R + col + v] : d.c;
+          acc.v[v] += c * xi.v[v] * f;
+        }
       }
-      dot0 += xi.x * acc0;
-      dot1 += xi.y * acc1;
-      Y[g0] = acc0;
-      if (ok1) Y[g1] = acc1;
+#pragma unroll
+      for (int v = 0; v < CPL; ++v) {
+        dot.v[v] += xi.v[v] * acc.v[v];
+        if (v >= q.skip) *yp[v] = acc.v[v];
+      }
     }
   }
   flush_to(a.n_sec, cur);
@@ -628,106 +571,127 @@ __global__ __launch_bounds__(kBlkThreads) void k_blk_capply2(
 
 // C = fb C - alpha fb B - beta fa A per column (fb, fa: the scales sB, sA of
 // the unnormalised blocks B and A, 1 when null; beta, A skipped when A is
-// null); |C_c|^2 partials.
+// null); |C_c|^2 partials per workgroup and sector.  Advances step (if given).
 __global__ __launch_bounds__(kBlkThreads) void k_blk_update(
     BlkArgs a, const double* __restrict__ A, const double* B,
     double* C, const double* __restrict__ alpha,
     const double* __restrict__ beta, double* __restrict__ partials,
-    const double* __restrict__ sA, const double* __restrict__ sB) {
-  const int lane = threadIdx.x & 63;
+    const double* __restrict__ sA, const double* __restrict__ sB, int* __restrict__ step) {
+  __shared__ double red[kBlkWaves][64];
   const int G = a.G, R = a.R;
-  const int grp = lane / G, col = lane % G;
-  const bool col_ok = col < R;
-  const int64_t wave = static_cast<int64_t>(blockIdx.x) * kBlkWaves + (threadIdx.x >> 6);
+  const ColLane<1> q(threadIdx.x & 63, G, R);
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int64_t n_waves = static_cast<int64_t>(gridDim.x) * kBlkWaves;
-  const int rows_per_pass = 64 / G;
-  double nrm[kMaxSectors];
-#pragma unroll
-  for (int k = 0; k < kMaxSectors; ++k) nrm[k] = 0.0;
-  for (int64_t t = wave; t < a.n_tiles; t += n_waves) {
-    const int s = find_sector(a, t);
+  ColVec<1> nrm{};
+  int flushed = 0;
+  auto flush_to = [&](int upto, int cur) {
+    for (; flushed < upto; ++flushed)
+      store_partials(red, q, G, R, flushed == cur ? nrm : ColVec<1>{},
+                     partials + (static_cast<int64_t>(flushed) * gridDim.x + blockIdx.x) * R);
+  };
+  int cur = -1;
+  for (int64_t tb0 = static_cast<int64_t>(blockIdx.x) * kBlkWaves; tb0 < a.n_tiles;
+       tb0 += n_waves) {
+    const int s = __builtin_amdgcn_readfirstlane(find_sector(a, tb0));  // the workgroup's
     const BlkSector& S = a.sec[s];
-    const int64_t r_begin = (t - S.tile_begin) * kTileRows;
-    const int64_t r_end = min<int64_t>(r_begin + kTileRows, S.b.dim);
-    const double al = col_ok && alpha ? alpha[s * R + col] : 0.0;
-    const double be = col_ok && A ? beta[s * R + col] : 0.0;
+    if (s != cur) {
+      flush_to(s, cur);
+      cur = s;
+      nrm = ColVec<1>{};
+    }
+    const int64_t t = tb0 + wv;
+    if (t >= a.n_tiles || !q.ok) continue;
+    const int64_t r_begin = (t - S.tile_begin) * a.tile_rows;
+    const int n_rows = static_cast<int>(min<int64_t>(a.tile_rows, S.b.dim - r_begin));
+    // the tile's elements, as uniform bases and 32-bit offsets
+    const int64_t base = (S.row_off + r_begin) * R;
+    double* Ct = C + base;
+    const double* Bt = B + base;
+    const double* At = A ? A + base : nullptr;
+    const double al = alpha ? alpha[s * R + q.col] : 0.0;
+    const double be = A ? beta[s * R + q.col] : 0.0;
     // the blocks hold unnormalised vectors: v_B = fb B, v_A = fa A, and C
     // holds H B, so H v_B = fb C
-    const double fb = col_ok && sB ? sB[s * R + col] : 1.0;
-    const double fa = col_ok && sA ? sA[s * R + col] : 1.0;
+    const double fb = sB ? sB[s * R + q.col] : 1.0;
+    const double fa = sA ? sA[s * R + q.col] : 1.0;
     const double alb = al * fb, bea = be * fa;
-    double part = 0.0;
     // eight rows per round: their loads are issued together; the norm is
     // still accumulated row by row in order
     constexpr int kU = 8;
-    for (int64_t i0 = r_begin + grp; i0 < r_end; i0 += kU * rows_per_pass) {
-      if (!col_ok) continue;
+    for (int i0 = q.grp; i0 < n_rows; i0 += kU * q.rpp) {
       double cv[kU], bv[kU], av[kU];
 #pragma unroll
       for (int u = 0; u < kU; ++u) {
-        const int64_t i = i0 + u * rows_per_pass;
-        const int64_t gi = (S.row_off + i) * R + col;
-        const bool in = i < r_end;
-        cv[u] = in ? C[gi] : 0.0;
-        bv[u] = in ? B[gi] : 0.0;
-        av[u] = in && A ? A[gi] : 0.0;
+        const int i = i0 + u * q.rpp;
+        const uint32_t gi = i * R + q.col;
+        const bool in = i < n_rows;
+        cv[u] = in ? Ct[gi] : 0.0;
+        bv[u] = in ? Bt[gi] : 0.0;
+        av[u] = in && A ? At[gi] : 0.0;
       }
 #pragma unroll
       for (int u = 0; u < kU; ++u) {
-        const int64_t i = i0 + u * rows_per_pass;
-        if (i >= r_end) continue;
-        const int64_t gi = (S.row_off + i) * R + col;
+        const int i = i0 + u * q.rpp;
+        if (i >= n_rows) continue;
+        const uint32_t gi = i * R + q.col;
         double w = fb * cv[u] - alb * bv[u];
         if (A) w -= bea * av[u];
         if (fb == 0.0) w = 0.0;  // a column whose beta underflowed stays zero
-        C[gi] = w;
-        part += w * w;
+        Ct[gi] = w;
+        nrm.v[0] += w * w;
       }
     }
-    for (int k = 0; k < kMaxSectors; ++k)
-      if (k == s) nrm[k] += part;
   }
-  for (int k = 0; k < a.n_sec; ++k) {
-    const double v = sum_over_groups(nrm[k], G);
-    if (grp == 0 && col_ok) partials[(k * n_waves + wave) * R + col] = v;
-  }
+  flush_to(a.n_sec, cur);
+  if (step && blockIdx.x == 0 && threadIdx.x == 0) step[0] += 1;
 }
 
-// One workgroup per (sector, column): fixed-order sum of the wave partials.
-// mode 0 (alpha): out[s*R+c] = sum, times sq[s*R+c]^2 when sq is given.  mode 1 (beta): out[s*R+c] = sqrt(sum),
-// out2[s*R+c] = 1/beta or 0.  hist (optional) receives the value at
-// hist[(s*R + c)*M + step[0]].
-__global__ __launch_bounds__(256) void k_blk_finalize(
-    const double* __restrict__ partials, int64_t n_waves, int R, int mode,
+// Fixed-order sums of the workgroups' partials, kFinCols columns of one sector
+// per workgroup (grid: ceil(R / kFinCols) x sectors): neighbouring threads read
+// neighbouring columns, and a workgroup's loads are in flight together (1024
+// partials of two sectors and 64 columns: 5.8 us, 10 us with a workgroup per
+// column and a partial per wavefront).
+// mode 0 (alpha): out[s*R+c] = sum, times sq[s*R+c]^2 when sq is given.  mode 1
+// (beta): out[s*R+c] = sqrt(sum), out2[s*R+c] = 1/beta or 0.  hist (optional) receives the value at
+// hist[(s*R + c)*M + step[0] - back].
+constexpr int kFinCols = 8;
+constexpr int kFinThreads = 1024;
+__global__ __launch_bounds__(kFinThreads) void k_blk_finalize(
+    const double* __restrict__ partials, int n_blocks, int R, int mode,
     double* __restrict__ out, double* __restrict__ out2, double* __restrict__ hist,
-    const int* __restrict__ step, int M, const double* __restrict__ sq) {
-  const int sc = blockIdx.x;  // s * R + c
-  const int s = sc / R, c = sc % R;
+    const int* __restrict__ step, int back, int M, const double* __restrict__ sq) {
+  constexpr int kRows = kFinThreads / kFinCols;
+  __shared__ double red[kRows][kFinCols];
+  const int s = blockIdx.y;
+  const int u = threadIdx.x % kFinCols, g = threadIdx.x / kFinCols;
+  const int c = blockIdx.x * kFinCols + u;
   double v = 0.0;
-  for (int64_t w = threadIdx.x; w < n_waves; w += 256)
-    v += partials[(s * n_waves + w) * R + c];
-  v = block_sum<256>(v);
-  if (threadIdx.x == 0) {
-    double r = v;
+  if (c < R) {
+    const double* p = partials + static_cast<int64_t>(s) * n_blocks * R + c;
+#pragma unroll 8
+    for (int w = g; w < n_blocks; w += kRows) v += p[static_cast<int64_t>(w) * R];
+  }
+  red[g][u] = v;
+  for (int h = kRows / 2; h > 0; h >>= 1) {
+    __syncthreads();
+    if (g < h) red[g][u] += red[g + h][u];
+  }
+  if (g == 0 && c < R) {
+    const int sc = s * R + c;
+    double r = red[0][u];
     if (mode == 0 && sq) r = r * sq[sc] * sq[sc];
     if (mode == 1) {
-      r = sqrt(v);
+      r = sqrt(r);
       out2[sc] = r > 1e-300 ? 1.0 / r : 0.0;
     }
     out[sc] = r;
-    if (hist) hist[static_cast<int64_t>(sc) * M + step[0]] = r;
+    if (hist) hist[static_cast<int64_t>(sc) * M + step[0] - back] = r;
   }
 }
 
-// Advances the step counter the coefficient history is indexed by.
-__global__ void k_blk_step(int* __restrict__ step) {
-  if (blockIdx.x == 0 && threadIdx.x == 0) step[0] += 1;
-}
-
-// C *= 1/beta per (sector, column); optionally advances the step counter.
+// C *= 1/beta per (sector, column).
 __global__ __launch_bounds__(kBlkThreads) void k_blk_scale(
-    BlkArgs a, double* __restrict__ C, const double* __restrict__ invb,
-    int* __restrict__ step) {
+    BlkArgs a, double* __restrict__ C, const double* __restrict__ invb) {
   const int lane = threadIdx.x & 63;
   const int G = a.G, R = a.R;
   const int grp = lane / G, col = lane % G;
@@ -738,8 +702,8 @@ __global__ __launch_bounds__(kBlkThreads) void k_blk_scale(
   for (int64_t t = wave; t < a.n_tiles; t += n_waves) {
     const int s = find_sector(a, t);
     const BlkSector& S = a.sec[s];
-    const int64_t r_begin = (t - S.tile_begin) * kTileRows;
-    const int64_t r_end = min<int64_t>(r_begin + kTileRows, S.b.dim);
+    const int64_t r_begin = (t - S.tile_begin) * a.tile_rows;
+    const int64_t r_end = min<int64_t>(r_begin + a.tile_rows, S.b.dim);
     if (!col_ok) continue;
     const double f = invb[s * R + col];
     constexpr int kU = 8;
@@ -757,10 +721,7 @@ __global__ __launch_bounds__(kBlkThreads) void k_blk_scale(
       }
     }
   }
-  if (step && blockIdx.x == 0 && threadIdx.x == 0) step[0] += 1;
 }
-
-
 
 struct DevMem {
   std::vector<void*> ptrs;
@@ -786,34 +747,48 @@ namespace {
 using BlkKernel = void (*)(BlkArgs, const double*, double*, double*);
 
 // Block-apply kernel of a configuration: cached kernels by gathers in flight
-// (4, 8, 16), one or two columns per lane; searching kernels by lookups in
-// flight (4, 2).
+// (4, 8, 16), searching kernels by lookups in flight (6 or 4 by the state's
+// words; 2); one or two columns per lane.
+template <int CPL>
+BlkKernel blk_kernel_t(int nw, bool cached, int k) {
+  if (cached) {
+    if (nw == 1)
+      return k == 0 ? k_blk_capply<1, 4, CPL>
+                    : (k == 2 ? k_blk_capply<1, 16, CPL> : k_blk_capply<1, 8, CPL>);
+    return k == 0 ? k_blk_capply<2, 4, CPL>
+                  : (k == 2 ? k_blk_capply<2, 16, CPL> : k_blk_capply<2, 8, CPL>);
+  }
+  if (nw == 1) return k == 2 ? k_blk_apply<1, 2, CPL> : k_blk_apply<1, 6, CPL>;
+  return k == 2 ? k_blk_apply<2, 2, CPL> : k_blk_apply<2, 4, CPL>;
+}
 BlkKernel blk_kernel(int nw, bool cached, int cfg, bool pairs) {
   const int k = blk_cfg_kernel(cfg);
-  if (cached && pairs) {
-    if (nw == 1) return k == 0 ? k_blk_capply2<1, 4> : (k == 2 ? k_blk_capply2<1, 16> : k_blk_capply2<1, 8>);
-    return k == 0 ? k_blk_capply2<2, 4> : (k == 2 ? k_blk_capply2<2, 16> : k_blk_capply2<2, 8>);
-  }
-  if (cached) {
-    if (nw == 1) return k == 0 ? k_blk_capply<1, 4> : (k == 2 ? k_blk_capply<1, 16> : k_blk_capply<1, 8>);
-    return k == 0 ? k_blk_capply<2, 4> : (k == 2 ? k_blk_capply<2, 16> : k_blk_capply<2, 8>);
-  }
-  if (pairs) {
-    if (nw == 1) return k == 2 ? k_blk_apply<1, 2, 2> : k_blk_apply<1, 6, 2>;
-    return k == 2 ? k_blk_apply<2, 2, 2> : k_blk_apply<2, 4, 2>;
-  }
-  if (nw == 1) return k == 2 ? k_blk_apply<1, 2, 1> : k_blk_apply<1, 6, 1>;
-  return k == 2 ? k_blk_apply<2, 2, 1> : k_blk_apply<2, 4, 1>;
+  return pairs ? blk_kernel_t<2>(nw, cached, k) : blk_kernel_t<1>(nw, cached, k);
 }
 
 }  // namespace
 
-bool blk_pairs(const BlkArgs& a, const double* X) {
-  return blk_cached(a) && blk_cfg_pairs(a.cfg) && a.R >= 2 && a.ldx % 2 == 0 &&
-         a.ldx >= a.R + (a.R & 1) && reinterpret_cast<uintptr_t>(X) % 16 == 0;
+void blk_set_tiles(BlkArgs& a) {
+  int64_t rows = 0;
+  for (int s = 0; s < a.n_sec; ++s) rows += a.sec[s].b.dim;
+  // rows of one pass of a wavefront, at most
+  const int pass = a.R >= 2 ? std::min(64, 128 / a.G) : 64 / a.G;
+  a.tile_rows = kTileRows;
+  const int64_t fill = blk_cached(a) ? kBlkFillCached : kBlkFillSearch;
+  while (a.tile_rows > std::max(pass, kTileRowsMin) && rows < fill * a.tile_rows) a.tile_rows /= 2;
+  int64_t tiles = 0;
+  for (int s = 0; s < a.n_sec; ++s) {
+    a.sec[s].tile_begin = tiles;
+    // whole workgroups of tiles (the last ones may be empty)
+    const int64_t wg = static_cast<int64_t>(a.tile_rows) * kBlkWaves;
+    tiles += (a.sec[s].b.dim + wg - 1) / wg * kBlkWaves;
+  }
+  a.n_tiles = tiles;
 }
 
-int blk_apply_blocks(int nw, int64_t n_tiles, bool cached, int cfg) {
+int blk_apply_blocks(const BlkArgs& a, int nw) {
+  const bool cached = blk_cached(a), pairs = blk_pairs(a);
+  const int cfg = a.cfg;
   // resident blocks per CU of each kernel: [cached][nw - 1][kernel][pairs];
   // atomics, as host threads may launch concurrently (they store equal
   // values).  The CU count is a function-local static, whose initialisation
@@ -827,7 +802,6 @@ int blk_apply_blocks(int nw, int64_t n_tiles, bool cached, int cfg) {
       cu = 256;
     return cu;
   }();
-  const bool pairs = !cached || blk_cfg_pairs(cfg);
   std::atomic<int>& occ = per_cu[cached ? 1 : 0][nw - 1][blk_cfg_kernel(cfg)][pairs ? 1 : 0];
   int o_cu = occ.load(std::memory_order_relaxed);
   if (o_cu == 0) {
@@ -839,40 +813,22 @@ int blk_apply_blocks(int nw, int64_t n_tiles, bool cached, int cfg) {
   }
   int64_t resident = static_cast<int64_t>(o_cu) * n_cu;
   if (blk_cfg_half(cfg)) resident = std::max<int64_t>(1, resident / 2);
-  const int64_t need = (n_tiles + kBlkWaves - 1) / kBlkWaves;
+  const int64_t need = (a.n_tiles + kBlkWaves - 1) / kBlkWaves;
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(need, resident)));
 }
 
 int launch_blk_apply(const BlkArgs& a, int nw, int n_blocks, const double* X, double* Y,
                      double* partials, hipStream_t s) {
-  if (!blk_cached(a) && a.R >= 2) {
-    // two columns per lane, a power of two of lanes per row
-    BlkArgs b = a;
-    b.G = 1;
-    while (2 * b.G < a.R) b.G <<= 1;
-    hipLaunchKernelGGL(blk_kernel(nw, false, a.cfg, true), dim3(n_blocks), dim3(kBlkThreads), 0,
-                       s, b, X, Y, partials);
-    QSI_CHECK_LAUNCH();
-    return QSI_OK;
-  }
-  if (blk_pairs(a, X)) {
-    // ceil(R / 2) lanes per row; a power of two when the partials cross
-    // row groups by butterfly
-    BlkArgs b = a;
-    const int w = (a.R + 1) / 2;
-    int G = w;
-    if (partials) {
-      G = 1;
-      while (G < w) G <<= 1;
-    }
-    b.G = G;
-    hipLaunchKernelGGL(blk_kernel(nw, true, a.cfg, true), dim3(n_blocks), dim3(kBlkThreads), 0,
-                       s, b, X, Y, partials);
-    QSI_CHECK_LAUNCH();
-    return QSI_OK;
-  }
-  hipLaunchKernelGGL(blk_kernel(nw, blk_cached(a), a.cfg, false), dim3(n_blocks),
-                     dim3(kBlkThreads), 0, s, a, X, Y, partials);
+  const bool cached = blk_cached(a), pairs = blk_pairs(a);
+  BlkArgs b = a;
+  // lanes per row: as many as hold the columns; a power of two in the
+  // searching kernels and where partials cross row groups by butterfly
+  const int w = pairs ? (a.R + 1) / 2 : a.R;
+  b.G = 1;
+  while (b.G < w) b.G <<= 1;
+  if (cached && !partials) b.G = w;
+  hipLaunchKernelGGL(blk_kernel(nw, cached, a.cfg, pairs), dim3(n_blocks), dim3(kBlkThreads), 0,
+                     s, b, X, Y, partials);
   QSI_CHECK_LAUNCH();
   return QSI_OK;
 }
@@ -988,7 +944,7 @@ BlkArgs sector_args(const qsi_op_t* ops, int n_sectors, int R, const double* con
   args.ldx = args.ldy = R;
   args.accumulate = 0;
   args.y_colmajor = 0;
-  int64_t tiles = 0, rows = 0;
+  int64_t rows = 0;
   for (int s = 0; s < n_sectors; ++s) {
     const qsi_op_s* op = ops[s];
     BlkSector& S = args.sec[s];
@@ -1004,13 +960,10 @@ BlkArgs sector_args(const qsi_op_t* ops, int n_sectors, int R, const double* con
     S.n_off = op->n_off;
     S.n_diag = op->n_diag;
     S.coeffs = d_coeffs ? d_coeffs[s] : nullptr;
-    S.tile_begin = tiles;
     S.row_off = rows;
-    // whole workgroups of tiles (the last ones may be empty)
-    tiles += (op->basis->dim + kTileRows * kBlkWaves - 1) / (kTileRows * kBlkWaves) * kBlkWaves;
     rows += op->basis->dim;
   }
-  args.n_tiles = tiles;
+  blk_set_tiles(args);
   args.cfg = ops[0]->blk_cfg;
   *rows_out = rows;
   return args;
@@ -1038,11 +991,9 @@ extern "C" int qsi_lanczos_block(const qsi_op_t* ops, int n_sectors, int R,
   }
   int64_t rows = 0;
   BlkArgs args = sector_args(ops, n_sectors, R, d_coeffs, &rows);
-  const int64_t tiles = args.n_tiles;
-  // persistent grid: enough wavefronts to fill the chip, never more than tiles
-  args.cfg = ops[0]->blk_cfg;
-  const int n_blocks = blk_apply_blocks(nw, tiles, blk_cached(args), args.cfg);
-  const int64_t n_waves = static_cast<int64_t>(n_blocks) * kBlkWaves;
+  // persistent grids: enough wavefronts to fill the chip, never more than tiles
+  const int n_blocks = blk_apply_blocks(args, nw);
+  const int n_vec = static_cast<int>(std::min<int64_t>(args.n_tiles / kBlkWaves, kBlkVecBlocks));
   const size_t blk = static_cast<size_t>(rows) * R;
   DevMem mem;
   double *A = nullptr, *B = nullptr, *C = nullptr, *part = nullptr;
@@ -1052,7 +1003,7 @@ extern "C" int qsi_lanczos_block(const qsi_op_t* ops, int n_sectors, int R,
   QSI_CHECK_HIP(mem.alloc(&A, blk));
   QSI_CHECK_HIP(mem.alloc(&B, blk));
   QSI_CHECK_HIP(mem.alloc(&C, blk));
-  QSI_CHECK_HIP(mem.alloc(&part, static_cast<size_t>(n_sectors) * n_waves * R));
+  QSI_CHECK_HIP(mem.alloc(&part, static_cast<size_t>(SR) * std::max(n_blocks, n_vec)));
   QSI_CHECK_HIP(mem.alloc(&alpha, SR));
   QSI_CHECK_HIP(mem.alloc(&beta, SR));
   QSI_CHECK_HIP(mem.alloc(&invb, SR));
@@ -1074,18 +1025,18 @@ extern "C" int qsi_lanczos_block(const qsi_op_t* ops, int n_sectors, int R,
   QSI_CHECK_HIP(hipMemsetAsync(beta, 0, SR * sizeof(double), st));
   QSI_CHECK_HIP(hipMemsetAsync(step, 0, sizeof(int), st));
   // normalise the start columns: B = B / |B_c|
-  hipLaunchKernelGGL(k_blk_update, dim3(n_blocks), dim3(kBlkThreads), 0, st, args,
+  const dim3 fin((R + kFinCols - 1) / kFinCols, n_sectors);
+  hipLaunchKernelGGL(k_blk_update, dim3(n_vec), dim3(kBlkThreads), 0, st, args,
                      static_cast<const double*>(nullptr), B, B, static_cast<const double*>(nullptr),
                      static_cast<const double*>(nullptr), part, static_cast<const double*>(nullptr),
-                     static_cast<const double*>(nullptr));
+                     static_cast<const double*>(nullptr), static_cast<int*>(nullptr));
   QSI_CHECK_LAUNCH();
   // (C = B - 0*B: the kernel writes back B unchanged and produces |B_c|^2)
-  hipLaunchKernelGGL(k_blk_finalize, dim3(SR), dim3(256), 0, st, part, n_waves, R, 1,
-                     beta, invb, static_cast<double*>(nullptr), static_cast<const int*>(nullptr), M,
-                     static_cast<const double*>(nullptr));
+  hipLaunchKernelGGL(k_blk_finalize, fin, dim3(kFinThreads), 0, st, part, n_vec, R, 1,
+                     beta, invb, static_cast<double*>(nullptr), static_cast<const int*>(nullptr), 0,
+                     M, static_cast<const double*>(nullptr));
   QSI_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_blk_scale, dim3(n_blocks), dim3(kBlkThreads), 0, st, args, B, invb,
-                     static_cast<int*>(nullptr));
+  hipLaunchKernelGGL(k_blk_scale, dim3(n_vec), dim3(kBlkThreads), 0, st, args, B, invb);
   QSI_CHECK_LAUNCH();
   QSI_CHECK_HIP(hipMemsetAsync(beta, 0, SR * sizeof(double), st));
 
@@ -1112,16 +1063,14 @@ extern "C" int qsi_lanczos_block(const qsi_op_t* ops, int n_sectors, int R,
     double* sc = scl[(p + 2) % 3];
     const int rc = launch_blk_apply(args, nw, n_blocks, b, c, part, st);
     if (rc != QSI_OK) return rc;
-    hipLaunchKernelGGL(k_blk_finalize, dim3(SR), dim3(256), 0, st, part, n_waves, R, 0,
-                       alpha, static_cast<double*>(nullptr), ha, step, M, sb);
+    hipLaunchKernelGGL(k_blk_finalize, fin, dim3(kFinThreads), 0, st, part, n_blocks, R, 0,
+                       alpha, static_cast<double*>(nullptr), ha, step, 0, M, sb);
     QSI_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_blk_update, dim3(n_blocks), dim3(kBlkThreads), 0, st, args, a, b, c,
-                       alpha, beta, part, sa, sb);
+    hipLaunchKernelGGL(k_blk_update, dim3(n_vec), dim3(kBlkThreads), 0, st, args, a, b, c,
+                       alpha, beta, part, sa, sb, step);
     QSI_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_blk_finalize, dim3(SR), dim3(256), 0, st, part, n_waves, R, 1,
-                       beta, sc, hb, step, M, static_cast<const double*>(nullptr));
-    QSI_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_blk_step, dim3(1), dim3(64), 0, st, step);
+    hipLaunchKernelGGL(k_blk_finalize, fin, dim3(kFinThreads), 0, st, part, n_vec, R, 1,
+                       beta, sc, hb, step, 1, M, static_cast<const double*>(nullptr));
     QSI_CHECK_LAUNCH();
     return QSI_OK;
   };
@@ -1233,7 +1182,7 @@ int tune_block(BlkArgs a, int nw, int reps, const double* X, double* Y, int* pic
     for (int cf = 0; cf < 2 * n_pairs; ++cf) {
       const int half = cf & 1, pairs = cf >> 1;
       a.cfg = k | (half << 2) | (pairs << 3);
-      const int nb = blk_apply_blocks(nw, a.n_tiles, cached, a.cfg);
+      const int nb = blk_apply_blocks(a, nw);
       double ms = 0.0;
       const int rc = time_ms([&]() { return launch_blk_apply(a, nw, nb, X, Y, nullptr, nullptr); },
                              reps, nullptr, &ms);

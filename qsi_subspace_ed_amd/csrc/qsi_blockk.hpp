@@ -14,7 +14,7 @@ namespace qsi {
 
 constexpr int kBlkThreads = 256;
 constexpr int kBlkWaves = kBlkThreads / 64;
-constexpr int kTileRows = 64;
+constexpr int kTileRows = 64;  // at most
 constexpr int kMaxSectors = 8;
 
 struct BlkSector {
@@ -27,7 +27,7 @@ struct BlkSector {
   int n_cls;             // 0: per-term coefficients
   int n_off;
   int n_diag;
-  int64_t tile_begin;  // first global tile of this sector, a multiple of kBlkWaves
+  int64_t tile_begin;  // first global tile of this sector, a multiple of kBlkWaves (blk_set_tiles)
   int64_t row_off;     // first row of this sector in the concatenated blocks
   // cached connectivity of the operator, or null (see qsi_op_s)
   const uint64_t* rowptr;
@@ -38,11 +38,11 @@ struct BlkSector {
 struct BlkArgs {
   BlkSector sec[kMaxSectors];
   int n_sec;
-  int64_t n_tiles;
+  int64_t n_tiles;  // tiles of all sectors (blk_set_tiles)
+  int tile_rows;    // rows per tile: a power of two, at most 64 (blk_set_tiles)
   int R;
-  int G;            // lanes per row group: a power of two >= R, or any width
-                    // >= R for the cached kernel without partials (the
-                    // column-pairs kernel sets its own, ceil(R / 2))
+  int G;            // lanes per row: a power of two >= R (launch_blk_apply sets
+                    // its own)
   int64_t ldx, ldy; // row strides of the X and Y blocks (>= R)
   int accumulate;   // Y += H X instead of Y = H X (apply kernel)
   int y_colmajor;   // Y stored column-major: Y[col * ldy + row] (apply kernel)
@@ -50,9 +50,10 @@ struct BlkArgs {
 };
 
 // Block-apply configuration: bits 0-1 pick the kernel (cached connectivity:
-// 4 / 8 / 16 gathers in flight per lane; searching: 4 / 4 / 2 lookups in
-// flight), bit 2 halves the persistent grid, bit 3 lets the cached kernel
-// serve two columns per lane (16-byte gathers) where X's rows allow it.
+// 4 / 8 / 16 gathers in flight per lane; searching: 6 or 4 lookups in flight
+// by the state's words, or 2), bit 2 halves the persistent grid, bit 3 lets the
+// cached kernel serve two columns per lane (16-byte gathers); the searching
+// kernel always does.
 constexpr int kBlkCfgDefault = 1;
 inline int blk_cfg_kernel(int cfg) { return cfg & 3; }
 inline bool blk_cfg_half(int cfg) { return (cfg >> 2) & 1; }
@@ -66,18 +67,22 @@ inline bool blk_cached(const BlkArgs& a) {
   return a.n_sec > 0;
 }
 
-// True when a cached block apply on X serves two columns per lane: the
-// configuration's pairs bit, R >= 2, an even ldx >= R rounded up to even and
-// a 16-byte aligned X.
-bool blk_pairs(const BlkArgs& a, const double* X);
+// True when a block apply serves two columns per lane: R >= 2 and, over cached
+// connectivity, the configuration's pairs bit.
+inline bool blk_pairs(const BlkArgs& a) {
+  return a.R >= 2 && (!blk_cached(a) || blk_cfg_pairs(a.cfg));
+}
 
-// Blocks of a persistent block-apply grid over n_tiles 64-row tiles: all
-// resident at once (occupancy x compute units), never more than the tiles
-// need.  `cached` picks the kernel (see blk_cached).
-int blk_apply_blocks(int nw, int64_t n_tiles, bool cached, int cfg);
+// Cuts the sectors (bases, R and G set) into tiles, one wavefront's work each:
+// tile_rows, every tile_begin and n_tiles.
+void blk_set_tiles(BlkArgs& a);
+
+// Blocks of a persistent block-apply grid over the tiles of `a`: all resident
+// at once (occupancy x compute units), never more than the tiles need.
+int blk_apply_blocks(const BlkArgs& a, int nw);
 
 // Y (+)= H X over the sectors of `a` (the block-apply kernels; see
-// qsi_block.hip).  partials: n_sec x (n_blocks * kBlkWaves) x R, or null.
+// qsi_block.hip).  partials: n_sec x n_blocks x R, or null.
 int launch_blk_apply(const BlkArgs& a, int nw, int n_blocks, const double* X, double* Y,
                      double* partials, hipStream_t s);
 

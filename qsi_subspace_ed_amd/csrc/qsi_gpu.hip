@@ -3526,9 +3526,9 @@ int qsi_op_apply_block(qsi_op_t op, const double* d_X, int64_t ldx, double* d_Y,
   a.sec[0].rowptr = op->d_rowptr;
   a.sec[0].cj = op->d_cj;
   a.sec[0].cm = op->d_cm;
-  a.n_tiles = (op->basis->dim + kTileRows - 1) / kTileRows;
+  blk_set_tiles(a);
   a.cfg = op->blk_cfg;
-  const int nb = blk_apply_blocks(op->basis->nw, a.n_tiles, blk_cached(a), a.cfg);
+  const int nb = blk_apply_blocks(a, op->basis->nw);
   return launch_blk_apply(a, op->basis->nw, nb, d_X, d_Y, nullptr,
                           static_cast<hipStream_t>(stream));
 }

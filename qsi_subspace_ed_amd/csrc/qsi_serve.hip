@@ -713,11 +713,10 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
   a.sec[0].cm = op->d_cm;
   a.sec[0].n_off = op->n_off;
   a.sec[0].n_diag = op->n_diag;
-  a.sec[0].tile_begin = 0;
   a.sec[0].row_off = 0;
-  a.n_tiles = (E->D + kTileRows - 1) / kTileRows;
+  blk_set_tiles(a);
   a.cfg = op->blk_cfg;
-  E->n_blocks = blk_apply_blocks(op->basis->nw, a.n_tiles, blk_cached(a), a.cfg);
+  E->n_blocks = blk_apply_blocks(a, op->basis->nw);
   const size_t R = static_cast<size_t>(E->R);
   hipError_t e = hipStreamCreateWithFlags(&E->st, hipStreamNonBlocking);
   const int ns = std::max(op->n_slots, 1);
@@ -881,10 +880,6 @@ int qsi_engine_step_begin(qsi_engine_t E, int* launched) {
   // output is column sl of Wc
   BlkArgs a = E->args;
   a.R = nact;
-  int G = 64;
-  while (G / 2 >= nact && G > 1) G >>= 1;
-  // the cached kernel takes any row-group width: one lane per live column
-  a.G = blk_cached(a) ? nact : G;
   a.ldx = ldx;
   rc = launch_blk_apply(a, E->op->basis->nw, E->n_blocks, E->X, E->Wc, nullptr, s);
   if (rc != QSI_OK) return rc;

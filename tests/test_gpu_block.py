@@ -68,3 +68,65 @@ def test_columns(cuda, words, bits, keep, n, n_cls):
         y = cuda.empty_like(x)
         op.apply_block(x, y)
         assert cuda.equal(y, alone)
+
+
+@pytest.mark.parametrize("words,bits,keep", [(1, 6, 17), (2, 7, 65), (1, 12, 1500), (1, 13, 8191)])
+@pytest.mark.parametrize("cfg", [0, 1, 2, 4, 8, 9, 10, 13])
+def test_cached_columns(cuda, words, bits, keep, cfg):
+    """Every configuration over cached connectivity gives the searching apply's
+    columns bit for bit, at every width, odd and strided blocks included."""
+    states, spins, W = _basis(words, bits, keep, keep)
+    H = _classed(_terms(spins, 130, bits, z=True, open_spins=False), 3)
+    basis = q.GpuBasis(states, W)
+    op, cached = q.GpuOp(basis, H), q.GpuOp(basis, H)
+    assert cached.cache_connectivity(True) > 0
+    cached.set_block_cfg(cfg)
+    D = basis.dim()
+    rng = np.random.default_rng(D)
+    x = cuda.from_numpy(rng.standard_normal((D, 64))).cuda()
+    y0 = cuda.from_numpy(rng.standard_normal((D, 64))).cuda()
+    for R in (1, 2, 3, 5, 7, 8, 16, 21, 33, 63, 64):
+        c0 = 1 if R < 64 else 0
+        for add in (False, True):
+            y, yc = y0.clone(), y0.clone()
+            op.apply_block(x[:, c0:c0 + R], y[:, c0:c0 + R], accumulate=add)
+            cached.apply_block(x[:, c0:c0 + R], yc[:, c0:c0 + R], accumulate=add)
+            assert cuda.equal(y, yc), (R, add)
+
+
+@pytest.mark.parametrize("R", [1, 3, 8, 21, 64])
+@pytest.mark.parametrize("cached", [False, True])
+def test_recurrence(cuda, R, cached):
+    """Block Lanczos over sectors of 1500, 17 and 4096 states (tiles cut short,
+    empty tiles, workgroups without a tile of some sector): each column's
+    coefficients are those of the three-term recurrence in float64 on the CPU.
+    Six steps; rounding grows with the condition of the steps before, so 1e-11
+    relative to the largest coefficient, as for the sectors run alone."""
+    from qsi_subspace_ed_amd import ftlm
+    ops, V, want = [], [], []
+    for bits, keep in ((12, 1500), (6, 17), (12, 4096)):
+        states, spins, W = _basis(1, bits, keep, keep)
+        H = _classed(_terms(spins, 40, 5, z=False, open_spins=False), 3)
+        ops.append(q.GpuOp(q.GpuBasis(states, W), H))
+        V.append(np.random.default_rng(keep).standard_normal((keep, R)))
+        if cached:
+            ops[-1].cache_connectivity(True)
+        r, c, v, d = ops[-1].connectivity()
+        A = np.diag(d)
+        np.add.at(A, (r, c), v)
+        b = V[-1] / np.linalg.norm(V[-1], axis=0)
+        a, be, al_s, be_s = np.zeros_like(b), np.zeros(R), [], []
+        for _ in range(6):
+            w = A @ b
+            al = np.sum(b * w, axis=0)
+            w -= al * b + be * a
+            be = np.linalg.norm(w, axis=0)
+            a, b = b, w / be
+            al_s.append(al)
+            be_s.append(be)
+        want.append((np.array(al_s).T, np.array(be_s).T))
+    al, be, _ = ftlm.lanczos_block(ops, [cuda.from_numpy(v).cuda() for v in V], 6)
+    for s, (wa, wb) in enumerate(want):
+        scale = max(np.abs(wa).max(), np.abs(wb).max())
+        assert np.abs(al[s] - wa).max() <= 1e-11 * scale, s
+        assert np.abs(be[s] - wb).max() <= 1e-11 * scale, s
