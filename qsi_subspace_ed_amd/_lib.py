@@ -139,6 +139,8 @@ SIGNATURES = {
     "qsi_ftlm_sample": (C.c_int, [_P, C.POINTER(_P), C.c_int, _P, C.c_int, _DP, C.c_int, _D,
                                   _DP, _DP, _DP, _DP, _DP, C.POINTER(C.c_int)]),
     "qsi_tridiag_eig": (C.c_int, [_DP, _DP, C.c_int, _DP, _DP]),
+    "qsi_tridiag_quadrature": (C.c_int, [_DP, C.c_int64, _DP, C.c_int64, C.POINTER(C.c_int),
+                                         C.c_int, _DP, _DP]),
     "qsi_lanczos_ritz": (C.c_int, [_DP, _DP, C.c_int, _D, C.c_int, _DP, _DP,
                                    C.POINTER(C.c_int), C.POINTER(C.c_int)]),
     "qsi_engine_create": (C.c_int, [_P, C.c_int, C.c_int, C.c_int, _D, C.c_int, C.POINTER(_P)]),

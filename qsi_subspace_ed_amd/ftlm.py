@@ -84,13 +84,34 @@ def quadrature(alpha, beta):
     (R, M) coefficient arrays of one sector.  A sample whose recurrence ended
     (beta_j == 0: its Krylov space is invariant, later coefficients are 0)
     keeps only its first j + 1 steps, as the C++ FtlmComputer does."""
-    out = []
-    for r in range(alpha.shape[0]):
-        b = np.asarray(beta[r])
-        z = np.flatnonzero(b == 0.0)
-        m = int(z[0]) + 1 if z.size else len(alpha[r])
-        out.append(tridiag_eig(alpha[r][:m], b[:m]))
-    return out
+    R = alpha.shape[0]
+    if not (R and alpha.ndim == 2 and isinstance(beta, np.ndarray) and beta.ndim == 2
+            and beta.shape[0] >= R and beta.shape[1] >= alpha.shape[1] - 1 >= 0):
+        # samples of different lengths, or couplings that end with their sample
+        out = []
+        for r in range(R):
+            b = np.asarray(beta[r])
+            z = np.flatnonzero(b == 0.0)
+            m = int(z[0]) + 1 if z.size else len(alpha[r])
+            out.append(tridiag_eig(alpha[r][:m], b[:m]))
+        return out
+    # all samples in one call, on several threads: 64 samples of 100 steps took
+    # 31 ms one after the other (half of a batched run of two 48-spin sectors),
+    # 5 ms on eight cores
+    M = alpha.shape[1]
+    d = np.ascontiguousarray(alpha, dtype=np.float64)
+    e = np.ascontiguousarray(beta, dtype=np.float64)
+    n = np.full(R, M, dtype=np.intc)
+    for r, j in zip(*np.nonzero(e[:R, :M] == 0.0)):
+        n[r] = min(n[r], j + 1)
+    w = np.empty((R, M))
+    f = np.empty((R, M))
+    P = C.POINTER(C.c_double)
+    check(_lib.load().qsi_tridiag_quadrature(
+        d.ctypes.data_as(P), M, e.ctypes.data_as(P), e.shape[1],
+        n.ctypes.data_as(C.POINTER(C.c_int)), R, w.ctypes.data_as(P), f.ctypes.data_as(P)),
+        "qsi_tridiag_quadrature")
+    return [(w[r, :m], f[r, :m]) for r, m in enumerate(n)]
 
 
 def thermodynamics(nodes, D, temps, e_ref=None, normalise=True):
