@@ -1544,16 +1544,6 @@ inline int vec_blocks(int64_t n) {
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(nb, 8192)));
 }
 
-// Workgroups of the projection passes (multi-dots over up to 64 columns):
-// about 16 rows per thread, but at least 1024 workgroups while there are 4
-// rows per thread to give them, so each workgroup's column sums (one block
-// reduction per column) are spread over more rows than in a plain vector
-// kernel and the chip still fills.
-inline int proj_blocks(int64_t n) {
-  const int64_t want = (n + kVecBlock * 16 - 1) / (kVecBlock * 16);
-  return static_cast<int>(std::min<int64_t>(vec_blocks(n), std::max<int64_t>(want, 1024)));
-}
-
 // The grid-stride dot, axpy-norm and device-scalar scale kernels take
 // kVecUnroll of a thread's elements per round, all loads first, and
 // accumulate in element order (the sums are the ones a one-element loop
@@ -1638,19 +1628,74 @@ __global__ __launch_bounds__(kVecBlock) void k_axpy_dev_norm(
 
 constexpr int kMaxCols = 64;
 
-// partials[blk * m + j] = sum over the workgroup's rows of V[:, j] * w
-__global__ __launch_bounds__(kVecBlock) void k_multidot(
+// Gram-Schmidt step of w against V[:, 0:m] in three kernels.  Each one that
+// needs a sum over all rows adds up the partials of the kernel before it by
+// itself: with at most kGsBlocks workgroups that is a few loads per lane from
+// the L2, where kernels of their own for the sums and for the tail's scalars
+// cost three launches of 3-4 us per step.  87 546 rows, ten columns on average:
+// 35 -> 14 us of kernels per step in 3 launches instead of 6; at 2.76 M rows
+// the reads of V bound passes 1 and 2 (42 and 48 us, 5.4 TB/s), and 256
+// workgroups of 512 threads keep enough of them in flight.
+// partials[j * gridDim.x + workgroup] is column j's.
+constexpr int kGsBlocks = 256;
+
+// Sums N values per lane over the wavefront by halving: lane l returns the
+// total of value l / (64 / N), in 2 N exchanges fewer than N full butterflies.
+template <int N, int O = kWave / 2>
+__device__ __forceinline__ double wave_sum_many(double* v, int lane) {
+  static_assert(N <= kWave && (N & (N - 1)) == 0);
+  if constexpr (N > 1) {
+    const bool up = (lane & O) != 0;
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      const double send = up ? v[i] : v[i + N / 2];
+      const double keep = up ? v[i + N / 2] : v[i];
+      v[i] = keep + __shfl_xor(send, O, kWave);
+    }
+    return wave_sum_many<N / 2, O / 2>(v, lane);
+  } else {
+    double t = v[0];
+#pragma unroll
+    for (int o = O; o > 0; o >>= 1) t += __shfl_xor(t, o, kWave);
+    return t;
+  }
+}
+
+// out[j] (LDS) = sum_b partials[j * nb + b] for j < m, by the whole workgroup
+// of T threads; ends with a barrier.
+template <int T>
+__device__ __forceinline__ void sum_partials(const double* __restrict__ partials, int nb, int m,
+                                             double* out) {
+  constexpr int W = T / kWave;
+  static_assert(kGsBlocks <= 4 * kWave);
+  const int lane = threadIdx.x % kWave;
+  for (int j = threadIdx.x / kWave; j < m; j += W) {
+    double v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int b = lane + k * kWave;
+      v[k] = b < nb ? partials[j * nb + b] : 0.0;
+    }
+    const double t = wave_sum((v[0] + v[1]) + (v[2] + v[3]));
+    if (lane == 0) out[j] = t;
+  }
+  __syncthreads();
+}
+
+// Pass 1: partials of V[:, 0:m]^T w, 16 columns at a time.
+template <int T>
+__global__ __launch_bounds__(T) void k_gs_dots(
     const double* __restrict__ V, int64_t ldv, int m, const double* __restrict__ w,
     int64_t n, double* __restrict__ partials) {
-  __shared__ double red[kVecBlock / kWave][16];
+  __shared__ double red[T / kWave][16];
   const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
   for (int j0 = 0; j0 < m; j0 += 16) {
     const int jn = min(16, m - j0);
     double acc[16];
 #pragma unroll
     for (int j = 0; j < 16; ++j) acc[j] = 0.0;
-    for (int64_t i = static_cast<int64_t>(blockIdx.x) * kVecBlock + threadIdx.x;
-         i < n; i += static_cast<int64_t>(gridDim.x) * kVecBlock) {
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * T + threadIdx.x; i < n;
+         i += static_cast<int64_t>(gridDim.x) * T) {
       // every load of the row first, then unpredicated updates (absent
       // columns load as 0 and leave their unused sums unchanged), so a lane
       // keeps all its column loads in flight
@@ -1661,68 +1706,39 @@ __global__ __launch_bounds__(kVecBlock) void k_multidot(
 #pragma unroll
       for (int j = 0; j < 16; ++j) acc[j] += v[j] * wi;
     }
-#pragma unroll
-    for (int j = 0; j < 16; ++j) {
-      const double v = wave_sum(acc[j]);
-      if (lane == 0) red[wid][j] = v;
-    }
+    const double t = wave_sum_many<16>(acc, lane);
+    if (lane % 4 == 0) red[wid][lane / 4] = t;
     __syncthreads();
     if (threadIdx.x < jn) {
       double r = 0.0;
-      for (int k = 0; k < kVecBlock / kWave; ++k) r += red[k][threadIdx.x];
-      partials[static_cast<int64_t>(blockIdx.x) * m + j0 + threadIdx.x] = r;
+#pragma unroll
+      for (int k = 0; k < T / kWave; ++k) r += red[k][threadIdx.x];
+      partials[static_cast<int64_t>(j0 + threadIdx.x) * gridDim.x + blockIdx.x] = r;
     }
     __syncthreads();
   }
 }
 
-// out[j] = sum_b partials[b * m + j], one workgroup per column j, fixed order
-__global__ __launch_bounds__(256) void k_finalize_cols(
-    const double* __restrict__ partials, int nb, int m, double* __restrict__ out,
-    double* __restrict__ acc_out) {
-  const int j = blockIdx.x;
-  double v = 0.0;
-  for (int b = threadIdx.x; b < nb; b += 256) v += partials[static_cast<int64_t>(b) * m + j];
-  v = block_sum<256>(v);
-  if (threadIdx.x == 0) {
-    out[j] = v;
-    if (acc_out) acc_out[j] += v;
-  }
-}
-
-// w -= V[:, 0:m] h
-__global__ __launch_bounds__(kVecBlock) void k_gemv_sub(
-    const double* __restrict__ V, int64_t ldv, int m, const double* __restrict__ h,
-    double* __restrict__ w, int64_t n) {
-  __shared__ double hs[kMaxCols];
-  if (threadIdx.x < m) hs[threadIdx.x] = h[threadIdx.x];
-  __syncthreads();
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kVecBlock + threadIdx.x;
-       i < n; i += static_cast<int64_t>(gridDim.x) * kVecBlock) {
-    double acc = 0.0;
-    for (int j = 0; j < m; ++j) acc += V[j * ldv + i] * hs[j];
-    w[i] -= acc;
-  }
-}
-
-// Second Gram-Schmidt pass fused with the check for a third: w -= V[:, 0:m] h
-// (the same sum order as k_gemv_sub), and from the same read of V the
-// per-workgroup partials of V[:, 0:m]^T w_new (columns 0..m-1) and of
-// w_new . w_new (column m), m <= MAXC.
-template <int MAXC>
-__global__ __launch_bounds__(kVecBlock) void k_gemv_sub_dots(
-    const double* __restrict__ V, int64_t ldv, int m, const double* __restrict__ h,
-    double* __restrict__ w, int64_t n, double* __restrict__ partials) {
+// Pass 2: h = pass 1's sums (written to hcol by one workgroup), w -= V[:, 0:m] h,
+// and from the same read of V the partials of V[:, 0:m]^T w_new (columns
+// 0..m-1) and of w_new . w_new (column m), m <= MAXC.
+template <int T, int MAXC>
+__global__ __launch_bounds__(T) void k_gs_sub_dots(
+    const double* __restrict__ V, int64_t ldv, int m, const double* __restrict__ part1,
+    double* __restrict__ hcol, double* __restrict__ w, int64_t n,
+    double* __restrict__ partials) {
   __shared__ double hs[MAXC];
-  __shared__ double red[kVecBlock / kWave][MAXC + 1];
+  __shared__ double red[T / kWave][MAXC + 1];
   const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
-  if (threadIdx.x < MAXC) hs[threadIdx.x] = threadIdx.x < m ? h[threadIdx.x] : 0.0;
+  if (threadIdx.x < MAXC) hs[threadIdx.x] = 0.0;
   __syncthreads();
-  double acc[MAXC + 1];
+  sum_partials<T>(part1, gridDim.x, m, hs);
+  if (blockIdx.x == 0 && threadIdx.x < m) hcol[threadIdx.x] = hs[threadIdx.x];
+  double acc[MAXC], nrm = 0.0;
 #pragma unroll
-  for (int j = 0; j <= MAXC; ++j) acc[j] = 0.0;
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kVecBlock + threadIdx.x;
-       i < n; i += static_cast<int64_t>(gridDim.x) * kVecBlock) {
+  for (int j = 0; j < MAXC; ++j) acc[j] = 0.0;
+  for (int64_t i = static_cast<int64_t>(blockIdx.x) * T + threadIdx.x; i < n;
+       i += static_cast<int64_t>(gridDim.x) * T) {
     // every load of the row first (absent columns load as 0, and their h is
     // 0, so the sum and the dots are unchanged), then the sums in column
     // order, so a lane keeps all its column loads in flight
@@ -1737,56 +1753,49 @@ __global__ __launch_bounds__(kVecBlock) void k_gemv_sub_dots(
     w[i] = wn;
 #pragma unroll
     for (int j = 0; j < MAXC; ++j) acc[j] += vr[j] * wn;
-    acc[MAXC] += wn * wn;
+    nrm += wn * wn;
   }
-#pragma unroll
-  for (int j = 0; j <= MAXC; ++j) {
-    const double v = wave_sum(acc[j]);
-    if (lane == 0) red[wid][j] = v;
-  }
+  nrm = wave_sum(nrm);
+  const double t = wave_sum_many<MAXC>(acc, lane);
+  if (lane % (kWave / MAXC) == 0) red[wid][lane / (kWave / MAXC)] = t;
+  if (lane == 0) red[wid][MAXC] = nrm;
   __syncthreads();
-  for (int j = threadIdx.x; j <= m; j += kVecBlock) {
+  for (int j = threadIdx.x; j <= m; j += T) {
     const int src = j == m ? MAXC : j;
     double r = 0.0;
-    for (int k = 0; k < kVecBlock / kWave; ++k) r += red[k][src];
-    partials[static_cast<int64_t>(blockIdx.x) * (m + 1) + j] = r;
+#pragma unroll
+    for (int k = 0; k < T / kWave; ++k) r += red[k][src];
+    partials[static_cast<int64_t>(j) * gridDim.x + blockIdx.x] = r;
   }
 }
 
-// After the fused pass: g[0..m) = V^T w, g[m] = w . w.  A third pass is
-// needed when |V^T w| > 1e-12 |w| (flag[0] = 1); its correction is added to
-// the projected column hcol[0..m) and the norm follows it.  beta[0] = |w|,
-// beta[1] = 1 / |w| (0 for a vanishing w).
-__global__ void k_gs_tail(const double* __restrict__ g, int m, double* __restrict__ hcol,
-                          int* __restrict__ flag, double* __restrict__ beta) {
-  __shared__ int need;
-  if (threadIdx.x == 0) {
-    double g2 = 0.0;
-    for (int j = 0; j < m; ++j) g2 += g[j] * g[j];
-    const double q = g[m];
-    need = (q > 0.0 && g2 > 1e-24 * q) ? 1 : 0;
-    const double b2 = need ? q - g2 : q;
-    const double b = b2 > 0.0 ? sqrt(b2) : 0.0;
-    beta[0] = b;
-    beta[1] = b > 0.0 ? 1.0 / b : 0.0;
-    flag[0] = need;
+// The tail of the step: g[0..m) = V^T w and g[m] = w . w from pass 2's
+// partials.  A third pass w -= V g is needed when |V^T w| > 1e-12 |w|; its
+// correction is added to the projected column hcol[0..m) and the norm follows
+// it.  Then w *= 1 / |w|, and one workgroup writes beta[0] = |w|, beta[1] =
+// 1 / |w| (0 for a vanishing w).
+template <int T>
+__global__ __launch_bounds__(T) void k_gs_tail(
+    const double* __restrict__ V, int64_t ldv, int m, const double* __restrict__ part2,
+    double* __restrict__ hcol, double* __restrict__ w, int64_t n, double* __restrict__ beta) {
+  __shared__ double g[kMaxCols + 1];
+  sum_partials<T>(part2, gridDim.x, m + 1, g);
+  double g2 = 0.0;
+  for (int j = 0; j < m; ++j) g2 += g[j] * g[j];
+  const double q = g[m];
+  const bool need = q > 0.0 && g2 > 1e-24 * q;
+  const double b2 = need ? q - g2 : q;
+  const double b = b2 > 0.0 ? sqrt(b2) : 0.0;
+  const double a = b > 0.0 ? 1.0 / b : 0.0;
+  if (blockIdx.x == 0) {
+    if (threadIdx.x == 0) {
+      beta[0] = b;
+      beta[1] = a;
+    }
+    if (need && threadIdx.x < m) hcol[threadIdx.x] += g[threadIdx.x];
   }
-  __syncthreads();
-  if (need)
-    for (int j = threadIdx.x; j < m; j += blockDim.x) hcol[j] += g[j];
-}
-
-// The conditional third pass fused with the normalisation: w -= V[:, 0:m] h
-// when flag[0] is set (a plain column-order sum), then w *= a = beta[1], the
-// scale k_gs_tail computed from the pass-2 sums, in one pass over w.
-__global__ __launch_bounds__(kVecBlock) void k_gemv_sub_scal(
-    const double* __restrict__ V, int64_t ldv, int m, const double* __restrict__ h,
-    double* __restrict__ w, int64_t n, const int* __restrict__ flag,
-    const double* __restrict__ beta) {
-  const bool need = flag[0] != 0;
-  const double a = beta[1];
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * kVecBlock;
-  int64_t i = static_cast<int64_t>(blockIdx.x) * kVecBlock + threadIdx.x;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * T;
+  int64_t i = static_cast<int64_t>(blockIdx.x) * T + threadIdx.x;
   if (!need) {
     for (; i + (kVecUnroll - 1) * stride < n; i += kVecUnroll * stride) {
       double xv[kVecUnroll];
@@ -1798,13 +1807,130 @@ __global__ __launch_bounds__(kVecBlock) void k_gemv_sub_scal(
     for (; i < n; i += stride) w[i] *= a;
     return;
   }
-  __shared__ double hs[kMaxCols];
-  if (threadIdx.x < m) hs[threadIdx.x] = h[threadIdx.x];
-  __syncthreads();
   for (; i < n; i += stride) {
     double acc = 0.0;
-    for (int j = 0; j < m; ++j) acc += V[j * ldv + i] * hs[j];
+    for (int j = 0; j < m; ++j) acc += V[j * ldv + i] * g[j];
     w[i] = (w[i] - acc) * a;
+  }
+}
+
+// ---- Rayleigh-Ritz of the thick-restart solvers -----------------------------
+// One workgroup per projected matrix (RitzArgs): all eigenpairs by Jacobi
+// rotations, kRitzThreads threads, matrix and vectors in LDS.  A sweep is N - 1
+// rounds of N / 2 rotations on disjoint index pairs (round robin), so a round
+// is one barrier for the angles and one for the 2 x 2 blocks of J^T A J and the
+// vectors' columns, where a cyclic sweep is N (N - 1) / 2 rotations one after
+// the other (20 to 24 vectors: about 300 us on a host core while the device
+// idles, 70 us here, and the vectors need not be sent back).
+constexpr int kRitzThreads = 256;
+__global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
+  constexpr int LD = kRitzMax + 1;
+  __shared__ double A[kRitzMax * LD];
+  __shared__ double U[kRitzMax * LD];
+  __shared__ double2 rot[kRitzMax / 2];
+  __shared__ double red[2][kRitzThreads / kWave];
+  const int t = threadIdx.x, lane = t % kWave, wid = t / kWave;
+  const int m = a.m, N = (m + 1) & ~1, H = N / 2;
+  const int job = a.job[blockIdx.x], k = a.kept[blockIdx.x];
+  const double* cols = a.cols + job * a.job_stride;
+  double* theta = a.theta + job * a.theta_stride;
+  // the kept Ritz values, their couplings to the first new vector, and the
+  // projections onto the new vectors (the rest is rounding noise)
+  for (int e = t; e < N * N; e += kRitzThreads) {
+    const int i = min(e / N, e % N), j = max(e / N, e % N);
+    double v = 0.0;
+    if (j < k) v = i == j ? theta[j] : 0.0;
+    else if (j < m && (i >= k || j == k)) v = cols[j * a.ldc + i];
+    A[(e / N) * LD + e % N] = v;
+    U[(e / N) * LD + e % N] = e / N == e % N ? 1.0 : 0.0;
+  }
+  __syncthreads();
+  for (int sweep = 0; sweep < 64; ++sweep) {
+    double off = 0.0, tot = 0.0;
+    for (int e = t; e < N * N; e += kRitzThreads) {
+      const double v = A[(e / N) * LD + e % N] * A[(e / N) * LD + e % N];
+      tot += v;
+      if (e / N != e % N) off += v;
+    }
+    off = wave_sum(off);
+    tot = wave_sum(tot);
+    if (lane == 0) {
+      red[0][wid] = off;
+      red[1][wid] = tot;
+    }
+    __syncthreads();
+    off = tot = 0.0;
+#pragma unroll
+    for (int w = 0; w < kRitzThreads / kWave; ++w) {
+      off += red[0][w];
+      tot += red[1][w];
+    }
+    if (off == 0.0 || off <= 1e-32 * tot) break;  // the same in every thread
+    for (int r = 0; r < N - 1; ++r) {
+      // pair u of the round: the last index stays, the others go around
+      auto pair = [&](int u, int& p, int& q) {
+        p = r + u;
+        p = p >= N - 1 ? p - (N - 1) : p;
+        q = r - u;
+        q = u == 0 ? N - 1 : (q < 0 ? q + N - 1 : q);
+      };
+      if (t < H) {
+        int p, q;
+        pair(t, p, q);
+        const double apq = A[p * LD + q];
+        double2 cs = make_double2(1.0, 0.0);
+        if (apq != 0.0) {
+          const double th = (A[q * LD + q] - A[p * LD + p]) / (2.0 * apq);
+          const double tt = copysign(1.0, th) / (fabs(th) + sqrt(th * th + 1.0));
+          cs.x = 1.0 / sqrt(tt * tt + 1.0);
+          cs.y = tt * cs.x;
+        }
+        rot[t] = cs;
+      }
+      __syncthreads();
+      for (int e = t; e < H * H; e += kRitzThreads) {
+        const int x = e / H, y = e % H;
+        int p, q, u, v;
+        pair(x, p, q);
+        pair(y, u, v);
+        const double2 R = rot[x], C = rot[y];
+        const double pu = A[p * LD + u], pv = A[p * LD + v];
+        const double qu = A[q * LD + u], qv = A[q * LD + v];
+        const double pu1 = C.x * pu - C.y * pv, pv1 = C.y * pu + C.x * pv;
+        const double qu1 = C.x * qu - C.y * qv, qv1 = C.y * qu + C.x * qv;
+        A[p * LD + u] = R.x * pu1 - R.y * qu1;
+        A[q * LD + u] = x == y && R.y != 0.0 ? 0.0 : R.y * pu1 + R.x * qu1;
+        A[p * LD + v] = x == y && R.y != 0.0 ? 0.0 : R.x * pv1 - R.y * qv1;
+        A[q * LD + v] = R.y * pv1 + R.x * qv1;
+      }
+      for (int e = t; e < m * H; e += kRitzThreads) {
+        const int i = e / H, y = e % H;
+        int u, v;
+        pair(y, u, v);
+        const double2 C = rot[y];
+        const double iu = U[i * LD + u], iv = U[i * LD + v];
+        U[i * LD + u] = C.x * iu - C.y * iv;
+        U[i * LD + v] = C.y * iu + C.x * iv;
+      }
+      __syncthreads();
+    }
+  }
+  // ascending order (ties by index); NaN values share ranks, within m
+  double* Y = a.Y + job * a.y_stride;
+  for (int e = t; e < m * m; e += kRitzThreads) {
+    const int j = e / m, i = e % m;
+    const double d = A[j * LD + j];
+    int rank = 0;
+    for (int u = 0; u < m; ++u) {
+      const double du = A[u * LD + u];
+      rank += du < d || (du == d && u < j) ? 1 : 0;
+    }
+    Y[rank * m + i] = U[i * LD + j];
+    if (i == 0) {
+      theta[rank] = d;
+      a.out_theta[blockIdx.x * a.out_stride + rank] = d;
+    }
+    if (i == m - 1) a.out_last[blockIdx.x * a.out_stride + rank] = U[i * LD + j];
   }
 }
 
@@ -1822,11 +1948,19 @@ __global__ __launch_bounds__(kVecBlock) void k_combine(
       double acc[8];
 #pragma unroll
       for (int c = 0; c < 8; ++c) acc[c] = 0.0;
-      for (int j = 0; j < m; ++j) {
-        const double vj = V[j * ldv + i];
+      // eight columns' loads in flight (one at a time: 181 us for 20 columns of
+      // 2.76 M rows onto 7, where the bytes take about 120)
+      for (int j0 = 0; j0 < m; j0 += 8) {
+        double vj[8];
 #pragma unroll
-        for (int c = 0; c < 8; ++c)
-          if (c0 + c < k) acc[c] += vj * ys[(c0 + c) * m + j];
+        for (int j = 0; j < 8; ++j) vj[j] = j0 + j < m ? V[(j0 + j) * ldv + i] : 0.0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          if (j0 + j >= m) break;
+#pragma unroll
+          for (int c = 0; c < 8; ++c)
+            if (c0 + c < k) acc[c] += vj[j] * ys[(c0 + c) * m + j0 + j];
+        }
       }
 #pragma unroll
       for (int c = 0; c < 8; ++c)
@@ -2491,62 +2625,40 @@ int launch_axpy_norm(const double* alpha_dev, const double* v, double* u,
 }
 
 int max_vec_partials() { return 8192; }
-int multidot_partials() { return 1 << 17; }
+int gs_partials() { return kGsBlocks * (2 * kMaxCols + 1); }
 
-int launch_multidot(const double* V, int64_t ldv, int m, const double* w,
-                    int64_t n, double* partials, double* out, double* acc_out,
-                    hipStream_t s) {
-  if (m <= 0) return QSI_OK;
-  if (m > kMaxCols) {
-    set_error("launch_multidot: too many columns");
-    return QSI_E_INVALID;
-  }
-  // one partial per (workgroup, column): the caller's buffer holds
-  // multidot_partials() doubles
-  const int nb = std::max(1, std::min(proj_blocks(n), multidot_partials() / std::max(m, 1)));
-  hipLaunchKernelGGL(k_multidot, dim3(nb), dim3(kVecBlock), 0, s, V, ldv, m, w,
-                     n, partials);
-  QSI_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_finalize_cols, dim3(m), dim3(256), 0, s, partials, nb, m,
-                     out, acc_out);
-  QSI_CHECK_LAUNCH();
-  return QSI_OK;
-}
-
-int launch_gemv_sub(const double* V, int64_t ldv, int m, const double* h,
-                    double* w, int64_t n, hipStream_t s) {
-  if (m <= 0) return QSI_OK;
-  hipLaunchKernelGGL(k_gemv_sub, dim3(vec_blocks(n)), dim3(kVecBlock), 0, s, V,
-                     ldv, m, h, w, n);
-  QSI_CHECK_LAUNCH();
-  return QSI_OK;
-}
-
-int launch_gs_reorth(const double* V, int64_t ldv, int m, const double* h, double* w,
-                     int64_t n, double* partials, double* g, double* hcol, int* flag,
-                     double* beta, hipStream_t s) {
+int launch_gs_step(const double* V, int64_t ldv, int m, double* w, int64_t n, double* partials,
+                   double* hcol, double* beta, hipStream_t s) {
   if (m <= 0 || m > kMaxCols) {
-    set_error("launch_gs_reorth: column count out of range");
+    set_error("launch_gs_step: column count out of range");
     return QSI_E_INVALID;
   }
-  const int nb = std::max(1, std::min(proj_blocks(n), multidot_partials() / (m + 1)));
-  if (m <= 16)
-    hipLaunchKernelGGL(k_gemv_sub_dots<16>, dim3(nb), dim3(kVecBlock), 0, s, V, ldv, m, h, w, n,
-                       partials);
-  else if (m <= 32)
-    hipLaunchKernelGGL(k_gemv_sub_dots<32>, dim3(nb), dim3(kVecBlock), 0, s, V, ldv, m, h, w, n,
-                       partials);
-  else
-    hipLaunchKernelGGL(k_gemv_sub_dots<64>, dim3(nb), dim3(kVecBlock), 0, s, V, ldv, m, h, w, n,
-                       partials);
+  double* part2 = partials + static_cast<int64_t>(kGsBlocks) * kMaxCols;
+  auto blocks = [&](int T) {
+    return static_cast<int>(std::min<int64_t>((n + T - 1) / T, kGsBlocks));
+  };
+#define QSI_GS(T_, C_)                                                                           \
+  do {                                                                                           \
+    const dim3 nb(blocks(T_));                                                                   \
+    hipLaunchKernelGGL(k_gs_dots<T_>, nb, dim3(T_), 0, s, V, ldv, m, w, n, partials);            \
+    hipLaunchKernelGGL((k_gs_sub_dots<T_, C_>), nb, dim3(T_), 0, s, V, ldv, m, partials, hcol, w, \
+                       n, part2);                                                                \
+    hipLaunchKernelGGL(k_gs_tail<T_>, nb, dim3(T_), 0, s, V, ldv, m, part2, hcol, w, n, beta);   \
+  } while (0)
+  if (m <= 16) QSI_GS(512, 16);
+  else if (m <= 32) QSI_GS(512, 32);
+  else QSI_GS(256, 64);
+#undef QSI_GS
   QSI_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_finalize_cols, dim3(m + 1), dim3(256), 0, s, partials, nb, m + 1, g,
-                     static_cast<double*>(nullptr));
-  QSI_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_gs_tail, dim3(1), dim3(64), 0, s, g, m, hcol, flag, beta);
-  QSI_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_gemv_sub_scal, dim3(vec_blocks(n)), dim3(kVecBlock), 0, s, V, ldv, m, g,
-                     w, n, flag, beta);
+  return QSI_OK;
+}
+
+int launch_ritz(const RitzArgs& a, int n_jobs, hipStream_t s) {
+  if (n_jobs < 1 || n_jobs > kMaxCols || a.m < 1 || a.m > kRitzMax) {
+    set_error("launch_ritz: size out of range");
+    return QSI_E_INVALID;
+  }
+  hipLaunchKernelGGL(k_ritz, dim3(n_jobs), dim3(kRitzThreads), 0, s, a);
   QSI_CHECK_LAUNCH();
   return QSI_OK;
 }

@@ -207,9 +207,9 @@ int launch_apply_scaled(const qsi_op_s* op, const double* x, double* y,
 int64_t apply_num_blocks(const qsi_op_s* op);
 
 // streaming vector kernels; partial buffers need max_vec_partials() doubles
-// (multidot_partials() for launch_multidot)
+// (gs_partials() for launch_gs_step)
 int max_vec_partials();
-int multidot_partials();
+int gs_partials();
 int launch_dot(const double* a, const double* b, int64_t n, double* partials,
                double* out, hipStream_t s);
 int launch_axpy(double alpha, const double* x, double* y, int64_t n,
@@ -220,23 +220,39 @@ int launch_scal(double alpha, double* x, int64_t n, hipStream_t s);
 int launch_axpy_norm(const double* alpha_dev, const double* v, double* u,
                      int64_t n, double* partials, double* nrm_out,
                      hipStream_t s, const double* vs_dev = nullptr);
-// out[j] = V[:, j] . w for j < m (V column-major, ld ldv); acc_out += out
-int launch_multidot(const double* V, int64_t ldv, int m, const double* w,
-                    int64_t n, double* partials, double* out, double* acc_out,
-                    hipStream_t s);
-// w -= V[:, 0:m] h
-int launch_gemv_sub(const double* V, int64_t ldv, int m, const double* h,
-                    double* w, int64_t n, hipStream_t s);
-// Second and (when needed) third classical Gram-Schmidt passes of w against
-// V[:, 0:m] after a first pass gave h = V^T w: w -= V h with g[0..m) =
-// V^T w_new and g[m] = |w_new|^2 from the same read (g: m + 1 doubles); if
-// |g[0..m)| > 1e-12 |w_new| then w -= V g, g is added to hcol[0..m) and
-// flag[0] = 1.  beta[0] = |w| at the end, beta[1] = 1 / beta[0] (0 if w
-// vanishes), and w is scaled by beta[1] in the same final pass.  All on the
-// device (no host synchronisation).
-int launch_gs_reorth(const double* V, int64_t ldv, int m, const double* h, double* w,
-                     int64_t n, double* partials, double* g, double* hcol, int* flag,
-                     double* beta, hipStream_t s);
+// Classical Gram-Schmidt of w against V[:, 0:m] (column-major, ld ldv) in two
+// passes and, when they leave |V^T w| > 1e-12 |w|, a third: hcol[0..m) receives
+// the projections (the third pass's correction included), beta[0] = |w| at the
+// end, beta[1] = 1 / beta[0] (0 if w vanishes), and w is scaled by beta[1].
+// partials: gs_partials() doubles.  All on the device (no host
+// synchronisation).
+int launch_gs_step(const double* V, int64_t ldv, int m, double* w, int64_t n, double* partials,
+                   double* hcol, double* beta, hipStream_t s);
+
+// Rayleigh-Ritz of n_jobs thick-restart Lanczos matrices of order m <= kRitzMax,
+// one workgroup each.  Workgroup b takes job[b], whose kept[b] first vectors
+// are Ritz vectors of the values theta[job * theta_stride + i] and whose column
+// j >= kept[b] of projections starts at cols[job * job_stride + j * ldc].  It
+// writes the ascending eigenvalues to theta (of the job) and out_theta
+// (out_stride apart by workgroup), the eigenvectors to Y + job * y_stride
+// (column-major m x m) and their last components to out_last.
+constexpr int kRitzMax = 48;
+struct RitzArgs {
+  const double* cols;
+  int64_t job_stride;
+  int ldc;
+  int m;
+  double* theta;
+  int64_t theta_stride;
+  double* Y;
+  int64_t y_stride;
+  double* out_theta;
+  double* out_last;
+  int64_t out_stride;
+  uint8_t job[64], kept[64];
+};
+int launch_ritz(const RitzArgs& a, int n_jobs, hipStream_t s);
+
 // out[:, 0:k] = V[:, 0:m] Y  (Y m x k column-major, device)
 int launch_combine(const double* V, int64_t ldv, int m, const double* Y, int k,
                    double* out, int64_t ldo, int64_t n, hipStream_t s);

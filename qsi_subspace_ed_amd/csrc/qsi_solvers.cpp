@@ -496,19 +496,20 @@ int qsi_eigsh(qsi_op_t op, int nev, int ncv, double tol, int max_restarts,
   DevBuf bV, bW, bpart, bscal;
   QSI_CHECK_HIP(bV.alloc(static_cast<size_t>(ld) * (ncv + 1) * sizeof(double)));
   QSI_CHECK_HIP(bW.alloc(static_cast<size_t>(ld) * (ncv + 1) * sizeof(double)));
-  QSI_CHECK_HIP(bpart.alloc(std::max(max_vec_partials(), multidot_partials()) * sizeof(double)));
+  QSI_CHECK_HIP(bpart.alloc(std::max(max_vec_partials(), gs_partials()) * sizeof(double)));
   QSI_CHECK_HIP(bscal.alloc(4 * sizeof(double)));
   DevBuf bY;  // Ritz coefficients of a restart (at most ncv x ncv)
   QSI_CHECK_HIP(bY.alloc(static_cast<size_t>(ncv) * ncv * sizeof(double)));
-  // projected columns (ncv + 1 per step: h and, from pass 1, |w|^2), per-step
-  // beta and 1/beta, the fused pass's sums and the third-pass flag, all
-  // device-resident so a restart cycle runs without host synchronisation
-  const int colw = ncv + 1;
-  DevBuf bT, bbeta, bg, bflag;
-  QSI_CHECK_HIP(bT.alloc(static_cast<size_t>(ncv) * colw * sizeof(double)));
-  QSI_CHECK_HIP(bbeta.alloc(static_cast<size_t>(2 * ncv) * sizeof(double)));
-  QSI_CHECK_HIP(bg.alloc(80 * sizeof(double)));
-  QSI_CHECK_HIP(bflag.alloc(sizeof(int)));
+  // projected columns (ncv per step), per-step beta and 1/beta, the Ritz values
+  // and their vectors' last components, all device-resident so a restart cycle
+  // runs without host synchronisation, and in one piece so it takes one copy
+  const size_t n_T = static_cast<size_t>(ncv) * ncv;
+  DevBuf bx, btheta;
+  QSI_CHECK_HIP(bx.alloc((n_T + 4 * ncv) * sizeof(double)));
+  QSI_CHECK_HIP(btheta.alloc(ncv * sizeof(double)));
+  double* dT = bx.d();
+  double* dbeta = dT + n_T;
+  const bool dev_ritz = ncv <= kRitzMax;
   double* V = bV.d();
   double* W = bW.d();
   int applies = 0;
@@ -530,38 +531,42 @@ int qsi_eigsh(qsi_op_t op, int nev, int ncv, double tol, int max_restarts,
 
   std::vector<double> T(static_cast<size_t>(ncv) * ncv, 0.0);
   auto Tat = [&](int i, int j) -> double& { return T[static_cast<size_t>(j) * ncv + i]; };
-  std::vector<double> theta, Y;
+  std::vector<double> theta;
   int k = 0;       // kept (locked + thick) vectors
   int nconv = 0;
   int m = ncv;     // current basis size
   double beta_last = 0.0;
   bool exhausted = false;
-  std::vector<double> hT(static_cast<size_t>(ncv) * colw), hbeta(2 * ncv);
+  std::vector<double> hx(n_T + 4 * ncv);
+  const double* hbeta = hx.data() + n_T;
   for (int restart = 0;; ++restart) {
     m = ncv;
     // the cycle: steps k..ncv-1 write v_{j+1} straight into V[:, j+1]
     for (int j = k; j < ncv; ++j) {
       const double* vj = V + static_cast<int64_t>(j) * ld;
       double* w = V + static_cast<int64_t>(j + 1) * ld;
-      double* hcol = bT.d() + static_cast<size_t>(j) * colw;
+      double* hcol = dT + static_cast<size_t>(j) * ncv;
       QSI_TRY(launch_apply(op, vj, w, nullptr, 0.0, nullptr, nullptr, s));
       ++applies;
-      // pass 1: h = V[:, 0..j]^T w (and w . w: column j + 1 is w itself)
-      QSI_TRY(launch_multidot(V, ld, j + 2, w, D, bpart.d(), hcol, nullptr, s));
-      // pass 2 fused with the norm and the test for pass 3; the conditional
-      // third pass and the normalisation share one final pass
-      QSI_TRY(launch_gs_reorth(V, ld, j + 1, hcol, w, D, bpart.d(), bg.d(), hcol,
-                               static_cast<int*>(bflag.p), bbeta.d() + 2 * j, s));
+      QSI_TRY(launch_gs_step(V, ld, j + 1, w, D, bpart.d(), hcol, dbeta + 2 * j, s));
     }
-    QSI_CHECK_HIP(hipMemcpyAsync(hT.data() + static_cast<size_t>(k) * colw,
-                                 bT.d() + static_cast<size_t>(k) * colw,
-                                 static_cast<size_t>(ncv - k) * colw * sizeof(double),
-                                 hipMemcpyDeviceToHost, s));
-    QSI_CHECK_HIP(hipMemcpyAsync(hbeta.data(), bbeta.d(), 2 * ncv * sizeof(double),
+    if (dev_ritz) {
+      RitzArgs r{};
+      r.cols = dT;
+      r.ldc = ncv;
+      r.m = ncv;
+      r.theta = btheta.d();
+      r.Y = bY.d();
+      r.out_theta = dbeta + 2 * ncv;
+      r.out_last = dbeta + 3 * ncv;
+      r.kept[0] = static_cast<uint8_t>(k);
+      QSI_TRY(launch_ritz(r, 1, s));
+    }
+    QSI_CHECK_HIP(hipMemcpyAsync(hx.data(), dT, hx.size() * sizeof(double),
                                  hipMemcpyDeviceToHost, s));
     QSI_CHECK_HIP(hipStreamSynchronize(s));
     for (int j = k; j < ncv; ++j) {
-      const double* hh = hT.data() + static_cast<size_t>(j) * colw;
+      const double* hh = hx.data() + static_cast<size_t>(j) * ncv;
       for (int i = 0; i <= j; ++i) {
         if (i < k && j == k) {
           Tat(i, j) = Tat(j, i) = hh[i];  // coupling to the kept Ritz vectors
@@ -582,16 +587,26 @@ int qsi_eigsh(qsi_op_t op, int nev, int ncv, double tol, int max_restarts,
       }
       beta_last = beta;
     }
-    // Rayleigh-Ritz on the m x m projected matrix
-    std::vector<double> Tm(static_cast<size_t>(m) * m);
-    for (int j = 0; j < m; ++j)
-      for (int i = 0; i < m; ++i) Tm[static_cast<size_t>(j) * m + i] = Tat(i, j);
-    hostla::sym_eig(Tm, m, theta, Y);
+    // Rayleigh-Ritz on the m x m projected matrix: the device's, or here where
+    // the subspace ended early or is larger than the device kernel takes
+    std::vector<double> last(m);
+    if (dev_ritz && m == ncv) {
+      theta.assign(hbeta + 2 * ncv, hbeta + 3 * ncv);
+      last.assign(hbeta + 3 * ncv, hbeta + 4 * ncv);
+    } else {
+      std::vector<double> Tm(static_cast<size_t>(m) * m), Y;
+      for (int j = 0; j < m; ++j)
+        for (int i = 0; i < m; ++i) Tm[static_cast<size_t>(j) * m + i] = Tat(i, j);
+      hostla::sym_eig(Tm, m, theta, Y);
+      for (int i = 0; i < m; ++i) last[i] = Y[static_cast<size_t>(i) * m + (m - 1)];
+      // Y goes away with this scope
+      QSI_CHECK_HIP(hipMemcpy(bY.d(), Y.data(), Y.size() * sizeof(double), hipMemcpyHostToDevice));
+    }
     const double eps23 = std::pow(std::numeric_limits<double>::epsilon(), 2.0 / 3.0);
     const int want = std::min(nev, m);
     nconv = 0;
     for (int i = 0; i < want; ++i) {
-      const double resid = beta_last * std::fabs(Y[static_cast<size_t>(i) * m + (m - 1)]);
+      const double resid = beta_last * std::fabs(last[i]);
       if (resid < tol * std::max(eps23, std::fabs(theta[i]))) ++nconv;
       else break;  // count the leading converged run
     }
@@ -599,15 +614,11 @@ int qsi_eigsh(qsi_op_t op, int nev, int ncv, double tol, int max_restarts,
     // thick restart: keep the k lowest Ritz vectors plus the residual vector
     int kn = nev + std::min(nconv, (m - nev) / 2);
     kn = std::max(1, std::min(kn, m - 1));
-    std::vector<double> Yk(Y.begin(), Y.begin() + static_cast<size_t>(kn) * m);
-    QSI_CHECK_HIP(hipMemcpyAsync(bY.d(), Yk.data(), Yk.size() * sizeof(double),
-                                 hipMemcpyHostToDevice, s));
     QSI_TRY(launch_combine(V, ld, m, bY.d(), kn, W, ld, D, s));
     QSI_CHECK_HIP(hipMemcpyAsync(W + static_cast<int64_t>(kn) * ld,
                                  V + static_cast<int64_t>(m) * ld,
                                  static_cast<size_t>(D) * sizeof(double),
                                  hipMemcpyDeviceToDevice, s));
-    QSI_CHECK_HIP(hipStreamSynchronize(s));
     std::swap(V, W);
     std::fill(T.begin(), T.end(), 0.0);
     for (int i = 0; i < kn; ++i) Tat(i, i) = theta[i];
@@ -618,9 +629,6 @@ int qsi_eigsh(qsi_op_t op, int nev, int ncv, double tol, int max_restarts,
     h_evals[i] = i < nout ? theta[i] : std::numeric_limits<double>::quiet_NaN();
   if (n_evecs > 0) {
     const int ne = std::min(n_evecs, m);
-    std::vector<double> Yk(Y.begin(), Y.begin() + static_cast<size_t>(ne) * m);
-    QSI_CHECK_HIP(hipMemcpyAsync(bY.d(), Yk.data(), Yk.size() * sizeof(double),
-                                 hipMemcpyHostToDevice, s));
     QSI_TRY(launch_combine(V, ld, m, bY.d(), ne, d_evecs, D, D, s));
     QSI_CHECK_HIP(hipStreamSynchronize(s));
   }

@@ -1,0 +1,48 @@
+"""The thick-restart solver's device passes at their edges, against a dense
+diagonalisation: search spaces on both sides of the projection kernels' 16 and
+32 columns and of the device Rayleigh-Ritz's 48, odd and even orders, the
+smallest ones, bases below one workgroup's rows and beyond, and subspaces that end
+early.  The solver stops at a relative residual of 1e-10: eigenvalues lie within
+that of the exact ones (times the norm of H), and vectors with a gap to the rest
+of the spectrum within 1e-10 * |H| / gap, checked as residuals below 1e-9 |H|."""
+import numpy as np
+import pytest
+
+import qsi_subspace_ed_amd as q
+from test_gpu_window import _basis, _terms
+
+pytestmark = pytest.mark.gpu
+
+
+def _dense(op):
+    r, c, v, d = op.connectivity()
+    A = np.diag(d).astype(np.float64)
+    np.add.at(A, (r, c), v)
+    return A
+
+
+@pytest.mark.parametrize("bits,keep", [(6, 40), (9, 500), (9, 512), (10, 513), (11, 1500)])
+@pytest.mark.parametrize("nev,ncv", [(1, 2), (1, 3), (2, 9), (3, 15), (5, 16), (5, 17), (6, 24),
+                                     (4, 32), (4, 33), (8, 47), (8, 48), (8, 49), (10, 63)])
+def test_lowest(cuda, bits, keep, nev, ncv):
+    if ncv < 9 and keep > 64:
+        keep, bits = 64, 6  # a search in two or three vectors takes hundreds of restarts
+    states, spins, W = _basis(1, bits, keep, keep)
+    H = _terms(spins, 24, bits, z=False, open_spins=False)
+    # a diagonal without repeated values: no degenerate levels
+    from qsi_subspace_ed_amd.operators import SymbolicPMROperator
+    for k, p in enumerate(spins):
+        H.add_term(0.37 * 1.61 ** (k % 7) + 0.011 * k, SymbolicPMROperator.from_ops("z", [p]))
+    op = q.GpuOp(q.GpuBasis(states, W), H)
+    A = _dense(op)
+    assert np.array_equal(A, A.T)  # every term is followed by its conjugate
+    want = np.linalg.eigvalsh(A)
+    norm = np.abs(want).max()
+    n = min(nev, keep - 1)
+    evals, vecs, _, _ = op.eigsh(nev=nev, ncv=ncv, tol=1e-10, max_restarts=20000, seed=3, n_evecs=n)
+    assert np.abs(evals[:n] - want[:n]).max() <= 1e-9 * norm
+    V = vecs.cpu().numpy()
+    for i in range(n):
+        v = V[:, i]
+        assert abs(np.linalg.norm(v) - 1.0) <= 1e-9
+        assert np.linalg.norm(A @ v - evals[i] * v) <= 1e-9 * norm
