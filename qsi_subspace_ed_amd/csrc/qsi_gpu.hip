@@ -1637,50 +1637,7 @@ constexpr int kMaxCols = 64;
 // the reads of V bound passes 1 and 2 (42 and 48 us, 5.4 TB/s), and 256
 // workgroups of 512 threads keep enough of them in flight.
 // partials[j * gridDim.x + workgroup] is column j's.
-constexpr int kGsBlocks = 256;
-
-// Sums N values per lane over the wavefront by halving: lane l returns the
-// total of value l / (64 / N), in 2 N exchanges fewer than N full butterflies.
-template <int N, int O = kWave / 2>
-__device__ __forceinline__ double wave_sum_many(double* v, int lane) {
-  static_assert(N <= kWave && (N & (N - 1)) == 0);
-  if constexpr (N > 1) {
-    const bool up = (lane & O) != 0;
-#pragma unroll
-    for (int i = 0; i < N / 2; ++i) {
-      const double send = up ? v[i] : v[i + N / 2];
-      const double keep = up ? v[i + N / 2] : v[i];
-      v[i] = keep + __shfl_xor(send, O, kWave);
-    }
-    return wave_sum_many<N / 2, O / 2>(v, lane);
-  } else {
-    double t = v[0];
-#pragma unroll
-    for (int o = O; o > 0; o >>= 1) t += __shfl_xor(t, o, kWave);
-    return t;
-  }
-}
-
-// out[j] (LDS) = sum_b partials[j * nb + b] for j < m, by the whole workgroup
-// of T threads; ends with a barrier.
-template <int T>
-__device__ __forceinline__ void sum_partials(const double* __restrict__ partials, int nb, int m,
-                                             double* out) {
-  constexpr int W = T / kWave;
-  static_assert(kGsBlocks <= 4 * kWave);
-  const int lane = threadIdx.x % kWave;
-  for (int j = threadIdx.x / kWave; j < m; j += W) {
-    double v[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const int b = lane + k * kWave;
-      v[k] = b < nb ? partials[j * nb + b] : 0.0;
-    }
-    const double t = wave_sum((v[0] + v[1]) + (v[2] + v[3]));
-    if (lane == 0) out[j] = t;
-  }
-  __syncthreads();
-}
+constexpr int kGsBlocks = kSumBlocks;
 
 // Pass 1: partials of V[:, 0:m]^T w, 16 columns at a time.
 template <int T>
@@ -1816,12 +1773,17 @@ __global__ __launch_bounds__(T) void k_gs_tail(
 
 // ---- Rayleigh-Ritz of the thick-restart solvers -----------------------------
 // One workgroup per projected matrix (RitzArgs): all eigenpairs by Jacobi
-// rotations, kRitzThreads threads, matrix and vectors in LDS.  A sweep is N - 1
-// rounds of N / 2 rotations on disjoint index pairs (round robin), so a round
-// is one barrier for the angles and one for the 2 x 2 blocks of J^T A J and the
-// vectors' columns, where a cyclic sweep is N (N - 1) / 2 rotations one after
-// the other (20 to 24 vectors: about 300 us on a host core while the device
-// idles, 70 us here, and the vectors need not be sent back).
+// rotations, matrix and vectors in LDS.  A sweep is N - 1 rounds of N / 2
+// rotations on disjoint index pairs (round robin), where a cyclic sweep is
+// N (N - 1) / 2 rotations one after the other.  A round is a chain of latencies
+// (LDS, the angle, two barriers), about 0.6 us; an angle need only be near the
+// one that annihilates its element (hardware reciprocals, about 26 bits): what
+// must be exact is c^2 + s^2 = 1, one Newton step of third order for c.  Blocks
+// on and above the diagonal are computed and mirrored: a matrix that rounding
+// makes unsymmetric keeps that difference in every rotation and never gets
+// diagonal.  Orders 8, 16, 24, 32: 30, 65, 120, 175 us; one matrix of order 15
+// takes 95 us on a host core, of order 20 to 24 about 300, while the device
+// idles.
 constexpr int kRitzThreads = 256;
 __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
   constexpr int LD = kRitzMax + 1;
@@ -1831,6 +1793,9 @@ __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
   __shared__ double red[2][kRitzThreads / kWave];
   const int t = threadIdx.x, lane = t % kWave, wid = t / kWave;
   const int m = a.m, N = (m + 1) & ~1, H = N / 2;
+  // thread (x0, y): pairs or rows x0, x0 + xs, ... and pair y of each round
+  const int lp = 32 - __builtin_clz(static_cast<unsigned>(max(H - 1, 1)));
+  const int y = t & ((1 << lp) - 1), x0 = t >> lp, xs = kRitzThreads >> lp;
   const int job = a.job[blockIdx.x], k = a.kept[blockIdx.x];
   const double* cols = a.cols + job * a.job_stride;
   double* theta = a.theta + job * a.theta_stride;
@@ -1847,10 +1812,14 @@ __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
   __syncthreads();
   for (int sweep = 0; sweep < 64; ++sweep) {
     double off = 0.0, tot = 0.0;
-    for (int e = t; e < N * N; e += kRitzThreads) {
-      const double v = A[(e / N) * LD + e % N] * A[(e / N) * LD + e % N];
-      tot += v;
-      if (e / N != e % N) off += v;
+    for (int x = x0; x < N && y < H; x += xs) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int z = 2 * y + h;
+        const double v = A[x * LD + z] * A[x * LD + z];
+        tot += v;
+        if (x != z) off += v;
+      }
     }
     off = wave_sum(off);
     tot = wave_sum(tot);
@@ -1877,40 +1846,45 @@ __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
       if (t < H) {
         int p, q;
         pair(t, p, q);
-        const double apq = A[p * LD + q];
+        // tt = tan of the smaller angle that annihilates A[p][q]
+        const double b = 2.0 * A[p * LD + q], d = A[q * LD + q] - A[p * LD + p];
+        const double h2 = d * d + b * b;
+        const double den = fabs(d) + h2 * __builtin_amdgcn_rsq(h2);
+        const double tt = (d < 0.0 ? -b : b) * __builtin_amdgcn_rcp(den);
         double2 cs = make_double2(1.0, 0.0);
-        if (apq != 0.0) {
-          const double th = (A[q * LD + q] - A[p * LD + p]) / (2.0 * apq);
-          const double tt = copysign(1.0, th) / (fabs(th) + sqrt(th * th + 1.0));
-          cs.x = 1.0 / sqrt(tt * tt + 1.0);
+        if (fabs(tt) < 2.0) {  // not for a vanishing or overflowing h2
+          const double z = tt * tt + 1.0, g = __builtin_amdgcn_rsq(z);
+          const double er = fma(-z * g, g, 1.0);
+          cs.x = fma(g * er, fma(0.375, er, 0.5), g);
           cs.y = tt * cs.x;
         }
         rot[t] = cs;
       }
       __syncthreads();
-      for (int e = t; e < H * H; e += kRitzThreads) {
-        const int x = e / H, y = e % H;
-        int p, q, u, v;
-        pair(x, p, q);
-        pair(y, u, v);
-        const double2 R = rot[x], C = rot[y];
-        const double pu = A[p * LD + u], pv = A[p * LD + v];
-        const double qu = A[q * LD + u], qv = A[q * LD + v];
-        const double pu1 = C.x * pu - C.y * pv, pv1 = C.y * pu + C.x * pv;
-        const double qu1 = C.x * qu - C.y * qv, qv1 = C.y * qu + C.x * qv;
-        A[p * LD + u] = R.x * pu1 - R.y * qu1;
-        A[q * LD + u] = x == y && R.y != 0.0 ? 0.0 : R.y * pu1 + R.x * qu1;
-        A[p * LD + v] = x == y && R.y != 0.0 ? 0.0 : R.x * pv1 - R.y * qv1;
-        A[q * LD + v] = R.y * pv1 + R.x * qv1;
-      }
-      for (int e = t; e < m * H; e += kRitzThreads) {
-        const int i = e / H, y = e % H;
+      if (y < H) {
         int u, v;
         pair(y, u, v);
         const double2 C = rot[y];
-        const double iu = U[i * LD + u], iv = U[i * LD + v];
-        U[i * LD + u] = C.x * iu - C.y * iv;
-        U[i * LD + v] = C.y * iu + C.x * iv;
+        for (int x = x0; x <= y; x += xs) {
+          int p, q;
+          pair(x, p, q);
+          const double2 R = rot[x];
+          const double pu = A[p * LD + u], pv = A[p * LD + v];
+          const double qu = A[q * LD + u], qv = A[q * LD + v];
+          const double pu1 = C.x * pu - C.y * pv, pv1 = C.y * pu + C.x * pv;
+          const double qu1 = C.x * qu - C.y * qv, qv1 = C.y * qu + C.x * qv;
+          const double a00 = R.x * pu1 - R.y * qu1, a10 = R.y * pu1 + R.x * qu1;
+          const double a01 = R.x * pv1 - R.y * qv1, a11 = R.y * pv1 + R.x * qv1;
+          A[p * LD + u] = A[u * LD + p] = a00;
+          A[p * LD + v] = A[v * LD + p] = a01;
+          A[q * LD + v] = A[v * LD + q] = a11;
+          if (x != y) A[q * LD + u] = A[u * LD + q] = a10;
+        }
+        for (int x = x0; x < m; x += xs) {
+          const double iu = U[x * LD + u], iv = U[x * LD + v];
+          U[x * LD + u] = C.x * iu - C.y * iv;
+          U[x * LD + v] = C.y * iu + C.x * iv;
+        }
       }
       __syncthreads();
     }

@@ -80,4 +80,48 @@ __global__ __launch_bounds__(BLOCK) void k_sum_chunks(double* partials, int64_t 
   if (threadIdx.x == 0) partials[lo] = v;
 }
 
+// Sums N values per lane over the wavefront by halving: lane l returns the
+// total of value l / (64 / N), in 2 N exchanges fewer than N full butterflies.
+template <int N, int O = kWave / 2>
+__device__ __forceinline__ double wave_sum_many(double* v, int lane) {
+  static_assert(N <= kWave && (N & (N - 1)) == 0);
+  if constexpr (N > 1) {
+    const bool up = (lane & O) != 0;
+#pragma unroll
+    for (int i = 0; i < N / 2; ++i) {
+      const double send = up ? v[i] : v[i + N / 2];
+      const double keep = up ? v[i + N / 2] : v[i];
+      v[i] = keep + __shfl_xor(send, O, kWave);
+    }
+    return wave_sum_many<N / 2, O / 2>(v, lane);
+  } else {
+    double t = v[0];
+#pragma unroll
+    for (int o = O; o > 0; o >>= 1) t += __shfl_xor(t, o, kWave);
+    return t;
+  }
+}
+
+// out[j] (LDS) = sum_b partials[j * nb + b] for j < m, nb <= kSumBlocks, by the
+// whole workgroup of T threads; ends with a barrier.
+constexpr int kSumBlocks = 256;
+template <int T>
+__device__ __forceinline__ void sum_partials(const double* __restrict__ partials, int nb, int m,
+                                             double* out) {
+  constexpr int W = T / kWave;
+  static_assert(kSumBlocks <= 4 * kWave);
+  const int lane = threadIdx.x % kWave;
+  for (int j = threadIdx.x / kWave; j < m; j += W) {
+    double v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int b = lane + k * kWave;
+      v[k] = b < nb ? partials[j * nb + b] : 0.0;
+    }
+    const double t = wave_sum((v[0] + v[1]) + (v[2] + v[3]));
+    if (lane == 0) out[j] = t;
+  }
+  __syncthreads();
+}
+
 }  // namespace qsi

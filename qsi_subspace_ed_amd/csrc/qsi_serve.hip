@@ -38,15 +38,16 @@ namespace qsi {
 namespace {
 
 constexpr int kSrvThreads = 256;
-// rows per workgroup of the reorthogonalisation kernels: D / 256 rounded up
-// to a multiple of 64, between 256 and 2048 (small bases still get many
-// workgroups; the grid stays a few hundred workgroups per column)
+// rows per workgroup of the reorthogonalisation kernels: D / kSumBlocks rounded
+// up to a multiple of 64, at least 256, so a column has at most kSumBlocks
+// workgroups and the next kernel's workgroups can add up their partials
+// themselves (kernels of their own for the sums, the norms, the flags and the
+// results were six of a step's twelve launches, 4 us each)
 constexpr int kSrvRowsMin = 256;
-constexpr int kSrvRowsMax = 2048;
 constexpr int kHMax = 64;
 // partials slot holding |u|^2 (projections use slots 0..ncv-1 <= 62)
 constexpr int kNormSlot = kHMax - 1;
-// the second Gram-Schmidt pass runs when |h2|^2 > kReorthTol2 |u|^2
+// the last Gram-Schmidt pass runs when |h2|^2 > kReorthTol2 |u|^2
 constexpr double kReorthTol2 = 1e-24;
 
 // Start of a step: for every apply slot sl < n_act (column c = slotcol[sl]),
@@ -90,11 +91,16 @@ __device__ __forceinline__ void srv_block_dots(double (&acc)[MMAX], int m, int c
                                                double* __restrict__ partials) {
   __shared__ double red[kSrvThreads / 64][MMAX];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  if constexpr ((MMAX & (MMAX - 1)) == 0) {
+    const double v = wave_sum_many<MMAX>(acc, lane);
+    if (lane % (64 / MMAX) == 0) red[wid][lane / (64 / MMAX)] = v;
+  } else {
 #pragma unroll
-  for (int i = 0; i < MMAX; ++i) {
-    if (i < m) {
-      const double v = wave_sum(acc[i]);
-      if (lane == 0) red[wid][i] = v;
+    for (int i = 0; i < MMAX; ++i) {
+      if (i < m) {
+        const double v = wave_sum(acc[i]);
+        if (lane == 0) red[wid][i] = v;
+      }
     }
   }
   __syncthreads();
@@ -141,6 +147,25 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_mdot(
   srv_block_dots<MMAX>(acc, m, c, gridDim.x, partials);
 }
 
+// hs[i] = vs_i h_i for i < m (0 up to MMAX), h_i = vs_i times pass 1's sum of
+// partials i; the column's first workgroup writes h to hacc.  Ends with a
+// barrier.
+template <int MMAX>
+__device__ __forceinline__ void srv_first_sums(const double* __restrict__ part1, int c, int m,
+                                               const double* __restrict__ vs,
+                                               double* __restrict__ hacc, double (&hs)[MMAX]) {
+  const int t = threadIdx.x;
+  if (t < MMAX) hs[t] = 0.0;
+  __syncthreads();
+  sum_partials<kSrvThreads>(part1 + static_cast<int64_t>(c) * kHMax * gridDim.x, gridDim.x, m, hs);
+  if (t < m) {
+    const double sc = vs[c * kHMax + t], v = hs[t] * sc;
+    if (blockIdx.x == 0) hacc[c * kHMax + t] = v;
+    hs[t] = v * sc;
+  }
+  __syncthreads();
+}
+
 // pass 1 -> 2: u_c = w_c - V_c h_c (h from pass 1) written to V_c[j_c + 1],
 // then partials of V_c^T u_c (slots 0..j_c) and of |u_c|^2 (kNormSlot).
 // Grid (nblk, n_act).  The block walks its rows in 64-row tiles; wave k holds
@@ -148,9 +173,10 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_mdot(
 // (V h)[row] meet in LDS, and each wave reuses its V entries for the dots.
 template <int MMAX>
 __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot(
-    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ h,
-    const double* __restrict__ vs, const int* __restrict__ colj, const int* __restrict__ slotcol,
-    int64_t D, int rpb, const double* __restrict__ Wc, double* __restrict__ partials) {
+    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ part1,
+    double* __restrict__ hacc, const double* __restrict__ vs, const int* __restrict__ colj,
+    const int* __restrict__ slotcol, int64_t D, int rpb, const double* __restrict__ Wc,
+    double* __restrict__ partials) {
   constexpr int NWV = kSrvThreads / 64;
   constexpr int Q = (MMAX + NWV - 1) / NWV;
   const int sl = blockIdx.y;
@@ -162,8 +188,7 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot(
   __shared__ double red[MMAX];
   __shared__ double nsh;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  if (threadIdx.x < m) hs[threadIdx.x] = h[c * kHMax + threadIdx.x] * vs[c * kHMax + threadIdx.x];
-  __syncthreads();
+  srv_first_sums<MMAX>(part1, c, m, vs, hacc, hs);
   const double* V = Vb + static_cast<int64_t>(c) * ncv1 * ld;
   double* out = Vb + (static_cast<int64_t>(c) * ncv1 + m) * ld;
   const double* w = Wc + static_cast<int64_t>(sl) * ld;
@@ -223,17 +248,22 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot(
 // (no workgroup barrier per row tile).
 template <int MMAX>
 __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot_rows(
-    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ h,
-    const double* __restrict__ vs, const int* __restrict__ colj, const int* __restrict__ slotcol,
-    int64_t D, int rpb, const double* __restrict__ Wc, double* __restrict__ partials) {
+    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ part1,
+    double* __restrict__ hacc, const double* __restrict__ vs, const int* __restrict__ colj,
+    const int* __restrict__ slotcol, int64_t D, int rpb, const double* __restrict__ Wc,
+    double* __restrict__ partials) {
   const int sl = blockIdx.y;
   const int c = slotcol[sl];
   const int m = colj[c] + 1;
-  // h in registers (uniform); entries i >= m are zero, so the loops below
-  // run unpredicated
+  __shared__ double hs[MMAX];
+  srv_first_sums<MMAX>(part1, c, m, vs, hacc, hs);
+  // h in scalar registers; entries i >= m are zero, so the loops below run
+  // unpredicated
   double hr[MMAX];
 #pragma unroll
-  for (int i = 0; i < MMAX; ++i) hr[i] = i < m ? h[c * kHMax + i] * vs[c * kHMax + i] : 0.0;
+  for (int i = 0; i < MMAX; ++i)
+    hr[i] = __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(hs[i])),
+                             __builtin_amdgcn_readfirstlane(__double2loint(hs[i])));
   const double* V = Vb + static_cast<int64_t>(c) * ncv1 * ld;
   double* out = Vb + (static_cast<int64_t>(c) * ncv1 + m) * ld;
   const double* w = Wc + static_cast<int64_t>(sl) * ld;
@@ -263,17 +293,27 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot_rows(
     partials[(static_cast<int64_t>(c) * kHMax + kNormSlot) * gridDim.x + blockIdx.x] = nrm;
 }
 
-// Thick restart of one column, in place: row by row, V[0..kn) = v[0..m) Y
-// (Y column-major m x kn; v_i = vsc_i V[i]) and V[kn] = V[m] (the residual
-// direction, unscaled).  Every thread reads its row's m + 1 entries before
-// writing any of them.
+// The columns of one round of thick restarts: column c keeps kn of its m
+// vectors.
+struct Restarts {
+  uint8_t c[64], m[64], kn[64];
+};
+
+// Thick restart of column q.c[blockIdx.y], in place: row by row, V[0..kn) =
+// v[0..m) Y (Y column-major m x kn; v_i = vsc_i V[i]) and V[kn] = V[m] (the
+// residual direction, unscaled).  Every thread reads its row's m + 1 entries
+// before writing any of them.
 template <int MMAX>
-__global__ __launch_bounds__(kSrvThreads) void k_srv_restart(double* __restrict__ V, int64_t ld,
-                                                              int m, int kn,
-                                                              const double* __restrict__ Y,
-                                                              const double* __restrict__ vsc,
+__global__ __launch_bounds__(kSrvThreads) void k_srv_restart(double* __restrict__ Vb, int64_t ld,
+                                                              int ncv1, Restarts q,
+                                                              const double* __restrict__ Yb,
+                                                              const double* __restrict__ vs,
                                                               int64_t D) {
   __shared__ double ys[MMAX * MMAX];
+  const int c = q.c[blockIdx.y], m = q.m[blockIdx.y], kn = q.kn[blockIdx.y];
+  double* V = Vb + static_cast<int64_t>(c) * ncv1 * ld;
+  const double* Y = Yb + static_cast<int64_t>(c) * kHMax * kHMax;
+  const double* vsc = vs + c * kHMax;
   for (int t = threadIdx.x; t < m * kn; t += kSrvThreads) ys[t] = Y[t] * vsc[t % m];
   __syncthreads();
   for (int64_t r = static_cast<int64_t>(blockIdx.x) * kSrvThreads + threadIdx.x; r < D;
@@ -296,57 +336,55 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_restart(double* __restrict_
   }
 }
 
-// After pass 2's projections h2_c are summed: beta_c = |u_c| from the
-// kNormSlot partials, the scale 1/beta_c of the new vector u_c, and flag_c = 1
-// when |h2_c|^2 > kReorthTol2 |u_c|^2 (u_c needs the second Gram-Schmidt
-// pass).  Grid R, one wave each.
-__global__ void k_srv_check(const double* __restrict__ partials, int nblk,
-                            const int* __restrict__ colj, const double* __restrict__ h,
-                            int* __restrict__ flag, double* __restrict__ beta,
-                            double* __restrict__ vs) {
-  const int c = blockIdx.x;
-  const int j = colj[c];
-  if (j < 0) return;
-  double n2 = 0.0;
-  for (int b = threadIdx.x; b < nblk; b += 64)
-    n2 += partials[(static_cast<int64_t>(c) * kHMax + kNormSlot) * nblk + b];
-  n2 = wave_sum(n2);
+// The tail of the step, grid (any, n_act): pass 2's projections h2_c and norm
+// |u_c|^2 from its partials; where |h2_c|^2 > kReorthTol2 |u_c|^2 the last
+// Gram-Schmidt pass u_c -= V_c h2_c in place in V_c[j_c + 1], and the norm
+// follows it.  The column's first workgroup writes the step's results: the
+// projections (both passes) to column j_c of T_c on the device and, with
+// beta_c = |u_c|, straight into mapped pinned memory (hh: R x kHMax, bb: R; no
+// copy engine), and the scale 1/beta_c of the new vector.
+template <int MMAX>
+__global__ __launch_bounds__(kSrvThreads) void k_srv_tail(
+    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ part2, int nblk,
+    const double* __restrict__ hacc, double* __restrict__ vs, const int* __restrict__ colj,
+    const int* __restrict__ slotcol, int64_t D, double* __restrict__ T, double* hh, double* bb) {
+  const int c = slotcol[blockIdx.y];
+  const int j = colj[c], m = j + 1;
+  __shared__ double hs[MMAX], nsum[1];
+  const int t = threadIdx.x;
+  if (t < MMAX) hs[t] = 0.0;
+  const double* p = part2 + static_cast<int64_t>(c) * kHMax * nblk;
+  sum_partials<kSrvThreads>(p + static_cast<int64_t>(kNormSlot) * nblk, nblk, 1, nsum);
+  sum_partials<kSrvThreads>(p, nblk, m, hs);
   double s2 = 0.0;
-  for (int i = threadIdx.x; i <= j; i += 64) {
-    const double v = h[c * kHMax + i];
+  for (int i = 0; i < m; ++i) {
+    const double v = hs[i] * vs[c * kHMax + i];
     s2 += v * v;
   }
-  s2 = wave_sum(s2);
-  if (threadIdx.x == 0) {
-    flag[c] = s2 > kReorthTol2 * n2 ? 1 : 0;
-    const double r = sqrt(n2);
-    beta[c] = r;
-    vs[c * kHMax + j + 1] = r > 1e-300 ? 1.0 / r : 0.0;
+  const double n2 = nsum[0];
+  const bool flag = s2 > kReorthTol2 * n2;
+  const double h2 = t < m ? hs[t] * vs[c * kHMax + t] : 0.0;
+  if (blockIdx.x == 0) {
+    if (t < m) {
+      const double v = hacc[c * kHMax + t] + h2;
+      T[(static_cast<int64_t>(c) * kHMax + j) * kHMax + t] = v;
+      hh[c * kHMax + t] = v;
+    }
+    if (t == 0) {
+      const double b2 = flag ? n2 - s2 : n2;
+      const double r = b2 > 0.0 ? sqrt(b2) : (b2 <= 0.0 ? 0.0 : b2);  // NaN stays
+      bb[c] = r;
+      vs[c * kHMax + j + 1] = r > 1e-300 ? 1.0 / r : 0.0;
+    }
   }
-}
-
-// pass 3, flagged columns only: u_c -= V_c h2_c in place in V_c[j_c + 1],
-// partials of |u_c|^2 in partials[c*nblk + b].  Grid (nblk, n_act).
-template <int MMAX>
-__global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_norm(
-    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ h,
-    const double* __restrict__ vs, const int* __restrict__ colj,
-    const int* __restrict__ slotcol, const int* __restrict__ flag, int64_t D, int rpb,
-    double* __restrict__ partials) {
-  const int c = slotcol[blockIdx.y];
-  if (!flag[c]) return;
-  const int m = colj[c] + 1;
-  __shared__ double hs[MMAX];
-  if (threadIdx.x < MMAX)
-    hs[threadIdx.x] =
-        threadIdx.x < m ? h[c * kHMax + threadIdx.x] * vs[c * kHMax + threadIdx.x] : 0.0;
+  if (!flag) return;
+  __syncthreads();
+  if (t < m) hs[t] = h2 * vs[c * kHMax + t];
   __syncthreads();
   const double* V = Vb + static_cast<int64_t>(c) * ncv1 * ld;
   double* u = Vb + (static_cast<int64_t>(c) * ncv1 + m) * ld;
-  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rpb;
-  const int64_t r1 = min<int64_t>(r0 + rpb, D);
-  double nrm = 0.0;
-  for (int64_t r = r0 + threadIdx.x; r < r1; r += kSrvThreads) {
+  for (int64_t r = static_cast<int64_t>(blockIdx.x) * kSrvThreads + t; r < D;
+       r += static_cast<int64_t>(gridDim.x) * kSrvThreads) {
     double a = 0.0;
     if constexpr (MMAX <= 32) {
       // all loads first, then the sum in column order (absent columns load
@@ -361,59 +399,8 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_norm(
       for (int i = 0; i < MMAX; ++i)
         if (i < m) a += V[i * ld + r] * hs[i];
     }
-    const double ur = u[r] - a;
-    u[r] = ur;
-    nrm += ur * ur;
+    u[r] -= a;
   }
-  nrm = block_sum<kSrvThreads>(nrm);
-  if (threadIdx.x == 0) partials[static_cast<int64_t>(c) * gridDim.x + blockIdx.x] = nrm;
-}
-
-// h[c*kHMax + i] = vs_i * sum_b partials (fixed order); acc[c*kHMax + i] = h
-// (first pass, add = 0) or += h.  Grid (R, kHMax), one workgroup each.
-__global__ __launch_bounds__(kSrvThreads) void k_srv_fin(const double* __restrict__ partials,
-                                                         int nblk, const int* __restrict__ colj,
-                                                         const double* __restrict__ vs,
-                                                         double* __restrict__ h,
-                                                         double* __restrict__ acc, int add) {
-  const int c = blockIdx.x, i = blockIdx.y;
-  const int j = colj[c];
-  if (j < 0 || i > j) return;
-  const double* p = partials + (static_cast<int64_t>(c) * kHMax + i) * nblk;
-  double v = 0.0;
-  for (int b = threadIdx.x; b < nblk; b += kSrvThreads) v += p[b];
-  v = block_sum<kSrvThreads>(v);
-  if (threadIdx.x == 0) {
-    v *= vs[c * kHMax + i];
-    h[c * kHMax + i] = v;
-    acc[c * kHMax + i] = add ? acc[c * kHMax + i] + v : v;
-  }
-}
-
-// Flagged columns after pass 3: beta[c] = sqrt(sum) and the new vector's
-// scale 1/beta (0 if it underflows).  Grid R.
-__global__ void k_srv_beta(const double* __restrict__ partials, int nblk,
-                           const int* __restrict__ colj, const int* __restrict__ flag,
-                           double* __restrict__ beta, double* __restrict__ vs) {
-  const int c = blockIdx.x;
-  if (colj[c] < 0 || !flag[c]) return;
-  double v = 0.0;
-  for (int b = threadIdx.x; b < nblk; b += 64) v += partials[static_cast<int64_t>(c) * nblk + b];
-  v = wave_sum(v);
-  if (threadIdx.x == 0) {
-    const double r = sqrt(v);
-    beta[c] = r;
-    vs[c * kHMax + colj[c] + 1] = r > 1e-300 ? 1.0 / r : 0.0;
-  }
-}
-
-// The step's results for the host, written by a kernel straight into mapped
-// pinned memory (no copy engine): hh = hacc (R x kHMax), bb = beta (R).
-__global__ void k_srv_out(const double* __restrict__ hacc, const double* __restrict__ beta,
-                          int R, double* hh, double* bb) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < R * kHMax) hh[t] = hacc[t];
-  if (t < R) bb[t] = beta[t];
 }
 
 // vs[c][0] = 1 / sqrt(*n2) (start vector normalisation).
@@ -421,14 +408,15 @@ __global__ void k_srv_setinv(const double* __restrict__ n2, int c, double* __res
   if (threadIdx.x == 0) vs[c * kHMax] = 1.0 / sqrt(*n2);
 }
 
-// After column c's restart: the kept Ritz vectors are normalised and the
+// After the restarts: a column's kept Ritz vectors are normalised and the
 // residual direction moved from index m to kn keeps its scale.
-__global__ void k_srv_rescale(double* __restrict__ vs, int c, int m, int kn) {
-  if (threadIdx.x == 0) {
-    const double sm = vs[c * kHMax + m];
-    for (int k = 0; k < kn; ++k) vs[c * kHMax + k] = 1.0;
-    vs[c * kHMax + kn] = sm;
-  }
+__global__ void k_srv_rescale(double* __restrict__ vs, Restarts q) {
+  const int c = q.c[blockIdx.x], m = q.m[blockIdx.x], kn = q.kn[blockIdx.x];
+  const int t = threadIdx.x;
+  const double sm = vs[c * kHMax + m];
+  __syncthreads();
+  if (t < kn) vs[c * kHMax + t] = 1.0;
+  if (t == kn) vs[c * kHMax + kn] = sm;
 }
 
 }  // namespace
@@ -465,16 +453,20 @@ struct qsi_engine_s {
   int64_t D = 0, ld = 0;
   int nblk = 0;
   int rpb = 0;  // rows per workgroup of the reorthogonalisation kernels
-  hipStream_t st = nullptr;
+  // The steps' stream, and the one of their Rayleigh-Ritz kernels: a column
+  // whose basis is full sits out the next step, which runs meanwhile.
+  hipStream_t st = nullptr, ritz_st = nullptr;
   // device: Krylov bases (column c: ncv + 1 vectors of stride ld), the
   // row-major apply input X (D x R), the apply output w (column-major),
   // slot coefficients, projections, norms and reduction partials
   double *Vb = nullptr, *X = nullptr, *Wc = nullptr, *coeffs = nullptr;
-  double *h = nullptr, *hacc = nullptr, *beta = nullptr, *vs = nullptr, *part = nullptr;
-  double* Ydev = nullptr;
-  int *colj_d = nullptr, *slot_d = nullptr, *flag_d = nullptr;
+  double *hacc = nullptr, *vs = nullptr, *part = nullptr;
+  // per column: projections (kHMax^2, column j of the projected matrix at j *
+  // kHMax), Ritz values of the kept vectors (kHMax), Ritz vectors (kHMax^2)
+  double *Tdev = nullptr, *theta = nullptr, *Ydev = nullptr;
+  int *colj_d = nullptr, *slot_d = nullptr;
   std::vector<void*> allocs;
-  // pinned staging of the restarts' Ritz coefficients, kHMax^2 per column
+  // pinned staging of Ritz coefficients found on the host, kHMax^2 per column
   double* Ystage = nullptr;
   // Up to two steps are in flight; each has its own pinned exchange (column
   // state down, projections and norms up) and completion event.
@@ -484,11 +476,15 @@ struct qsi_engine_s {
     double* coeffs_p = nullptr;
     double* hh_p = nullptr;
     double* bb_p = nullptr;
-    double* hh_dev = nullptr;  // device addresses of hh_p / bb_p (mapped)
+    double* rv_p = nullptr;    // R x kHMax Ritz values, then as many last components
+    double* hh_dev = nullptr;  // device addresses of hh_p, bb_p, rv_p (mapped)
     double* bb_dev = nullptr;
+    double* rv_dev = nullptr;
     hipEvent_t ev = nullptr;   // recorded after the step's last command
+    hipEvent_t tail = nullptr; // recorded after its last kernel on the main stream
     std::vector<int> colj;     // j of each column in this step (-1: not in it)
     std::vector<int64_t> req;  // request of each column when it was enqueued
+    std::vector<int> ritz;     // its row of rv_p when the step fills its basis, or -1
   };
   StepBuf sb[2];
   void* pin = nullptr;
@@ -496,6 +492,7 @@ struct qsi_engine_s {
   int next_buf = 0;
   struct Restart {
     int c, m, kn;
+    bool staged;  // Ritz vectors in Ystage rather than on the device
   };
   std::vector<Restart> restarts;
   // host
@@ -510,11 +507,14 @@ struct qsi_engine_s {
 
   ~qsi_engine_s() {
     if (st) (void)hipStreamSynchronize(st);
+    if (ritz_st) (void)hipStreamSynchronize(ritz_st);
     for (void* p : allocs) (void)hipFree(p);
     if (Ystage) (void)hipHostFree(Ystage);
     if (pin) (void)hipHostFree(pin);
     for (auto& b : sb)
-      if (b.ev) (void)hipEventDestroy(b.ev);
+      for (hipEvent_t ev : {b.ev, b.tail})
+        if (ev) (void)hipEventDestroy(ev);
+    if (ritz_st) (void)hipStreamDestroy(ritz_st);
     if (st) (void)hipStreamDestroy(st);
   }
   template <typename T>
@@ -555,21 +555,31 @@ int engine_admit(qsi_engine_s* E) {
   return QSI_OK;
 }
 
-// Rayleigh-Ritz, convergence test and thick restart of column c whose basis
-// holds m vectors (V_c[m], the residual direction, still unnormalised).
-int engine_ritz(qsi_engine_s* E, int c, int m, bool exhausted) {
+// Convergence test and thick restart of column c whose basis holds m vectors
+// (V_c[m], the residual direction, still unnormalised).  theta, last: the Ritz
+// values and last components that the device found, or null (a basis that
+// ended early, or is larger than the device kernel takes): found here.
+int engine_ritz(qsi_engine_s* E, int c, int m, bool exhausted, const double* dtheta,
+                const double* dlast) {
   auto& col = E->cols[c];
   const int ncv = E->ncv;
-  std::vector<double> Tm(static_cast<size_t>(m) * m), theta, Y;
-  for (int j = 0; j < m; ++j)
-    for (int i = 0; i < m; ++i)
-      Tm[static_cast<size_t>(j) * m + i] = col.T[static_cast<size_t>(j) * ncv + i];
-  hostla::sym_eig(Tm, m, theta, Y);
+  std::vector<double> theta, last(m), Y;
+  if (dtheta) {
+    theta.assign(dtheta, dtheta + m);
+    last.assign(dlast, dlast + m);
+  } else {
+    std::vector<double> Tm(static_cast<size_t>(m) * m);
+    for (int j = 0; j < m; ++j)
+      for (int i = 0; i < m; ++i)
+        Tm[static_cast<size_t>(j) * m + i] = col.T[static_cast<size_t>(j) * ncv + i];
+    hostla::sym_eig(Tm, m, theta, Y);
+    for (int i = 0; i < m; ++i) last[i] = Y[static_cast<size_t>(i) * m + (m - 1)];
+  }
   const double eps23 = std::pow(std::numeric_limits<double>::epsilon(), 2.0 / 3.0);
   const int want = std::min(E->nev, m);
   int nconv = 0;
   for (int i = 0; i < want; ++i) {
-    const double resid = col.beta_last * std::fabs(Y[static_cast<size_t>(i) * m + (m - 1)]);
+    const double resid = col.beta_last * std::fabs(last[i]);
     if (resid < E->tol * std::max(eps23, std::fabs(theta[i]))) ++nconv;
     else break;
   }
@@ -589,9 +599,10 @@ int engine_ritz(qsi_engine_s* E, int c, int m, bool exhausted) {
   // device side runs after every column's host work (engine_restarts)
   int kn = E->nev + std::min(nconv, (m - E->nev) / 2);
   kn = std::max(1, std::min(kn, m - 1));
-  std::copy(Y.begin(), Y.begin() + static_cast<size_t>(kn) * m,
-            E->Ystage + static_cast<size_t>(c) * kHMax * kHMax);
-  E->restarts.push_back({c, m, kn});
+  if (!dtheta)
+    std::copy(Y.begin(), Y.begin() + static_cast<size_t>(kn) * m,
+              E->Ystage + static_cast<size_t>(c) * kHMax * kHMax);
+  E->restarts.push_back({c, m, kn, dtheta == nullptr});
   std::fill(col.T.begin(), col.T.end(), 0.0);
   for (int i = 0; i < kn; ++i) col.T[static_cast<size_t>(i) * ncv + i] = theta[i];
   col.k = kn;
@@ -604,60 +615,62 @@ int engine_ritz(qsi_engine_s* E, int c, int m, bool exhausted) {
 // V_c[0..kn) = V_c[0..m) Y_c and V_c[kn] = V_c[m] for the staged restarts.
 // The staging buffer is rewritten only after the next step synchronises.
 int engine_restarts(qsi_engine_s* E) {
+  if (E->restarts.empty()) return QSI_OK;
   const size_t per = static_cast<size_t>(kHMax) * kHMax;
-  const uint32_t grid = static_cast<uint32_t>(
-      std::min<int64_t>((E->D + kSrvThreads - 1) / kSrvThreads, 4096));
-  for (const auto& r : E->restarts) {
-    double* V = E->Vb + static_cast<int64_t>(r.c) * E->ncv1 * E->ld;
-    double* Yd = E->Ydev + r.c * per;
-    const double* vsc = E->vs + r.c * kHMax;
-    QSI_CHECK_HIP(hipMemcpyAsync(Yd, E->Ystage + r.c * per,
-                                 static_cast<size_t>(r.kn) * r.m * sizeof(double),
-                                 hipMemcpyHostToDevice, E->st));
-    if (E->mmax == 16)
-      hipLaunchKernelGGL(k_srv_restart<16>, dim3(grid), dim3(kSrvThreads), 0, E->st, V, E->ld,
-                         r.m, r.kn, Yd, vsc, E->D);
-    else if (E->mmax == 24)
-      hipLaunchKernelGGL(k_srv_restart<24>, dim3(grid), dim3(kSrvThreads), 0, E->st, V, E->ld,
-                         r.m, r.kn, Yd, vsc, E->D);
-    else if (E->mmax == 32)
-      hipLaunchKernelGGL(k_srv_restart<32>, dim3(grid), dim3(kSrvThreads), 0, E->st, V, E->ld,
-                         r.m, r.kn, Yd, vsc, E->D);
-    else
-      hipLaunchKernelGGL(k_srv_restart<64>, dim3(grid), dim3(kSrvThreads), 0, E->st, V, E->ld,
-                         r.m, r.kn, Yd, vsc, E->D);
-    QSI_CHECK_LAUNCH();
-    hipLaunchKernelGGL(k_srv_rescale, dim3(1), dim3(64), 0, E->st, E->vs, r.c, r.m, r.kn);
-    QSI_CHECK_LAUNCH();
+  Restarts q{};
+  const int n = static_cast<int>(E->restarts.size());  // at most one per column
+  for (int i = 0; i < n; ++i) {
+    const auto& r = E->restarts[i];
+    q.c[i] = static_cast<uint8_t>(r.c);
+    q.m[i] = static_cast<uint8_t>(r.m);
+    q.kn[i] = static_cast<uint8_t>(r.kn);
+    if (r.staged)
+      QSI_CHECK_HIP(hipMemcpyAsync(E->Ydev + r.c * per, E->Ystage + r.c * per,
+                                   static_cast<size_t>(r.kn) * r.m * sizeof(double),
+                                   hipMemcpyHostToDevice, E->st));
   }
+  const dim3 grid(static_cast<uint32_t>(
+                      std::min<int64_t>((E->D + kSrvThreads - 1) / kSrvThreads, 4096)),
+                  n);
+  if (E->mmax == 16)
+    hipLaunchKernelGGL(k_srv_restart<16>, grid, dim3(kSrvThreads), 0, E->st, E->Vb, E->ld,
+                       E->ncv1, q, E->Ydev, E->vs, E->D);
+  else if (E->mmax == 24)
+    hipLaunchKernelGGL(k_srv_restart<24>, grid, dim3(kSrvThreads), 0, E->st, E->Vb, E->ld,
+                       E->ncv1, q, E->Ydev, E->vs, E->D);
+  else if (E->mmax == 32)
+    hipLaunchKernelGGL(k_srv_restart<32>, grid, dim3(kSrvThreads), 0, E->st, E->Vb, E->ld,
+                       E->ncv1, q, E->Ydev, E->vs, E->D);
+  else
+    hipLaunchKernelGGL(k_srv_restart<64>, grid, dim3(kSrvThreads), 0, E->st, E->Vb, E->ld,
+                       E->ncv1, q, E->Ydev, E->vs, E->D);
+  QSI_CHECK_LAUNCH();
+  hipLaunchKernelGGL(k_srv_rescale, dim3(n), dim3(64), 0, E->st, E->vs, q);
+  QSI_CHECK_LAUNCH();
   E->restarts.clear();
   return QSI_OK;
 }
 
 template <int MMAX>
-void launch_reorth(qsi_engine_s* E, dim3 gcol, hipStream_t s) {
-  const int R = E->R;
+void launch_reorth(qsi_engine_s* E, int nact, const qsi_engine_s::StepBuf& B, hipStream_t s) {
+  const dim3 gcol(E->nblk, nact);
+  double* part2 = E->part + static_cast<size_t>(E->R) * E->nblk * kHMax;
   hipLaunchKernelGGL(k_srv_mdot<MMAX>, gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld, E->ncv1,
                      E->Wc, E->colj_d, E->slot_d, E->D, E->rpb, E->part);
-  hipLaunchKernelGGL(k_srv_fin, dim3(R, kHMax), dim3(kSrvThreads), 0, s, E->part, E->nblk,
-                     E->colj_d, E->vs, E->h, E->hacc, 0);
   if constexpr (MMAX <= 24)
     hipLaunchKernelGGL(k_srv_gemv_mdot_rows<MMAX>, gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld,
-                       E->ncv1, E->h, E->vs, E->colj_d, E->slot_d, E->D, E->rpb, E->Wc,
-                       E->part);
+                       E->ncv1, E->part, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb, E->Wc,
+                       part2);
   else
     hipLaunchKernelGGL(k_srv_gemv_mdot<MMAX>, gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld,
-                       E->ncv1, E->h, E->vs, E->colj_d, E->slot_d, E->D, E->rpb, E->Wc,
-                       E->part);
-  hipLaunchKernelGGL(k_srv_fin, dim3(R, kHMax), dim3(kSrvThreads), 0, s, E->part, E->nblk,
-                     E->colj_d, E->vs, E->h, E->hacc, 1);
-  hipLaunchKernelGGL(k_srv_check, dim3(R), dim3(64), 0, s, E->part, E->nblk, E->colj_d, E->h,
-                     E->flag_d, E->beta, E->vs);
-  hipLaunchKernelGGL(k_srv_gemv_norm<MMAX>, gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld,
-                     E->ncv1, E->h, E->vs, E->colj_d, E->slot_d, E->flag_d, E->D, E->rpb,
-                     E->part);
-  hipLaunchKernelGGL(k_srv_beta, dim3(R), dim3(64), 0, s, E->part, E->nblk, E->colj_d,
-                     E->flag_d, E->beta, E->vs);
+                       E->ncv1, E->part, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb, E->Wc,
+                       part2);
+  // enough workgroups for the last pass over the flagged columns, and few
+  // where there is none to make
+  const int nt = std::min(E->nblk, std::max(32, 512 / nact));
+  hipLaunchKernelGGL(k_srv_tail<MMAX>, dim3(nt, nact), dim3(kSrvThreads), 0, s, E->Vb, E->ld,
+                     E->ncv1, part2, E->nblk, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->Tdev,
+                     B.hh_dev, B.bb_dev);
 }
 
 }  // namespace
@@ -687,8 +700,8 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
   E->max_restarts = max_restarts;
   E->ld = (E->D + 63) / 64 * 64;
   {
-    int64_t rpb = ((E->D + 255) / 256 + 63) / 64 * 64;
-    rpb = std::min<int64_t>(std::max<int64_t>(rpb, kSrvRowsMin), kSrvRowsMax);
+    int64_t rpb = ((E->D + kSumBlocks - 1) / kSumBlocks + 63) / 64 * 64;
+    rpb = std::max<int64_t>(rpb, kSrvRowsMin);
     E->rpb = static_cast<int>(rpb);
     E->nblk = static_cast<int>((E->D + rpb - 1) / rpb);
   }
@@ -719,6 +732,7 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
   E->n_blocks = blk_apply_blocks(a, op->basis->nw);
   const size_t R = static_cast<size_t>(E->R);
   hipError_t e = hipStreamCreateWithFlags(&E->st, hipStreamNonBlocking);
+  if (e == hipSuccess) e = hipStreamCreateWithFlags(&E->ritz_st, hipStreamNonBlocking);
   const int ns = std::max(op->n_slots, 1);
   if (e == hipSuccess) e = E->alloc(&E->Vb, R * E->ncv1 * E->ld);
   if (e == hipSuccess) e = E->alloc(&E->X, static_cast<size_t>(E->D) * R);
@@ -732,19 +746,21 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
     E->colj_d = reinterpret_cast<int*>(down + static_cast<size_t>(ns) * R);
     E->slot_d = E->colj_d + R;
   }
-  if (e == hipSuccess) e = E->alloc(&E->h, R * kHMax);
   if (e == hipSuccess) e = E->alloc(&E->hacc, R * kHMax);
-  if (e == hipSuccess) e = E->alloc(&E->beta, R);
+  if (e == hipSuccess) e = E->alloc(&E->Tdev, R * kHMax * kHMax);
+  if (e == hipSuccess) e = E->alloc(&E->theta, R * kHMax);
   if (e == hipSuccess) e = E->alloc(&E->vs, R * kHMax);
   if (e == hipSuccess)
-    e = E->alloc(&E->part, std::max<size_t>(R * E->nblk * kHMax, static_cast<size_t>(max_vec_partials()) + 8));
+    e = E->alloc(&E->part, std::max<size_t>(2 * R * E->nblk * kHMax,
+                                            static_cast<size_t>(max_vec_partials()) + 8));
   if (e == hipSuccess) e = E->alloc(&E->Ydev, R * kHMax * kHMax);
   if (e == hipSuccess)
     e = hipHostMalloc(reinterpret_cast<void**>(&E->Ystage), R * kHMax * kHMax * sizeof(double),
                       hipHostMallocDefault);
   // pinned: per step buffer hh (R x kHMax), bb (R), coeffs (ns x R), colj and
-  // slotcol (R ints each, in R more doubles)
-  const size_t per_buf = R * (kHMax + 2 + ns);
+  // slotcol (R ints each, in R more doubles), Ritz values and last components
+  // (R x kHMax each)
+  const size_t per_buf = R * (3 * kHMax + 2 + ns);
   if (e == hipSuccess)
     e = hipHostMalloc(&E->pin, 2 * per_buf * sizeof(double),
                       hipHostMallocMapped | hipHostMallocCoherent);
@@ -757,13 +773,16 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
     B.coeffs_p = B.bb_p + R;
     B.colj_p = reinterpret_cast<int*>(B.coeffs_p + R * ns);
     B.slot_p = B.colj_p + R;
+    B.rv_p = B.hh_p + R * (kHMax + 2 + ns);
     B.hh_dev = static_cast<double*>(dp) + b * per_buf;
     B.bb_dev = B.hh_dev + R * kHMax;
+    B.rv_dev = B.hh_dev + R * (kHMax + 2 + ns);
     B.colj.assign(R, -1);
     B.req.assign(R, -1);
+    B.ritz.assign(R, -1);
     e = hipEventCreateWithFlags(&B.ev, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventCreateWithFlags(&B.tail, hipEventDisableTiming);
   }
-  if (e == hipSuccess) e = E->alloc(&E->flag_d, R);
   // on the engine's own stream: it does not wait for the null stream, so a
   // null-stream memset could still be running under the first step
   if (e == hipSuccess) e = hipMemsetAsync(E->Vb, 0, R * E->ncv1 * E->ld * sizeof(double), E->st);
@@ -883,18 +902,46 @@ int qsi_engine_step_begin(qsi_engine_t E, int* launched) {
   a.ldx = ldx;
   rc = launch_blk_apply(a, E->op->basis->nw, E->n_blocks, E->X, E->Wc, nullptr, s);
   if (rc != QSI_OK) return rc;
-  const dim3 gcol(E->nblk, nact);
   // hacc is written by the first projection pass (entries past a column's
   // j are stale and never read)
-  if (E->mmax == 16) launch_reorth<16>(E, gcol, s);
-  else if (E->mmax == 24) launch_reorth<24>(E, gcol, s);
-  else if (E->mmax == 32) launch_reorth<32>(E, gcol, s);
-  else launch_reorth<64>(E, gcol, s);
+  if (E->mmax == 16) launch_reorth<16>(E, nact, B, s);
+  else if (E->mmax == 24) launch_reorth<24>(E, nact, B, s);
+  else if (E->mmax == 32) launch_reorth<32>(E, nact, B, s);
+  else launch_reorth<64>(E, nact, B, s);
   QSI_CHECK_LAUNCH();
-  hipLaunchKernelGGL(k_srv_out, dim3((R * kHMax + 255) / 256), dim3(256), 0, s, E->hacc, E->beta,
-                     R, B.hh_dev, B.bb_dev);
-  QSI_CHECK_LAUNCH();
-  QSI_CHECK_HIP(hipEventRecord(B.ev, s));
+  // Rayleigh-Ritz of the columns whose basis this step fills, beside the next
+  // step (65 us for 15 vectors; a fifth of the device's time when in line)
+  hipStream_t last = s;
+  std::fill(B.ritz.begin(), B.ritz.end(), -1);
+  if (E->ncv <= kRitzMax) {
+    RitzArgs q{};
+    int n = 0;
+    for (int c = 0; c < R; ++c) {
+      if (E->colj[c] != E->ncv - 1) continue;
+      q.job[n] = static_cast<uint8_t>(c);
+      q.kept[n] = static_cast<uint8_t>(E->cols[c].k);
+      B.ritz[c] = n++;
+    }
+    if (n > 0) {
+      q.cols = E->Tdev;
+      q.job_stride = q.y_stride = static_cast<int64_t>(kHMax) * kHMax;
+      q.ldc = kHMax;
+      q.m = E->ncv;
+      q.theta = E->theta;
+      q.theta_stride = q.out_stride = kHMax;
+      q.Y = E->Ydev;
+      q.out_theta = B.rv_dev;
+      q.out_last = B.rv_dev + static_cast<size_t>(R) * kHMax;
+      // it reads and writes only what belongs to these columns; their restarts
+      // are enqueued by step_end, which waits for B.ev first
+      QSI_CHECK_HIP(hipEventRecord(B.tail, s));
+      QSI_CHECK_HIP(hipStreamWaitEvent(E->ritz_st, B.tail, 0));
+      rc = launch_ritz(q, n, E->ritz_st);
+      if (rc != QSI_OK) return rc;
+      last = E->ritz_st;
+    }
+  }
+  QSI_CHECK_HIP(hipEventRecord(B.ev, last));
   for (int c = 0; c < R; ++c) {
     B.colj[c] = E->colj[c];
     B.req[c] = E->cols[c].req;
@@ -944,7 +991,11 @@ int qsi_engine_step_end(qsi_engine_t E, int* n_active) {
       const bool exhausted = beta <= 1e-13 * std::max(tn, 1e-300);
       col.beta_last = exhausted ? 0.0 : beta;
       if (j + 1 == ncv || exhausted) {
-        const int rc = engine_ritz(E, c, j + 1, exhausted);
+        // an exhausted column ends here, with the values of its own subspace
+        const int b = j + 1 == ncv ? B.ritz[c] : -1;
+        const double* th = b >= 0 ? B.rv_p + static_cast<size_t>(b) * kHMax : nullptr;
+        const double* last = th ? th + static_cast<size_t>(E->R) * kHMax : nullptr;
+        const int rc = engine_ritz(E, c, j + 1, exhausted, th, last);
         if (rc != QSI_OK) return rc;
       }
     }

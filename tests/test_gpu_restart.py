@@ -46,3 +46,40 @@ def test_lowest(cuda, bits, keep, nev, ncv):
         v = V[:, i]
         assert abs(np.linalg.norm(v) - 1.0) <= 1e-9
         assert np.linalg.norm(A @ v - evals[i] * v) <= 1e-9 * norm
+
+
+@pytest.mark.parametrize("bits,keep", [(6, 40), (10, 513)])
+@pytest.mark.parametrize("nev,ncv", [(1, 6), (3, 15), (3, 16), (3, 17), (4, 24), (4, 32), (4, 33),
+                                     (5, 48), (5, 49), (5, 63)])
+def test_engine(cuda, bits, keep, nev, ncv):
+    """Seven points on three columns of the solve engine, on both sides of its
+    kernels' column limits and of the device Rayleigh-Ritz's: columns that
+    restart in different steps, are refilled, and (small basis, large search
+    space) exhaust their space."""
+    from qsi_subspace_ed_amd import serve
+    from qsi_subspace_ed_amd.operators import SymbolicOpSum, SymbolicPMROperator
+    states, spins, W = _basis(1, bits, keep, keep)
+    H = SymbolicOpSum()
+    # conjugate pairs share a slot; a field without repeated values
+    for k, (_, o, _) in enumerate(_terms(spins, 24, bits, z=False, open_spins=False).off_diag_terms):
+        H.add_term(1.0, o, slot=k // 2 % 4)
+    for k, p in enumerate(spins):
+        H.add_term(0.37 * 1.61 ** (k % 7) + 0.011 * k, SymbolicPMROperator.from_ops("z", [p]))
+    op = q.GpuOp(q.GpuBasis(states, W), H)
+    pts = np.random.default_rng(ncv).uniform(-1.0, -0.2, size=(op.n_slots, 7))
+    eng = serve.Engine(op, max_cols=3, nev=nev, ncv=ncv, tol=1e-10, max_restarts=20000)
+    ids = [eng.submit(pts[:, k], 11 + k) for k in range(7)]
+    got = {f.id: f.evals for f in eng.run_all()}
+    for k, i in enumerate(ids):
+        A = np.empty((keep, keep))
+        for c0 in range(0, keep, 64):
+            R = min(64, keep - c0)
+            c = cuda.from_numpy(np.repeat(pts[:, k:k + 1], R, axis=1)).cuda()
+            y = cuda.empty((keep, R), dtype=cuda.float64, device="cuda")
+            op.apply_block(cuda.eye(keep, dtype=cuda.float64, device="cuda")[:, c0:c0 + R]
+                           .contiguous(), y, coeffs=c)
+            A[:, c0:c0 + R] = y.cpu().numpy()
+        assert np.array_equal(A, A.T)
+        want = np.linalg.eigvalsh(A)
+        n = min(nev, keep - 1)
+        assert np.abs(got[i][:n] - want[:n]).max() <= 1e-9 * np.abs(want).max()
