@@ -312,6 +312,12 @@ __device__ __forceinline__ State<NW> staged_target(const LowTermsLds<NW>& tl,
   return r;
 }
 
+// v of one lane, in all.
+__device__ __forceinline__ double read_lane(double v, int lane) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                          __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
 // y[i] = yscale * y_in[i] + sum_t H_{i,t} x[...] + d(s_i) x[i]
 // If DOT, partials[block] = sum over the block's rows of x[i] * y[i].
 // Lane variant: every lane walks its own row's connected states and runs a
@@ -444,6 +450,63 @@ __attribute__((amdgpu_waves_per_eu(G >= 8 ? 3 : G >= 4 ? 5 : 8))) void k_apply_l
     const double bs = block_sum<kApplyBlock>(prod);
     if (threadIdx.x == 0) partials[blk] = bs;
   }
+}
+
+// Row variant, for bases that leave the lane variant with a wavefront or two on
+// each compute unit: one wavefront per row, one term per lane.  All of a row's
+// lookups go through the table, the bisection and the gather at once, so the
+// kernel is one chain of dependent loads where a lane that walks its row's
+// terms four at a time waits for that chain two to eight times.  The
+// contributions are then added by every lane alike, in term order and with the
+// lane variant's multiply-adds, so y is bit-identical.
+template <int NW, bool HAS_Z>
+__global__ __launch_bounds__(kApplyBlock) void k_apply_row(
+    BasisView b, const OffTerm* __restrict__ off, int n_off,
+    const DiagTerm* __restrict__ dg, int n_diag, const double* __restrict__ x,
+    double* y, const double* y_in, double yscale, const double* __restrict__ yscale_dev) {
+  const int lane = threadIdx.x % kWave;
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * (kApplyBlock / kWave) +
+                    __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  if (i >= b.dim) return;
+  if (yscale_dev) yscale *= yscale_dev[0];
+  const State<NW> s = load_state_cached<NW>(b.states, i);
+  const double xi = x[i];
+  double acc = y_in ? yscale * y_in[i] : 0.0;
+  for (int t0 = 0; t0 < n_off; t0 += kWave) {
+    const bool in = t0 + lane < n_off;
+    const OffTerm& T = off[in ? t0 + lane : 0];
+    bool hit = in && term_ok<NW>(T, s);
+    const State<NW> key = xor_state<NW>(s, T.X);
+    double c = T.c * T.sgn;
+    if constexpr (HAS_Z) {
+      if (parity_notz<NW>(s, T.Z)) c = -c;
+    }
+    uint32_t lo = 0, n = 0;
+    if (hit) {
+      uint2 p;
+      __builtin_memcpy(&p, b.table + bucket_key<NW>(b, key), sizeof(uint2));
+      lo = p.x;
+      n = p.y - p.x;
+    }
+    while (n > 1) {
+      const uint32_t half = n >> 1;
+      if (st_le<NW>(load_state_cached<NW>(b.states, lo + half), key)) lo += half;
+      n -= half;
+    }
+    double xj = 0.0;
+    if (n == 1) {
+      const State<NW> f = load_state_cached<NW>(b.states, lo);
+      xj = x[lo];
+      if (!st_eq<NW>(f, key)) xj = 0.0;
+    }
+    for (uint64_t mask = __ballot(fabs(xj) > kApplyTol); mask; mask &= mask - 1) {
+      const int l = __builtin_ctzll(mask);
+      const double cl = read_lane(c, l), xl = read_lane(xj, l);
+      acc += cl * xl;
+    }
+  }
+  acc = diag_accumulate<NW>(acc, xi, s, dg, n_diag);
+  if (lane == 0) y[i] = acc;
 }
 
 // Low-key variant (QSI_APPLY_LOW*): as the lane variant, but the bisection
@@ -987,6 +1050,7 @@ template <int NW, bool CHECK>
 constexpr int kWinWaves = NW == 1 ? 7 : 5;
 // AUTO takes the window kernel from this many states on; against LOW8 on two-word
 // states only from the second
+constexpr int64_t kRowMaxDim = int64_t{1} << 14;
 constexpr int64_t kWinMinDim = int64_t{1} << 21;
 constexpr int64_t kWinMinDimLow2 = int64_t{1} << 28;
 constexpr int kWinRows = 128;  // rows of a wavefront, and ranks of a window
@@ -2318,7 +2382,11 @@ static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
   const dim3 wgrid(static_cast<uint32_t>((nb + 1) / 2));
   const auto v = op->basis->view();
   int variant = op->variant;
-  // AUTO: the cached connectivity when it exists.  Else, without low keys whose
+  // AUTO: the cached connectivity when it exists.  Else, on bases of a few
+  // thousand states, a wavefront per row (call to call, a call's host side being
+  // 7.8 us, row / LANE4 / LOW8 in us: 2970 states 7.8 / 12.4 / 11.9, 13122 states
+  // 9.1 / 14.5 / 14.7, 87546 states 54 / 20 / 19), but not for the dot-product
+  // instances, whose partials are sums over 256 rows.  Else, without low keys whose
   // candidates need no compare, the window kernel on bases large enough to fill
   // the chip with its 128-row wavefronts (WINDOW / LANE4 / LOW4 in us: 32 spins
   // 35 / 12 / 13, 293394 states 33 / 25 / 25, 1062882 states 55 / 52 / 53, 64 spins 200 /
@@ -2331,6 +2399,15 @@ static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
   // 80 spins 9.47 / 9.38, 96 spins 278 / 292 ms).
   if (variant == QSI_APPLY_AUTO) {
     const int64_t dim = op->basis->dim;
+    if constexpr (!DOT) {
+      if (dim <= kRowMaxDim && op->conn_nnz < 0) {
+        const int64_t rb = kApplyBlock / kWave;
+        hipLaunchKernelGGL((k_apply_row<NW, HAS_Z>), dim3(static_cast<uint32_t>((dim + rb - 1) / rb)),
+                           block, 0, s, v, op->d_off, op->n_off, op->d_diag, op->n_diag, x, y, y_in,
+                           yscale, yscale_dev);
+        return;
+      }
+    }
     const bool trusted = op->basis->d_lowkeys && op->lowkeys_check == kLowTrusted;
     const bool window = 
         dim >= kWinMinDim && op->ordered &&
