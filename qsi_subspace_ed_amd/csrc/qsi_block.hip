@@ -95,9 +95,9 @@ __device__ __forceinline__ ColVec<CPL> load_cols(const double* p) {
 }
 
 // A wavefront's place in a row-major block: G lanes per row, CPL neighbouring
-// columns each.  An odd last column is computed by a lane that also reads the
-// column before it and leaves that one alone (R >= 2), so every load stays
-// inside its row.
+// columns each (R >= CPL).  The last columns, where CPL does not divide R, are
+// computed by a lane that also reads the columns before them and leaves those
+// alone, so every load stays inside its row.
 template <int CPL>
 struct ColLane {
   int grp;    // row within the pass
@@ -475,7 +475,7 @@ __device__ __forceinline__ void load_entries(const BlkSector& S, uint64_t e, uin
 }
 
 // The block apply over cached connectivity: same arithmetic, order and
-// results as k_blk_apply.  G lanes per row, CPL columns each, PIPE entries'
+// results as k_blk_apply.  G lanes per row, CPL columns each (blk_cpl), PIPE entries'
 // gathers in flight.  G may be any width up to 64 when no partials are asked
 // for (a wavefront then serves floor(64 / G) rows per pass); with partials it
 // must be a power of two (the per-column sums cross row groups by butterfly).
@@ -749,26 +749,44 @@ namespace {
 using BlkKernel = void (*)(BlkArgs, const double*, double*, double*);
 
 // Block-apply kernel of a configuration: cached kernels by gathers in flight
-// (4, 8, 16), searching kernels by lookups in flight (6 or 4 by the state's
-// words; 2); one or two columns per lane.
+// (4, 8, 16; half as many of four columns), searching kernels by lookups in
+// flight (6 or 4 by the state's words; 2); cpl columns per lane (blk_cpl).
 template <int CPL>
-BlkKernel blk_kernel_t(int nw, bool cached, int k) {
-  if (cached) {
-    if (nw == 1)
-      return k == 0 ? k_blk_capply<1, 4, CPL>
-                    : (k == 2 ? k_blk_capply<1, 16, CPL> : k_blk_capply<1, 8, CPL>);
-    return k == 0 ? k_blk_capply<2, 4, CPL>
-                  : (k == 2 ? k_blk_capply<2, 16, CPL> : k_blk_capply<2, 8, CPL>);
-  }
+BlkKernel cached_kernel(int nw, int k) {
+  constexpr int P8 = CPL == 4 ? 4 : 8, P16 = CPL == 4 ? 8 : 16;
+  if (nw == 1)
+    return k == 0 ? k_blk_capply<1, 4, CPL>
+                  : (k == 2 ? k_blk_capply<1, P16, CPL> : k_blk_capply<1, P8, CPL>);
+  return k == 0 ? k_blk_capply<2, 4, CPL>
+                : (k == 2 ? k_blk_capply<2, P16, CPL> : k_blk_capply<2, P8, CPL>);
+}
+template <int CPL>
+BlkKernel search_kernel(int nw, int k) {
   if (nw == 1) return k == 2 ? k_blk_apply<1, 2, CPL> : k_blk_apply<1, 6, CPL>;
   return k == 2 ? k_blk_apply<2, 2, CPL> : k_blk_apply<2, 4, CPL>;
 }
-BlkKernel blk_kernel(int nw, bool cached, int cfg, bool pairs) {
+BlkKernel blk_kernel(int nw, bool cached, int cfg, int cpl) {
   const int k = blk_cfg_kernel(cfg);
-  return pairs ? blk_kernel_t<2>(nw, cached, k) : blk_kernel_t<1>(nw, cached, k);
+  if (!cached) return cpl == 1 ? search_kernel<1>(nw, k) : search_kernel<2>(nw, k);
+  return cpl == 1   ? cached_kernel<1>(nw, k)
+         : cpl == 2 ? cached_kernel<2>(nw, k)
+                    : cached_kernel<4>(nw, k);
 }
 
 }  // namespace
+
+int blk_cpl(const BlkArgs& a) {
+  const bool cached = blk_cached(a);
+  if (a.R < 2 || (cached && !blk_cfg_pairs(a.cfg))) return 1;
+  // Four columns per lane halve the instructions per entry and column, and
+  // with them the wavefronts that share a row: worth it from 12 columns on,
+  // where enough passes of 64 lanes are left to fill the chip (64 columns of
+  // 2.76 M, 87 546 rows: 2.75 -> 2.55 ms, 77 -> 68 us; but 16 columns of 87 546
+  // rows 24 -> 30 us, 8 columns of 2.76 M 410 -> 421 us).
+  int64_t rows = 0;
+  for (int s = 0; s < a.n_sec; ++s) rows += a.sec[s].b.dim;
+  return cached && a.R >= 12 && rows * a.R >= int64_t{1} << 22 ? 4 : 2;
+}
 
 void blk_set_tiles(BlkArgs& a) {
   int64_t rows = 0;
@@ -789,13 +807,13 @@ void blk_set_tiles(BlkArgs& a) {
 }
 
 int blk_apply_blocks(const BlkArgs& a, int nw) {
-  const bool cached = blk_cached(a), pairs = blk_pairs(a);
-  const int cfg = a.cfg;
-  // resident blocks per CU of each kernel: [cached][nw - 1][kernel][pairs];
+  const bool cached = blk_cached(a);
+  const int cpl = blk_cpl(a), cfg = a.cfg;
+  // resident blocks per CU of each kernel: [cached][nw - 1][kernel][columns per lane];
   // atomics, as host threads may launch concurrently (they store equal
   // values).  The CU count is a function-local static, whose initialisation
   // is thread-safe, so no thread can see an occupancy without it.
-  static std::atomic<int> per_cu[2][2][3][2];
+  static std::atomic<int> per_cu[2][2][3][5];
   static const int n_cu = [] {
     int dev = 0, cu = 0;
     (void)hipGetDevice(&dev);
@@ -804,12 +822,12 @@ int blk_apply_blocks(const BlkArgs& a, int nw) {
       cu = 256;
     return cu;
   }();
-  std::atomic<int>& occ = per_cu[cached ? 1 : 0][nw - 1][blk_cfg_kernel(cfg)][pairs ? 1 : 0];
+  std::atomic<int>& occ = per_cu[cached ? 1 : 0][nw - 1][blk_cfg_kernel(cfg)][cpl];
   int o_cu = occ.load(std::memory_order_relaxed);
   if (o_cu == 0) {
     int o = 0;
     const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-        &o, blk_kernel(nw, cached, cfg, pairs), kBlkThreads, 0);
+        &o, blk_kernel(nw, cached, cfg, cpl), kBlkThreads, 0);
     o_cu = (e == hipSuccess && o > 0) ? o : 4;
     occ.store(o_cu, std::memory_order_relaxed);
   }
@@ -821,15 +839,16 @@ int blk_apply_blocks(const BlkArgs& a, int nw) {
 
 int launch_blk_apply(const BlkArgs& a, int nw, int n_blocks, const double* X, double* Y,
                      double* partials, hipStream_t s) {
-  const bool cached = blk_cached(a), pairs = blk_pairs(a);
+  const bool cached = blk_cached(a);
+  const int cpl = blk_cpl(a);
   BlkArgs b = a;
   // lanes per row: as many as hold the columns; a power of two in the
   // searching kernels and where partials cross row groups by butterfly
-  const int w = pairs ? (a.R + 1) / 2 : a.R;
+  const int w = (a.R + cpl - 1) / cpl;
   b.G = 1;
   while (b.G < w) b.G <<= 1;
   if (cached && !partials) b.G = w;
-  hipLaunchKernelGGL(blk_kernel(nw, cached, a.cfg, pairs), dim3(n_blocks), dim3(kBlkThreads), 0,
+  hipLaunchKernelGGL(blk_kernel(nw, cached, a.cfg, cpl), dim3(n_blocks), dim3(kBlkThreads), 0,
                      s, b, X, Y, partials);
   QSI_CHECK_LAUNCH();
   return QSI_OK;

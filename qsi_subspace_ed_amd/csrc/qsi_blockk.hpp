@@ -52,8 +52,8 @@ struct BlkArgs {
 // Block-apply configuration: bits 0-1 pick the kernel (cached connectivity:
 // 4 / 8 / 16 gathers in flight per lane; searching: 6 or 4 lookups in flight
 // by the state's words, or 2), bit 2 halves the persistent grid, bit 3 lets the
-// cached kernel serve two columns per lane (16-byte gathers); the searching
-// kernel always does.
+// cached kernel serve several columns per lane (16-byte gathers; blk_cpl); the
+// searching kernel always does.
 constexpr int kBlkCfgDefault = 1;
 inline int blk_cfg_kernel(int cfg) { return cfg & 3; }
 inline bool blk_cfg_half(int cfg) { return (cfg >> 2) & 1; }
@@ -67,11 +67,10 @@ inline bool blk_cached(const BlkArgs& a) {
   return a.n_sec > 0;
 }
 
-// True when a block apply serves two columns per lane: R >= 2 and, over cached
-// connectivity, the configuration's pairs bit.
-inline bool blk_pairs(const BlkArgs& a) {
-  return a.R >= 2 && (!blk_cached(a) || blk_cfg_pairs(a.cfg));
-}
+// Columns per lane of a block apply (1, 2 or 4, at most R): one without the
+// configuration's bit over cached connectivity, else two, or four in wide cached
+// applies of large bases.
+int blk_cpl(const BlkArgs& a);
 
 // Cuts the sectors (bases, R and G set) into tiles, one wavefront's work each:
 // tile_rows, every tile_begin and n_tiles.

@@ -32,7 +32,7 @@ struct OffTerm {
 // Off-diagonal terms of one coefficient class share their per-column
 // coefficient in a block apply: slot `slot` of the column (or `c` when the
 // apply has no per-column coefficients or slot < 0).  Block applies keep the
-// classes' coefficients in registers instead of loading each term's.
+// classes' coefficients in LDS instead of loading each term's.
 struct CoefClass {
   double c;
   int32_t slot;

@@ -130,3 +130,29 @@ def test_recurrence(cuda, R, cached):
         scale = max(np.abs(wa).max(), np.abs(wb).max())
         assert np.abs(al[s] - wa).max() <= 1e-11 * scale, s
         assert np.abs(be[s] - wb).max() <= 1e-11 * scale, s
+
+
+@pytest.mark.parametrize("R", [31, 32, 63, 64])
+@pytest.mark.parametrize("cfg", [8, 9, 10])
+def test_cached_wide(cuda, R, cfg):
+    """Blocks large enough for four columns per lane (the last lane repeats up to
+    three), beside the same columns sixteen at a time, which are not."""
+    from qsi_subspace_ed_amd import latgen
+    jd = latgen.Supercell((1, 3, 4)).to_dict()
+    H = q.build_hamiltonian_g(jd, [-0.9, -0.5, -0.3, -0.7])
+    q.add_local_field(H, jd, [0.05, -0.02, 0.07])
+    op = q.GpuOp(q.enumerate_basis_device(jd, 0), H)
+    assert op.cache_connectivity(True) > 0
+    op.set_block_cfg(cfg)
+    D = op.rows()
+    assert D * R >= 1 << 22 > D * 16
+    x = cuda.randn(D, R + 1, dtype=cuda.float64, device="cuda",
+                   generator=cuda.Generator(device="cuda").manual_seed(R))
+    y = cuda.full_like(x, 7.0)
+    op.apply_block(x[:, 1:], y[:, 1:])
+    assert bool((y[:, 0] == 7.0).all())
+    for c0 in range(1, R + 1, 16):
+        w = min(16, R + 1 - c0)
+        z = cuda.empty((D, w), dtype=cuda.float64, device="cuda")
+        op.apply_block(x[:, c0:c0 + w].contiguous(), z)
+        assert cuda.equal(y[:, c0:c0 + w], z), c0
