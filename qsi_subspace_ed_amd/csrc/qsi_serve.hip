@@ -44,6 +44,7 @@ constexpr int kSrvThreads = 256;
 // themselves (kernels of their own for the sums, the norms, the flags and the
 // results were six of a step's twelve launches, 4 us each)
 constexpr int kSrvRowsMin = 256;
+constexpr int kSrvRowsMax = 2048;  // plain steps
 constexpr int kHMax = 64;
 // partials slot holding |u|^2 (projections use slots 0..ncv-1 <= 62)
 constexpr int kNormSlot = kHMax - 1;
@@ -147,14 +148,19 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_mdot(
   srv_block_dots<MMAX>(acc, m, c, gridDim.x, partials);
 }
 
-// hs[i] = vs_i h_i for i < m (0 up to MMAX), h_i = vs_i times pass 1's sum of
-// partials i; the column's first workgroup writes h to hacc.  Ends with a
-// barrier.
-template <int MMAX>
+// hs[i] = vs_i h_i for i < m (0 up to MMAX).  FUSED: h_i = vs_i times pass 1's sum
+// of partials i, and the column's first workgroup writes h to hacc; else part1
+// is h (R x kHMax).  Ends with a barrier.
+template <int MMAX, bool FUSED>
 __device__ __forceinline__ void srv_first_sums(const double* __restrict__ part1, int c, int m,
                                                const double* __restrict__ vs,
                                                double* __restrict__ hacc, double (&hs)[MMAX]) {
   const int t = threadIdx.x;
+  if constexpr (!FUSED) {
+    if (t < MMAX) hs[t] = t < m ? part1[c * kHMax + t] * vs[c * kHMax + t] : 0.0;
+    __syncthreads();
+    return;
+  }
   if (t < MMAX) hs[t] = 0.0;
   __syncthreads();
   sum_partials<kSrvThreads>(part1 + static_cast<int64_t>(c) * kHMax * gridDim.x, gridDim.x, m, hs);
@@ -171,7 +177,7 @@ __device__ __forceinline__ void srv_first_sums(const double* __restrict__ part1,
 // Grid (nblk, n_act).  The block walks its rows in 64-row tiles; wave k holds
 // basis vectors i = k, k + 4, ... in registers, the four waves' parts of
 // (V h)[row] meet in LDS, and each wave reuses its V entries for the dots.
-template <int MMAX>
+template <int MMAX, bool FUSED>
 __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot(
     double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ part1,
     double* __restrict__ hacc, const double* __restrict__ vs, const int* __restrict__ colj,
@@ -188,7 +194,7 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot(
   __shared__ double red[MMAX];
   __shared__ double nsh;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  srv_first_sums<MMAX>(part1, c, m, vs, hacc, hs);
+  srv_first_sums<MMAX, FUSED>(part1, c, m, vs, hacc, hs);
   const double* V = Vb + static_cast<int64_t>(c) * ncv1 * ld;
   double* out = Vb + (static_cast<int64_t>(c) * ncv1 + m) * ld;
   const double* w = Wc + static_cast<int64_t>(sl) * ld;
@@ -246,7 +252,7 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot(
 // Pass 1 -> 2 as k_srv_gemv_mdot for MMAX <= 24: one thread per row keeps
 // the row's m basis entries in registers for both the update and the dots
 // (no workgroup barrier per row tile).
-template <int MMAX>
+template <int MMAX, bool FUSED>
 __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot_rows(
     double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ part1,
     double* __restrict__ hacc, const double* __restrict__ vs, const int* __restrict__ colj,
@@ -256,7 +262,7 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot_rows(
   const int c = slotcol[sl];
   const int m = colj[c] + 1;
   __shared__ double hs[MMAX];
-  srv_first_sums<MMAX>(part1, c, m, vs, hacc, hs);
+  srv_first_sums<MMAX, FUSED>(part1, c, m, vs, hacc, hs);
   // h in scalar registers; entries i >= m are zero, so the loops below run
   // unpredicated
   double hr[MMAX];
@@ -335,6 +341,135 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_restart(double* __restrict_
     V[kn * ld + r] = res;
   }
 }
+
+// ---- steps of operators that are not symmetric ------------------------------
+// An operator whose terms lack their reverses (rings of a cluster one cell wide
+// pass through a spin twice) is not symmetric; thick-restart Lanczos does not
+// converge on it, so what a request returns at its restart limit depends on the
+// rounding of every step.  Those steps keep sums in kernels of their own and
+// Rayleigh-Ritz on the host.
+
+// After pass 2's projections h2_c are summed: beta_c = |u_c| from the
+// kNormSlot partials, the scale 1/beta_c of the new vector u_c, and flag_c = 1
+// when |h2_c|^2 > kReorthTol2 |u_c|^2 (u_c needs the second Gram-Schmidt
+// pass).  Grid R, one wave each.
+__global__ void k_srv_check(const double* __restrict__ partials, int nblk,
+                            const int* __restrict__ colj, const double* __restrict__ h,
+                            int* __restrict__ flag, double* __restrict__ beta,
+                            double* __restrict__ vs) {
+  const int c = blockIdx.x;
+  const int j = colj[c];
+  if (j < 0) return;
+  double n2 = 0.0;
+  for (int b = threadIdx.x; b < nblk; b += 64)
+    n2 += partials[(static_cast<int64_t>(c) * kHMax + kNormSlot) * nblk + b];
+  n2 = wave_sum(n2);
+  double s2 = 0.0;
+  for (int i = threadIdx.x; i <= j; i += 64) {
+    const double v = h[c * kHMax + i];
+    s2 += v * v;
+  }
+  s2 = wave_sum(s2);
+  if (threadIdx.x == 0) {
+    flag[c] = s2 > kReorthTol2 * n2 ? 1 : 0;
+    const double r = sqrt(n2);
+    beta[c] = r;
+    vs[c * kHMax + j + 1] = r > 1e-300 ? 1.0 / r : 0.0;
+  }
+}
+
+// pass 3, flagged columns only: u_c -= V_c h2_c in place in V_c[j_c + 1],
+// partials of |u_c|^2 in partials[c*nblk + b].  Grid (nblk, n_act).
+template <int MMAX>
+__global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_norm(
+    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ h,
+    const double* __restrict__ vs, const int* __restrict__ colj,
+    const int* __restrict__ slotcol, const int* __restrict__ flag, int64_t D, int rpb,
+    double* __restrict__ partials) {
+  const int c = slotcol[blockIdx.y];
+  if (!flag[c]) return;
+  const int m = colj[c] + 1;
+  __shared__ double hs[MMAX];
+  if (threadIdx.x < MMAX)
+    hs[threadIdx.x] =
+        threadIdx.x < m ? h[c * kHMax + threadIdx.x] * vs[c * kHMax + threadIdx.x] : 0.0;
+  __syncthreads();
+  const double* V = Vb + static_cast<int64_t>(c) * ncv1 * ld;
+  double* u = Vb + (static_cast<int64_t>(c) * ncv1 + m) * ld;
+  const int64_t r0 = static_cast<int64_t>(blockIdx.x) * rpb;
+  const int64_t r1 = min<int64_t>(r0 + rpb, D);
+  double nrm = 0.0;
+  for (int64_t r = r0 + threadIdx.x; r < r1; r += kSrvThreads) {
+    double a = 0.0;
+    if constexpr (MMAX <= 32) {
+      // all loads first, then the sum in column order (absent columns load
+      // as 0 against a zero h), so a lane keeps its column loads in flight
+      double v[MMAX];
+#pragma unroll
+      for (int i = 0; i < MMAX; ++i) v[i] = i < m ? V[i * ld + r] : 0.0;
+#pragma unroll
+      for (int i = 0; i < MMAX; ++i) a += v[i] * hs[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < MMAX; ++i)
+        if (i < m) a += V[i * ld + r] * hs[i];
+    }
+    const double ur = u[r] - a;
+    u[r] = ur;
+    nrm += ur * ur;
+  }
+  nrm = block_sum<kSrvThreads>(nrm);
+  if (threadIdx.x == 0) partials[static_cast<int64_t>(c) * gridDim.x + blockIdx.x] = nrm;
+}
+
+// h[c*kHMax + i] = vs_i * sum_b partials (fixed order); acc[c*kHMax + i] = h
+// (first pass, add = 0) or += h.  Grid (R, kHMax), one workgroup each.
+__global__ __launch_bounds__(kSrvThreads) void k_srv_fin(const double* __restrict__ partials,
+                                                         int nblk, const int* __restrict__ colj,
+                                                         const double* __restrict__ vs,
+                                                         double* __restrict__ h,
+                                                         double* __restrict__ acc, int add) {
+  const int c = blockIdx.x, i = blockIdx.y;
+  const int j = colj[c];
+  if (j < 0 || i > j) return;
+  const double* p = partials + (static_cast<int64_t>(c) * kHMax + i) * nblk;
+  double v = 0.0;
+  for (int b = threadIdx.x; b < nblk; b += kSrvThreads) v += p[b];
+  v = block_sum<kSrvThreads>(v);
+  if (threadIdx.x == 0) {
+    v *= vs[c * kHMax + i];
+    h[c * kHMax + i] = v;
+    acc[c * kHMax + i] = add ? acc[c * kHMax + i] + v : v;
+  }
+}
+
+// Flagged columns after pass 3: beta[c] = sqrt(sum) and the new vector's
+// scale 1/beta (0 if it underflows).  Grid R.
+__global__ void k_srv_beta(const double* __restrict__ partials, int nblk,
+                           const int* __restrict__ colj, const int* __restrict__ flag,
+                           double* __restrict__ beta, double* __restrict__ vs) {
+  const int c = blockIdx.x;
+  if (colj[c] < 0 || !flag[c]) return;
+  double v = 0.0;
+  for (int b = threadIdx.x; b < nblk; b += 64) v += partials[static_cast<int64_t>(c) * nblk + b];
+  v = wave_sum(v);
+  if (threadIdx.x == 0) {
+    const double r = sqrt(v);
+    beta[c] = r;
+    vs[c * kHMax + colj[c] + 1] = r > 1e-300 ? 1.0 / r : 0.0;
+  }
+}
+
+// The step's results for the host, written by a kernel straight into mapped
+// pinned memory (no copy engine): hh = hacc (R x kHMax), bb = beta (R).
+__global__ void k_srv_out(const double* __restrict__ hacc, const double* __restrict__ beta,
+                          int R, double* hh, double* bb) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t < R * kHMax) hh[t] = hacc[t];
+  if (t < R) bb[t] = beta[t];
+}
+
+// ---- the fused step's tail ---------------------------------------------------
 
 // The tail of the step, grid (any, n_act): pass 2's projections h2_c and norm
 // |u_c|^2 from its partials; where |h2_c|^2 > kReorthTol2 |u_c|^2 the last
@@ -461,6 +596,9 @@ struct qsi_engine_s {
   // slot coefficients, projections, norms and reduction partials
   double *Vb = nullptr, *X = nullptr, *Wc = nullptr, *coeffs = nullptr;
   double *hacc = nullptr, *vs = nullptr, *part = nullptr;
+  double *h = nullptr, *beta = nullptr;  // plain steps
+  int* flag_d = nullptr;
+  bool plain = false;  // the operator is not symmetric: unfused steps, Ritz on the host
   // per column: projections (kHMax^2, column j of the projected matrix at j *
   // kHMax), Ritz values of the kept vectors (kHMax), Ritz vectors (kHMax^2)
   double *Tdev = nullptr, *theta = nullptr, *Ydev = nullptr;
@@ -658,11 +796,11 @@ void launch_reorth(qsi_engine_s* E, int nact, const qsi_engine_s::StepBuf& B, hi
   hipLaunchKernelGGL(k_srv_mdot<MMAX>, gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld, E->ncv1,
                      E->Wc, E->colj_d, E->slot_d, E->D, E->rpb, E->part);
   if constexpr (MMAX <= 24)
-    hipLaunchKernelGGL(k_srv_gemv_mdot_rows<MMAX>, gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld,
+    hipLaunchKernelGGL((k_srv_gemv_mdot_rows<MMAX, true>), gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld,
                        E->ncv1, E->part, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb, E->Wc,
                        part2);
   else
-    hipLaunchKernelGGL(k_srv_gemv_mdot<MMAX>, gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld,
+    hipLaunchKernelGGL((k_srv_gemv_mdot<MMAX, true>), gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld,
                        E->ncv1, E->part, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb, E->Wc,
                        part2);
   // enough workgroups for the last pass over the flagged columns, and few
@@ -671,6 +809,43 @@ void launch_reorth(qsi_engine_s* E, int nact, const qsi_engine_s::StepBuf& B, hi
   hipLaunchKernelGGL(k_srv_tail<MMAX>, dim3(nt, nact), dim3(kSrvThreads), 0, s, E->Vb, E->ld,
                      E->ncv1, part2, E->nblk, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->Tdev,
                      B.hh_dev, B.bb_dev);
+}
+
+// The same step for an operator that is not symmetric (E->plain).
+template <int MMAX>
+void launch_reorth_plain(qsi_engine_s* E, int nact, const qsi_engine_s::StepBuf& B,
+                         hipStream_t s) {
+  const dim3 gcol(E->nblk, nact);
+  const int R = E->R;
+  hipLaunchKernelGGL(k_srv_mdot<MMAX>, gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld, E->ncv1,
+                     E->Wc, E->colj_d, E->slot_d, E->D, E->rpb, E->part);
+  hipLaunchKernelGGL(k_srv_fin, dim3(R, kHMax), dim3(kSrvThreads), 0, s, E->part, E->nblk,
+                     E->colj_d, E->vs, E->h, E->hacc, 0);
+  if constexpr (MMAX <= 24)
+    hipLaunchKernelGGL((k_srv_gemv_mdot_rows<MMAX, false>), gcol, dim3(kSrvThreads), 0, s, E->Vb,
+                       E->ld, E->ncv1, E->h, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb,
+                       E->Wc, E->part);
+  else
+    hipLaunchKernelGGL((k_srv_gemv_mdot<MMAX, false>), gcol, dim3(kSrvThreads), 0, s, E->Vb,
+                       E->ld, E->ncv1, E->h, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb,
+                       E->Wc, E->part);
+  hipLaunchKernelGGL(k_srv_fin, dim3(R, kHMax), dim3(kSrvThreads), 0, s, E->part, E->nblk,
+                     E->colj_d, E->vs, E->h, E->hacc, 1);
+  hipLaunchKernelGGL(k_srv_check, dim3(R), dim3(64), 0, s, E->part, E->nblk, E->colj_d, E->h,
+                     E->flag_d, E->beta, E->vs);
+  hipLaunchKernelGGL(k_srv_gemv_norm<MMAX>, gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld,
+                     E->ncv1, E->h, E->vs, E->colj_d, E->slot_d, E->flag_d, E->D, E->rpb,
+                     E->part);
+  hipLaunchKernelGGL(k_srv_beta, dim3(R), dim3(64), 0, s, E->part, E->nblk, E->colj_d,
+                     E->flag_d, E->beta, E->vs);
+  hipLaunchKernelGGL(k_srv_out, dim3((R * kHMax + 255) / 256), dim3(256), 0, s, E->hacc, E->beta,
+                     R, B.hh_dev, B.bb_dev);
+}
+
+template <int MMAX>
+void launch_step(qsi_engine_s* E, int nact, const qsi_engine_s::StepBuf& B, hipStream_t s) {
+  if (E->plain) launch_reorth_plain<MMAX>(E, nact, B, s);
+  else launch_reorth<MMAX>(E, nact, B, s);
 }
 
 }  // namespace
@@ -702,6 +877,8 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
   {
     int64_t rpb = ((E->D + kSumBlocks - 1) / kSumBlocks + 63) / 64 * 64;
     rpb = std::max<int64_t>(rpb, kSrvRowsMin);
+    E->plain = !op->paired;
+    if (E->plain) rpb = std::min<int64_t>(rpb, kSrvRowsMax);
     E->rpb = static_cast<int>(rpb);
     E->nblk = static_cast<int>((E->D + rpb - 1) / rpb);
   }
@@ -747,6 +924,9 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
     E->slot_d = E->colj_d + R;
   }
   if (e == hipSuccess) e = E->alloc(&E->hacc, R * kHMax);
+  if (e == hipSuccess && E->plain) e = E->alloc(&E->h, R * kHMax);
+  if (e == hipSuccess && E->plain) e = E->alloc(&E->beta, R);
+  if (e == hipSuccess && E->plain) e = E->alloc(&E->flag_d, R);
   if (e == hipSuccess) e = E->alloc(&E->Tdev, R * kHMax * kHMax);
   if (e == hipSuccess) e = E->alloc(&E->theta, R * kHMax);
   if (e == hipSuccess) e = E->alloc(&E->vs, R * kHMax);
@@ -904,16 +1084,16 @@ int qsi_engine_step_begin(qsi_engine_t E, int* launched) {
   if (rc != QSI_OK) return rc;
   // hacc is written by the first projection pass (entries past a column's
   // j are stale and never read)
-  if (E->mmax == 16) launch_reorth<16>(E, nact, B, s);
-  else if (E->mmax == 24) launch_reorth<24>(E, nact, B, s);
-  else if (E->mmax == 32) launch_reorth<32>(E, nact, B, s);
-  else launch_reorth<64>(E, nact, B, s);
+  if (E->mmax == 16) launch_step<16>(E, nact, B, s);
+  else if (E->mmax == 24) launch_step<24>(E, nact, B, s);
+  else if (E->mmax == 32) launch_step<32>(E, nact, B, s);
+  else launch_step<64>(E, nact, B, s);
   QSI_CHECK_LAUNCH();
   // Rayleigh-Ritz of the columns whose basis this step fills, beside the next
   // step (65 us for 15 vectors; a fifth of the device's time when in line)
   hipStream_t last = s;
   std::fill(B.ritz.begin(), B.ritz.end(), -1);
-  if (E->ncv <= kRitzMax) {
+  if (!E->plain && E->ncv <= kRitzMax) {
     RitzArgs q{};
     int n = 0;
     for (int c = 0; c < R; ++c) {

@@ -83,3 +83,27 @@ def test_engine(cuda, bits, keep, nev, ncv):
         want = np.linalg.eigvalsh(A)
         n = min(nev, keep - 1)
         assert np.abs(got[i][:n] - want[:n]).max() <= 1e-9 * np.abs(want).max()
+
+
+@pytest.mark.parametrize("nev,ncv", [(1, 8), (3, 15), (3, 20), (4, 40)])
+def test_engine_not_symmetric(cuda, nev, ncv):
+    """A cluster one cell wide: its rings pass through a spin twice, H is not
+    symmetric and requests end at their restart limit.  The engine's unfused
+    steps give a request the same bits alone and among others."""
+    from qsi_subspace_ed_amd import latgen, serve
+    jd = latgen.Supercell((1, 2, 2)).to_dict()
+    basis = q.enumerate_basis_device(jd, 0)
+    pts = np.random.default_rng(ncv).uniform(-1.0, -0.2, size=(serve.N_SLOTS, 5))
+    pts[4:] *= 0.1
+
+    def run(ks):
+        op = q.GpuOp(basis, serve.slotted_hamiltonian(jd))
+        eng = serve.Engine(op, max_cols=5, nev=nev, ncv=ncv, tol=1e-10, max_restarts=7,
+                           autotune=False)
+        ids = [eng.submit(pts[:, k], 11 + k) for k in ks]
+        got = {f.id: f.evals for f in eng.run_all()}
+        return [got[i] for i in ids]
+
+    together = run(range(5))
+    for k in range(5):
+        assert np.array_equal(run([k])[0], together[k])
