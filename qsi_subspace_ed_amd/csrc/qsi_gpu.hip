@@ -1874,6 +1874,7 @@ __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
     U[(e / N) * LD + e % N] = e / N == e % N ? 1.0 : 0.0;
   }
   __syncthreads();
+  bool bad = false;  // a NaN in the matrix
   for (int sweep = 0; sweep < 64; ++sweep) {
     double off = 0.0, tot = 0.0;
     for (int x = x0; x < N && y < H; x += xs) {
@@ -1898,7 +1899,9 @@ __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
       off += red[0][w];
       tot += red[1][w];
     }
-    if (off == 0.0 || off <= 1e-32 * tot) break;  // the same in every thread
+    // the same in every thread
+    bad = tot != tot;
+    if (bad || off == 0.0 || off <= 1e-32 * tot) break;
     for (int r = 0; r < N - 1; ++r) {
       // pair u of the round: the last index stays, the others go around
       auto pair = [&](int u, int& p, int& q) {
@@ -1953,7 +1956,10 @@ __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
       __syncthreads();
     }
   }
-  // ascending order (ties by index); NaN values share ranks, within m
+  // ascending order, NaN behind every number, ties by index: every index has a
+  // rank of its own, so every output is written.  A matrix with a NaN has no
+  // eigenpairs: all its outputs are NaN (a request's values stand where an
+  // earlier one's stood)
   double* Y = a.Y + job * a.y_stride;
   for (int e = t; e < m * m; e += kRitzThreads) {
     const int j = e / m, i = e % m;
@@ -1961,14 +1967,16 @@ __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
     int rank = 0;
     for (int u = 0; u < m; ++u) {
       const double du = A[u * LD + u];
-      rank += du < d || (du == d && u < j) ? 1 : 0;
+      rank += (d != d ? du == du : du < d) || ((du == d || (d != d && du != du)) && u < j) ? 1 : 0;
     }
-    Y[rank * m + i] = U[i * LD + j];
+    const double nan = __builtin_nan("");
+    const double w = bad ? nan : U[i * LD + j], th = bad ? nan : d;
+    Y[rank * m + i] = w;
     if (i == 0) {
-      theta[rank] = d;
-      a.out_theta[blockIdx.x * a.out_stride + rank] = d;
+      theta[rank] = th;
+      a.out_theta[blockIdx.x * a.out_stride + rank] = th;
     }
-    if (i == m - 1) a.out_last[blockIdx.x * a.out_stride + rank] = U[i * LD + j];
+    if (i == m - 1) a.out_last[blockIdx.x * a.out_stride + rank] = w;
   }
 }
 
