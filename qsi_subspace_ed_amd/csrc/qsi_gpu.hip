@@ -1840,9 +1840,12 @@ __global__ __launch_bounds__(T) void k_gs_tail(
 // rotations, matrix and vectors in LDS.  A sweep is N - 1 rounds of N / 2
 // rotations on disjoint index pairs (round robin), where a cyclic sweep is
 // N (N - 1) / 2 rotations one after the other.  A round is a chain of latencies
-// (LDS, the angle, two barriers), about 0.6 us; an angle need only be near the
-// one that annihilates its element (hardware reciprocals, about 26 bits): what
-// must be exact is c^2 + s^2 = 1, one Newton step of third order for c.  Blocks
+// (LDS, the angle, two barriers).  The vectors of a thick restart are kept for
+// good and never normalised again, so c must round to either side alike: from
+// the hardware's reciprocal root with one Newton step it came out 2^-53 too large
+// for every tangent of 1e-8 to 1e-5, and kept vectors grew by 2e-14 a restart
+// (square norm, order 40; eigenvalues with them), where host rotations leave them
+// within 1e-15 on average.  Blocks
 // on and above the diagonal are computed and mirrored: a matrix that rounding
 // makes unsymmetric keeps that difference in every rotation and never gets
 // diagonal.  Orders 8, 16, 24, 32: 30, 65, 120, 175 us; one matrix of order 15
@@ -1913,16 +1916,16 @@ __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
       if (t < H) {
         int p, q;
         pair(t, p, q);
-        // tt = tan of the smaller angle that annihilates A[p][q]
+        // tt = tan of the smaller angle that annihilates A[p][q]; c = (1 + tt^2)^-1/2
+        // with the rounding errors of 1 + tt^2 and of z r put back
         const double b = 2.0 * A[p * LD + q], d = A[q * LD + q] - A[p * LD + p];
-        const double h2 = d * d + b * b;
-        const double den = fabs(d) + h2 * __builtin_amdgcn_rsq(h2);
-        const double tt = (d < 0.0 ? -b : b) * __builtin_amdgcn_rcp(den);
         double2 cs = make_double2(1.0, 0.0);
-        if (fabs(tt) < 2.0) {  // not for a vanishing or overflowing h2
-          const double z = tt * tt + 1.0, g = __builtin_amdgcn_rsq(z);
-          const double er = fma(-z * g, g, 1.0);
-          cs.x = fma(g * er, fma(0.375, er, 0.5), g);
+        if (b != 0.0) {
+          const double tt = (d < 0.0 ? -b : b) / (fabs(d) + hypot(d, b));
+          const double z = fma(tt, tt, 1.0), zl = fma(tt, tt, 1.0 - z);
+          const double r0 = 1.0 / sqrt(z), zr = z * r0, zrl = fma(z, r0, -zr);
+          const double er = fma(-zr, r0, 1.0) - fma(zl * r0, r0, zrl * r0);
+          cs.x = fma(0.5 * r0, er, r0);
           cs.y = tt * cs.x;
         }
         rot[t] = cs;

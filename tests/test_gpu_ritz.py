@@ -38,3 +38,25 @@ def test_engine_not_finite(cuda, value, slot, ncv):
         assert np.array_equal(got[k].evals, want[w])
     for k in (1, 4):
         assert np.isnan(got[k].evals).all() and got[k].nconv == 0
+
+
+@pytest.mark.parametrize("nev,ncv", [(8, 32), (10, 40), (12, 47), (12, 48)])
+def test_vectors_keep_their_norm(cuda, nev, ncv):
+    """A thick restart keeps Ritz vectors without normalising them again, so the
+    rotations that form their coefficients must not grow or shrink vectors on
+    average: an error of one sign in c^2 + s^2 adds up.  A vector sees about ten
+    sweeps of ncv rotations in each of four cycles, each rounding its square norm
+    by 2^-53 (root mean square) either way: a random walk of sqrt(40 ncv) 2^-53,
+    and 1 / sqrt(nev) of that for the mean of nev vectors.  Six of these are
+    allowed."""
+    from test_gpu_restart import _basis, _terms
+    from qsi_subspace_ed_amd.operators import SymbolicPMROperator
+    states, spins, W = _basis(1, 10, 513, 513)
+    H = _terms(spins, 24, 10, z=False, open_spins=False)
+    for k, p in enumerate(spins):
+        H.add_term(0.37 * 1.61 ** (k % 7) + 0.011 * k, SymbolicPMROperator.from_ops("z", [p]))
+    op = q.GpuOp(q.GpuBasis(states, W), H)
+    _, vecs, _, _ = op.eigsh(nev=nev, ncv=ncv, tol=1e-30, max_restarts=3, seed=3, n_evecs=nev,
+                             raise_on_noconv=False)
+    off = ((vecs * vecs).sum(0) - 1.0).cpu().numpy()
+    assert abs(off.mean()) <= 6 * np.sqrt(40 * ncv / nev) * 2.0 ** -53, off
