@@ -3440,6 +3440,35 @@ int qsi_op_create(qsi_basis_t b, const qsi_term_t* terms, int n_terms,
     for (auto& o : op->h_off) have.insert(key(o, false));
     for (auto& o : op->h_off) op->paired = op->paired && have.count(key(o, true)) != 0;
   }
+  // symmetric: the terms are the reversed terms, with their coefficients, slots,
+  // Z strings and signs.  A Z on a spin that the projector fixes is a sign; a Z on
+  // a flipped one changes the reverse's sign.
+  {
+    auto full = [](const OffTerm& o, bool rev) {
+      std::array<uint64_t, 10> k{};
+      int odd = o.sgn < 0.0 ? 1 : 0;
+      for (int w = 0; w < 2; ++w) {
+        const uint64_t z = o.Z[w] & ~o.m[w];
+        odd += __builtin_popcountll(o.Z[w] & o.m[w] & ~o.v[w]);
+        if (rev) odd += __builtin_popcountll(z & o.X[w]);
+        k[w] = o.X[w];
+        k[2 + w] = o.m[w];
+        k[4 + w] = rev ? o.v[w] ^ (o.X[w] & o.m[w]) : o.v[w];
+        k[6 + w] = z;
+      }
+      std::memcpy(&k[8], &o.c, sizeof(double));
+      k[9] = static_cast<uint64_t>(static_cast<int64_t>(o.slot)) << 1 | (odd & 1);
+      return k;
+    };
+    std::vector<std::array<uint64_t, 10>> a, r;
+    for (auto& o : op->h_off) {
+      a.push_back(full(o, false));
+      r.push_back(full(o, true));
+    }
+    std::sort(a.begin(), a.end());
+    std::sort(r.begin(), r.end());
+    op->symmetric = a == r;
+  }
   // the terms field by field and as TermRec records, behind the full records
   // and padded to whole chunks of 64
   op->n_plane = op->n_off / 64 * 64 + 64;

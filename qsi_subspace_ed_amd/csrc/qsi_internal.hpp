@@ -148,7 +148,8 @@ struct qsi_op_s {
   uint64_t* d_planes = nullptr;  // TermPlanes data (in the allocation of d_off)
   int n_plane = 0;
   bool ordered = false;          // every off-diagonal term's X lies under its m
-  bool paired = false;           // every off-diagonal term's reverse is a term too
+  bool paired = false;           // every off-diagonal term's reverse flip is a term's too
+  bool symmetric = false;        // ... with the same coefficient, slot, sign and Z string
   bool mostly_closed = false;    // sampled: most connected states are in the basis
   std::vector<qsi::OffTerm> h_off;
   std::vector<qsi::DiagTerm> h_diag;

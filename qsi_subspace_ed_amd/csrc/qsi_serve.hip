@@ -344,10 +344,11 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_restart(double* __restrict_
 
 // ---- steps of operators that are not symmetric ------------------------------
 // An operator whose terms lack their reverses (rings of a cluster one cell wide
-// pass through a spin twice) is not symmetric; thick-restart Lanczos does not
-// converge on it, so what a request returns at its restart limit depends on the
-// rounding of every step.  Those steps keep sums in kernels of their own and
-// Rayleigh-Ritz on the host.
+// pass through a spin twice), or whose reverses differ in coefficient, slot, sign
+// or Z string, is not symmetric; thick-restart Lanczos does not converge on it,
+// so what a request returns at its restart limit depends on the rounding of every
+// step.  Those steps keep sums in kernels of their own and Rayleigh-Ritz on the
+// host.
 
 // After pass 2's projections h2_c are summed: beta_c = |u_c| from the
 // kNormSlot partials, the scale 1/beta_c of the new vector u_c, and flag_c = 1
@@ -877,7 +878,7 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
   {
     int64_t rpb = ((E->D + kSumBlocks - 1) / kSumBlocks + 63) / 64 * 64;
     rpb = std::max<int64_t>(rpb, kSrvRowsMin);
-    E->plain = !op->paired;
+    E->plain = !op->symmetric;
     if (E->plain) rpb = std::min<int64_t>(rpb, kSrvRowsMax);
     E->rpb = static_cast<int>(rpb);
     E->nblk = static_cast<int>((E->D + rpb - 1) / rpb);

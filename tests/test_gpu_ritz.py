@@ -1,10 +1,13 @@
-"""What the solve engine returns where a request's projected matrix is not finite,
-on both sides of the order up to which the device diagonalises it."""
+"""The thick-restart solvers' Rayleigh-Ritz: what the solve engine returns where a
+request's projected matrix is not finite, on both sides of the order up to which
+the device diagonalises it; vectors that keep their norm over restarts; and
+operators that are not symmetric."""
 import numpy as np
 import pytest
 
 import qsi_subspace_ed_amd as q
 from qsi_subspace_ed_amd import latgen, serve
+from qsi_subspace_ed_amd.operators import SymbolicOpSum, SymbolicPMROperator
 
 pytestmark = pytest.mark.gpu
 
@@ -50,7 +53,6 @@ def test_vectors_keep_their_norm(cuda, nev, ncv):
     and 1 / sqrt(nev) of that for the mean of nev vectors.  Six of these are
     allowed."""
     from test_gpu_restart import _basis, _terms
-    from qsi_subspace_ed_amd.operators import SymbolicPMROperator
     states, spins, W = _basis(1, 10, 513, 513)
     H = _terms(spins, 24, 10, z=False, open_spins=False)
     for k, p in enumerate(spins):
@@ -60,3 +62,79 @@ def test_vectors_keep_their_norm(cuda, nev, ncv):
                              raise_on_noconv=False)
     off = ((vecs * vecs).sum(0) - 1.0).cpu().numpy()
     assert abs(off.mean()) <= 6 * np.sqrt(40 * ncv / nev) * 2.0 ** -53, off
+
+
+# Operators that are not symmetric: thick-restart Lanczos does not converge on
+# them, and what is returned at the restart limit follows from the rounding of
+# every step.  The values are what the solvers with one kernel per sum and
+# Rayleigh-Ritz on the host return; they are kept to the bit.
+def _hamiltonian(jd):
+    H = q.build_hamiltonian_g(jd, [-0.9, -0.5, -0.3, -0.7])
+    q.add_local_field(H, jd, [0.05, -0.02, 0.07])
+    return H
+
+
+def _operator(kind, slots):
+    """An operator that is not symmetric: rings of a cluster one cell wide pass
+    through a spin twice and lack their reverses ("unpaired"); or flips whose
+    reverses have another coefficient, slot, sign or Z string."""
+    if kind == "unpaired":
+        jd = latgen.Supercell((1, 2, 2)).to_dict()
+        H = serve.slotted_hamiltonian(jd) if slots else _hamiltonian(jd)
+        return q.GpuOp(q.enumerate_basis_device(jd, 0), H)
+    rng = np.random.default_rng(5)
+    states = np.zeros((513, 2), dtype=np.uint64)
+    states[:, 0] = np.sort(rng.choice(1 << 10, 513, replace=False))
+    H = SymbolicOpSum()
+    for k in range(16):
+        at = [int(v) for v in rng.choice(10, 3, replace=False)]
+        a = str(rng.choice(["+", "-"]))
+        b = "-" if a == "+" else "+"
+        slot = k % 4
+        c = float(rng.standard_normal())
+        O = SymbolicPMROperator.from_ops([a, b, "z"], at)
+        R = SymbolicPMROperator.from_ops([b, a, "z"], at)
+        if kind == "coefficient":
+            H.add_term(c, O)
+            H.add_term(c if k else 0.7 * c, R)
+        elif kind == "slot":
+            H.add_term(1.0, O, slot=slot)
+            H.add_term(1.0, R, slot=slot if k else 1)
+        elif kind == "sign":
+            R.sign = R.sign if k else -R.sign
+            H.add_term(1.0, O, slot=slot)
+            H.add_term(1.0, R, slot=slot)
+        else:
+            H.add_term(c, O)
+            H.add_term(c, R if k else SymbolicPMROperator.from_ops([b, a], at[:2]) *
+                       SymbolicPMROperator.from_ops("z", [(at[2] + 1) % 10]))
+    for p in range(10):
+        H.add_term(0.3 + 0.11 * p, SymbolicPMROperator.from_ops("z", [p]))
+    return q.GpuOp(q.GpuBasis(states, 10), H)
+
+
+ENGINE = {
+    ("unpaired", 1, 8): ["-0x1.9fe0d4c2c7c0cp+1", "-0x1.7072c5b6d0d7cp+1"],
+    ("unpaired", 3, 15): ["-0x1.9bf524818ecb4p+1", "-0x1.6fa7a1920b2adp+1"],
+    ("unpaired", 4, 40): ["-0x1.e14f6f44a4fd6p+1", "-0x1.6ff32dbf933dap+1"],
+    ("coefficient", 3, 15): ["-0x1.16f86942d6129p+3", "-0x1.17086c65509b9p+3"],
+    ("coefficient", 4, 40): ["-0x1.16f88457e3d0ap+3", "-0x1.17086e0fb5686p+3"],
+    ("slot", 3, 15): ["-0x1.1877479e14638p+3", "-0x1.0bc5c954f6703p+3"],
+    ("slot", 4, 40): ["-0x1.187747d8455e1p+3", "-0x1.0bc682daf1cdap+3"],
+    ("sign", 3, 15): ["-0x1.15c12481f49a8p+3", "-0x1.0b422f2ee88dbp+3"],
+    ("sign", 4, 40): ["-0x1.15c104ff95c17p+3", "-0x1.0b43c0a9874dap+3"],
+    ("z", 3, 15): ["-0x1.16f0dd958dff8p+3", "-0x1.170022242d1f7p+3"],
+    ("z", 4, 40): ["-0x1.16f0d32ec16c0p+3", "-0x1.17001f54ce088p+3"],
+}
+
+
+@pytest.mark.parametrize("kind,nev,ncv", list(ENGINE))
+def test_engine_not_symmetric(cuda, kind, nev, ncv):
+    """The first and the last of five requests on three columns."""
+    op = _operator(kind, True)
+    eng = serve.Engine(op, max_cols=3, nev=nev, ncv=ncv, tol=1e-10, max_restarts=4,
+                       autotune=False, cache_connectivity=False)
+    c = np.random.default_rng(2).uniform(-1.0, -0.2, size=(5, op.n_slots))
+    ids = [eng.submit(c[k], 11 + k) for k in range(5)]
+    got = {f.id: f.evals[0] for f in eng.run_all()}
+    assert [float(got[ids[k]]).hex() for k in (0, 4)] == ENGINE[kind, nev, ncv]
