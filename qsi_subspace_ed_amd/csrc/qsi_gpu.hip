@@ -1608,6 +1608,14 @@ inline int vec_blocks(int64_t n) {
   return static_cast<int>(std::max<int64_t>(1, std::min<int64_t>(nb, 8192)));
 }
 
+// Workgroups of the projection passes that leave their sums to a kernel of
+// their own: about 16 rows per thread, but at least 1024 workgroups while there
+// are 4 rows per thread to give them.
+inline int proj_blocks(int64_t n) {
+  const int64_t want = (n + kVecBlock * 16 - 1) / (kVecBlock * 16);
+  return static_cast<int>(std::min<int64_t>(vec_blocks(n), std::max<int64_t>(want, 1024)));
+}
+
 // The grid-stride dot, axpy-norm and device-scalar scale kernels take
 // kVecUnroll of a thread's elements per round, all loads first, and
 // accumulate in element order (the sums are the ones a one-element loop
@@ -1701,6 +1709,8 @@ constexpr int kMaxCols = 64;
 // the reads of V bound passes 1 and 2 (42 and 48 us, 5.4 TB/s), and 256
 // workgroups of 512 threads keep enough of them in flight.
 // partials[j * gridDim.x + workgroup] is column j's.
+// SUMS = false (operators that are not symmetric, whose results depend on every
+// rounding): the sums are k_finalize_cols's, over more workgroups.
 constexpr int kGsBlocks = kSumBlocks;
 
 // Pass 1: partials of V[:, 0:m]^T w, 16 columns at a time.
@@ -1740,10 +1750,20 @@ __global__ __launch_bounds__(T) void k_gs_dots(
   }
 }
 
-// Pass 2: h = pass 1's sums (written to hcol by one workgroup), w -= V[:, 0:m] h,
-// and from the same read of V the partials of V[:, 0:m]^T w_new (columns
+// out[j] = sum_b partials[j * nb + b], one workgroup per column j, fixed order
+__global__ __launch_bounds__(256) void k_finalize_cols(const double* __restrict__ partials,
+                                                       int nb, double* __restrict__ out) {
+  const double* p = partials + static_cast<int64_t>(blockIdx.x) * nb;
+  double v = 0.0;
+  for (int b = threadIdx.x; b < nb; b += 256) v += p[b];
+  v = block_sum<256>(v);
+  if (threadIdx.x == 0) out[blockIdx.x] = v;
+}
+
+// Pass 2: h = pass 1's sums (written to hcol by one workgroup; part1 itself
+// without SUMS), w -= V[:, 0:m] h, and from the same read of V the partials of V[:, 0:m]^T w_new (columns
 // 0..m-1) and of w_new . w_new (column m), m <= MAXC.
-template <int T, int MAXC>
+template <int T, int MAXC, bool SUMS>
 __global__ __launch_bounds__(T) void k_gs_sub_dots(
     const double* __restrict__ V, int64_t ldv, int m, const double* __restrict__ part1,
     double* __restrict__ hcol, double* __restrict__ w, int64_t n,
@@ -1751,10 +1771,12 @@ __global__ __launch_bounds__(T) void k_gs_sub_dots(
   __shared__ double hs[MAXC];
   __shared__ double red[T / kWave][MAXC + 1];
   const int lane = threadIdx.x % kWave, wid = threadIdx.x / kWave;
-  if (threadIdx.x < MAXC) hs[threadIdx.x] = 0.0;
+  if (threadIdx.x < MAXC) hs[threadIdx.x] = !SUMS && threadIdx.x < m ? part1[threadIdx.x] : 0.0;
   __syncthreads();
-  sum_partials<T>(part1, gridDim.x, m, hs);
-  if (blockIdx.x == 0 && threadIdx.x < m) hcol[threadIdx.x] = hs[threadIdx.x];
+  if constexpr (SUMS) {
+    sum_partials<T>(part1, gridDim.x, m, hs);
+    if (blockIdx.x == 0 && threadIdx.x < m) hcol[threadIdx.x] = hs[threadIdx.x];
+  }
   double acc[MAXC], nrm = 0.0;
 #pragma unroll
   for (int j = 0; j < MAXC; ++j) acc[j] = 0.0;
@@ -1791,16 +1813,21 @@ __global__ __launch_bounds__(T) void k_gs_sub_dots(
 }
 
 // The tail of the step: g[0..m) = V^T w and g[m] = w . w from pass 2's
-// partials.  A third pass w -= V g is needed when |V^T w| > 1e-12 |w|; its
+// partials (part2 itself without SUMS).  A third pass w -= V g is needed when |V^T w| > 1e-12 |w|; its
 // correction is added to the projected column hcol[0..m) and the norm follows
 // it.  Then w *= 1 / |w|, and one workgroup writes beta[0] = |w|, beta[1] =
 // 1 / |w| (0 for a vanishing w).
-template <int T>
+template <int T, bool SUMS>
 __global__ __launch_bounds__(T) void k_gs_tail(
     const double* __restrict__ V, int64_t ldv, int m, const double* __restrict__ part2,
     double* __restrict__ hcol, double* __restrict__ w, int64_t n, double* __restrict__ beta) {
   __shared__ double g[kMaxCols + 1];
-  sum_partials<T>(part2, gridDim.x, m + 1, g);
+  if constexpr (SUMS) {
+    sum_partials<T>(part2, gridDim.x, m + 1, g);
+  } else {
+    if (threadIdx.x <= m) g[threadIdx.x] = part2[threadIdx.x];
+    __syncthreads();
+  }
   double g2 = 0.0;
   for (int j = 0; j < m; ++j) g2 += g[j] * g[j];
   const double q = g[m];
@@ -2687,30 +2714,60 @@ int launch_axpy_norm(const double* alpha_dev, const double* v, double* u,
 }
 
 int max_vec_partials() { return 8192; }
-int gs_partials() { return kGsBlocks * (2 * kMaxCols + 1); }
+constexpr int kPlainPartials = 1 << 17;
+int gs_partials(bool plain) {
+  return plain ? kPlainPartials + kMaxCols + 1 : kGsBlocks * (2 * kMaxCols + 1);
+}
+
+namespace {
+// Pass 2 of 16, 32 or 64 columns at most.
+template <int T, bool SUMS>
+void launch_gs_sub_dots(int nb, const double* V, int64_t ldv, int m, const double* part1,
+                        double* hcol, double* w, int64_t n, double* part2, hipStream_t s) {
+  if (m <= 16)
+    hipLaunchKernelGGL((k_gs_sub_dots<T, 16, SUMS>), dim3(nb), dim3(T), 0, s, V, ldv, m, part1,
+                       hcol, w, n, part2);
+  else if (m <= 32)
+    hipLaunchKernelGGL((k_gs_sub_dots<T, 32, SUMS>), dim3(nb), dim3(T), 0, s, V, ldv, m, part1,
+                       hcol, w, n, part2);
+  else if constexpr (T <= kVecBlock)
+    hipLaunchKernelGGL((k_gs_sub_dots<T, 64, SUMS>), dim3(nb), dim3(T), 0, s, V, ldv, m, part1,
+                       hcol, w, n, part2);
+}
+
+template <int T>
+void launch_gs(const double* V, int64_t ldv, int m, double* w, int64_t n, double* partials,
+               double* hcol, double* beta, hipStream_t s) {
+  double* part2 = partials + static_cast<int64_t>(kGsBlocks) * kMaxCols;
+  const int nb = static_cast<int>(std::min<int64_t>((n + T - 1) / T, kGsBlocks));
+  hipLaunchKernelGGL(k_gs_dots<T>, dim3(nb), dim3(T), 0, s, V, ldv, m, w, n, partials);
+  launch_gs_sub_dots<T, true>(nb, V, ldv, m, partials, hcol, w, n, part2, s);
+  hipLaunchKernelGGL((k_gs_tail<T, true>), dim3(nb), dim3(T), 0, s, V, ldv, m, part2, hcol, w, n,
+                     beta);
+}
+}  // namespace
 
 int launch_gs_step(const double* V, int64_t ldv, int m, double* w, int64_t n, double* partials,
-                   double* hcol, double* beta, hipStream_t s) {
+                   double* hcol, double* beta, bool plain, hipStream_t s) {
   if (m <= 0 || m > kMaxCols) {
     set_error("launch_gs_step: column count out of range");
     return QSI_E_INVALID;
   }
-  double* part2 = partials + static_cast<int64_t>(kGsBlocks) * kMaxCols;
-  auto blocks = [&](int T) {
-    return static_cast<int>(std::min<int64_t>((n + T - 1) / T, kGsBlocks));
-  };
-#define QSI_GS(T_, C_)                                                                           \
-  do {                                                                                           \
-    const dim3 nb(blocks(T_));                                                                   \
-    hipLaunchKernelGGL(k_gs_dots<T_>, nb, dim3(T_), 0, s, V, ldv, m, w, n, partials);            \
-    hipLaunchKernelGGL((k_gs_sub_dots<T_, C_>), nb, dim3(T_), 0, s, V, ldv, m, partials, hcol, w, \
-                       n, part2);                                                                \
-    hipLaunchKernelGGL(k_gs_tail<T_>, nb, dim3(T_), 0, s, V, ldv, m, part2, hcol, w, n, beta);   \
-  } while (0)
-  if (m <= 16) QSI_GS(512, 16);
-  else if (m <= 32) QSI_GS(512, 32);
-  else QSI_GS(256, 64);
-#undef QSI_GS
+  if (plain) {
+    double* g = partials + kPlainPartials;
+    const int nb = std::max(1, std::min(proj_blocks(n), kPlainPartials / (m + 1)));
+    hipLaunchKernelGGL(k_gs_dots<kVecBlock>, dim3(nb), dim3(kVecBlock), 0, s, V, ldv, m, w, n,
+                       partials);
+    hipLaunchKernelGGL(k_finalize_cols, dim3(m), dim3(256), 0, s, partials, nb, hcol);
+    launch_gs_sub_dots<kVecBlock, false>(nb, V, ldv, m, hcol, nullptr, w, n, partials, s);
+    hipLaunchKernelGGL(k_finalize_cols, dim3(m + 1), dim3(256), 0, s, partials, nb, g);
+    hipLaunchKernelGGL((k_gs_tail<kVecBlock, false>), dim3(vec_blocks(n)), dim3(kVecBlock), 0, s,
+                       V, ldv, m, g, hcol, w, n, beta);
+  } else if (m <= 32) {
+    launch_gs<512>(V, ldv, m, w, n, partials, hcol, beta, s);
+  } else {
+    launch_gs<kVecBlock>(V, ldv, m, w, n, partials, hcol, beta, s);
+  }
   QSI_CHECK_LAUNCH();
   return QSI_OK;
 }

@@ -210,7 +210,7 @@ int64_t apply_num_blocks(const qsi_op_s* op);
 // streaming vector kernels; partial buffers need max_vec_partials() doubles
 // (gs_partials() for launch_gs_step)
 int max_vec_partials();
-int gs_partials();
+int gs_partials(bool plain);
 int launch_dot(const double* a, const double* b, int64_t n, double* partials,
                double* out, hipStream_t s);
 int launch_axpy(double alpha, const double* x, double* y, int64_t n,
@@ -226,9 +226,10 @@ int launch_axpy_norm(const double* alpha_dev, const double* v, double* u,
 // the projections (the third pass's correction included), beta[0] = |w| at the
 // end, beta[1] = 1 / beta[0] (0 if w vanishes), and w is scaled by beta[1].
 // partials: gs_partials() doubles.  All on the device (no host
-// synchronisation).
+// synchronisation).  plain: the sums in kernels of their own, for operators that
+// are not symmetric (their results at the restart limit depend on every rounding).
 int launch_gs_step(const double* V, int64_t ldv, int m, double* w, int64_t n, double* partials,
-                   double* hcol, double* beta, hipStream_t s);
+                   double* hcol, double* beta, bool plain, hipStream_t s);
 
 // Rayleigh-Ritz of n_jobs thick-restart Lanczos matrices of order m <= kRitzMax,
 // one workgroup each.  Workgroup b takes job[b], whose kept[b] first vectors

@@ -493,10 +493,12 @@ int qsi_eigsh(qsi_op_t op, int nev, int ncv, double tol, int max_restarts,
   n_evecs = std::min(n_evecs, nev);
   const int64_t ld = (D + 63) / 64 * 64;
   hipStream_t s = nullptr;
+  // operators that are not symmetric: as the solve engine's plain steps
+  const bool plain = !op->symmetric;
   DevBuf bV, bW, bpart, bscal;
   QSI_CHECK_HIP(bV.alloc(static_cast<size_t>(ld) * (ncv + 1) * sizeof(double)));
   QSI_CHECK_HIP(bW.alloc(static_cast<size_t>(ld) * (ncv + 1) * sizeof(double)));
-  QSI_CHECK_HIP(bpart.alloc(std::max(max_vec_partials(), gs_partials()) * sizeof(double)));
+  QSI_CHECK_HIP(bpart.alloc(std::max(max_vec_partials(), gs_partials(plain)) * sizeof(double)));
   QSI_CHECK_HIP(bscal.alloc(4 * sizeof(double)));
   DevBuf bY;  // Ritz coefficients of a restart (at most ncv x ncv)
   QSI_CHECK_HIP(bY.alloc(static_cast<size_t>(ncv) * ncv * sizeof(double)));
@@ -509,7 +511,7 @@ int qsi_eigsh(qsi_op_t op, int nev, int ncv, double tol, int max_restarts,
   QSI_CHECK_HIP(btheta.alloc(ncv * sizeof(double)));
   double* dT = bx.d();
   double* dbeta = dT + n_T;
-  const bool dev_ritz = ncv <= kRitzMax;
+  const bool dev_ritz = !plain && ncv <= kRitzMax;
   double* V = bV.d();
   double* W = bW.d();
   int applies = 0;
@@ -548,7 +550,8 @@ int qsi_eigsh(qsi_op_t op, int nev, int ncv, double tol, int max_restarts,
       double* hcol = dT + static_cast<size_t>(j) * ncv;
       QSI_TRY(launch_apply(op, vj, w, nullptr, 0.0, nullptr, nullptr, s));
       ++applies;
-      QSI_TRY(launch_gs_step(V, ld, j + 1, w, D, bpart.d(), hcol, dbeta + 2 * j, s));
+      QSI_TRY(launch_gs_step(V, ld, j + 1, w, D, bpart.d(), hcol, dbeta + 2 * j, plain,
+                             s));
     }
     if (dev_ritz) {
       RitzArgs r{};
@@ -588,7 +591,8 @@ int qsi_eigsh(qsi_op_t op, int nev, int ncv, double tol, int max_restarts,
       beta_last = beta;
     }
     // Rayleigh-Ritz on the m x m projected matrix: the device's, or here where
-    // the subspace ended early or is larger than the device kernel takes
+    // the subspace ended early or is larger than the device kernel takes, or the
+    // operator is not symmetric
     std::vector<double> last(m);
     if (dev_ritz && m == ncv) {
       theta.assign(hbeta + 2 * ncv, hbeta + 3 * ncv);

@@ -138,3 +138,37 @@ def test_engine_not_symmetric(cuda, kind, nev, ncv):
     ids = [eng.submit(c[k], 11 + k) for k in range(5)]
     got = {f.id: f.evals[0] for f in eng.run_all()}
     assert [float(got[ids[k]]).hex() for k in (0, 4)] == ENGINE[kind, nev, ncv]
+
+
+EIGSH = {
+    ("unpaired", 1, 8): ["-0x1.85801080438b4p+1"],
+    ("unpaired", 3, 15): [
+        "-0x1.880140e659e0dp+1", "-0x1.5db61958a620cp+1", "-0x1.2ec5de7bffba5p+1"],
+    ("unpaired", 4, 40): [
+        "-0x1.7d7baec051c76p+1", "-0x1.737b84701f64fp+1", "-0x1.5cb90754572f2p+1",
+        "-0x1.04f10d5fb1ff0p+1"],
+    ("coefficient", 3, 15): [
+        "-0x1.16f77984bc2c1p+3", "-0x1.032bf7a933870p+3", "-0x1.01d9850bfff13p+3"],
+    ("coefficient", 4, 40): [
+        "-0x1.16f77963bde57p+3", "-0x1.03281b4ccf654p+3", "-0x1.01d90e88b3bc8p+3",
+        "-0x1.fde173ff380d4p+2"],
+    ("slot", 3, 15): ["-0x1.4dd4ce9d6be9ep+3", "-0x1.1e06b85639decp+3", "-0x1.0bb6c10d340aap+3"],
+    ("slot", 4, 40): [
+        "-0x1.4dd4ce9d6bea4p+3", "-0x1.1e06b85639dd3p+3", "-0x1.0bb6c10d8a04fp+3",
+        "-0x1.0381eccf9cf2ep+3"],
+    ("sign", 3, 15): ["-0x1.49cfdf30570c4p+3", "-0x1.1830bca798542p+3", "-0x1.0b9e600ddbccap+3"],
+    ("sign", 4, 40): [
+        "-0x1.49cf772b4be51p+3", "-0x1.1858fbe961848p+3", "-0x1.064ca6a064eb2p+3",
+        "-0x1.ee510a93e7c47p+2"],
+    ("z", 3, 15): ["-0x1.16e5d80e0ad31p+3", "-0x1.03a0d26f18c47p+3", "-0x1.01a406039092dp+3"],
+    ("z", 4, 40): [
+        "-0x1.16e5e0820c03ap+3", "-0x1.039f3c19c5468p+3", "-0x1.01ace8cf41a5cp+3",
+        "-0x1.fdbfc88094235p+2"],
+}
+
+
+@pytest.mark.parametrize("kind,nev,ncv", list(EIGSH))
+def test_eigsh_not_symmetric(cuda, kind, nev, ncv):
+    evals = _operator(kind, False).eigsh(nev=nev, ncv=ncv, tol=1e-10, max_restarts=4, seed=3,
+                                         raise_on_noconv=False)[0]
+    assert [float(v).hex() for v in evals] == EIGSH[kind, nev, ncv]
