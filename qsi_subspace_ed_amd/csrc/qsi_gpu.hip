@@ -1055,6 +1055,20 @@ constexpr int64_t kWinMinDim = int64_t{1} << 21;
 constexpr int64_t kWinMinDimLow2 = int64_t{1} << 28;
 constexpr int kWinRows = 128;  // rows of a wavefront, and ranks of a window
 constexpr int kWinMax = 8;     // windows of one term (a wider range: per-row lookups)
+// Windows of a term whose first and last target have ranks la and lz in a basis of
+// dim states; 0 (per-row lookups) if they are too many, pass the end of the
+// arrays, or the targets do not keep the rows' order.  With la <= lz < dim <=
+// 2^32 - 512 the end of the last one does not pass 2^32.
+__host__ __device__ constexpr uint32_t win_count(uint32_t la, uint32_t lz, uint32_t dim) {
+  const uint32_t n = (lz - la) / kWinRows + 1;
+  return la <= lz && n <= kWinMax && la + n * kWinRows <= dim ? n : 0;
+}
+static_assert(win_count(0, 127, 128) == 1 && win_count(1, 127, 128) == 0 &&
+              win_count(0, 128, 256) == 2 && win_count(0, 1024, 4096) == 0 &&
+              win_count(5, 4, 4096) == 0);
+// a last target far before the first one wraps to a short range there
+static_assert(win_count(0xFFFFFDFEu, 0, 0xFFFFFE00u) == 0 &&
+              win_count(0xFFFFFDFFu, 1, 0xFFFFFE00u) == 0);
 __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -1389,9 +1403,8 @@ __attribute__((amdgpu_waves_per_eu(kWinWaves<NW, CHECK>))) void k_apply_win(
           good = st_eq<NW>(fa, ka) && st_eq<NW>(fz, kz);
         }
       }
-      // every window of the term lies inside the arrays
-      uint32_t n_win = (lz - la) / kWinRows + 1;
-      good = good && n_win <= kWinMax && la + n_win * kWinRows <= dim32;
+      uint32_t n_win = win_count(la, lz, dim32);
+      good = good && n_win != 0;
       if constexpr (CHECK) {
         const int bad = __popcll(__builtin_amdgcn_ballot_w64(has && !good));
         if (2 * bad > __popcll(__builtin_amdgcn_ballot_w64(has))) {
