@@ -2901,9 +2901,11 @@ int launch_observe(const qsi_basis_s* basis, const ObserveArgs& q, const double*
   const int nb = (q.P + 15) / 16, blocks = observe_blocks(basis->dim);
   const size_t lds = static_cast<size_t>(16 * nb + (q.same ? 0 : 16)) * kObsLd * sizeof(double);
   auto kern = basis->nw == 1 ? k_observe<1> : k_observe<2>;
+  // the attribute is the process's: every call sets the most that any call needs,
+  // or a thread with fewer columns could lower it under another's launch
   QSI_CHECK_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                     hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    static_cast<int>(lds)));
+                                    (kObsCols + 16) * kObsLd * static_cast<int>(sizeof(double))));
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), lds, s, basis->view(), q, psi, ld, partials);
   QSI_CHECK_LAUNCH();
   hipLaunchKernelGGL(k_gram_sum<16>, dim3(q.tiles * 8), dim3(256), 0, s, partials, blocks, q.P,
