@@ -165,9 +165,10 @@ int qsi_op_n_diag(qsi_op_t op);
  * bucket on the basis's low keys (qsi_basis_build_lowkeys); setting one
  * requires them, and without them later the apply falls back to LANE* of the
  * same depth.  AUTO = CACHED when the connectivity is cached; else WINDOW on
- * bases of at least 2^21 states whose connected states are mostly in the basis
- * and whose terms flip no spin outside their projectors (after
- * qsi_op_verify_lowkeys found mode 2: one-word states, or at least 2^28
+ * bases of at least 2^21 states where at most one in 32 sampled pairs of 128 rows
+ * and a term leads out of the basis (one in 64, and one-word states, after
+ * qsi_op_verify_lowkeys found mode 1) and whose terms flip no spin outside their
+ * projectors (after mode 2: one-word states, or at least 2^28
  * of two words, and a term list that holds every flip's reverse); else, when the
  * basis has low keys, LOW8 after mode 2 and LOW4 otherwise, else LANE4.
  * All give bit-identical y. */

@@ -169,22 +169,31 @@ __global__ void k_verify_lowkeys(BasisView b, const OffTerm* __restrict__ off, i
   if (clash || absent) atomicOr(bad, (clash ? 1u : 0u) | (absent ? 2u : 0u));
 }
 
-// cnt[0] += connecting (row, term) pairs of gridDim.x * blockDim.x rows spread
-// evenly over the basis, cnt[1] += those whose target is in the basis.
+// cnt[0] += (tile, term) pairs that connect, of gridDim.x tiles of 128 rows spread
+// evenly over the basis; cnt[1] += those with a target that is not in the basis.
+// One tile per workgroup, its wavefronts taking every fourth term.
 template <int NW>
-__global__ void k_sample_closed(BasisView b, const OffTerm* __restrict__ off, int n_off,
-                                unsigned int* __restrict__ cnt) {
-  const int64_t n = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  const int64_t k = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  const State<NW> s = load_state_cached<NW>(b.states, b.dim / n * k);
-  unsigned int conn = 0, found = 0;
-  for (int t = 0; t < n_off; ++t) {
-    if (!term_ok<NW>(off[t], s)) continue;
+__global__ __launch_bounds__(256) void k_sample_closed(BasisView b,
+                                                       const OffTerm* __restrict__ off, int n_off,
+                                                       unsigned int* __restrict__ cnt) {
+  const int lane = threadIdx.x % kWave;
+  const int64_t r0 = b.dim / 128 / gridDim.x * blockIdx.x * 128 + lane;
+  const State<NW> s0 = load_state_cached<NW>(b.states, r0);
+  const State<NW> s1 = load_state_cached<NW>(b.states, r0 + 64);
+  unsigned int conn = 0, missing = 0;
+  for (int t = threadIdx.x / kWave; t < n_off; t += 4) {
+    const OffTerm& T = off[t];
+    const bool c0 = term_ok<NW>(T, s0), c1 = term_ok<NW>(T, s1);
+    if (!__any(c0 || c1)) continue;
+    const bool miss = (c0 && basis_lookup<NW>(b, xor_state<NW>(s0, T.X)) < 0) ||
+                      (c1 && basis_lookup<NW>(b, xor_state<NW>(s1, T.X)) < 0);
     ++conn;
-    found += basis_lookup<NW>(b, xor_state<NW>(s, off[t].X)) >= 0 ? 1u : 0u;
+    missing += __any(miss) ? 1u : 0u;
   }
-  atomicAdd(cnt, conn);
-  atomicAdd(cnt + 1, found);
+  if (lane == 0) {
+    atomicAdd(cnt, conn);
+    atomicAdd(cnt + 1, missing);
+  }
 }
 
 // lowkeys[i] = low key of state i (qsi_basis_build_lowkeys)
@@ -2442,8 +2451,15 @@ static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
   // the chip with its 128-row wavefronts (WINDOW / LANE4 / LOW4 in us: 32 spins
   // 35 / 12 / 13, 293394 states 33 / 25 / 25, 1062882 states 55 / 52 / 53, 64 spins 200 /
   // 266 / 273, 72 spins 1467 / 2089 / 1831; 80 spins 10.1 / 17.6 / 14.3 and 96 spins
-  // 301 / 543 ms), if the sampled rows' targets are mostly in the basis (64 spins
-  // with single flips, which all leave it, 678 / 456).  With them LOW8, except where WINDOW
+  // 301 / 543 ms), if few of the sampled (tile, term) pairs have a target outside
+  // the basis: such a term is done again by per-row lookups.  By the share of such
+  // pairs, WINDOW / LANE4 / LOW4 unverified / LOW4 after mode 1: 60 spins at 0 171 /
+  // 224 / 218 / - us, 2 % 201 / 221 / 214 / 202, 5 % 238 / 224 / 215 / 202; 64 spins, one
+  // pair, 1 % 356 / 522 / - / 449; 64 spins, 4 % 254 / 271 / - / 235, 11 % 312 / 269 / - / 233,
+  // 30 % 428 / 268 / - / 231; 72 spins, one pair, 1 % 2.92 / 4.20 / 3.57 / 2.82 ms, 2 %
+  // 3.27 / 4.21 / 3.57 / 2.82, 5 % 3.93 / 4.21 / 3.57 / 2.82; 64 spins, two pairs, 32 %
+  // 115 / 91 ms.  So up to 1/32, with key compares (mode 1) up to 1/64 and one-word
+  // states only.  With low keys that need no compare LOW8, except where WINDOW
   // without its compare is the faster: one-word states on large bases (WINDOW /
   // LOW8: 293394 states 33 / 21, 64 spins 181 / 190, 60 spins 166 / 191 us) and bases so
   // large that the 31-bit bucket key leaves long bisections (72 spins 1.21 / 1.18,
@@ -2459,10 +2475,12 @@ static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
         return;
       }
     }
-    const bool trusted = op->basis->d_lowkeys && op->lowkeys_check == kLowTrusted;
-    const bool window = 
-        dim >= kWinMinDim && op->ordered &&
-        (trusted ? op->paired && (NW == 1 || dim >= kWinMinDimLow2) : op->mostly_closed);
+    const int check = op->basis->d_lowkeys ? op->lowkeys_check : kLowCmpState;
+    const bool trusted = check == kLowTrusted;
+    bool window = dim >= kWinMinDim && op->ordered;
+    if (trusted) window = window && op->paired && (NW == 1 || dim >= kWinMinDimLow2);
+    else if (check == kLowCmpKey) window = window && NW == 1 && op->miss_share <= 1.0f / 64;
+    else window = window && op->miss_share <= 1.0f / 32;
     variant = op->conn_nnz >= 0        ? QSI_APPLY_CACHED
               : window                 ? QSI_APPLY_WINDOW
               : trusted                ? QSI_APPLY_LOW8
@@ -3609,18 +3627,18 @@ int qsi_op_create(qsi_basis_t b, const qsi_term_t* terms, int n_terms,
     return e == hipErrorOutOfMemory ? QSI_E_NOMEM : QSI_E_HIP;
   }
   if (b->dim >= kWinMinDim && op->n_off > 0) {
-    // whether the terms mostly stay in the basis, by 4096 rows: AUTO's choice
-    // between kernels of equal results
+    // how many of the window kernel's (tile, term) pairs have a target outside the
+    // basis, by 64 tiles: AUTO's choice between kernels of equal results
     unsigned int* cnt = nullptr;
     unsigned int h[2] = {0, 0};
     e = hipMalloc(&cnt, sizeof(h));
     if (e == hipSuccess) e = hipMemset(cnt, 0, sizeof(h));
     if (e == hipSuccess) {
       if (nw == 1)
-        hipLaunchKernelGGL(k_sample_closed<1>, dim3(64), dim3(64), 0, 0, b->view(), op->d_off,
+        hipLaunchKernelGGL(k_sample_closed<1>, dim3(64), dim3(256), 0, 0, b->view(), op->d_off,
                            op->n_off, cnt);
       else
-        hipLaunchKernelGGL(k_sample_closed<2>, dim3(64), dim3(64), 0, 0, b->view(), op->d_off,
+        hipLaunchKernelGGL(k_sample_closed<2>, dim3(64), dim3(256), 0, 0, b->view(), op->d_off,
                            op->n_off, cnt);
       e = hipGetLastError();
     }
@@ -3634,7 +3652,7 @@ int qsi_op_create(qsi_basis_t b, const qsi_term_t* terms, int n_terms,
       set_error(std::string("qsi_op_create: ") + hipGetErrorString(e));
       return QSI_E_HIP;
     }
-    op->mostly_closed = h[1] >= h[0] - h[0] / 8;
+    op->miss_share = h[0] ? static_cast<float>(h[1]) / static_cast<float>(h[0]) : 0.0f;
   }
   basis_retain(b);
   op->basis = b;

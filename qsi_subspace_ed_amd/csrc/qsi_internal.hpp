@@ -150,7 +150,9 @@ struct qsi_op_s {
   bool ordered = false;          // every off-diagonal term's X lies under its m
   bool paired = false;           // every off-diagonal term's reverse flip is a term's too
   bool symmetric = false;        // ... with the same coefficient, slot, sign and Z string
-  bool mostly_closed = false;    // sampled: most connected states are in the basis
+  // sampled on large bases: of the pairs of 128 rows and a term that connect, the
+  // share with a target outside the basis
+  float miss_share = 0.0f;
   std::vector<qsi::OffTerm> h_off;
   std::vector<qsi::DiagTerm> h_diag;
   int n_cls = 0;  // coefficient classes (0: more than kMaxCoefClasses)

@@ -1,0 +1,59 @@
+"""The automatic choice of the apply kernel against the kernels it chooses from:
+it is not left behind by the fixed choices where it was measured to lose."""
+import numpy as np
+import pytest
+
+import qsi_subspace_ed_amd as q
+from qsi_subspace_ed_amd import latgen
+
+pytestmark = pytest.mark.gpu
+
+
+def _times(cuda, ops, n=20, rounds=5):
+    """Shortest time (us) of n applies of each of ops, taken in turn."""
+    x = cuda.randn(ops[0].rows(), dtype=cuda.float64, device="cuda")
+    y = cuda.empty_like(x)
+    best = [np.inf] * len(ops)
+    for _ in range(rounds + 1):
+        for k, op in enumerate(ops):
+            a, b = (cuda.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(n):
+                op.evaluate(x, y)
+            b.record()
+            b.synchronize()
+            best[k] = min(best[k], a.elapsed_time(b) / n * 1e3)
+    return best
+
+
+def _ops(basis, H, variants):
+    out = []
+    for v in variants:
+        op = q.GpuOp(basis, H)
+        op.set_variant(v)
+        out.append(op)
+    return out
+
+
+@pytest.mark.parametrize("missing", [0.0, 0.01, 0.03, 0.1])
+def test_scattered_misses(cuda, missing):
+    """64 spins with states left out at random: where terms lead out of the basis
+    all over, the window kernel takes up to twice the lane kernel's time."""
+    jd = latgen.Supercell((2, 2, 4)).to_dict()
+    H = q.build_hamiltonian_g(jd, [-0.9, -0.5, -0.3, -0.7])
+    states = q.enumerate_basis_device(jd, 0).states()
+    keep = np.random.default_rng(1).random(states.shape[0]) >= missing
+    basis = q.GpuBasis(np.ascontiguousarray(states[keep]), 64)
+    auto, lane = _times(cuda, _ops(basis, H, ("auto", "lane4")))
+    assert auto <= 1.2 * lane, (auto, lane)
+    if missing == 0.0:
+        assert auto <= 0.9 * lane, (auto, lane)
+
+
+def test_one_pair_sector(cuda):
+    """A sector that few terms lead out of, together, stays on the window kernel."""
+    jd = latgen.Supercell((1, 3, 5)).to_dict()
+    H = q.build_hamiltonian_g(jd, [-0.9, -0.5, -0.3, -0.7])
+    basis = q.enumerate_basis_device(jd, 1)
+    auto, lane = _times(cuda, _ops(basis, H, ("auto", "lane4")))
+    assert auto <= 0.9 * lane, (auto, lane)
