@@ -164,7 +164,8 @@ int qsi_op_n_diag(qsi_op_t op);
  * LANE4 (SLOT4) or LANE2.  QSI_APPLY_LOW{2,4,8}: as LANE*, bisecting each
  * bucket on the basis's low keys (qsi_basis_build_lowkeys); setting one
  * requires them, and without them later the apply falls back to LANE* of the
- * same depth.  AUTO = CACHED when the connectivity is cached; else WINDOW on
+ * same depth.  AUTO = CACHED when the connectivity is cached; else, up to 2^14
+ * states and without a dot product, a wavefront per row; else WINDOW on
  * bases of at least 2^21 states where at most one in 32 sampled pairs of 128 rows
  * and a term leads out of the basis (one in 64, and one-word states, after
  * qsi_op_verify_lowkeys found mode 1) and whose terms flip no spin outside their
@@ -265,7 +266,8 @@ int qsi_op_get_block_cfg(qsi_op_t op);
 /* Autotuner: times the apply kernels on this operator (reps calls each, after
  * a warm-up, with HIP events) and keeps the fastest.  R = 0 tunes the
  * single-vector kernel (the QSI_APPLY_* variants that apply: hash variants
- * when the basis has a hash index, CACHED when the connectivity is cached)
+ * when the basis has a hash index, CACHED when the connectivity is cached,
+ * AUTO where it has a kernel of its own, on small bases without the cache)
  * and sets the operator's variant; R in [1, 64] tunes the block apply for R
  * columns (kernel depth and grid size) used by qsi_op_apply_block,
  * qsi_lanczos_block and qsi_engine_create.  d_x, d_y: scratch of D (R = 0)

@@ -1320,6 +1320,9 @@ extern "C" int qsi_op_autotune(qsi_op_t op, int R, int reps, double* d_x, double
   if (R == 0) {
     std::vector<int> cand = {QSI_APPLY_LANE, QSI_APPLY_LANE2, QSI_APPLY_LANE4, QSI_APPLY_LANE8,
                              QSI_APPLY_WINDOW};
+    // a kernel that only AUTO takes (2970 states: 7.3 us where the best of the
+    // others takes 12.4)
+    if (auto_takes_rows(op)) cand.push_back(QSI_APPLY_AUTO);
     if (op->basis->d_hash) {
       cand.push_back(QSI_APPLY_HASH);
       cand.push_back(QSI_APPLY_HASH4);

@@ -2431,6 +2431,10 @@ static void launch_cached_t(const qsi_op_s* op, dim3 grid, dim3 block, const Bas
                      op->d_cm, op->d_diag, op->n_diag, x, y, y_in, yscale, yscale_dev, partials, xs_dev, ys_dev);
 }
 
+bool auto_takes_rows(const qsi_op_s* op) {
+  return op->basis->dim <= kRowMaxDim && op->conn_nnz < 0;
+}
+
 template <int NW, bool HAS_Z, bool DOT>
 static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
                            const double* y_in, double yscale,
@@ -2467,7 +2471,7 @@ static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
   if (variant == QSI_APPLY_AUTO) {
     const int64_t dim = op->basis->dim;
     if constexpr (!DOT) {
-      if (dim <= kRowMaxDim && op->conn_nnz < 0) {
+      if (auto_takes_rows(op)) {
         const int64_t rb = kApplyBlock / kWave;
         hipLaunchKernelGGL((k_apply_row<NW, HAS_Z>), dim3(static_cast<uint32_t>((dim + rb - 1) / rb)),
                            block, 0, s, v, op->d_off, op->n_off, op->d_diag, op->n_diag, x, y, y_in,

@@ -208,6 +208,8 @@ int launch_apply_scaled(const qsi_op_s* op, const double* x, double* y,
                         const double* xs_dev, const double* ys_dev, double* dot_partials,
                         double* dot_out, hipStream_t s);
 int64_t apply_num_blocks(const qsi_op_s* op);
+// AUTO takes the wavefront-per-row kernel, which no other variant names
+bool auto_takes_rows(const qsi_op_s* op);
 
 // streaming vector kernels; partial buffers need max_vec_partials() doubles
 // (gs_partials() for launch_gs_step)

@@ -305,8 +305,9 @@ class GpuOp:
         """Time the apply kernels and keep the fastest (qsi_op_autotune):
         R = 0 the single-vector variant, R >= 1 the block apply for R
         columns.  x, y: optional CUDA float64 scratch (D or D x R).  Returns
-        (choice, ms per apply); the choice is a variant name for R = 0 and a
-        block configuration number otherwise."""
+        (choice, ms per apply); the choice is a variant name for R = 0 ('auto'
+        on small bases, where it has a kernel of its own) and a block
+        configuration number otherwise."""
         best = C.c_int(-1)
         ms = C.c_double(0.0)
         check(_lib.load().qsi_op_autotune(self._h, int(R), int(reps),
@@ -314,7 +315,7 @@ class GpuOp:
                                           _ptr(y) if y is not None else None,
                                           C.byref(best), C.byref(ms)), "qsi_op_autotune")
         if R == 0:
-            names = {v: k for k, v in _lib.VARIANTS.items() if k != "auto"}
+            names = {v: k for k, v in _lib.VARIANTS.items()}
             return names.get(best.value, best.value), ms.value
         return best.value, ms.value
 

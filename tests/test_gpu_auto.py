@@ -57,3 +57,16 @@ def test_one_pair_sector(cuda):
     basis = q.enumerate_basis_device(jd, 1)
     auto, lane = _times(cuda, _ops(basis, H, ("auto", "lane4")))
     assert auto <= 0.9 * lane, (auto, lane)
+
+
+@pytest.mark.parametrize("repeats", [(2, 2, 2), (1, 3, 3)])
+def test_autotuned_small(cuda, repeats):
+    """Tuning an operator on a small basis, where the automatic choice has a kernel
+    of its own, does not leave it slower than before."""
+    jd = latgen.Supercell(repeats).to_dict()
+    H = q.build_hamiltonian_g(jd, [-0.9, -0.5, -0.3, -0.7])
+    basis = q.enumerate_basis_device(jd, 0)
+    tuned, auto = _ops(basis, H, ("auto", "auto"))
+    assert tuned.autotune(0, reps=3)[0] in q._lib.VARIANTS
+    a, b = _times(cuda, (tuned, auto), n=100)
+    assert a <= 1.2 * b, (a, b)
