@@ -2807,6 +2807,20 @@ int launch_gs_step(const double* V, int64_t ldv, int m, double* w, int64_t n, do
   return QSI_OK;
 }
 
+int launch_multidot(const double* V, int64_t ldv, int m, const double* w, int64_t n,
+                    double* partials, double* out, hipStream_t s) {
+  for (int j0 = 0; j0 < m; j0 += kMaxCols) {
+    const int jn = std::min(kMaxCols, m - j0);
+    const int nb = std::max(1, std::min(proj_blocks(n), kPlainPartials / jn));
+    hipLaunchKernelGGL(k_gs_dots<kVecBlock>, dim3(nb), dim3(kVecBlock), 0, s, V + j0 * ldv, ldv,
+                       jn, w, n, partials);
+    QSI_CHECK_LAUNCH();
+    hipLaunchKernelGGL(k_finalize_cols, dim3(jn), dim3(256), 0, s, partials, nb, out + j0);
+    QSI_CHECK_LAUNCH();
+  }
+  return QSI_OK;
+}
+
 int launch_ritz(const RitzArgs& a, int n_jobs, hipStream_t s) {
   if (n_jobs < 1 || n_jobs > kMaxCols || a.m < 1 || a.m > kRitzMax) {
     set_error("launch_ritz: size out of range");
@@ -2872,9 +2886,12 @@ int64_t gram_pairs(int pa, int pb, bool same) {
   const int64_t na = (pa + kGramCols - 1) / kGramCols, nb = (pb + kGramCols - 1) / kGramCols;
   return same ? na * (na + 1) / 2 : na * nb;
 }
-// Rows of a slab: 1024 workgroups over all pairs, at least 256 rows each.
+// Rows of a slab: 1024 workgroups over all pairs, at least 256 rows each; 352 on
+// smaller bases, where allocating more partial sums than 11 MB takes longer than
+// it gives (24 long operators on 3 vectors of 48 spins: 2.03 -> 1.69 ms).
 int64_t gram_slab(int pa, int pb, bool same, int64_t n) {
-  const int64_t want = std::max<int64_t>(1, 1024 / gram_pairs(pa, pb, same));
+  const int64_t groups = n > 1 << 20 ? 1024 : 352;
+  const int64_t want = std::max<int64_t>(1, groups / gram_pairs(pa, pb, same));
   return std::max<int64_t>(256, ((n + want - 1) / want + 63) / 64 * 64);
 }
 }  // namespace
@@ -2902,8 +2919,16 @@ int launch_gram(const double* A, int64_t lda, int pa, const double* B, int64_t l
   return QSI_OK;
 }
 
-bool observe_fits(int P, int n_vec, bool gram) {
-  return P <= kObsCols && (gram || n_vec <= kObsVecs);
+bool observe_fits(const qsi_basis_s* basis, int P, int n_vec, bool gram) {
+  // From three columns on.  Its wavefronts wait for one lookup after the other,
+  // and with fewer operators than wavefronts most of them wait for the rest:
+  // expectations of one ring, this pass / an apply and a multi-dot: 48 spins 71 / 46
+  // us, 64 spins 217 / 101, 72 spins 1598 / 510; four rings on 48 spins 72 / 91.  On
+  // large bases of two-word states the lookups take longer: 72 spins, 16 columns
+  // 3.3 / 2.9 ms, 32 columns 4.3 / 6.5; correlations of 8 columns 2.77 / 2.72, of 16
+  // 3.5 / 7.4.
+  const int few = basis->nw == 2 && basis->dim >= int64_t{1} << 22 ? (gram ? 8 : 16) : 2;
+  return P > few && P <= kObsCols && (gram || n_vec <= kObsVecs);
 }
 
 int observe_blocks(int64_t n) {

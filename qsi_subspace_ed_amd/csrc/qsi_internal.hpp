@@ -234,6 +234,9 @@ int launch_axpy_norm(const double* alpha_dev, const double* v, double* u,
 // are not symmetric (their results at the restart limit depend on every rounding).
 int launch_gs_step(const double* V, int64_t ldv, int m, double* w, int64_t n, double* partials,
                    double* hcol, double* beta, bool plain, hipStream_t s);
+// out[j] = V[:, j] . w for j < m; partials: gs_partials(true) doubles
+int launch_multidot(const double* V, int64_t ldv, int m, const double* w, int64_t n,
+                    double* partials, double* out, hipStream_t s);
 
 // Rayleigh-Ritz of n_jobs thick-restart Lanczos matrices of order m <= kRitzMax,
 // one workgroup each.  Workgroup b takes job[b], whose kept[b] first vectors
@@ -302,7 +305,7 @@ struct ObserveArgs {
   int off_begin[5], diag_begin[5], col_begin[5];
   int P, n_vec, same, tiles;
 };
-bool observe_fits(int P, int n_vec, bool gram);
+bool observe_fits(const qsi_basis_s* basis, int P, int n_vec, bool gram);
 int observe_blocks(int64_t n);
 int observe_tiles(int P, bool gram);
 // out[b * P + a] as launch_gram; partials: observe_blocks() * observe_tiles() * 256

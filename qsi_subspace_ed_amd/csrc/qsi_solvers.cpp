@@ -656,6 +656,9 @@ namespace {
 // its own costs 4 us and a launch each.  Longer ones keep the apply kernels,
 // which have several lookups in flight per row.
 constexpr int kEachTerms = 16;
+// Up to this many columns the short operators have an apply of their own, too
+// (observe_fits says why).
+constexpr int kFewCols = 16;
 
 // Y[:, l*n_vec + i] = O_l psi_i for every operator and vector (Y column-major
 // with leading dimension ldy), then out[b*P + a] = Y[:, a] . W[:, b] for the
@@ -678,7 +681,7 @@ int observe(const qsi_op_t* ops, int n_ops, const double* d_psi, int64_t ld, int
   QSI_CHECK_HIP(bout.alloc(static_cast<size_t>(P) * n_w * sizeof(double)));
   bool small = true;
   for (int l = 0; l < n_ops; ++l) small = small && ops[l]->n_off <= kEachTerms;
-  if (small && observe_fits(P, n_vec, gram)) {
+  if (small && observe_fits(basis, P, n_vec, gram)) {
     // four lists of operators, dealt round robin, in one upload
     std::vector<OffTerm> off;
     std::vector<EachOp> diag;
@@ -726,9 +729,17 @@ int observe(const qsi_op_t* ops, int n_ops, const double* d_psi, int64_t ld, int
     return QSI_OK;
   }
   QSI_CHECK_HIP(bY.alloc(static_cast<size_t>(ldy) * P * sizeof(double)));
-  QSI_CHECK_HIP(bpart.alloc(gram_partials(P, n_w, gram, D) * sizeof(double)));
+  // few columns of W: a multi-dot each, with 1 MB of partials where the 64 x 64
+  // products leave up to 33 (one operator of 96 terms on 1, 2 vectors: 48 spins 62,
+  // 108 us for 117, 153; 64 spins 359, 681 for 442, 968; 24 operators on one vector of
+  // 48 spins 647 for 695, and their correlations 1051 for 694)
+  const bool few = P <= kFewCols && small;
+  const bool dots = few || n_w * ((P + 63) / 64) <= 3;
+  QSI_CHECK_HIP(bpart.alloc((dots ? static_cast<size_t>(gs_partials(true))
+                                  : gram_partials(P, n_w, gram, D)) *
+                            sizeof(double)));
   double* Y = bY.d();
-  if (small) {
+  if (small && !few) {
     std::vector<EachOp> each(n_ops);
     for (int l = 0; l < n_ops; ++l)
       each[l] = {ops[l]->d_off, ops[l]->d_diag, ops[l]->n_off, ops[l]->n_diag, 0};
@@ -747,8 +758,14 @@ int observe(const qsi_op_t* ops, int n_ops, const double* d_psi, int64_t ld, int
                              Y + static_cast<int64_t>(l * n_vec + i) * ldy, nullptr, 0.0, nullptr,
                              nullptr, s));
   }
-  QSI_TRY(launch_gram(Y, ldy, P, gram ? Y : d_psi, gram ? ldy : ld, n_w, D, bpart.d(), bout.d(),
-                      s));
+  if (dots) {
+    for (int b = 0; b < n_w; ++b)
+      QSI_TRY(launch_multidot(Y, ldy, P, gram ? Y + b * ldy : d_psi + b * ld, D, bpart.d(),
+                              bout.d() + static_cast<int64_t>(b) * P, s));
+  } else {
+    QSI_TRY(launch_gram(Y, ldy, P, gram ? Y : d_psi, gram ? ldy : ld, n_w, D, bpart.d(), bout.d(),
+                        s));
+  }
   out.resize(static_cast<size_t>(P) * n_w);
   QSI_CHECK_HIP(hipMemcpy(out.data(), bout.d(), out.size() * sizeof(double), hipMemcpyDeviceToHost));
   *P_out = P;
