@@ -165,12 +165,14 @@ int qsi_op_n_diag(qsi_op_t op);
  * bucket on the basis's low keys (qsi_basis_build_lowkeys); setting one
  * requires them, and without them later the apply falls back to LANE* of the
  * same depth.  AUTO = CACHED when the connectivity is cached; else, up to 2^14
- * states and without a dot product, a wavefront per row; else WINDOW on
+ * states (2^12 for fewer than 16 terms) and without a dot product, a wavefront
+ * per row; else WINDOW on
  * bases of at least 2^21 states where at most one in 32 sampled pairs of 128 rows
  * and a term leads out of the basis (one in 64, and one-word states, after
- * qsi_op_verify_lowkeys found mode 1) and whose terms flip no spin outside their
- * projectors (after mode 2: one-word states, or at least 2^28
- * of two words, and a term list that holds every flip's reverse); else, when the
+ * qsi_op_verify_lowkeys found mode 1), for at least 32 terms, which flip no spin
+ * outside their projectors (after mode 2: any number of them, one-word states, or
+ * at least 2^28 of two words, and a term list that holds every flip's reverse);
+ * else, when the
  * basis has low keys, LOW8 after mode 2 and LOW4 otherwise, else LANE4.
  * All give bit-identical y. */
 enum {

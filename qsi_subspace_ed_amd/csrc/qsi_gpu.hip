@@ -1057,11 +1057,15 @@ template <int NW, bool CHECK>
 constexpr int kWinItems = NW == 1 ? 4 : 2;
 template <int NW, bool CHECK>
 constexpr int kWinWaves = NW == 1 ? 7 : 5;
-// AUTO takes the window kernel from this many states on; against LOW8 on two-word
-// states only from the second
-constexpr int64_t kRowMaxDim = int64_t{1} << 14;
+// AUTO takes the window kernel from this many states and (against kernels that
+// compare) terms on; against LOW8 on two-word states only from the second
 constexpr int64_t kWinMinDim = int64_t{1} << 21;
 constexpr int64_t kWinMinDimLow2 = int64_t{1} << 28;
+constexpr int kWinMinTerms = 32;
+// and the row kernel up to this many states, for few terms up to the second number
+constexpr int64_t kRowMaxDim = int64_t{1} << 14;
+constexpr int64_t kRowMaxDimFew = int64_t{1} << 12;
+constexpr int kRowMinTerms = 16;
 constexpr int kWinRows = 128;  // rows of a wavefront, and ranks of a window
 constexpr int kWinMax = 8;     // windows of one term (a wider range: per-row lookups)
 // Windows of a term whose first and last target have ranks la and lz in a basis of
@@ -2432,7 +2436,8 @@ static void launch_cached_t(const qsi_op_s* op, dim3 grid, dim3 block, const Bas
 }
 
 bool auto_takes_rows(const qsi_op_s* op) {
-  return op->basis->dim <= kRowMaxDim && op->conn_nnz < 0;
+  return op->conn_nnz < 0 &&
+         op->basis->dim <= (op->n_off < kRowMinTerms ? kRowMaxDimFew : kRowMaxDim);
 }
 
 template <int NW, bool HAS_Z, bool DOT>
@@ -2450,7 +2455,10 @@ static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
   // thousand states, a wavefront per row (call to call, a call's host side being
   // 7.8 us, row / LANE4 / LOW8 in us: 2970 states 7.8 / 12.4 / 11.9, 13122 states
   // 9.1 / 14.5 / 14.7, 87546 states 54 / 20 / 19), but not for the dot-product
-  // instances, whose partials are sums over 256 rows.  Else, without low keys whose
+  // instances, whose partials are sums over 256 rows, nor on more than 4096 states
+  // for few terms, which a lane does in a round or two (13122 states, 1 / 4 / 8 / 16
+  // / 32 terms, row / LANE4: 4.5 / 3.3, 4.8 / 3.7, 5.1 / 4.2, 5.5 / 5.4, 5.8 / 7.9).
+  // Else, without low keys whose
   // candidates need no compare, the window kernel on bases large enough to fill
   // the chip with its 128-row wavefronts (WINDOW / LANE4 / LOW4 in us: 32 spins
   // 35 / 12 / 13, 293394 states 33 / 25 / 25, 1062882 states 55 / 52 / 53, 64 spins 200 /
@@ -2463,7 +2471,9 @@ static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
   // 30 % 428 / 268 / - / 231; 72 spins, one pair, 1 % 2.92 / 4.20 / 3.57 / 2.82 ms, 2 %
   // 3.27 / 4.21 / 3.57 / 2.82, 5 % 3.93 / 4.21 / 3.57 / 2.82; 64 spins, two pairs, 32 %
   // 115 / 91 ms.  So up to 1/32, with key compares (mode 1) up to 1/64 and one-word
-  // states only.  With low keys that need no compare LOW8, except where WINDOW
+  // states only; and from 32 terms on (1 / 8 / 16 / 32 / 64 of them, WINDOW / LANE4 in
+  // us: 64 spins 27 / 19, 39 / 30, 49 / 38, 66 / 68, 111 / 132; 72 spins 134 / 130, 241 /
+  // 231, 310 / 296, 434 / 488, 703 / 943).  With low keys that need no compare LOW8, except where WINDOW
   // without its compare is the faster: one-word states on large bases (WINDOW /
   // LOW8: 293394 states 33 / 21, 64 spins 181 / 190, 60 spins 166 / 191 us) and bases so
   // large that the 31-bit bucket key leaves long bisections (72 spins 1.21 / 1.18,
@@ -2483,6 +2493,7 @@ static void launch_apply_t(const qsi_op_s* op, const double* x, double* y,
     const bool trusted = check == kLowTrusted;
     bool window = dim >= kWinMinDim && op->ordered;
     if (trusted) window = window && op->paired && (NW == 1 || dim >= kWinMinDimLow2);
+    else if (op->n_off < kWinMinTerms) window = false;
     else if (check == kLowCmpKey) window = window && NW == 1 && op->miss_share <= 1.0f / 64;
     else window = window && op->miss_share <= 1.0f / 32;
     variant = op->conn_nnz >= 0        ? QSI_APPLY_CACHED

@@ -26,6 +26,31 @@ def _times(cuda, ops, n=20, rounds=5):
     return best
 
 
+def _graph_times(cuda, ops, n=50, rounds=5):
+    """The same for the applies of a graph of n."""
+    x = cuda.randn(ops[0].rows(), dtype=cuda.float64, device="cuda")
+    y = cuda.empty_like(x)
+    best, graphs = [], []
+    for op in ops:
+        op.evaluate(x, y)
+        cuda.cuda.synchronize()
+        g = cuda.cuda.CUDAGraph()
+        with cuda.cuda.graph(g):
+            for _ in range(n):
+                op.evaluate(x, y)
+        graphs.append(g)
+        best.append(np.inf)
+    for _ in range(rounds + 1):
+        for k, g in enumerate(graphs):
+            a, b = (cuda.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            g.replay()
+            b.record()
+            b.synchronize()
+            best[k] = min(best[k], a.elapsed_time(b) / n * 1e3)
+    return best
+
+
 def _ops(basis, H, variants):
     out = []
     for v in variants:
@@ -70,3 +95,22 @@ def test_autotuned_small(cuda, repeats):
     assert tuned.autotune(0, reps=3)[0] in q._lib.VARIANTS
     a, b = _times(cuda, (tuned, auto), n=100)
     assert a <= 1.2 * b, (a, b)
+
+
+def _first_terms(H, n):
+    out = q.SymbolicOpSum()
+    for c, o, _ in H.off_diag_terms[:n]:
+        out.add_term(c, o)
+    return out
+
+
+@pytest.mark.parametrize("repeats", [(1, 3, 3), (2, 2, 4)])
+@pytest.mark.parametrize("n", [1, 4, 8])
+def test_few_terms(cuda, repeats, n):
+    """Operators of few terms: a row does them in a round or two.  Applies of a
+    captured graph: on their own those of the smaller basis take the host's time."""
+    jd = latgen.Supercell(repeats).to_dict()
+    H = _first_terms(q.build_hamiltonian_g(jd, [-0.9, -0.5, -0.3, -0.7]), n)
+    basis = q.enumerate_basis_device(jd, 0)
+    auto, lane = _graph_times(cuda, _ops(basis, H, ("auto", "lane4")))
+    assert auto <= 1.15 * lane, (auto, lane)
