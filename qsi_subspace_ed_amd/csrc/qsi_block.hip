@@ -482,7 +482,9 @@ __device__ __forceinline__ void load_entries(const BlkSector& S, uint64_t e, uin
 // The class's coefficients come from LDS: one read of CPL columns instead of a
 // choice among eight registers per column and entry (2.76 M rows of 64 spins, 16
 // columns in pairs 0.87 -> 0.68 ms, 64 columns 3.4 -> 2.7 ms; then bound by the
-// gathers' L2 misses, 15.5 GB of X's rows at 5.7 TB/s).
+// gathers' L2 misses, 15.5 GB of X's rows at 5.7 TB/s).  One column per lane keeps
+// the choice, where an LDS read per entry serves one product (64 spins, 3 / 8 / 16
+// columns: 270 / 486 / 920 us, from LDS 309 / 572 / 1008).
 template <int NW, int PIPE, int CPL>
 __global__ __launch_bounds__(kBlkThreads) void k_blk_capply(
     BlkArgs a, const double* __restrict__ X, double* __restrict__ Y,
@@ -503,6 +505,7 @@ __global__ __launch_bounds__(kBlkThreads) void k_blk_capply(
                      partials + (static_cast<int64_t>(flushed) * gridDim.x + blockIdx.x) * R);
   };
   int cur = -1;
+  double cc[kMaxCoefClasses];  // this lane's column (CPL == 1)
   for (int64_t tb0 = static_cast<int64_t>(blockIdx.x) * kBlkWaves; tb0 < a.n_tiles;
        tb0 += n_waves) {
     const int s = __builtin_amdgcn_readfirstlane(find_sector(a, tb0));  // the workgroup's
@@ -514,6 +517,10 @@ __global__ __launch_bounds__(kBlkThreads) void k_blk_capply(
       __syncthreads();  // no wavefront still reads the last sector's
       load_coefs(coef, S, R);
       __syncthreads();
+      if constexpr (CPL == 1) {
+#pragma unroll
+        for (int c = 0; c < kMaxCoefClasses; ++c) cc[c] = c < S.n_cls ? coef[c][q.col] : 0.0;
+      }
     }
     const int64_t t = tb0 + wv;
     const int64_t r_begin = (t - S.tile_begin) * a.tile_rows;
@@ -543,7 +550,15 @@ __global__ __launch_bounds__(kBlkThreads) void k_blk_capply(
 #pragma unroll
         for (int u = 0; u < PIPE; ++u) {
           if (J[u] == kNoRank) continue;
-          const ColVec<CPL> c = load_cols<CPL>(&coef[mt[u] & 0x7F][col]);
+          ColVec<CPL> c;
+          if constexpr (CPL == 1) {
+            c.v[0] = cc[0];
+#pragma unroll
+            for (int z = 1; z < kMaxCoefClasses; ++z)
+              if ((mt[u] & 0x7F) == z) c.v[0] = cc[z];
+          } else {
+            c = load_cols<CPL>(&coef[mt[u] & 0x7F][col]);
+          }
 #pragma unroll
           for (int v = 0; v < CPL; ++v)
             if (fabs(xj[u].v[v]) > kApplyTol)

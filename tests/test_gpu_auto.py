@@ -1,5 +1,6 @@
-"""The automatic choice of the apply kernel against the kernels it chooses from:
-it is not left behind by the fixed choices where it was measured to lose."""
+"""Choices of kernels against the kernels they choose from: the automatic one is
+not left behind by the fixed ones where it was measured to lose, and the default
+block configuration not by the other."""
 import numpy as np
 import pytest
 
@@ -114,3 +115,26 @@ def test_few_terms(cuda, repeats, n):
     basis = q.enumerate_basis_device(jd, 0)
     auto, lane = _graph_times(cuda, _ops(basis, H, ("auto", "lane4")))
     assert auto <= 1.15 * lane, (auto, lane)
+
+
+def test_default_block(cuda):
+    """Eight cached columns, one per lane (the default configuration): at most 1.28
+    times as long as in pairs, of whose gathers it makes twice as many."""
+    jd = latgen.Supercell((2, 2, 4)).to_dict()
+    op = q.GpuOp(q.enumerate_basis_device(jd, 0),
+                 q.build_hamiltonian_g(jd, [-0.9, -0.5, -0.3, -0.7]))
+    op.cache_connectivity()
+    X = cuda.randn(op.rows(), 8, dtype=cuda.float64, device="cuda")
+    Y = cuda.empty_like(X)
+    best = {}
+    for _ in range(5):
+        for cfg in (1, 9):
+            op.set_block_cfg(cfg)
+            a, b = (cuda.cuda.Event(enable_timing=True) for _ in range(2))
+            a.record()
+            for _ in range(10):
+                op.apply_block(X, Y)
+            b.record()
+            b.synchronize()
+            best[cfg] = min(best.get(cfg, np.inf), a.elapsed_time(b))
+    assert best[1] <= 1.28 * best[9], best
