@@ -42,9 +42,15 @@ constexpr int kSrvThreads = 256;
 // up to a multiple of 64, at least 256, so a column has at most kSumBlocks
 // workgroups and the next kernel's workgroups can add up their partials
 // themselves (kernels of their own for the sums, the norms, the flags and the
-// results were six of a step's twelve launches, 4 us each)
+// results were six of a step's twelve launches, 4 us each).  Above kSumBlocks
+// times 2048 rows they are too few to fill the chip for one or two columns of many
+// vectors: there 2048 rows, at most kSrvBlocksMax workgroups, and a launch for
+// each pass's sums (2.76 M rows, four cycles of 32 vectors: one column 85.6 -> 46.9
+// ms, two 112.6 -> 79.2, four 159.9 -> 142.6; of 15 vectors 13.8 -> 13.3, 16 columns
+// 153 -> 138)
 constexpr int kSrvRowsMin = 256;
-constexpr int kSrvRowsMax = 2048;  // plain steps
+constexpr int kSrvRowsMax = 2048;
+constexpr int kSrvBlocksMax = 2048;
 constexpr int kHMax = 64;
 // partials slot holding |u|^2 (projections use slots 0..ncv-1 <= 62)
 constexpr int kNormSlot = kHMax - 1;
@@ -148,11 +154,26 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_mdot(
   srv_block_dots<MMAX>(acc, m, c, gridDim.x, partials);
 }
 
+// out[c * kHMax + i] = sum of column c's nblk partials of slot i, in a fixed order,
+// for the slots up to j_c and kNormSlot.  Grid (kHMax, n_act).
+__global__ __launch_bounds__(kSrvThreads) void k_srv_sums(const double* __restrict__ partials,
+                                                          int nblk, const int* __restrict__ colj,
+                                                          const int* __restrict__ slotcol,
+                                                          double* __restrict__ out) {
+  const int c = slotcol[blockIdx.y], i = blockIdx.x;
+  if (i > colj[c] && i != kNormSlot) return;
+  const double* p = partials + (static_cast<int64_t>(c) * kHMax + i) * nblk;
+  double v = 0.0;
+  for (int b = threadIdx.x; b < nblk; b += kSrvThreads) v += p[b];
+  v = block_sum<kSrvThreads>(v);
+  if (threadIdx.x == 0) out[c * kHMax + i] = v;
+}
+
 // hs[i] = vs_i h_i for i < m (0 up to MMAX).  FUSED: h_i = vs_i times pass 1's sum
-// of partials i, and the column's first workgroup writes h to hacc; else part1
-// is h (R x kHMax).  Ends with a barrier.
+// of partials i (nb of them), and the column's first workgroup writes h to hacc;
+// else part1 is h (R x kHMax).  Ends with a barrier.
 template <int MMAX, bool FUSED>
-__device__ __forceinline__ void srv_first_sums(const double* __restrict__ part1, int c, int m,
+__device__ __forceinline__ void srv_first_sums(const double* __restrict__ part1, int nb, int c, int m,
                                                const double* __restrict__ vs,
                                                double* __restrict__ hacc, double (&hs)[MMAX]) {
   const int t = threadIdx.x;
@@ -163,7 +184,7 @@ __device__ __forceinline__ void srv_first_sums(const double* __restrict__ part1,
   }
   if (t < MMAX) hs[t] = 0.0;
   __syncthreads();
-  sum_partials<kSrvThreads>(part1 + static_cast<int64_t>(c) * kHMax * gridDim.x, gridDim.x, m, hs);
+  sum_partials<kSrvThreads>(part1 + static_cast<int64_t>(c) * kHMax * nb, nb, m, hs);
   if (t < m) {
     const double sc = vs[c * kHMax + t], v = hs[t] * sc;
     if (blockIdx.x == 0) hacc[c * kHMax + t] = v;
@@ -179,7 +200,7 @@ __device__ __forceinline__ void srv_first_sums(const double* __restrict__ part1,
 // (V h)[row] meet in LDS, and each wave reuses its V entries for the dots.
 template <int MMAX, bool FUSED>
 __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot(
-    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ part1,
+    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ part1, int nb1,
     double* __restrict__ hacc, const double* __restrict__ vs, const int* __restrict__ colj,
     const int* __restrict__ slotcol, int64_t D, int rpb, const double* __restrict__ Wc,
     double* __restrict__ partials) {
@@ -194,7 +215,7 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot(
   __shared__ double red[MMAX];
   __shared__ double nsh;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  srv_first_sums<MMAX, FUSED>(part1, c, m, vs, hacc, hs);
+  srv_first_sums<MMAX, FUSED>(part1, nb1, c, m, vs, hacc, hs);
   const double* V = Vb + static_cast<int64_t>(c) * ncv1 * ld;
   double* out = Vb + (static_cast<int64_t>(c) * ncv1 + m) * ld;
   const double* w = Wc + static_cast<int64_t>(sl) * ld;
@@ -254,7 +275,7 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot(
 // (no workgroup barrier per row tile).
 template <int MMAX, bool FUSED>
 __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot_rows(
-    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ part1,
+    double* __restrict__ Vb, int64_t ld, int ncv1, const double* __restrict__ part1, int nb1,
     double* __restrict__ hacc, const double* __restrict__ vs, const int* __restrict__ colj,
     const int* __restrict__ slotcol, int64_t D, int rpb, const double* __restrict__ Wc,
     double* __restrict__ partials) {
@@ -262,7 +283,7 @@ __global__ __launch_bounds__(kSrvThreads) void k_srv_gemv_mdot_rows(
   const int c = slotcol[sl];
   const int m = colj[c] + 1;
   __shared__ double hs[MMAX];
-  srv_first_sums<MMAX, FUSED>(part1, c, m, vs, hacc, hs);
+  srv_first_sums<MMAX, FUSED>(part1, nb1, c, m, vs, hacc, hs);
   // h in scalar registers; entries i >= m are zero, so the loops below run
   // unpredicated
   double hr[MMAX];
@@ -597,6 +618,7 @@ struct qsi_engine_s {
   // slot coefficients, projections, norms and reduction partials
   double *Vb = nullptr, *X = nullptr, *Wc = nullptr, *coeffs = nullptr;
   double *hacc = nullptr, *vs = nullptr, *part = nullptr;
+  double* sums = nullptr;  // pass 1's and pass 2's (R x kHMax each), on large bases
   double *h = nullptr, *beta = nullptr;  // plain steps
   int* flag_d = nullptr;
   bool plain = false;  // the operator is not symmetric: unfused steps, Ritz on the host
@@ -794,21 +816,36 @@ template <int MMAX>
 void launch_reorth(qsi_engine_s* E, int nact, const qsi_engine_s::StepBuf& B, hipStream_t s) {
   const dim3 gcol(E->nblk, nact);
   double* part2 = E->part + static_cast<size_t>(E->R) * E->nblk * kHMax;
+  // more partials than the next kernel's workgroups add up themselves: one launch
+  // sums them, and that kernel finds a single one
+  const double *sum1 = E->part, *sum2 = part2;
+  int nb = E->nblk;
+  auto reduce = [&](const double* part, double* sums) {
+    hipLaunchKernelGGL(k_srv_sums, dim3(kHMax, nact), dim3(kSrvThreads), 0, s, part, E->nblk,
+                       E->colj_d, E->slot_d, sums);
+  };
   hipLaunchKernelGGL(k_srv_mdot<MMAX>, gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld, E->ncv1,
                      E->Wc, E->colj_d, E->slot_d, E->D, E->rpb, E->part);
+  if (E->sums) {
+    sum1 = E->sums;
+    sum2 = E->sums + static_cast<size_t>(E->R) * kHMax;
+    nb = 1;
+    reduce(E->part, E->sums);
+  }
   if constexpr (MMAX <= 24)
     hipLaunchKernelGGL((k_srv_gemv_mdot_rows<MMAX, true>), gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld,
-                       E->ncv1, E->part, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb, E->Wc,
+                       E->ncv1, sum1, nb, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb, E->Wc,
                        part2);
   else
     hipLaunchKernelGGL((k_srv_gemv_mdot<MMAX, true>), gcol, dim3(kSrvThreads), 0, s, E->Vb, E->ld,
-                       E->ncv1, E->part, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb, E->Wc,
+                       E->ncv1, sum1, nb, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb, E->Wc,
                        part2);
+  if (E->sums) reduce(part2, E->sums + static_cast<size_t>(E->R) * kHMax);
   // enough workgroups for the last pass over the flagged columns, and few
   // where there is none to make
   const int nt = std::min(E->nblk, std::max(32, 512 / nact));
   hipLaunchKernelGGL(k_srv_tail<MMAX>, dim3(nt, nact), dim3(kSrvThreads), 0, s, E->Vb, E->ld,
-                     E->ncv1, part2, E->nblk, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->Tdev,
+                     E->ncv1, sum2, nb, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->Tdev,
                      B.hh_dev, B.bb_dev);
 }
 
@@ -824,11 +861,11 @@ void launch_reorth_plain(qsi_engine_s* E, int nact, const qsi_engine_s::StepBuf&
                      E->colj_d, E->vs, E->h, E->hacc, 0);
   if constexpr (MMAX <= 24)
     hipLaunchKernelGGL((k_srv_gemv_mdot_rows<MMAX, false>), gcol, dim3(kSrvThreads), 0, s, E->Vb,
-                       E->ld, E->ncv1, E->h, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb,
+                       E->ld, E->ncv1, E->h, 1, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb,
                        E->Wc, E->part);
   else
     hipLaunchKernelGGL((k_srv_gemv_mdot<MMAX, false>), gcol, dim3(kSrvThreads), 0, s, E->Vb,
-                       E->ld, E->ncv1, E->h, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb,
+                       E->ld, E->ncv1, E->h, 1, E->hacc, E->vs, E->colj_d, E->slot_d, E->D, E->rpb,
                        E->Wc, E->part);
   hipLaunchKernelGGL(k_srv_fin, dim3(R, kHMax), dim3(kSrvThreads), 0, s, E->part, E->nblk,
                      E->colj_d, E->vs, E->h, E->hacc, 1);
@@ -875,10 +912,13 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
   E->tol = tol;
   E->max_restarts = max_restarts;
   E->ld = (E->D + 63) / 64 * 64;
+  bool large = false;  // sums in kernels of their own
   {
-    int64_t rpb = ((E->D + kSumBlocks - 1) / kSumBlocks + 63) / 64 * 64;
-    rpb = std::max<int64_t>(rpb, kSrvRowsMin);
     E->plain = !op->symmetric;
+    large = !E->plain && E->D > int64_t{kSumBlocks} * kSrvRowsMax;
+    const int64_t blocks = large ? kSrvBlocksMax : kSumBlocks;
+    int64_t rpb = ((E->D + blocks - 1) / blocks + 63) / 64 * 64;
+    rpb = std::max<int64_t>(rpb, large ? kSrvRowsMax : kSrvRowsMin);
     if (E->plain) rpb = std::min<int64_t>(rpb, kSrvRowsMax);
     E->rpb = static_cast<int>(rpb);
     E->nblk = static_cast<int>((E->D + rpb - 1) / rpb);
@@ -925,6 +965,7 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
     E->slot_d = E->colj_d + R;
   }
   if (e == hipSuccess) e = E->alloc(&E->hacc, R * kHMax);
+  if (e == hipSuccess && large) e = E->alloc(&E->sums, 2 * R * kHMax);
   if (e == hipSuccess && E->plain) e = E->alloc(&E->h, R * kHMax);
   if (e == hipSuccess && E->plain) e = E->alloc(&E->beta, R);
   if (e == hipSuccess && E->plain) e = E->alloc(&E->flag_d, R);
@@ -932,7 +973,7 @@ int qsi_engine_create(qsi_op_t op, int max_cols, int nev, int ncv, double tol,
   if (e == hipSuccess) e = E->alloc(&E->theta, R * kHMax);
   if (e == hipSuccess) e = E->alloc(&E->vs, R * kHMax);
   if (e == hipSuccess)
-    e = E->alloc(&E->part, std::max<size_t>(2 * R * E->nblk * kHMax,
+    e = E->alloc(&E->part, std::max<size_t>((E->plain ? 1 : 2) * R * E->nblk * kHMax,
                                             static_cast<size_t>(max_vec_partials()) + 8));
   if (e == hipSuccess) e = E->alloc(&E->Ydev, R * kHMax * kHMax);
   if (e == hipSuccess)
