@@ -410,7 +410,8 @@ int qsi_ftlm_sample(qsi_op_t H, const qsi_op_t *ops, int n_ops, const double *d_
 int qsi_tridiag_eig(const double *d, const double *e, int n, double *evals,
                     double *first_row);
 
-/* Gauss quadratures of R tridiagonals at once, on up to 16 host threads: row r
+/* Gauss quadratures of R tridiagonals at once, on up to 16 host threads (and the cores of
+ * the process): row r
  * is d[r * ldd + 0 .. n[r]) and e[r * lde + 0 .. n[r] - 1); nodes[r * ldd + k]
  * receives its ascending eigenvalues and weights[r * ldd + k] the squared first
  * components, as qsi_tridiag_eig gives them.  1 <= n[r] <= ldd, n[r] - 1 <= lde.

@@ -20,6 +20,7 @@
 // No pass rewrites a block to normalise it.  The four launches of a step are
 // captured once per rotation phase as a HIP graph and replayed.
 #include <hip/hip_runtime.h>
+#include <sched.h>
 
 #include <algorithm>
 #include <atomic>
@@ -1452,8 +1453,12 @@ extern "C" int qsi_tridiag_quadrature(const double* d, int64_t ldd, const double
     }
   };
   // one sample costs about 50 ns per n^2, starting a thread about 20 us: 0.4 ms
-  // of work per thread
-  const int cores = static_cast<int>(std::max(1u, std::thread::hardware_concurrency()));
+  // of work per thread; no more of them than the process may run on (ranks that
+  // share a node are confined to their cores)
+  cpu_set_t set;
+  const int cores = sched_getaffinity(0, sizeof(set), &set) == 0
+                        ? std::max(1, CPU_COUNT(&set))
+                        : static_cast<int>(std::max(1u, std::thread::hardware_concurrency()));
   const int nt = std::min({16, cores, R, 1 + static_cast<int>(std::min(work / 8192.0, 64.0))});
   std::vector<std::thread> pool;
   try {
