@@ -218,6 +218,13 @@ void k_blk_apply(
        tb0 += n_waves) {
     const int s = __builtin_amdgcn_readfirstlane(find_sector(a, tb0));  // the workgroup's
     const BlkSector& S = a.sec[s];
+    // the rows' states are on their way while the sector's terms are staged
+    const int64_t t = tb0 + wv;
+    const int64_t r_begin = (t - S.tile_begin) * a.tile_rows;
+    const int n_rows = static_cast<int>(min<int64_t>(a.tile_rows, S.b.dim - r_begin));
+    const bool live = t < a.n_tiles && n_rows > 0;  // not a padding tile
+    const bool row_ok = live && lane < n_rows;
+    const State<NW> st = load_state_cached<NW>(S.b.states, row_ok ? r_begin + lane : 0);
     if (s != cur) {
       flush_to(s, cur);
       cur = s;
@@ -231,12 +238,7 @@ void k_blk_apply(
       }
       __syncthreads();
     }
-    const int64_t t = tb0 + wv;
-    const int64_t r_begin = (t - S.tile_begin) * a.tile_rows;
-    const int n_rows = static_cast<int>(min<int64_t>(a.tile_rows, S.b.dim - r_begin));
-    if (t >= a.n_tiles || n_rows <= 0) continue;  // padding tiles
-    const bool row_ok = lane < n_rows;
-    const State<NW> st = load_state_cached<NW>(S.b.states, r_begin + (row_ok ? lane : 0));
+    if (!live) continue;
     const uint32_t ks = bucket_key<NW>(S.b, st);
     const int n_sc = max(1, (S.n_off + kBlkSuper - 1) / kBlkSuper);
     for (int sc = 0; sc < n_sc; ++sc) {
@@ -334,22 +336,29 @@ void k_blk_apply(
                 xj[u] = J[u] != kNoRank
                             ? load_cols<CPL>(X + (S.row_off + static_cast<int64_t>(J[u])) * a.ldx + col)
                             : ColVec<CPL>{};
-#pragma unroll
-              for (int u = 0; u < kPipe; ++u) {
-                if (J[u] == kNoRank) continue;
-                ColVec<CPL> c;
-                if (S.n_cls > 0) {
-                  c = load_cols<CPL>(&coef[mt[u] & 255][col]);
-                } else {
-                  const OffTerm& T = S.off[tb + static_cast<int>(mt[u] & 255)];
-#pragma unroll
-                  for (int v = 0; v < CPL; ++v)
-                    c.v[v] = (S.coeffs && T.slot >= 0) ? S.coeffs[T.slot * R + col + v] : T.c;
-                }
+              auto add = [&](int u, const ColVec<CPL>& c) {
 #pragma unroll
                 for (int v = 0; v < CPL; ++v)
                   if (fabs(xj[u].v[v]) > kApplyTol)
                     acc.v[v] += (mt[u] & 256 ? -c.v[v] : c.v[v]) * xj[u].v[v];
+              };
+              if (S.n_cls > 0) {
+#pragma unroll
+                for (int u = 0; u < kPipe; ++u)
+                  if (J[u] != kNoRank) add(u, load_cols<CPL>(&coef[mt[u] & 255][col]));
+              } else {
+                // a coefficient per term: all of them before the first is used
+                ColVec<CPL> c[kPipe];
+#pragma unroll
+                for (int u = 0; u < kPipe; ++u) {
+                  const OffTerm& T = S.off[tb + static_cast<int>(mt[u] & 255)];
+#pragma unroll
+                  for (int v = 0; v < CPL; ++v)
+                    c[u].v[v] = (S.coeffs && T.slot >= 0) ? S.coeffs[T.slot * R + col + v] : T.c;
+                }
+#pragma unroll
+                for (int u = 0; u < kPipe; ++u)
+                  if (J[u] != kNoRank) add(u, c[u]);
               }
             }
             if (sc == n_sc - 1) {
