@@ -25,7 +25,6 @@
 #include <cstring>
 #include <mutex>
 #include <new>
-#include <set>
 #include <vector>
 
 #include "qsi_blockk.hpp"
@@ -3550,32 +3549,15 @@ int qsi_op_create(qsi_basis_t b, const qsi_term_t* terms, int n_terms,
   op->n_off = static_cast<int>(op->h_off.size());
   op->n_diag = static_cast<int>(op->h_diag.size());
   op->n_slots = n_slots;
-  // every flipped spin is under the term's projector, so targets keep the
-  // rows' order; and every term's reverse (the same flip from the flipped
-  // projector values) is a term too
-  op->ordered = op->paired = true;
+  // ordered: every flipped spin is under the term's projector, so targets keep the
+  // rows' order.  paired: every term's reverse (the same flip from the flipped
+  // projector values) is a term too.  symmetric: with the same coefficient, slot, Z
+  // string and sign, the terms being the reversed terms.  A Z on a spin that the
+  // projector fixes is a sign; a Z on a flipped one changes the reverse's sign.
   {
-    for (auto& o : op->h_off)
-      op->ordered = op->ordered && ((o.X[0] & ~o.m[0]) | (o.X[1] & ~o.m[1])) == 0;
+    using Key = std::array<uint64_t, 10>;  // X, m, v; Z, coefficient, slot and sign
     auto key = [](const OffTerm& o, bool rev) {
-      std::array<uint64_t, 6> k{};
-      for (int w = 0; w < 2; ++w) {
-        k[w] = o.X[w];
-        k[2 + w] = o.m[w];
-        k[4 + w] = rev ? o.v[w] ^ (o.X[w] & o.m[w]) : o.v[w];
-      }
-      return k;
-    };
-    std::set<std::array<uint64_t, 6>> have;
-    for (auto& o : op->h_off) have.insert(key(o, false));
-    for (auto& o : op->h_off) op->paired = op->paired && have.count(key(o, true)) != 0;
-  }
-  // symmetric: the terms are the reversed terms, with their coefficients, slots,
-  // Z strings and signs.  A Z on a spin that the projector fixes is a sign; a Z on
-  // a flipped one changes the reverse's sign.
-  {
-    auto full = [](const OffTerm& o, bool rev) {
-      std::array<uint64_t, 10> k{};
+      Key k{};
       int odd = o.sgn < 0.0 ? 1 : 0;
       for (int w = 0; w < 2; ++w) {
         const uint64_t z = o.Z[w] & ~o.m[w];
@@ -3590,14 +3572,29 @@ int qsi_op_create(qsi_basis_t b, const qsi_term_t* terms, int n_terms,
       k[9] = static_cast<uint64_t>(static_cast<int64_t>(o.slot)) << 1 | (odd & 1);
       return k;
     };
-    std::vector<std::array<uint64_t, 10>> a, r;
+    std::vector<Key> have;
+    have.reserve(op->h_off.size());
+    for (auto& o : op->h_off) have.push_back(key(o, false));
+    std::sort(have.begin(), have.end());
+    const bool once = std::adjacent_find(have.begin(), have.end()) == have.end();
+    std::vector<Key> rev;
+    op->ordered = op->paired = op->symmetric = true;
     for (auto& o : op->h_off) {
-      a.push_back(full(o, false));
-      r.push_back(full(o, true));
+      op->ordered = op->ordered && ((o.X[0] & ~o.m[0]) | (o.X[1] & ~o.m[1])) == 0;
+      if (!op->paired) continue;
+      Key k = key(o, true), flip{};
+      std::copy(k.begin(), k.begin() + 6, flip.begin());
+      const auto at = std::lower_bound(have.begin(), have.end(), flip);
+      op->paired = at != have.end() && std::equal(flip.begin(), flip.begin() + 6, at->begin());
+      // terms listed once: as many different reverses, so each a term is enough
+      op->symmetric = op->symmetric && op->paired &&
+                      (!once || std::binary_search(at, have.end(), k));
+      if (!once) rev.push_back(k);
     }
-    std::sort(a.begin(), a.end());
-    std::sort(r.begin(), r.end());
-    op->symmetric = a == r;
+    if (!once && op->symmetric) {
+      std::sort(rev.begin(), rev.end());
+      op->symmetric = have == rev;
+    }
   }
   // the terms field by field and as TermRec records, behind the full records
   // and padded to whole chunks of 64
