@@ -1894,8 +1894,8 @@ __global__ __launch_bounds__(T) void k_gs_tail(
 // N (N - 1) / 2 rotations one after the other.  A round is a chain of latencies
 // (LDS, the angle, two barriers).  The vectors of a thick restart are kept for
 // good and never normalised again, so c must round to either side alike: from
-// the hardware's reciprocal root with one Newton step it came out 2^-53 too large
-// for every tangent of 1e-8 to 1e-5, and kept vectors grew by 2e-14 a restart
+// the hardware's reciprocal root with a single Newton step it came out 2^-53 too
+// large for every tangent of 1e-8 to 1e-5, and kept vectors grew by 2e-14 a restart
 // (square norm, order 40; eigenvalues with them), where host rotations leave them
 // within 1e-15 on average.  Blocks
 // on and above the diagonal are computed and mirrored: a matrix that rounding
@@ -1968,16 +1968,23 @@ __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
       if (t < H) {
         int p, q;
         pair(t, p, q);
-        // tt = tan of the smaller angle that annihilates A[p][q]; c = (1 + tt^2)^-1/2
-        // with the rounding errors of 1 + tt^2 and of z r put back
+        // tt = tan of the smaller angle that annihilates A[p][q]
         const double b = 2.0 * A[p * LD + q], d = A[q * LD + q] - A[p * LD + p];
         double2 cs = make_double2(1.0, 0.0);
         if (b != 0.0) {
-          const double tt = (d < 0.0 ? -b : b) / (fabs(d) + hypot(d, b));
+          const double h2 = fma(d, d, b * b);
+          const double h = h2 > 1e-290 && h2 < 1e290 ? sqrt(h2) : hypot(d, b);
+          const double tt = (d < 0.0 ? -b : b) / (fabs(d) + h);
+          // c = (1 + tt^2)^-1/2: the hardware's reciprocal root, a Newton step of
+          // third order, and one with the rounding errors of 1 + tt^2 and of z g put
+          // back
           const double z = fma(tt, tt, 1.0), zl = fma(tt, tt, 1.0 - z);
-          const double r0 = 1.0 / sqrt(z), zr = z * r0, zrl = fma(z, r0, -zr);
-          const double er = fma(-zr, r0, 1.0) - fma(zl * r0, r0, zrl * r0);
-          cs.x = fma(0.5 * r0, er, r0);
+          double g = __builtin_amdgcn_rsq(z);
+          const double e = fma(-z * g, g, 1.0);
+          g = fma(g * e, fma(0.375, e, 0.5), g);
+          const double zg = z * g, zgl = fma(z, g, -zg);
+          const double er = fma(-zg, g, 1.0) - fma(zl * g, g, zgl * g);
+          cs.x = fma(0.5 * g, er, g);
           cs.y = tt * cs.x;
         }
         rot[t] = cs;
