@@ -43,14 +43,24 @@ _VARIANT_KERNEL = {"lane": ("lane", 1), "lane2": ("lane", 2), "lane4": ("lane", 
                    "hash4": ("hash", 4)}
 
 
-def variant_kernel(variant, nw, cached_pipe=None, low_mode=0):
+def window_compares(H, low_mode):
+    """Whether the window kernel compares the states it matches: not after a
+    mode-2 check of an operator that lists every flip's reverse and flips only
+    spins under its projectors."""
+    flips = {(o.X, o.up | o.down, o.up ^ (o.X & (o.up | o.down))) for _, o, _ in H.off_diag_terms}
+    plain = all((X & ~m) == 0 and (X, m, v ^ X) in flips for X, m, v in flips)
+    return not (low_mode == 2 and plain)
+
+
+def variant_kernel(variant, nw, cached_pipe=None, low_mode=0, H=None):
     """Kernel-name prefix of an apply variant (cached: by gather depth; low
-    keys: by how candidates are confirmed, qsi_op_verify_lowkeys' mode)."""
+    keys: by how candidates are confirmed, qsi_op_verify_lowkeys' mode; window:
+    by the operator H, too)."""
     if variant == "cached":
         return f"k_apply_cached<{nw}, false, {cached_pipe},"
     kind, g = _VARIANT_KERNEL[variant]
-    if kind == "win":  # without the compare after a mode-2 check
-        return f"k_apply_win<{nw}, false, false, {'false' if low_mode == 2 else 'true'}>"
+    if kind == "win":
+        return f"k_apply_win<{nw}, false, false, {str(window_compares(H, low_mode)).lower()}>"
     if kind == "low":
         return f"k_apply_low<{nw}, false, false, {g}, {int(low_mode or 0)}>"
     return f"k_apply_{kind}<{nw}, false, false, {g}>"
@@ -571,7 +581,7 @@ def bench_96(args):
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": measured_traffic(PMC_SUMMARY_96, variant_kernel(
                          tuned[0] if tuned else args.variant, 2,
-                         low_mode=lowkeys_mode))},
+                         low_mode=lowkeys_mode, H=H))},
         "apply_kernel_ms": kern_s * 1e3,
         "apply_variant": tuned[0] if tuned else args.variant,
         "autotuned": tuned is not None,
@@ -854,7 +864,7 @@ def bench_64(args):
                      "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
                      "traffic": measured_traffic(PMC_SUMMARY, variant_kernel(
                          tuned[0] if tuned else args.variant, 1,
-                         low_mode=lowkeys_mode))},
+                         low_mode=lowkeys_mode, H=H))},
         "apply_kernel_us": kern_s * 1e6,
         "apply_variant": tuned[0] if tuned else args.variant,
         "low_keys_mode": lowkeys_mode,
