@@ -101,9 +101,11 @@ def quadrature(alpha, beta):
     M = alpha.shape[1]
     d = np.ascontiguousarray(alpha, dtype=np.float64)
     e = np.ascontiguousarray(beta, dtype=np.float64)
+    zero = e[:R, :M] == 0.0
     n = np.full(R, M, dtype=np.intc)
-    for r, j in zip(*np.nonzero(e[:R, :M] == 0.0)):
-        n[r] = min(n[r], j + 1)
+    ended = zero.any(axis=1)
+    if ended.any():
+        n[ended] = zero[ended].argmax(axis=1) + 1
     w = np.empty((R, M))
     f = np.empty((R, M))
     P = C.POINTER(C.c_double)
