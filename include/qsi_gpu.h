@@ -257,8 +257,8 @@ int qsi_op_connectivity_padding(qsi_op_t op);
 int qsi_op_set_cached_pipe(qsi_op_t op, int pipe);
 int qsi_op_get_cached_pipe(qsi_op_t op);
 /* Block-apply configuration (bits 0-1: kernel 0-2, bit 2: half-size grid,
- * bit 3: two columns per lane in the cached kernel, used when X's rows are
- * 16-byte aligned and hold an even number of columns) of
+ * bit 3: two or four columns per lane in the cached kernel; the searching one
+ * always takes two) of
  * qsi_op_apply_block, qsi_lanczos_block (the first sector's) and engines
  * created afterwards.  Chosen by qsi_op_autotune / qsi_block_autotune; set it
  * to pin one.  No counterpart in the reference. */
@@ -410,12 +410,11 @@ int qsi_ftlm_sample(qsi_op_t H, const qsi_op_t *ops, int n_ops, const double *d_
 int qsi_tridiag_eig(const double *d, const double *e, int n, double *evals,
                     double *first_row);
 
-/* Gauss quadratures of R tridiagonals at once, on up to 16 host threads (and the cores of
- * the process): row r
- * is d[r * ldd + 0 .. n[r]) and e[r * lde + 0 .. n[r] - 1); nodes[r * ldd + k]
- * receives its ascending eigenvalues and weights[r * ldd + k] the squared first
- * components, as qsi_tridiag_eig gives them.  1 <= n[r] <= ldd, n[r] - 1 <= lde.
- * Host only. */
+/* Gauss quadratures of R tridiagonals at once, on up to 16 host threads (at most
+ * the cores the process may run on): row r is d[r * ldd + 0 .. n[r]) and
+ * e[r * lde + 0 .. n[r] - 1); nodes[r * ldd + k] receives its ascending
+ * eigenvalues and weights[r * ldd + k] the squared first components, as
+ * qsi_tridiag_eig gives them.  1 <= n[r] <= ldd, n[r] - 1 <= lde.  Host only. */
 int qsi_tridiag_quadrature(const double *d, int64_t ldd, const double *e, int64_t lde,
                            const int *n, int R, double *nodes, double *weights);
 

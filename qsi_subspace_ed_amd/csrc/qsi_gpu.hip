@@ -1037,9 +1037,11 @@ __global__ __launch_bounds__(kApplyBlock) void k_apply_hash(
 // beyond kWinMax windows is done by per-row lookups.  Without CHECK (every
 // connected state is in the basis, every flip's reverse is a term too, every
 // flipped spin under the projector) only the last can be.
-// What bounds it is the L2's misses: states and x of a window are 16 or 24 bytes
-// a rank, a third of them matched, and the rows in flight on an XCD reach more
-// ranks than its L2 holds (72 spins: 8.4 GB per apply at 7 TB/s).  Wider tiles,
+// What bounds it on two-word states is the L2's misses: states and x of a window
+// are 24 bytes a rank, a third of them matched, and the rows in flight on an XCD
+// reach more ranks than its L2 holds (96 spins: 1.98 TB per apply at 7.0 TB/s, 39 %
+// hits; 72 spins 8.4 GB at 7 TB/s).  At 64 spins no unit is at its limit (0.80 GB at
+// 4.4 TB/s, texture units busy 70 and 88 %, VALU issue 69 %).  Wider tiles,
 // fewer or more windows in flight and fewer wavefronts measured no better.
 // Against four lookups in flight per row (LANE4, no low keys): 64 spins 266 ->
 // 200 us, 72 spins 2.09 -> 1.47 ms, 80 spins 17.6 -> 10.1 ms, 96 spins 543 -> 301 ms.
@@ -1900,8 +1902,8 @@ __global__ __launch_bounds__(T) void k_gs_tail(
 // within 1e-15 on average.  Blocks
 // on and above the diagonal are computed and mirrored: a matrix that rounding
 // makes unsymmetric keeps that difference in every rotation and never gets
-// diagonal.  Orders 8, 16, 24, 32: 30, 65, 120, 175 us; one matrix of order 15
-// takes 95 us on a host core, of order 20 to 24 about 300, while the device
+// diagonal.  Orders 8, 16, 24, 32, 48: 33, 80, 150, 218, 662 us; one matrix of order
+// 15 takes 95 us on a host core, of order 20 to 24 about 300, while the device
 // idles.
 constexpr int kRitzThreads = 256;
 __global__ __launch_bounds__(kRitzThreads) void k_ritz(RitzArgs a) {
@@ -2290,8 +2292,8 @@ __global__ __launch_bounds__(256) void k_gram_sum(const double* __restrict__ par
 // holds the workgroup's sums.  With stored columns the products read every
 // column once per output column and 64-column block: 48 operators on two 48-spin
 // vectors took 6.9 ms for expectations and correlations, 96 launches of 4 us and
-// 98 of 28 us each; this way 0.38 ms, 2 x 80 us of it on the device, bound by the
-// latency of the lookups.  Columns [0, P) are the operators', and for
+// 98 of 28 us each; this way 0.37 ms, 2 x 63 us of it in this kernel, bound by the
+// latency of the lookups, and 2 x 12 us in the sums.  Columns [0, P) are the operators', and for
 // expectations (same = 0) n_vec columns of psi follow at the next multiple of 16.
 constexpr int kObsCols = 128;  // most columns of the operators
 constexpr int kObsVecs = 16;   // most columns of psi for expectations

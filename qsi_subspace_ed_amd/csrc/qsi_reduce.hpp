@@ -81,7 +81,8 @@ __global__ __launch_bounds__(BLOCK) void k_sum_chunks(double* partials, int64_t 
 }
 
 // Sums N values per lane over the wavefront by halving: lane l returns the
-// total of value l / (64 / N), in 2 N exchanges fewer than N full butterflies.
+// total of value l / (64 / N), in N - 1 + log2(64 / N) exchanges where N full
+// butterflies take 6 N.  Each total is the butterfly's, bit for bit.
 template <int N, int O = kWave / 2>
 __device__ __forceinline__ double wave_sum_many(double* v, int lane) {
   static_assert(N <= kWave && (N & (N - 1)) == 0);

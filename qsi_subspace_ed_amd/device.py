@@ -210,7 +210,8 @@ class GpuOp:
 
     def set_variant(self, variant):
         """Choose the apply kernel: 'auto' ('cached' when the connectivity is
-        cached, else 'window' on large bases, else with low keys 'low8' after
+        cached, else a wavefront per row on small bases, else 'window' on large
+        ones that few terms lead out of, else with low keys 'low8' after
         verify_lowkeys() gave 2 and 'low4' otherwise, else 'lane4'),
         'cached', 'hash', 'hash4' (hash-index lookups; the basis needs
         hash_index=True), 'lane', 'lane2', 'lane4',
